@@ -122,6 +122,24 @@ def lib() -> ctypes.CDLL:
     return l
 
 
+_host = None
+
+
+def host():
+    """The host module (csrc/host_ops.cpp: allocation, launches and autograd nodes in C++), loaded once; it calls the
+    HIP library, whose absence raises first."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from lorafusion_amd import _host as module
+        except ImportError as e:
+            raise RuntimeError("lorafusion_amd/_host.so is missing or does not load: build it with `python -m lorafusion_amd.csrc.build`. "
+                               "There is no non-HIP fallback.") from e
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         raise RuntimeError(f"{what} failed: {lib().lf_strerror(rc).decode()} (code {rc})")

@@ -1276,27 +1276,27 @@ static DysPlan dys_plan(int M, int N, int R, const LfSegTable& seg) {
 // ---- work split of the ring kernels.  Workgroups (slice x chunk) of w tiles each run on `slots` resident slots; the
 // pass lasts about as long as its busiest slot.  Two upper bounds of that (in tiles): whole rounds of the largest
 // workgroup, and the list-scheduling bound sum / slots + largest; the smaller one is the estimate.
-struct RingSplit { long wgs; long chunks; int max_chunks; double span; };
-static RingSplit ring_split(const int* blocks, int nseg, int g, int T, int nsl, int slots) {
-  RingSplit r{0, 0, 1, 0.0};
-  const int t_max = (T + nsl - 1) / nsl;
-  long total = 0;
-  int big = 0;
+struct GroupStats { long chunks, total; int max_chunks, big; };   // of one chunk length: independent of the slices
+static GroupStats group_stats(const int* blocks, int nseg, int g) {
+  GroupStats r{0, 0, 1, 0};
   for (int s = 0; s < nseg; s++) {
     const int c = (blocks[s] + g - 1) / g;
     if (c <= 0) continue;
     r.chunks += c;
     r.max_chunks = c > r.max_chunks ? c : r.max_chunks;
     const int sz = (blocks[s] + c - 1) / c;
-    big = sz > big ? sz : big;
-    total += blocks[s];
+    r.big = sz > r.big ? sz : r.big;
+    r.total += blocks[s];
   }
-  r.wgs = r.chunks * nsl;
-  const double sum = (double)total * T / slots, largest = (double)big * t_max;
-  const double by_rounds = (double)((r.wgs + slots - 1) / slots) * largest, by_list = sum + largest;
-  r.span = by_rounds < by_list ? by_rounds : by_list;
-  if (r.span < sum) r.span = sum;
   return r;
+}
+static double ring_span(const GroupStats& r, int T, int nsl, int slots) {
+  const int t_max = (T + nsl - 1) / nsl;
+  const long wgs = r.chunks * nsl;
+  const double sum = (double)r.total * T / slots, largest = (double)r.big * t_max;
+  const double by_rounds = (double)((wgs + slots - 1) / slots) * largest, by_list = sum + largest;
+  const double span = by_rounds < by_list ? by_rounds : by_list;
+  return span < sum ? sum : span;
 }
 static void seg_block_counts(int M, const LfSegTable& seg, int* blocks, int& nseg) {
   nseg = seg.table ? seg.n_seg : 1;
@@ -1307,6 +1307,18 @@ static void seg_block_counts(int M, const LfSegTable& seg, int* blocks, int& nse
   }
 }
 static const int kGroups[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 64};
+constexpr int kNGroups = 11;
+// Chunk lengths worth pricing: up to the longest segment (longer ones repeat its figures).
+static int all_group_stats(const int* blocks, int nseg, GroupStats (&st)[kNGroups]) {
+  int longest = 0;
+  for (int s = 0; s < nseg; s++) longest = blocks[s] > longest ? blocks[s] : longest;
+  int n = 0;
+  for (; n < kNGroups; n++) {
+    st[n] = group_stats(blocks, nseg, kGroups[n]);
+    if (kGroups[n] >= longest) return n + 1;
+  }
+  return n;
+}
 
 constexpr int dysr_tpw(int rt) { return rt >= 2 ? 12 : 16; }
 constexpr int dysr_ns(int rt) { return rt >= 4 ? 5 : 3; }
@@ -1324,15 +1336,17 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
   const double tile_bytes = TILE_BYTES + 64.0 * R * 2;
   DysRingPlan best{1, 1, 1};
   if (T < 2) return best;   // fewer than two column tiles: nothing to split (and no division by a zero slice count)
+  GroupStats stats[kNGroups];
+  const int ng = all_group_stats(blocks, nseg, stats);
   double best_cost = 1e300;
   for (int t = dysr_tpw(rt); t >= 2; t--) {   // tiles of the longest slice -> fewest slices that reach it
     const int nsl = (T + t - 1) / t;
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
-    for (int g : kGroups) {
-      const RingSplit sp = ring_split(blocks, nseg, g, T, nsl, slots);
-      const double cost = sp.span * slots * tile_bytes + 0.5 * (double)sp.wgs * g * ROWS * R * 2 +
-                          2.0 * 4.0 * R * ((double)nsl * rows + (double)sp.chunks * N);
-      if (cost < best_cost) { best_cost = cost; best = DysRingPlan{nsl, g, sp.max_chunks}; }
+    for (int k = 0; k < ng; k++) {
+      const GroupStats& st = stats[k];
+      const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
+                          2.0 * 4.0 * R * ((double)nsl * rows + (double)st.chunks * N);
+      if (cost < best_cost) { best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks}; }
     }
   }
   return best;
@@ -1512,14 +1526,17 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg) {
   const double tile_bytes = TILE_BYTES + da_mask_tile_bytes(maskfmt);
   DaPlan best{1, 1, 1};
   if (T < 2) return best;   // as in dysr_plan
+  GroupStats stats[kNGroups];
+  const int ng = all_group_stats(blocks, nseg, stats);
   double best_cost = 1e300;
   for (int t = da_tpw(rt); t >= 2; t--) {   // tiles of the longest slice -> fewest slices that reach it
     const int nsl = (T + t - 1) / t;
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
-    for (int g : kGroups) {
-      const RingSplit sp = ring_split(blocks, nseg, g, T, nsl, slots);
-      const double cost = sp.span * slots * tile_bytes + 0.5 * (double)sp.wgs * g * ROWS * R * 2 + 2.0 * 4.0 * R * K * (double)sp.chunks;
-      if (cost < best_cost) { best_cost = cost; best = DaPlan{nsl, g, sp.max_chunks}; }
+    for (int k = 0; k < ng; k++) {
+      const GroupStats& st = stats[k];
+      const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
+                          2.0 * 4.0 * R * K * (double)st.chunks;
+      if (cost < best_cost) { best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks}; }
     }
   }
   return best;

@@ -497,49 +497,20 @@ def fused_multi_lora_dyw_dsa(dy, w, ds, a_list, routing: MultiRouting, dropout_m
 
 def lora_forward(x, w, a_list, b_list, routing_c, R, mask, bias):
     """One C call: S = drop(x) A^T, then y = x w^T + scale S B^T + bias.  Returns (y, s)."""
-    M, K = x.shape
-    N = w.shape[0]
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    s = torch.empty((M, R), dtype=x.dtype, device=x.device)
-    ws, nbytes = _ws(L.LF_OP_FWD, M, N, K, R, routing_c, x.device)
-    rc = L.lib().lf_lora_fwd(L.ptr(x), L.ptr(w), L.ptr(bias), L.ptr(mask), L.ptr_array(a_list), L.ptr_array(b_list),
-                             L.ptr(y), L.ptr(s), L.ptr(ws), nbytes, M, N, K, R, routing_c, _dt(x, mask, K),
-                             L.stream_of(x))
-    L.check(rc, "lf_lora_fwd")
-    return y, s
+    return L.host().forward(x, w, 0, w.shape[0], a_list, b_list, ctypes.addressof(routing_c), R, mask, None, True, bias, False)[:2]
 
 
 def lora_forward_seeded(x, w, a_list, b_list, routing_c, R, seed: int, bias, *, packed: bool = True):
     """As ``lora_forward`` with the keep-mask drawn inside the rank-r kernel from ``seed``.
     Returns (y, s, mask).  The mask comes back bit-packed (uint8 ``[M, K // 8]``, the format the backward kernels read
     fastest; ``packed=False``: bool ``[M, K]``); unpacked it equals ``make_dropout_mask`` for the same seed and routing."""
-    M, K = x.shape
-    N = w.shape[0]
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    s = torch.empty((M, R), dtype=x.dtype, device=x.device)
-    mask = torch.empty((M, K // 8), dtype=torch.uint8, device=x.device) if packed else torch.empty((M, K), dtype=torch.bool, device=x.device)
-    ws, nbytes = _ws(L.LF_OP_FWD, M, N, K, R, routing_c, x.device)
-    rc = L.lib().lf_lora_fwd_seeded(L.ptr(x), L.ptr(w), L.ptr(bias), L.ptr(mask), L.ptr_array(a_list), L.ptr_array(b_list),
-                                    L.ptr(y), L.ptr(s), L.ptr(ws), nbytes, M, N, K, R, routing_c,
-                                    ctypes.c_uint64(int(seed) & 0xFFFFFFFFFFFFFFFF), _dt(x, mask, K), L.stream_of(x))
-    L.check(rc, "lf_lora_fwd_seeded")
-    return y, s, mask
+    return L.host().forward(x, w, 0, w.shape[0], a_list, b_list, ctypes.addressof(routing_c), R, None, int(seed) & 0xFFFFFFFFFFFFFFFF,
+                            packed, bias, False)[:3]
 
 
 def lora_backward(dy, x, w, a_list, b_list, s, routing_c, R, mask, rank_list, requires_dx: bool = True):
     """One C call: dS/dB, dA and (optionally) dX.  Returns (dx | None, da_list, db_list)."""
-    M, N = dy.shape
-    K = x.shape[1]
-    dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device) if requires_dx else None
-    da_list = [torch.empty((r, K), dtype=dy.dtype, device=dy.device) for r in rank_list]
-    db_list = [torch.empty((N, r), dtype=dy.dtype, device=dy.device) for r in rank_list]
-    ds = torch.empty((M, R), dtype=dy.dtype, device=dy.device)
-    ws, nbytes = _ws(L.LF_OP_BWD, M, N, K, R, routing_c, dy.device)
-    rc = L.lib().lf_lora_bwd(L.ptr(dy), L.ptr(x), L.ptr(w), L.ptr(mask), L.ptr(s), L.ptr_array(a_list),
-                             L.ptr_array(b_list), L.ptr(dx), L.ptr_array(da_list), L.ptr_array(db_list), L.ptr(ds),
-                             L.ptr(ws), nbytes, M, N, K, R, routing_c, _dt(dy, mask, K), L.stream_of(dy))
-    L.check(rc, "lf_lora_bwd")
-    return dx, da_list, db_list
+    return L.host().backward(dy, x, w, 0, a_list, b_list, s, ctypes.addressof(routing_c), R, mask, None, requires_dx)
 
 
 def nf4_lora_forward(x, wref, a_list, b_list, routing_c, R, mask, bias, *, keep_dense: bool = False):
@@ -547,17 +518,8 @@ def nf4_lora_forward(x, wref, a_list, b_list, routing_c, R, mask, bias, *, keep_
     and runs the forward on it.  Returns (y, s), or (y, s, dense) with ``keep_dense``: the dequantised
     weight then goes into a tensor of its own instead of the call's workspace, for a backward that
     follows while it is still around (``nf4_lora_backward(..., dense=dense)``)."""
-    M, K = x.shape
-    N = wref.shape[0]
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    s = torch.empty((M, R), dtype=x.dtype, device=x.device)
-    dense = torch.empty((N, K), dtype=x.dtype, device=x.device) if keep_dense else None
-    wc = wref.with_dense(dense, valid=False)
-    ws, nbytes = _ws(L.LF_OP_FWD if keep_dense else L.LF_OP_NF4_FWD, M, N, K, R, routing_c, x.device)
-    rc = L.lib().lf_nf4_lora_fwd(L.ptr(x), ctypes.byref(wc), L.ptr(bias), L.ptr(mask), L.ptr_array(a_list),
-                                 L.ptr_array(b_list), L.ptr(y), L.ptr(s), L.ptr(ws), nbytes, M, N, K, R, routing_c,
-                                 _dt(x, mask, K), L.stream_of(x))
-    L.check(rc, "lf_nf4_lora_fwd")
+    y, s, _, dense = L.host().forward(x, None, ctypes.addressof(wref.c), wref.shape[0], a_list, b_list, ctypes.addressof(routing_c), R, mask,
+                                      None, True, bias, keep_dense)
     return (y, s, dense) if keep_dense else (y, s)
 
 
@@ -565,23 +527,10 @@ def nf4_lora_backward(dy, x, wref, a_list, b_list, s, routing_c, R, mask, rank_l
                       dense: torch.Tensor | None = None):
     """``lora_backward`` with the base weight given as NF4.  ``dense``: the dequantised weight a forward with
     ``keep_dense`` left behind (nothing is dequantised then).  Returns (dx | None, da_list, db_list)."""
-    M, N = dy.shape
-    K = x.shape[1]
-    dx = torch.empty((M, K), dtype=dy.dtype, device=dy.device) if requires_dx else None
-    da_list = [torch.empty((r, K), dtype=dy.dtype, device=dy.device) for r in rank_list]
-    db_list = [torch.empty((N, r), dtype=dy.dtype, device=dy.device) for r in rank_list]
-    ds = torch.empty((M, R), dtype=dy.dtype, device=dy.device)
+    N, K = dy.shape[1], x.shape[1]
     if dense is not None and (tuple(dense.shape) != (N, K) or dense.dtype != dy.dtype or not dense.is_contiguous()):
         raise ValueError(f"dense must be a contiguous [{N}, {K}] tensor of dtype {dy.dtype}.")
-    wc = wref.with_dense(dense, valid=True)
-    # no weight-sized head in the workspace when the weight is handed over, or not needed at all (no dX)
-    lean = dense is not None or not requires_dx
-    ws, nbytes = _ws(L.LF_OP_BWD if lean else L.LF_OP_NF4_BWD, M, N, K, R, routing_c, dy.device)
-    rc = L.lib().lf_nf4_lora_bwd(L.ptr(dy), L.ptr(x), ctypes.byref(wc), L.ptr(mask), L.ptr(s), L.ptr_array(a_list),
-                                 L.ptr_array(b_list), L.ptr(dx), L.ptr_array(da_list), L.ptr_array(db_list), L.ptr(ds),
-                                 L.ptr(ws), nbytes, M, N, K, R, routing_c, _dt(dy, mask, K), L.stream_of(dy))
-    L.check(rc, "lf_nf4_lora_bwd")
-    return dx, da_list, db_list
+    return L.host().backward(dy, x, None, ctypes.addressof(wref.c), a_list, b_list, s, ctypes.addressof(routing_c), R, mask, dense, requires_dx)
 
 
 def gemm(a: torch.Tensor, b: torch.Tensor, *, trans_b: bool = True, bias=None, tile_cfg: int = -1) -> torch.Tensor:

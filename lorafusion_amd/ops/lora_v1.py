@@ -1,7 +1,8 @@
 """Single-adapter fused LoRA linear: ``fused_linear_lora`` / ``FusedLinearLoRA``.
 
-Same call signature and gradient contract as lorafusion/ops/lora_v1.py:173-297; the work is two
-C calls (forward: ``lf_lora_fwd``, backward: ``lf_lora_bwd``) into the HIP library.
+Same call signature and gradient contract as lorafusion/ops/lora_v1.py:173-297; the work is one call into the host
+module (csrc/host_ops.cpp: ``lf_lora_fwd`` / ``lf_lora_fwd_seeded``, and an autograd node whose backward is
+``lf_lora_bwd``).
 
 Differences from the reference, all deliberate:
  * the dropped input ``where(mask, x/(1-p), 0)`` is never stored: backward rebuilds it from
@@ -21,11 +22,6 @@ import torch
 
 from lorafusion_amd import _lib as L
 from lorafusion_amd.ops import hip_ops
-
-
-def _validate(x2d, linear_w, lora_a, lora_b, linear_bias, dropout_p):
-    L.require_gpu(linear_w, "linear_w")
-    return _validate_shapes(x2d, tuple(linear_w.shape), linear_w.dtype, lora_a, lora_b, linear_bias, dropout_p)
 
 
 def _validate_shapes(x2d, w_shape, w_dtype, lora_a, lora_b, linear_bias, dropout_p):
@@ -54,68 +50,16 @@ def _validate_shapes(x2d, w_shape, w_dtype, lora_a, lora_b, linear_bias, dropout
     return M, N, K, r
 
 
-class FusedLinearLoRA(torch.autograd.Function):
+class FusedLinearLoRA:
     """``y = x W^T + alpha * (drop(x) A^T) B^T + bias`` with the LoRA term fused into the GEMMs."""
 
     @staticmethod
-    def forward(ctx, x, linear_w, lora_a, lora_b, alpha, dropout_p, seed=None, linear_bias=None, dropout_mask=None):
-        if x.ndim == 3:
-            lead = x.shape[:2]
-            x2d = x.reshape(lead[0] * lead[1], -1)
-        elif x.ndim == 2:
-            lead = None
-            x2d = x
-        else:
-            raise ValueError(f"Expected x to have 2 or 3 dimensions, got {x.ndim}.")
-        x2d = x2d.contiguous()
-        linear_w, lora_a, lora_b = linear_w.contiguous(), lora_a.contiguous(), lora_b.contiguous()
-        M, N, K, r = _validate(x2d, linear_w, lora_a, lora_b, linear_bias, dropout_p)
-
-        R = L.round_rank(r)
-        bias = linear_bias.contiguous() if linear_bias is not None else None
-        mask = None
+    def apply(x, linear_w, lora_a, lora_b, alpha, dropout_p, seed=None, linear_bias=None, dropout_mask=None):
+        draw = None
         if dropout_p > 0 and dropout_mask is None:
             # the reference's default path: the keep-mask is drawn while X streams through the rank-r pass
-            if seed is None:
-                seed = random.randrange(int(1e6))  # noqa: S311
-            routing = L.single_routing(r, alpha, dropout_p)
-            y, s, mask = hip_ops.lora_forward_seeded(x2d, linear_w, [lora_a], [lora_b], routing, R, seed, bias)
-        else:
-            if dropout_p > 0:
-                mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
-                if not hip_ops.is_packed_mask(mask, K):
-                    mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-            routing = L.single_routing(r, alpha, dropout_p if mask is not None else 0.0)
-            y, s = hip_ops.lora_forward(x2d, linear_w, [lora_a], [lora_b], routing, R, mask, bias)
-
-        ctx.save_for_backward(x2d, linear_w, lora_a, lora_b, mask, s)
-        ctx.alpha = alpha
-        ctx.dropout_p = dropout_p if mask is not None else 0.0
-        ctx.seed = seed
-        ctx.lead = lead
-        return y if lead is None else y.reshape(*lead, N)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x2d, linear_w, lora_a, lora_b, mask, s = ctx.saved_tensors
-        if dy.ndim == 3:
-            dy2d = dy.reshape(dy.shape[0] * dy.shape[1], -1)
-        elif dy.ndim == 2:
-            dy2d = dy
-        else:
-            raise ValueError(f"Expected dy to have 2 or 3 dimensions, got {dy.ndim}.")
-        dy2d = dy2d.contiguous()
-        r = lora_a.shape[0]
-        routing = L.single_routing(r, ctx.alpha, ctx.dropout_p)
-        dx, da_list, db_list = hip_ops.lora_backward(
-            dy2d, x2d, linear_w, [lora_a], [lora_b], s, routing, L.round_rank(r), mask, [r],
-            requires_dx=ctx.needs_input_grad[0],
-        )
-        if dx is not None and ctx.lead is not None:
-            dx = dx.reshape(*ctx.lead, -1)
-        da = da_list[0] if ctx.needs_input_grad[2] else None
-        db = db_list[0] if ctx.needs_input_grad[3] else None
-        return dx, None, da, db, None, None, None, None, None
+            draw = (random.randrange(int(1e6)) if seed is None else int(seed)) & 0xFFFFFFFFFFFFFFFF  # noqa: S311
+        return L.host().linear_lora(x, linear_w, lora_a, lora_b, alpha, dropout_p, draw, linear_bias, dropout_mask)
 
 
 def fused_linear_lora(

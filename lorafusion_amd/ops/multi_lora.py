@@ -18,6 +18,7 @@ Differences from the reference, all deliberate:
 
 from __future__ import annotations
 
+import ctypes
 import random
 from collections import deque
 from dataclasses import dataclass
@@ -194,25 +195,18 @@ def batch_info_from_micro_batch(
     return info
 
 
-class FusedLinearMultiLoRA(torch.autograd.Function):
+class FusedLinearMultiLoRA:
     """Packed multi-adapter LoRA linear.  Adapter tensors are passed as ``*a_list, *b_list``."""
 
     @staticmethod
-    def forward(ctx, padded_x, linear_w, linear_bias, dropout_mask, seed, routing: MultiRouting, quant_state,
-                keep_dequantized, n_adapters, *ab):
+    def apply(padded_x, linear_w, linear_bias, dropout_mask, seed, routing: MultiRouting, quant_state, keep_dequantized, n_adapters, *ab):
         if padded_x.ndim == THREE_DIM:
             if padded_x.shape[0] != 1:
                 raise ValueError("currently, we only support batch size 1 for multi-linear LoRA")
-            x2d = padded_x.reshape(padded_x.shape[1], padded_x.shape[2])
-            lead = True
-        elif padded_x.ndim == 2:
-            x2d, lead = padded_x, False
-        else:
+        elif padded_x.ndim != 2:
             raise ValueError(f"padded_x must be a 3D tensor, but got {padded_x.ndim}")
-        x2d = x2d.contiguous()
-        linear_w = linear_w.contiguous()
-        a_list = [t.contiguous() for t in ab[:n_adapters]]
-        b_list = [t.contiguous() for t in ab[n_adapters:]]
+        x2d = padded_x.detach().contiguous().view(padded_x.shape[-2], padded_x.shape[-1])
+        a_list, b_list = list(ab[:n_adapters]), list(ab[n_adapters:])
         M, K = x2d.shape
         wref = None
         if quant_state is not None:
@@ -222,6 +216,7 @@ class FusedLinearMultiLoRA(torch.autograd.Function):
             wref = NF4WeightRef(linear_w, quant_state)
             w_shape, w_dtype = tuple(wref.shape), wref.dtype
         else:
+            linear_w = linear_w.contiguous()
             w_shape, w_dtype = tuple(linear_w.shape), linear_w.dtype
         if M != routing.M:
             raise ValueError(f"padded_x has {M} rows but the batch info covers {routing.M}.")
@@ -231,9 +226,11 @@ class FusedLinearMultiLoRA(torch.autograd.Function):
         L.require_gpu(x2d, "padded_x")
         L.dtype_id(x2d.dtype)
         hip_ops._check_dims(M, N, K)
-        hip_ops._check_adapters(a_list, b_list, routing, K, N, x2d.dtype)
+        host = L.host()
+        host.check_adapters(a_list, b_list, routing.rank_list, K, N, x2d)
         if linear_bias is not None and (tuple(linear_bias.shape) != (N,) or linear_bias.dtype != x2d.dtype):
             raise ValueError(f"linear_bias must have shape [{N}] and dtype {x2d.dtype}.")
+        a_run, b_run = [t.contiguous() for t in a_list], [t.contiguous() for t in b_list]
 
         mask, dense = None, None
         bias = linear_bias.contiguous() if linear_bias is not None else None
@@ -244,60 +241,22 @@ class FusedLinearMultiLoRA(torch.autograd.Function):
                 mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
                 if not hip_ops.is_packed_mask(mask, K):
                     mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-            if keep_dequantized:
-                y, s, dense = hip_ops.nf4_lora_forward(x2d, wref, a_list, b_list, routing.c, routing.R, mask, bias,
-                                                       keep_dense=True)
-            else:
-                y, s = hip_ops.nf4_lora_forward(x2d, wref, a_list, b_list, routing.c, routing.R, mask, bias)
+            y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing.c, routing.R, mask, bias, keep_dense=keep_dequantized)
+            dense = kept[0] if kept else None
         elif routing.enable_dropout and dropout_mask is None:
             # per-block p from the routing table, mask drawn inside the rank-r pass
             if seed is None:
                 seed = random.randrange(int(1e6))  # noqa: S311
-            y, s, mask = hip_ops.lora_forward_seeded(x2d, linear_w, a_list, b_list, routing.c, routing.R, seed, bias)
+            y, s, mask = hip_ops.lora_forward_seeded(x2d, linear_w, a_run, b_run, routing.c, routing.R, seed, bias)
         else:
             if routing.enable_dropout:
                 mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
                 if not hip_ops.is_packed_mask(mask, K):
                     mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-            y, s = hip_ops.lora_forward(x2d, linear_w, a_list, b_list, routing.c, routing.R, mask, bias)
-
-        ctx.save_for_backward(x2d, linear_w, mask, s, dense, *a_list, *b_list)
-        ctx.routing = routing
-        ctx.quant_state = quant_state
-        ctx.n_adapters = n_adapters
-        ctx.lead = lead
-        return y.reshape(1, M, N) if lead else y
-
-    @staticmethod
-    def backward(ctx, dy):
-        x2d, linear_w, mask, s, dense, *ab = ctx.saved_tensors
-        n = ctx.n_adapters
-        a_list, b_list = list(ab[:n]), list(ab[n:])
-        routing = ctx.routing
-        if dy.ndim == THREE_DIM:
-            if dy.shape[0] != 1:
-                raise ValueError("currently, we only support batch size 1 for multi-linear LoRA")
-            dy2d = dy.reshape(dy.shape[1], dy.shape[2])
-        elif dy.ndim == 2:
-            dy2d = dy
-        else:
-            raise ValueError(f"dy must be a 3D tensor, but got {dy.ndim}")
-        dy2d = dy2d.contiguous()
-        if ctx.quant_state is not None:
-            from lorafusion_amd.ops.nf4 import NF4WeightRef
-
-            dx, da_list, db_list = hip_ops.nf4_lora_backward(
-                dy2d, x2d, NF4WeightRef(linear_w, ctx.quant_state), a_list, b_list, s, routing.c, routing.R, mask,
-                routing.rank_list, requires_dx=ctx.needs_input_grad[0], dense=dense,
-            )
-        else:
-            dx, da_list, db_list = hip_ops.lora_backward(
-                dy2d, x2d, linear_w, a_list, b_list, s, routing.c, routing.R, mask, routing.rank_list,
-                requires_dx=ctx.needs_input_grad[0],
-            )
-        if dx is not None and ctx.lead:
-            dx = dx.reshape(1, *dx.shape)
-        return (dx, None, None, None, None, None, None, None, None, *da_list, *db_list)
+            y, s = hip_ops.lora_forward(x2d, linear_w, a_run, b_run, routing.c, routing.R, mask, bias)
+        nf4, keep = (ctypes.addressof(wref.c), wref.keep) if wref is not None else (0, [])
+        return host.attach(y, [padded_x], x2d, linear_w, nf4, [t for t in keep if t is not None], a_list, b_list, mask, s, dense, [],
+                           ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
 
 
 def fused_linear_multi_lora(

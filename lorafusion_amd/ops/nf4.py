@@ -10,6 +10,7 @@ dependency here).
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -178,7 +179,7 @@ def quantize_nf4(w: torch.Tensor, blocksize: int = 64, compress_statistics: bool
     return packed, QuantState(shape, out_dtype, blocksize, absq, offset, QuantState2(absmax2, code, blocksize2))
 
 
-class FusedLinearLoRANF4(torch.autograd.Function):
+class FusedLinearLoRANF4:
     """QLoRA linear: NF4 base weight dequantised on the fly, bf16/fp16 adapters.
 
     Forward and backward each dequantise the weight into the call's workspace
@@ -188,23 +189,16 @@ class FusedLinearLoRANF4(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, x, packed_w, quant_state, lora_a, lora_b, alpha, dropout_p, seed, linear_bias, dropout_mask,
-                keep_dequantized=False):
+    def apply(x, packed_w, quant_state, lora_a, lora_b, alpha, dropout_p, seed, linear_bias, dropout_mask, keep_dequantized=False):
         from lorafusion_amd.ops import hip_ops
         from lorafusion_amd.ops.lora_v1 import _validate_shapes
 
-        if x.ndim == 3:
-            lead = x.shape[:2]
-            x2d = x.reshape(lead[0] * lead[1], -1)
-        elif x.ndim == 2:
-            lead, x2d = None, x
-        else:
+        if x.ndim not in (2, 3):
             raise ValueError(f"Expected x to have 2 or 3 dimensions, got {x.ndim}.")
-        x2d = x2d.contiguous()
+        x2d = x.detach().contiguous().view(-1, x.shape[-1])
         if quant_state.dtype != x2d.dtype:
             raise ValueError(f"quant_state.dtype {quant_state.dtype} must match x.dtype {x2d.dtype}.")
         wref = NF4WeightRef(packed_w, quant_state)
-        lora_a, lora_b = lora_a.contiguous(), lora_b.contiguous()
         M, N, K, r = _validate_shapes(x2d, tuple(wref.shape), x2d.dtype, lora_a, lora_b, linear_bias, dropout_p)
         mask = None
         bias = linear_bias.contiguous() if linear_bias is not None else None
@@ -214,33 +208,11 @@ class FusedLinearLoRANF4(torch.autograd.Function):
             mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
             if not hip_ops.is_packed_mask(mask, K):
                 mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-        p_eff = dropout_p if mask is not None else 0.0
-        routing = L.single_routing(r, alpha, p_eff)
-        dense = None
-        if keep_dequantized:
-            y, s, dense = hip_ops.nf4_lora_forward(x2d, wref, [lora_a], [lora_b], routing, L.round_rank(r), mask, bias,
-                                                   keep_dense=True)
-        else:
-            y, s = hip_ops.nf4_lora_forward(x2d, wref, [lora_a], [lora_b], routing, L.round_rank(r), mask, bias)
-        ctx.save_for_backward(x2d, packed_w, lora_a, lora_b, mask, s, dense)
-        ctx.quant_state, ctx.alpha, ctx.p, ctx.lead = quant_state, alpha, p_eff, lead
-        return y if lead is None else y.reshape(*lead, N)
-
-    @staticmethod
-    def backward(ctx, dy):
-        from lorafusion_amd.ops import hip_ops
-
-        x2d, packed_w, lora_a, lora_b, mask, s, dense = ctx.saved_tensors
-        dy2d = dy.reshape(-1, dy.shape[-1]).contiguous()
-        r = lora_a.shape[0]
-        wref = NF4WeightRef(packed_w, ctx.quant_state)
-        routing = L.single_routing(r, ctx.alpha, ctx.p)
-        dx, da_list, db_list = hip_ops.nf4_lora_backward(dy2d, x2d, wref, [lora_a], [lora_b], s, routing,
-                                                         L.round_rank(r), mask, [r],
-                                                         requires_dx=ctx.needs_input_grad[0], dense=dense)
-        if dx is not None and ctx.lead is not None:
-            dx = dx.reshape(*ctx.lead, -1)
-        return dx, None, None, da_list[0], db_list[0], None, None, None, None, None, None
+        routing, R = L.single_routing(r, alpha, dropout_p if mask is not None else 0.0), L.round_rank(r)
+        y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, [lora_a.contiguous()], [lora_b.contiguous()], routing, R, mask, bias,
+                                               keep_dense=keep_dequantized)
+        return L.host().attach(y, [x], x2d, packed_w, ctypes.addressof(wref.c), [t for t in wref.keep if t is not None], [lora_a], [lora_b],
+                               mask, s, kept[0] if kept else None, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
 
 
 def fused_linear_lora_nf4(x, packed_w, quant_state, lora_a, lora_b, alpha, seed=None, dropout_p=0.0,

@@ -19,7 +19,6 @@ import torch
 from lorafusion_amd import _lib as L
 from lorafusion_amd.ops import hip_ops
 from lorafusion_amd.ops.hip_ops import MultiRouting
-from lorafusion_amd.ops.norm_act import _silu_bwd
 
 
 def _swiglu_lora_forward(gate, up, ld, w, a_list, b_list, routing_c, R, mask, draw_seed, bias):
@@ -48,36 +47,33 @@ def _rows2d(t: torch.Tensor) -> torch.Tensor:
     return t2 if ok else t2.contiguous()
 
 
-class FusedSwiGLULinearLoRA(torch.autograd.Function):
+class FusedSwiGLULinearLoRA:
     """``y = X W^T + scale_i (drop(X) A_i^T) B_i^T + bias`` with ``X = silu(gate) * up`` taken from a merged
     ``[.., 2K]`` gate/up tensor or from two ``[.., K]`` tensors.  ``routing`` is a ``MultiRouting`` (packed
     multi-adapter batch) or ``None`` (one adapter: ``alpha`` and ``dropout_p`` apply to all rows)."""
 
     @staticmethod
-    def forward(ctx, gate, up, linear_w, linear_bias, dropout_mask, seed, routing, alpha, dropout_p, n_adapters, *ab):
+    def apply(gate, up, linear_w, linear_bias, dropout_mask, seed, routing, alpha, dropout_p, n_adapters, *ab):
         # up is None: `gate` is the merged [.., 2K] tensor (gate half first)
-        merged = up is None
-        if merged:
+        if up is None:
             if gate.shape[-1] % 256 != 0:
                 raise ValueError(f"the merged gate/up width must be a multiple of 256, got {gate.shape[-1]}.")
-            lead = gate.shape[:-1]
-            g2 = gate.reshape(-1, gate.shape[-1])
-            g2 = g2 if g2.is_contiguous() else g2.contiguous()
+            inputs = [gate]
+            g2 = gate.detach().contiguous().view(-1, gate.shape[-1])
             K = g2.shape[1] // 2
             gv, uv, ld = g2[:, :K], g2[:, K:], 2 * K
-            saved_in = (g2,)
+            saved_in = [g2]
         else:
             if gate.shape != up.shape or gate.dtype != up.dtype:
                 raise ValueError(f"gate and up differ: {tuple(gate.shape)} {gate.dtype} vs {tuple(up.shape)} {up.dtype}.")
-            lead = gate.shape[:-1]
-            gv, uv = _rows2d(gate), _rows2d(up)
+            inputs = [gate, up]
+            gv, uv = _rows2d(gate.detach()), _rows2d(up.detach())
             if gv.stride(0) != uv.stride(0):
                 gv, uv = gv.contiguous(), uv.contiguous()
             K, ld = gv.shape[1], gv.stride(0) if gv.shape[0] > 1 else gv.shape[1]
-            saved_in = (gv, uv)
+            saved_in = [gv, uv]
         linear_w = linear_w.contiguous()
-        a_list = [t.contiguous() for t in ab[:n_adapters]]
-        b_list = [t.contiguous() for t in ab[n_adapters:]]
+        a_list, b_list = [t.detach().contiguous() for t in ab[:n_adapters]], [t.detach().contiguous() for t in ab[n_adapters:]]
         M = gv.shape[0]
         N = linear_w.shape[0]
         L.require_gpu(gv, "gate")
@@ -112,38 +108,9 @@ class FusedSwiGLULinearLoRA(torch.autograd.Function):
         p_used = dropout_p if dropout else 0.0
         routing_c = routing.c if routing is not None else L.single_routing(rank_list[0], alpha, p_used)
         x, y, s, mask = _swiglu_lora_forward(gv, uv, ld, linear_w, a_list, b_list, routing_c, R, mask, draw, bias)
-        ctx.save_for_backward(x, linear_w, mask, s, *saved_in, *a_list, *b_list)
-        ctx.routing, ctx.alpha, ctx.p_used = routing, alpha, p_used
-        ctx.R, ctx.rank_list, ctx.n_adapters, ctx.lead, ctx.merged = R, rank_list, n_adapters, lead, merged
-        return y.reshape(*lead, N)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, linear_w, mask, s, *rest = ctx.saved_tensors
-        n_in = 1 if ctx.merged else 2
-        inputs, ab = rest[:n_in], rest[n_in:]
-        n = ctx.n_adapters
-        a_list, b_list = list(ab[:n]), list(ab[n:])
-        dy2 = dy.reshape(-1, dy.shape[-1]).contiguous()
-        routing_c = ctx.routing.c if ctx.routing is not None else L.single_routing(ctx.rank_list[0], ctx.alpha, ctx.p_used)
-        need_dg = ctx.needs_input_grad[0] or (not ctx.merged and ctx.needs_input_grad[1])
-        dx, da_list, db_list = hip_ops.lora_backward(dy2, x, linear_w, a_list, b_list, s, routing_c, ctx.R, mask,
-                                                     ctx.rank_list, requires_dx=need_dg)
-        dg, du = None, None
-        if need_dg:
-            M, K = x.shape
-            if ctx.merged:
-                (g2,) = inputs
-                dg = torch.empty_like(g2)
-                _silu_bwd(dx, K, g2[:, :K], 2 * K, g2[:, K:], 2 * K, dg[:, :K], 2 * K, dg[:, K:], 2 * K)
-                dg = dg.reshape(*ctx.lead, 2 * K)
-            else:
-                gv, uv = inputs
-                dg = torch.empty((M, K), dtype=x.dtype, device=x.device)
-                du = torch.empty((M, K), dtype=x.dtype, device=x.device)
-                _silu_bwd(dx, K, gv, gv.stride(0) if M > 1 else K, uv, uv.stride(0) if M > 1 else K, dg, K, du, K)
-                dg, du = dg.reshape(*ctx.lead, K), du.reshape(*ctx.lead, K)
-        return (dg, du, None, None, None, None, None, None, None, None, *da_list, *db_list)
+        tables = [routing.table, routing.scale, routing.p] if routing is not None else []
+        return L.host().attach(y, inputs, x, linear_w, 0, [], list(ab[:n_adapters]), list(ab[n_adapters:]), mask, s, None, saved_in,
+                               ctypes.addressof(routing_c), tables, R, "FusedSwiGLULinearLoRABackward")
 
 
 def fused_swiglu_linear_lora(gate_up, linear_w, lora_a, lora_b, alpha: float, seed: int | None = None,
