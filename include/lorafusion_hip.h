@@ -98,9 +98,11 @@ typedef struct lf_routing {
 int lf_version(void);
 const char* lf_strerror(int code);
 /* Bytes of `workspace` the entry point(s) behind `op` use for this shape: the fp32 partial sums of
- * the rank-r passes, which a call must be given, and for LF_OP_FWD / BWD / NF4_* the fp32 partial
- * tiles of a split contraction (launches with few tiles and a long K: left-over rows of a packed
- * batch, short batches), which a call skips when the workspace is smaller or NULL.  0 also for a
+ * the backward's rank-r passes, which a call must be given, and what a call does without when the
+ * workspace is smaller or NULL: for LF_OP_FWD / BWD / NF4_* the fp32 partial tiles of a split
+ * contraction (launches with few tiles and a long K: left-over rows of a packed batch, short
+ * batches), for LF_OP_XA / FWD / NF4_FWD the slices of the forward's rank-r pass (more than 32 rank
+ * columns, short batches), for LF_OP_FWD / NF4_FWD the slices of a short batch's single pass. 0 also for a
  * shape or routing the entry point itself would refuse (M <= 0, R not a multiple of 16 in 16..128, a tiled dimension
  * -- N for DYS_DYB / BWD / NF4_*, K for XA / DA / FWD / BWD / NF4_* -- that is not a positive multiple
  * of 128, bad routing): the size query never fails harder than the call. */

@@ -860,6 +860,7 @@ int lf_pin_tile_cfg(int cfg) {
   pinned_cfg.store(cfg, std::memory_order_relaxed);
   return LF_OK;
 }
+bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; }
 
 // The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned: rows [0, *rows_head)
 // with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).

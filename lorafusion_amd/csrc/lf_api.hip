@@ -5,8 +5,13 @@
 
 int lf_launch_nf4_dequant(const uint8_t*, const void*, const float*, const float*, const float*, void*, int64_t,
                           int, int, int, hipStream_t);
-int lf_launch_xa(const void*, const void*, int64_t, void*, const uint8_t*, uint8_t*, int, uint64_t, void*, int, int, int, const LfSegTable&, int,
-                 hipStream_t);
+int lf_launch_xa(const void*, const void*, int64_t, void*, const uint8_t*, uint8_t*, int, uint64_t, void*, void*, size_t, int, int, int,
+                 const LfSegTable&, int, hipStream_t);
+bool lf_xa_streams(int M, int R, bool masked, const LfSegTable& seg);
+bool lf_short_fwd_applies(int M, int N);
+size_t lf_short_fwd_workspace(int M, int N, int K, int rank);
+int lf_launch_short_fwd(const void*, const void*, const void*, const void*, float, const void*, void*, void*, void*, int, int, int, int, int,
+                        const LfSegTable&, int, hipStream_t);
 int lf_launch_mask_pack(const uint8_t*, uint8_t*, int64_t, hipStream_t);
 int lf_launch_mask_unpack(const uint8_t*, uint8_t*, int64_t, hipStream_t);
 int lf_launch_dys_dyb(const void*, const void*, void*, void*, size_t, int, int, int, const LfSegTable&, int, hipStream_t);
@@ -86,6 +91,21 @@ int take_mask_bits(int& dtype) {
 bool bad_tiled_dim(int v) { return v <= 0 || v % 128 != 0; }
 bool bad_rank_cols(int R) { return R <= 0 || R % 16 != 0 || R > LF_MAX_RANK; }
 
+// Scratch of a forward: the rank-r pass's slices and, behind them, a split contraction's partial tiles (Y = [M,N] over K); or the
+// short forward's slices.
+size_t fwd_workspace(int M, int N, int K, int R, int rb, const LfSegTable& t) {
+  const size_t sliced = !t.table && lf_short_fwd_applies(M, N) && !bad_tiled_dim(N) ? lf_short_fwd_workspace(M, N, K, t.rank[0]) : 0;
+  return std::max(sliced, align256(lf_xa_workspace(M, K, R, t)) + lf_gemm_ksplit_bytes(M, N, K, rb));
+}
+// What is left of a forward's workspace behind the rank-r pass's slices.
+void behind_xa(void*& ws, size_t& bytes, int M, int K, int R, const lf_routing* routing) {
+  LfSegTable t;
+  if (ws == nullptr || make_seg(routing, M, nullptr, nullptr, t) != LF_OK) return;
+  const size_t head = align256(lf_xa_workspace(M, K, R, t));
+  bytes = bytes > head ? bytes - head : 0;
+  ws = bytes > 0 ? (char*)ws + head : nullptr;
+}
+
 }  // namespace
 
 extern "C" {
@@ -121,13 +141,12 @@ size_t lf_workspace_bytes(int op, int M, int N, int K, int R, const lf_routing* 
     case LF_OP_DYS_DYB: return align256(lf_dys_dyb_workspace(M, N, R, t));
     case LF_OP_DA: return align256(lf_da_workspace(M, K, R, t));
     // (the products of the whole-pass entry points may split their contraction: Y = [M,N] over K, dX = [M,K] over N)
-    case LF_OP_FWD: return align256(std::max(lf_xa_workspace(M, K, R, t), lf_gemm_ksplit_bytes(M, N, K, rb)));
+    case LF_OP_FWD: return align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_BWD: {
       size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
       return align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb)));
     }
-    case LF_OP_NF4_FWD:
-      return align256((size_t)N * K * 2) + align256(std::max(lf_xa_workspace(M, K, R, t), lf_gemm_ksplit_bytes(M, N, K, rb)));
+    case LF_OP_NF4_FWD: return align256((size_t)N * K * 2) + align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_NF4_BWD: {
       size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
       return align256((size_t)N * K * 2) + align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb)));
@@ -144,24 +163,29 @@ int lf_lora_xa(const void* X, const uint8_t* mask, const void* const* a_ptrs, vo
   int rc = make_seg(routing, M, a_ptrs, nullptr, t);
   if (rc != LF_OK) return rc;
   for (int s = 0; s < t.n_seg; s++) if (!t.ptr[s]) return LF_EINVAL;
-  (void)workspace; (void)ws_bytes;  // no partial sums leave the workgroups
-  return lf_launch_xa(X, nullptr, 0, nullptr, mask, nullptr, mb, 0, S, M, K, R, t, dtype, (hipStream_t)stream);
+  return lf_launch_xa(X, nullptr, 0, nullptr, mask, nullptr, mb, 0, S, workspace, workspace ? ws_bytes : 0, M, K, R, t, dtype, (hipStream_t)stream);
 }
 
-int lf_lora_xa_seeded(const void* X, uint8_t* mask_out, const void* const* a_ptrs, void* S, int M, int K, int R,
-                      const lf_routing* routing, uint64_t seed, int dtype, void* stream) {
+static int xa_seeded_ws(const void* X, uint8_t* mask_out, const void* const* a_ptrs, void* S, void* workspace, size_t ws_bytes, int M,
+                        int K, int R, const lf_routing* routing, uint64_t seed, int dtype, void* stream) {
   const int mb = take_mask_bits(dtype);
   if (bad_dtype(dtype) || !a_ptrs || !mask_out) return LF_EINVAL;
   LfSegTable t;
   int rc = make_seg(routing, M, a_ptrs, nullptr, t);
   if (rc != LF_OK) return rc;
   for (int s = 0; s < t.n_seg; s++) if (!t.ptr[s]) return LF_EINVAL;
-  return lf_launch_xa(X, nullptr, 0, nullptr, nullptr, mask_out, mb, seed, S, M, K, R, t, dtype, (hipStream_t)stream);
+  return lf_launch_xa(X, nullptr, 0, nullptr, nullptr, mask_out, mb, seed, S, workspace, workspace ? ws_bytes : 0, M, K, R, t, dtype,
+                      (hipStream_t)stream);
 }
 
-int lf_lora_xa_silu_mul(const void* G, const void* U, int64_t ld, void* X_out, const uint8_t* mask, uint8_t* mask_out,
-                        uint64_t seed, const void* const* a_ptrs, void* S, int M, int K, int R, const lf_routing* routing,
-                        int dtype, void* stream) {
+int lf_lora_xa_seeded(const void* X, uint8_t* mask_out, const void* const* a_ptrs, void* S, int M, int K, int R,
+                      const lf_routing* routing, uint64_t seed, int dtype, void* stream) {
+  return xa_seeded_ws(X, mask_out, a_ptrs, S, nullptr, 0, M, K, R, routing, seed, dtype, stream);
+}
+
+static int xa_silu_mul_ws(const void* G, const void* U, int64_t ld, void* X_out, const uint8_t* mask, uint8_t* mask_out, uint64_t seed,
+                          const void* const* a_ptrs, void* S, void* workspace, size_t ws_bytes, int M, int K, int R, const lf_routing* routing,
+                          int dtype, void* stream) {
   const int mb = take_mask_bits(dtype);
   if (bad_dtype(dtype) || !a_ptrs || !G || !U || !X_out) return LF_EINVAL;
   if (mask && mask_out) return LF_EINVAL;
@@ -169,7 +193,21 @@ int lf_lora_xa_silu_mul(const void* G, const void* U, int64_t ld, void* X_out, c
   int rc = make_seg(routing, M, a_ptrs, nullptr, t);
   if (rc != LF_OK) return rc;
   for (int s = 0; s < t.n_seg; s++) if (!t.ptr[s]) return LF_EINVAL;
-  return lf_launch_xa(G, U, ld, X_out, mask, mask_out, mb, seed, S, M, K, R, t, dtype, (hipStream_t)stream);
+  // (what the fused kernel refuses is refused here too; where the sliced pass takes the product, the activation is a pass of its own)
+  if (M > 0 && K > 0 && S != nullptr && lf_xa_streams(M, R, mask != nullptr || mask_out != nullptr, t)) {
+    if (K % 128 != 0 || bad_rank_cols(R) || ld < K || ld % 8 != 0 || (((uintptr_t)G | (uintptr_t)U | (uintptr_t)X_out) & 15) != 0) return LF_ESHAPE;
+    rc = lf_silu_mul_fwd(G, U, X_out, M, K, ld, ld, K, dtype, stream);
+    if (rc != LF_OK) return rc;
+    return lf_launch_xa(X_out, nullptr, 0, nullptr, mask, mask_out, mb, seed, S, workspace, workspace ? ws_bytes : 0, M, K, R, t, dtype,
+                        (hipStream_t)stream);
+  }
+  return lf_launch_xa(G, U, ld, X_out, mask, mask_out, mb, seed, S, nullptr, 0, M, K, R, t, dtype, (hipStream_t)stream);
+}
+
+int lf_lora_xa_silu_mul(const void* G, const void* U, int64_t ld, void* X_out, const uint8_t* mask, uint8_t* mask_out,
+                        uint64_t seed, const void* const* a_ptrs, void* S, int M, int K, int R, const lf_routing* routing,
+                        int dtype, void* stream) {
+  return xa_silu_mul_ws(G, U, ld, X_out, mask, mask_out, seed, a_ptrs, S, nullptr, 0, M, K, R, routing, dtype, stream);
 }
 
 // lf_lora_xw_sb / lf_lora_dyw_dsa with a workspace for the split contraction of under-filled launches (the whole
@@ -199,12 +237,35 @@ int lf_lora_xw_sb(const void* X, const void* W, const void* bias, const void* S,
   return xw_sb_ws(X, W, bias, S, b_ptrs, Y, nullptr, 0, M, N, K, R, routing, dtype, stream);
 }
 
+// The forward of a short batch of one adapter without a keep-mask: one pass over W and A together (lora_stream.hip).
+// False where it does not apply, or where the general path refuses the call itself; a pinned tile stays as pinned.
+static bool short_fwd(const void* X, const void* W, const void* bias, const void* const* a_ptrs, const void* const* b_ptrs, void* Y, void* S,
+                      void* workspace, size_t ws_bytes, int M, int N, int K, int R, const lf_routing* routing, int dtype, void* stream, int* rc) {
+  dtype &= ~LF_MASK_BITS;
+  if (lf_tile_pinned() || bad_dtype(dtype) || !X || !W || !Y || !S || !a_ptrs || !b_ptrs || M <= 0 || bad_tiled_dim(N) || bad_tiled_dim(K) ||
+      bad_rank_cols(R) || (((uintptr_t)Y | (uintptr_t)S) & 15) != 0)
+    return false;
+  LfSegTable t;
+  if (make_seg(routing, M, a_ptrs, nullptr, t) != LF_OK || t.table || !lf_short_fwd_applies(M, N) || !t.ptr[0] || !b_ptrs[0] || t.rank[0] > R) return false;
+  if (!workspace || ws_bytes < lf_short_fwd_workspace(M, N, K, t.rank[0])) return false;
+  *rc = lf_launch_short_fwd(X, W, t.ptr[0], b_ptrs[0], t.scale, bias, Y, S, workspace, M, N, K, t.rank[0], R, t, dtype, (hipStream_t)stream);
+  return true;
+}
+
 int lf_swiglu_lora_fwd(const void* G, const void* U, int64_t ld, void* X_out, const void* W, const void* bias,
                        const uint8_t* mask, uint8_t* mask_out, uint64_t seed, const void* const* a_ptrs,
                        const void* const* b_ptrs, void* Y, void* S_out, void* workspace, size_t ws_bytes, int M, int N,
                        int K, int R, const lf_routing* routing, int dtype, void* stream) {
-  int rc = lf_lora_xa_silu_mul(G, U, ld, X_out, mask, mask_out, seed, a_ptrs, S_out, M, K, R, routing, dtype, stream);
+  const int et = dtype & ~LF_MASK_BITS;
+  // (as lf_lora_fwd on the activation's output would: short batches without a mask take the single pass)
+  if (!mask && !mask_out && routing && !routing->block_table && lf_short_fwd_applies(M, N) && G && U && X_out && !bad_tiled_dim(K)) {
+    int rc = lf_silu_mul_fwd(G, U, X_out, M, K, ld, ld, K, et, stream);
+    if (rc != LF_OK) return rc;
+    return lf_lora_fwd(X_out, W, bias, nullptr, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, et, stream);
+  }
+  int rc = xa_silu_mul_ws(G, U, ld, X_out, mask, mask_out, seed, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;
+  behind_xa(workspace, ws_bytes, M, K, R, routing);
   return xw_sb_ws(X_out, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);
 }
 
@@ -258,17 +319,20 @@ int lf_lora_dyw_dsa(const void* dY, const void* W, const void* dS, const void* c
 int lf_lora_fwd(const void* X, const void* W, const void* bias, const uint8_t* mask, const void* const* a_ptrs,
                 const void* const* b_ptrs, void* Y, void* S_out, void* workspace, size_t ws_bytes, int M, int N,
                 int K, int R, const lf_routing* routing, int dtype, void* stream) {
-  int rc = lf_lora_xa(X, mask, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
+  int rc;
+  if (mask == nullptr && short_fwd(X, W, bias, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, dtype, stream, &rc)) return rc;
+  rc = lf_lora_xa(X, mask, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;
-  // (the rank-r pass is done with the workspace: the product's split contraction may have it)
+  behind_xa(workspace, ws_bytes, M, K, R, routing);
   return xw_sb_ws(X, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);
 }
 
 int lf_lora_fwd_seeded(const void* X, const void* W, const void* bias, uint8_t* mask_out, const void* const* a_ptrs,
                        const void* const* b_ptrs, void* Y, void* S_out, void* workspace, size_t ws_bytes, int M, int N,
                        int K, int R, const lf_routing* routing, uint64_t seed, int dtype, void* stream) {
-  int rc = lf_lora_xa_seeded(X, mask_out, a_ptrs, S_out, M, K, R, routing, seed, dtype, stream);
+  int rc = xa_seeded_ws(X, mask_out, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, seed, dtype, stream);
   if (rc != LF_OK) return rc;
+  behind_xa(workspace, ws_bytes, M, K, R, routing);
   return xw_sb_ws(X, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);
 }
 

@@ -65,6 +65,7 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
 int lf_launch_gemm_big(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int tile_rows, hipStream_t st);  // persistent tiles of 256 or 128 rows x 256 columns
 int lf_cu_count();
 int lf_pin_tile_cfg(int cfg);  // -1: automatic choice
+bool lf_tile_pinned();
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail);
 size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block);  // workspace of the split contraction for this product
 

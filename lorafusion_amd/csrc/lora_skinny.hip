@@ -30,76 +30,10 @@
 // its column's 4 rows).
 #include "lf_common.h"
 #include "act_math.h"
-#include "philox.h"
+#include "rank_common.h"
 #include <type_traits>
 
 namespace {
-
-constexpr int ROWS = 128;  // rows per workgroup = one routing block
-
-template <typename T> struct Mfma16;
-template <> struct Mfma16<__bf16> {
-  static __device__ __forceinline__ lf_f32x4 run(lf_u32x4 a, lf_u32x4 b, lf_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lf_bf16x8, a), __builtin_bit_cast(lf_bf16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t cvt(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
-};
-template <> struct Mfma16<_Float16> {
-  static __device__ __forceinline__ lf_f32x4 run(lf_u32x4 a, lf_u32x4 b, lf_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lf_f16x8, a), __builtin_bit_cast(lf_f16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t cvt(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
-};
-
-struct BlockInfo {
-  int rank, valid, seg;
-  float scale, p;
-};
-
-// Routing of the 128-row block `blk` (wave-uniform).
-__device__ __forceinline__ BlockInfo block_info(const LfSegTable& seg, int blk, int M) {
-  BlockInfo b;
-  if (seg.table == nullptr) {
-    b.rank = seg.rank[0];
-    b.valid = min(ROWS, M - blk * ROWS);
-    b.seg = 0;
-    b.scale = seg.scale;
-    b.p = seg.p;
-  } else {
-    b.rank = seg.table[3 * blk + 0];
-    b.valid = seg.table[3 * blk + 1];
-    const int fb = seg.table[3 * blk + 2];
-    int s = 0;
-    for (int i = 1; i < seg.n_seg; i++) s = (seg.first_block[i] == fb) ? i : s;
-    b.seg = s;
-    b.scale = seg.block_scale ? seg.block_scale[blk] : 1.f;
-    b.p = seg.block_p ? seg.block_p[blk] : 0.f;
-  }
-  return b;
-}
-
-// keep ? x : 0 on 8 packed 16-bit elements given their 8 mask bytes.
-__device__ __forceinline__ lf_u32x4 apply_mask8(lf_u32x4 x, lf_u32x2 m) {
-  lf_u32x4 r;
-#pragma unroll
-  for (int d = 0; d < 4; d++) {
-    const uint32_t mw = d < 2 ? m[0] : m[1];
-    const uint32_t two = (mw >> (16 * (d & 1))) & 0xffffu;           // bytes (2d, 2d+1)
-    const uint32_t sel = ((two & 0xffu) ? 0x0000ffffu : 0u) | ((two & 0xff00u) ? 0xffff0000u : 0u);
-    r[d] = x[d] & sel;
-  }
-  return r;
-}
-
-// Bit-packed keep-masks: element k of a row = bit k & 7 of byte k >> 3 of the row (K / 8 bytes per row).
-// The eight keep bytes (0/1 each, `lo` = the first four) as eight bits, and back: one multiply gathers / spreads four
-// single bits (no two partial products meet in one bit position, so nothing carries).
-__device__ __forceinline__ uint32_t pack_keep8(uint32_t lo, uint32_t hi) {
-  return ((lo * 0x01020408u) >> 24) | (((hi * 0x01020408u) >> 24) << 4);
-}
-__device__ __forceinline__ lf_u32x2 expand_keep8(uint32_t b) {
-  return lf_u32x2{((b & 0xfu) * 0x00204081u) & 0x01010101u, (((b >> 4) & 0xfu) * 0x00204081u) & 0x01010101u};
-}
 
 __device__ __forceinline__ lf_u32x4 tr_read8(const char* p, int pitch) {
   // 8 contraction elements (rows r..r+3 and r+4..r+7) of this lane's column
@@ -307,25 +241,24 @@ lora_xa_kernel(const T* __restrict__ X, const T* __restrict__ U, int64_t ldx, T*
             xv[b][u][i] = silu_mul8<T>(xv[b][u][i], uv[b][u][i]);
             if (row_real[i]) __builtin_nontemporal_store(xv[b][u][i], (lf_u32x4*)(act_out + erow[i] + s * 64));
           }
+          lf_u32x4 kept = xv[b][u][i];
           if constexpr (GEN) {
-            uint32_t klo, khi;
-            lf_keep8((uint64_t)(erow[i] + s * 64) >> 3, thr, seed_lo, seed_hi, klo, khi);
-            mv[b][u][i] = lf_u32x2{klo, khi};
+            uint32_t bits = 0xffu;
+            if (thr > 0) kept &= draw8((uint64_t)(erow[i] + s * 64) >> 3, thr, seed_lo, seed_hi, bits);   // (p = 0: everything is kept)
             if (mask_bits) {
               // this lane's eight bits are byte lg of the row's eight bytes of the step: the four lanes of a quad join
               // theirs (two cross-lane moves) and one of them stores the dword
-              uint32_t w = pack_keep8(klo, khi) << (8 * (lg & 3));
+              uint32_t w = bits << (8 * (lg & 3));
               w |= (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xB1, 0xf, 0xf, true);   // lanes 1 0 3 2
               w |= (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x4E, 0xf, 0xf, true);   // lanes 2 3 0 1
               if (row_real[i] && (lg & 3) == 0) *(uint32_t*)(mask_out + ((erow[i] + s * 64) >> 3)) = w;
             } else {
-              if (row_real[i]) *(lf_u32x2*)(mask_out + erow[i] + s * 64) = mv[b][u][i];
+              if (row_real[i]) *(lf_u32x2*)(mask_out + erow[i] + s * 64) = expand_keep8(bits);
             }
+          } else {
+            if (use_mask) kept = mask_bits ? kept & select8(mv[b][u][i][0]) : apply_mask8(kept, mv[b][u][i]);
           }
-          if constexpr (!GEN) {
-            if (use_mask && mask_bits) mv[b][u][i] = expand_keep8(mv[b][u][i][0]);
-          }
-          *(lf_u32x4*)(patch + (i >> 1) * 2048 + wr_off[i & 1]) = use_mask ? apply_mask8(xv[b][u][i], mv[b][u][i]) : xv[b][u][i];
+          *(lf_u32x4*)(patch + (i >> 1) * 2048 + wr_off[i & 1]) = kept;
         }
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -390,35 +323,6 @@ lora_xa_kernel(const T* __restrict__ X, const T* __restrict__ U, int64_t ldx, T*
 }
 
 // S[row][col] = cast( mult * sum_p part[p][row][col] ), zero for padded rows / rank columns.
-// Sum of `n` fp32x4 partials `stride` floats apart, in index order (deterministic).
-__device__ __forceinline__ lf_f32x4 sum_parts(const float* __restrict__ p, int64_t stride, int n) {
-  // Up to sixteen partials are requested before the first is added: these second stages are short launches whose
-  // time is the chain of memory round trips of one thread, and with four loads in flight a sum of sixteen was four
-  // round trips long (5 us for a few hundred KB).  The order of the additions is the index order either way.
-  lf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  int i = 0;
-  for (; i + 16 <= n; i += 16) {
-    lf_f32x4 t[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) t[k] = *(const lf_f32x4*)(p + (int64_t)(i + k) * stride);
-#pragma unroll
-    for (int k = 0; k < 16; k++) v += t[k];
-  }
-  if (i < n) {
-    lf_f32x4 t[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) t[k] = (i + k < n) ? *(const lf_f32x4*)(p + (int64_t)(i + k) * stride) : lf_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 16; k++) v += t[k];   // (adding the zeros beyond n changes nothing: x + 0 = x, and -0 cannot arise from a sum that started at +0)
-  }
-  return v;
-}
-template <typename T>
-__device__ __forceinline__ lf_u32x2 pack4(lf_f32x4 v) {
-  return lf_u32x2{(uint32_t)Mfma16<T>::cvt(v[0]) | ((uint32_t)Mfma16<T>::cvt(v[1]) << 16),
-                  (uint32_t)Mfma16<T>::cvt(v[2]) | ((uint32_t)Mfma16<T>::cvt(v[3]) << 16)};
-}
-
 template <typename T>
 __device__ __forceinline__ void reduce_rows_body(int bx, const float* __restrict__ part, T* __restrict__ out, int nparts, int M, int R,
                    int mode /*0: times 1/(1-p); 1: times scale*/, const LfSegTable seg) {
@@ -797,37 +701,7 @@ lora_da_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, int ma
 // every iteration (past the end: the last tile again, unconsumed), and drains the ring before the workgroup ends.
 // Rows past the end of a matrix are not clamped: every tile gets a buffer descriptor that ends where the matrix
 // ends, and lanes beyond it read zeros, which add nothing to a sum over rows.
-__device__ __forceinline__ uint32_t to_sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-
-__device__ __forceinline__ lf_u32x4 window_rsrc(const void* base, int64_t bytes) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  const int64_t n = bytes > 0xffffffffll ? 0xffffffffll : bytes;   // (never negative: a window starts inside its matrix)
-  return lf_u32x4{to_sgpr((uint32_t)a), to_sgpr((uint32_t)(a >> 32)) & 0xffffu, to_sgpr((uint32_t)n), 0x00020000u};
-}
-// one wave instruction: lane l fetches 16 bytes at window offset `voff` into LDS byte lds_addr + 16 l
-__device__ __forceinline__ void dma16(const lf_u32x4& rsrc, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
-}
-// one wave instruction: lane l fetches 4 bytes at window offset `voff` into LDS byte lds_addr + 4 l
-__device__ __forceinline__ void dma4(const lf_u32x4& rsrc, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
-}
 constexpr int da_mask_tile_bytes(int fmt) { return fmt == 1 ? ROWS * 64 : fmt == 2 ? ROWS * 8 : 0; }
-template <int N>
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// at most `groups` groups of G operations each may still be outstanding
-template <int G>
-__device__ __forceinline__ void wait_groups(int groups) {
-  switch (groups) {
-    case 0: wait_vm<0>(); break;
-    case 1: wait_vm<G>(); break;
-    case 2: wait_vm<2 * G>(); break;
-    case 3: wait_vm<3 * G>(); break;
-    default: wait_vm<4 * G>(); break;
-  }
-}
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Per-thread window offsets of a 128-row x 64-column tile of a 16-bit matrix with `ld` elements per row, in the LDS
 // layout the fragment readers expect (position p = i*256 + tid: row p>>3, slot p&7 holds granule slot ^ tile_key(row)).
 __device__ __forceinline__ void tile_voffs(uint32_t (&v)[4], int64_t ld, int tid) {
@@ -1204,11 +1078,7 @@ lora_dys_dyb_ring_kernel(const T* __restrict__ dY, const T* __restrict__ S, floa
     }
 }
 
-int rt_of(int R) { return R <= 16 ? 1 : R <= 32 ? 2 : R <= 64 ? 4 : 8; }
-
 }  // namespace
-
-static int n_row_blocks(int M, const LfSegTable& seg) { return seg.table ? seg.n_blocks : (M + ROWS - 1) / ROWS; }
 
 // Split of a length-`len` axis into slices (multiples of 64) so that blocks * split fills the
 // chip; `min_split` bounds the slice length from above.
@@ -1226,10 +1096,6 @@ static int pick_tiles_per_wg(int max_t, int slots, Count count) {
     if (cost <= best_cost) { best_cost = cost; best = t; }
   }
   return best;
-}
-static int lds_slots(int smem_bytes) {
-  const int per_cu = (160 * 1024) / smem_bytes;
-  return 256 * (per_cu > 0 ? per_cu : 1);
 }
 static int dys_smem(int rt) { return 2 * TILE_BYTES + ROWS * (rt * 32 + 32) + 2 * 64 * (rt * 32 + 32); }
 // Shape of a dys_dyb launch: tiles per workgroup (<= the kernel's TPW), row blocks per chunk, chunks of the longest
@@ -1352,7 +1218,23 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
   return best;
 }
 
-size_t lf_xa_workspace(int, int, int, const LfSegTable&) { return 0; }
+// (lora_stream.hip)
+size_t lf_xa_stream_workspace(int, int, int, const LfSegTable&);
+int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, void*, float*, int, int, int, const LfSegTable&, int, hipStream_t);
+
+// The sliced pass (lora_stream.hip) in place of lora_xa_kernel: above 32 rank columns, where that kernel reads the adapter matrix
+// once per 16-64 rows through wave-private patches and has too few workgroups (1000 x 4096, rank 64, keep bits read: 22.5 ->
+// 10.1 us; 3000 x 5120, rank 128: 67 -> 19; 8576 x 28672, rank 64: 201 -> 148; 8576 x 8192: 40.6 -> 38.9), and with a
+// keep-mask up to 1024 rows, where drawing it on a few compute units is what takes the time (300 x 4096, rank 16: -2.5 us
+// drawn, level when read).  Elsewhere the second stage costs more than the slices give (4096 x 4096, rank 16: 7.9 against
+// 9.6 us).  The same choice for every mask format, drawn or read: S does not depend on how the mask came.
+bool lf_xa_streams(int M, int R, bool masked, const LfSegTable& seg) {
+  const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
+  return R > 32 || (masked && rows <= 1024);
+}
+size_t lf_xa_workspace(int M, int K, int R, const LfSegTable& seg) {
+  return lf_xa_streams(M, R, true, seg) ? lf_xa_stream_workspace(M, K, R, seg) : 0;
+}
 
 template <typename T, int RT>
 static int xa_launch(const void* X, const void* U, int64_t ldx, void* act_out, const uint8_t* mask, uint8_t* mask_out, int mask_bits,
@@ -1388,7 +1270,7 @@ static int xa_impl(const void* X, const void* U, int64_t ldx, void* act_out, con
 // U != nullptr: X and U are the gate and up halves (rows ldx elements apart) and the pass's input
 // round16(round16(silu(X)) * U) is written to act_out [rows, K]; otherwise X [rows, K] is dense.
 int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const uint8_t* mask, uint8_t* mask_out, int mask_bits,
-                 uint64_t seed, void* S, int M, int K, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
+                 uint64_t seed, void* S, void* ws, size_t ws_bytes, int M, int K, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
   if (!X || !S || M <= 0 || K <= 0) return LF_EINVAL;
   if (K % 128 != 0 || R % 16 != 0 || R <= 0 || R > LF_MAX_RANK) return LF_ESHAPE;
   if (seg.table && seg.block_size_m != ROWS) return LF_ESHAPE;
@@ -1398,6 +1280,9 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
     if (ldx < K || ldx % 8 != 0 || (((uintptr_t)X | (uintptr_t)U | (uintptr_t)act_out) & 15) != 0) return LF_ESHAPE;
   } else {
     ldx = K;
+    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_streams(M, R, mask != nullptr || mask_out != nullptr, seg))
+      return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, seg) ? (float*)ws : nullptr, M, K,
+                                 R, seg, dtype, st);
   }
   if (dtype == LF_BF16) return xa_impl<__bf16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);
   if (dtype == LF_F16) return xa_impl<_Float16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);

@@ -1,0 +1,410 @@
+// Products of a long streamed operand with a matrix of few rows, split along the contraction, for gfx950.
+//
+//   D[row][c] = sum_k keep(row, k) * P[row][k] * Q[c][k]       P: many rows, read once; Q: at most 128 rows
+//
+// Two uses:
+//   xa      : P = X, Q = A_i:             S = drop(X) A^T     (seeded_dropout + `masked_scaled_x @ lora_a.T`,
+//             lorafusion/ops/lora_v1.py:111-119; the multi-adapter product, multi_lora.py:481-513)
+//   forward : P = the rows of W followed by the rows of A, Q = X of at most 128 rows: one pass over the weight gives the
+//             base product and the rank-r product of a short batch; a second kernel adds the slices and forms
+//             Y = X W^T + scale (X A^T) B^T + bias (fused_lora_xw_sb, triton_ops/fused_lora_xw_sb.py:74-206)
+//
+// Both are bound by the stream of P (the forward of 8 rows moves 34 MB of weights for 0.3 GFLOP), so what counts is how
+// many bytes the chip has on order.  A workgroup (4 waves) owns 64 rows of P and a slice of K: the slices are what
+// gives every compute unit two workgroups when P has few rows, or when Q is so tall that a workgroup which walks all of K
+// (lora_xa_kernel) would read it once per 16 rows of P.  P (64 rows x 64 columns, 8 KB), Q (up to 16 KB) and the keep
+// bits of a step arrive by direct-to-LDS loads in a ring of NS stages; a wave reads the rows it loaded itself, the keep
+// bits are applied to the fragment in registers (every element of P belongs to exactly one lane), so the only thing the
+// waves share is Q and the one barrier of a step.
+#include "lf_common.h"
+#include "act_math.h"
+#include "rank_common.h"
+
+namespace {
+
+constexpr int SROWS = 64;                                              // rows of P per workgroup, 16 per wave
+constexpr int st_q_bytes(int rt) { return rt == 1 ? 4096 : rt * 2048; }   // rank 16: four rows per wave, padded to a load's 1 KB
+constexpr int st_bytes(int rt, int mode) { return SROWS * 128 + st_q_bytes(rt) + (mode == 2 ? 1024 : mode == 1 ? 4096 : 0); }
+constexpr int st_ns(int rt, int mode) { return mode == 1 ? (rt <= 2 ? 5 : rt == 4 ? 4 : 2) : (rt <= 2 ? 6 : rt == 4 ? 4 : 3); }   // stages: two workgroups per CU
+constexpr int st_smem(int rt, int mode) { return st_ns(rt, mode) * st_bytes(rt, mode) + (mode == 3 ? 4096 : 0); }
+
+struct StreamArgs {
+  const void* p0;        // rows [0, n0) of P
+  const void* p1;        // rows [n0, n0 + n1) (forward: the adapter's rows), or nullptr
+  int n0, n1, K, n_slices;
+  int folded;            // no memory for the slices' sums: one workgroup walks all slices and adds their sums in the order the second stage would
+  const uint8_t* mask;   // keep-mask read: bits [rows, K / 8] (MODE 2) or bytes [rows, K] (MODE 1)
+  uint8_t* mask_out;     //           or drawn and written (MODE 3), as bits or as bytes
+  int mask_bytes;
+  uint32_t seed_lo, seed_hi;
+  float* part;           // xa: [slice][row][R]; forward: [slice][m][pitch]; nullptr (xa, one slice or folded): S is written directly
+  int64_t pitch;
+  void* S;
+  int M, R;              // xa: rows given, columns of S.  forward: M = rows of Q
+  const void* q;         // forward: X [M, K]
+};
+
+// grid (64-row groups of P, slices of K).  MODE: 0 no keep-mask, 1 keep bytes read, 2 keep bits read, 3 mask drawn and written.
+// FWD: Q = X (the second use above), D is stored transposed, [m][row of P].
+template <typename T, int RT, int MODE, bool FWD>
+__global__ void __launch_bounds__(256, 2)
+lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
+  constexpr int NS = st_ns(RT, MODE), STAGE = st_bytes(RT, MODE), QB = st_q_bytes(RT);
+  constexpr int NQ = RT == 1 ? 1 : RT / 2;              // loads of Q per wave and step
+  constexpr int G = 2 + NQ + (MODE == 1 || MODE == 2 ? 1 : 0);       // loads per wave and step
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int tid = threadIdx.x, lane = tid & 63, wave = to_sgpr(tid >> 6);
+  const int li = lane & 15, qq = lane >> 4;
+  const int grp = blockIdx.x, sl = blockIdx.y, K = a.K;
+  // this slice (or all of them): whole pairs of steps (128 columns), balanced
+  const int np = K / 128;
+  auto slice_begin = [&](int i) { return (int)((int64_t)np * i / a.n_slices); };
+  const int k_lo = a.folded ? 0 : slice_begin(sl), k_hi = a.folded ? np : slice_begin(sl + 1);
+  const int nsteps = 2 * (k_hi - k_lo);
+
+  int row0 = grp * SROWS, rows_all = a.n0;   // within p0 or p1
+  const char* pb = (const char*)a.p0;
+  const char* qb = (const char*)a.q;
+  int q_rows = a.M;
+  BlockInfo bi{};
+  if constexpr (FWD) {
+    if (row0 >= a.n0) { row0 -= a.n0; rows_all = a.n1; pb = (const char*)a.p1; }
+  } else {
+    bi = block_info(seg, row0 / ROWS, a.M);
+    qb = (const char*)seg.ptr[bi.seg];
+    q_rows = bi.rank;
+  }
+  const bool use_mask = MODE > 0 && bi.p > 0.f;   // (rows of a block without dropout keep everything)
+  const uint32_t thr = lf_keep_threshold(bi.p);
+
+  // loader: 8 lanes cover the 128 bytes of a row; granule g of row r goes to slot g ^ ((r >> 1) & 7)
+  const int lrow = lane >> 3, slot = lane & 7;
+  uint32_t pv[2], qv[NQ], mv = 0;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int r = i * 8 + lrow;
+    pv[i] = (uint32_t)(((int64_t)(wave * 16 + r) * K) * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
+  }
+#pragma unroll
+  for (int i = 0; i < NQ; i++) {
+    // rank 16: a wave fetches four rows (lanes 0..31), else eight rows per load
+    const int r = RT == 1 ? wave * 4 + (lrow & 3) : (wave * NQ + i) * 8 + lrow;
+    qv[i] = (uint32_t)(((int64_t)r * K) * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
+    if (RT == 1 && lane >= 32) qv[i] = 0xffffff00u;   // beyond the window: nothing is fetched
+  }
+  if constexpr (MODE == 1) mv = (uint32_t)((wave * 16 + (lane >> 2)) * (int64_t)K + (lane & 3) * 16);
+  if constexpr (MODE == 2) mv = lane < 32 ? (uint32_t)((wave * 16 + (lane >> 1)) * (K >> 3) + (lane & 1) * 4) : 0xffffff00u;
+
+  const int64_t k0 = (int64_t)k_lo * 128;
+  pb += ((int64_t)row0 * K + k0) * 2;
+  int64_t pleft = ((int64_t)(rows_all - row0) * K - k0) * 2;
+  qb += k0 * 2;
+  int64_t qleft = ((int64_t)q_rows * K - k0) * 2;
+  const char* mb = (const char*)a.mask + (((int64_t)row0 * K + k0) >> (MODE == 2 ? 3 : 0));
+  int64_t mleft = ((int64_t)(rows_all - row0) * K - k0) >> (MODE == 2 ? 3 : 0);
+  int ord = 0, ist = 0;   // steps ordered so far (behind the last one: that one again, unconsumed), stage of the next
+  auto issue = [&]() {
+    const uint32_t st = lds0 + ist * STAGE;
+    const lf_u32x4 rp = window_rsrc(pb, pleft), rq = window_rsrc(qb, qleft);
+#pragma unroll
+    for (int i = 0; i < 2; i++) dma16(rp, pv[i], st + wave * 2048 + i * 1024);
+#pragma unroll
+    for (int i = 0; i < NQ; i++) dma16(rq, qv[i], st + SROWS * 128 + (wave * NQ + i) * 1024);
+    if constexpr (MODE == 1) dma16(window_rsrc(mb, mleft), mv, st + SROWS * 128 + QB + wave * 1024);
+    if constexpr (MODE == 2) dma4(window_rsrc(mb, mleft), mv, st + SROWS * 128 + QB + wave * 256);
+    ist = ist + 1 == NS ? 0 : ist + 1;
+    if (++ord < nsteps) {
+      pb += 128, pleft -= 128, qb += 128, qleft -= 128;
+      if constexpr (MODE == 1) mb += 64, mleft -= 64;
+      if constexpr (MODE == 2) mb += 8, mleft -= 8;
+    }
+  };
+#pragma unroll 1
+  for (int i = 0; i < NS - 1; i++) issue();
+
+  lf_f32x4 acc[RT], sum[RT];
+#pragma unroll
+  for (int c = 0; c < RT; c++) acc[c] = sum[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
+  int fold_at = 2 * slice_begin(1), fold_next = 2;   // folded: first step of the next slice
+  const int key = (li >> 1) & 7;
+  char* bits_buf = lds + NS * STAGE + wave * 1024;   // MODE 3: 16 rows x 64 bytes = eight steps of this wave's keep bits
+  const int64_t my_row = row0 + wave * 16 + li;
+  const uint64_t ctr0 = (uint64_t)(my_row * K + k0) >> 3;
+
+  int cst = 0;
+  for (int s = 0; s < nsteps; s++) {
+    wait_groups<G>(NS - 2);
+    ring_barrier();   // this step's stage has landed for every wave; everyone is done with the stage refilled next
+    issue();
+    if (!FWD && a.folded && s == fold_at) {
+#pragma unroll
+      for (int c = 0; c < RT; c++) sum[c] += acc[c], acc[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
+      fold_at = 2 * slice_begin(fold_next++);
+    }
+    const char* x = lds + cst * STAGE + wave * 2048;
+    const char* q = lds + cst * STAGE + SROWS * 128;
+    lf_u32x4 xf[2], qf[2][RT];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int fo = ((h * 4 + qq) ^ key) << 4;
+      xf[h] = *(const lf_u32x4*)(x + li * 128 + fo);
+#pragma unroll
+      for (int c = 0; c < RT; c++)
+        qf[h][c] = *(const lf_u32x4*)(RT == 1 ? q + (li >> 2) * 1024 + (li & 3) * 128 + fo : q + (c * 16 + li) * 128 + fo);
+    }
+    if constexpr (MODE == 1) {
+      if (use_mask) {
+        const char* mt = lds + cst * STAGE + SROWS * 128 + QB + wave * 1024;
+#pragma unroll
+        for (int h = 0; h < 2; h++) xf[h] = apply_mask8(xf[h], *(const lf_u32x2*)(mt + li * 64 + (h * 4 + qq) * 8));
+      }
+    }
+    if constexpr (MODE == 2) {
+      if (use_mask) {
+        const char* mt = lds + cst * STAGE + SROWS * 128 + QB + wave * 256;
+#pragma unroll
+        for (int h = 0; h < 2; h++) xf[h] &= select8(*(const uint8_t*)(mt + li * 8 + h * 4 + qq));
+      }
+    }
+    if constexpr (MODE == 3) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        uint32_t bits = 0xffu;
+        if (use_mask && thr > 0) xf[h] &= draw8(ctr0 + (uint64_t)(s * 8 + h * 4 + qq), thr, a.seed_lo, a.seed_hi, bits);
+        bits_buf[li * 64 + (s & 7) * 8 + h * 4 + qq] = (char)bits;
+        if (a.mask_bytes && my_row < rows_all) *(lf_u32x2*)(a.mask_out + my_row * K + k0 + s * 64 + (h * 4 + qq) * 8) = expand_keep8(bits);
+      }
+      if (!a.mask_bytes && ((s & 7) == 7 || s + 1 == nsteps)) {
+        // (same-wave LDS traffic is ordered.)  Lane l: row l>>2, 16-byte piece l&3 = two steps
+        const int r = lane >> 2, pc = lane & 3, first = s & ~7;
+        const lf_u32x4 v = *(const lf_u32x4*)(bits_buf + r * 64 + pc * 16);
+        const int64_t gr = row0 + wave * 16 + r;
+        if (gr < rows_all && first + 2 * pc <= s) __builtin_nontemporal_store(v, (lf_u32x4*)(a.mask_out + ((gr * K + k0) >> 3) + first * 8 + pc * 16));
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int c = 0; c < RT; c++)
+        acc[c] = FWD ? Mfma16<T>::run(qf[h][c], xf[h], acc[c]) : Mfma16<T>::run(xf[h], qf[h][c], acc[c]);
+    cst = cst + 1 == NS ? 0 : cst + 1;
+  }
+  wait_vm<0>();   // the unconsumed loads behind the last step must not land in another workgroup's LDS
+  if constexpr (FWD) {
+    // lane: row li of P, rows 4 qq + e of Q
+    if (row0 + wave * 16 + li < rows_all) {
+      float* po = a.part + (int64_t)sl * a.M * a.pitch + grp * SROWS + wave * 16 + li;
+#pragma unroll
+      for (int c = 0; c < RT; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int m = c * 16 + qq * 4 + e;
+          if (m < a.M) po[(int64_t)m * a.pitch] = acc[c][e];
+        }
+    }
+  } else {
+    // lane: column li of each 16, rows 4 qq + e of the wave
+    const float mult = use_mask ? 1.f / (1.f - bi.p) : 1.f;
+#pragma unroll
+    for (int c = 0; c < RT; c++) acc[c] = sum[c] + acc[c];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int64_t row = row0 + wave * 16 + qq * 4 + e;
+      if (row < rows_all) {
+        const bool real = (int)(row & (ROWS - 1)) < bi.valid;
+#pragma unroll
+        for (int c = 0; c < RT; c++) {
+          const int col = c * 16 + li;
+          if (c * 16 < a.R) {
+            if (a.part != nullptr) a.part[((int64_t)sl * rows_all + row) * a.R + col] = acc[c][e];
+            else ((uint16_t*)a.S)[row * a.R + col] = real && col < bi.rank ? Mfma16<T>::cvt(acc[c][e] * mult) : (uint16_t)0;
+          }
+        }
+      }
+    }
+  }
+}
+
+// Second stage of a sliced xa: S = cast(1/(1-p) * sum of the slices), zero in padded rows and beyond the rank.
+template <typename T>
+__global__ void __launch_bounds__(256)
+stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_slices, int M, int R, int dropout, const LfSegTable seg) {
+  const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
+  const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (idx >= rows * R) return;
+  const int row = (int)(idx / R), col = (int)(idx % R);
+  const BlockInfo bi = block_info(seg, row / ROWS, M);
+  lf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (row % ROWS < bi.valid && col < bi.rank) {
+    v = sum_parts(part + idx, rows * R, n_slices);
+    if (dropout && bi.p > 0.f) v *= 1.f / (1.f - bi.p);
+  }
+  *(lf_u32x2*)((uint16_t*)S + idx) = pack4<T>(v);
+}
+
+// Second stage of the short forward.  grid (64-column tiles of Y, groups of 16 rows), 16 lanes per row.  A short launch is
+// as long as its chain of memory round trips: the slices of Y and the rows of B are requested before the S rows that the
+// workgroup needs are added up and rounded (each workgroup its own, r <= 128 columns, from L2; the first column tile
+// stores them).
+template <typename T>
+__global__ void __launch_bounds__(256)
+short_fwd_finish_kernel(const float* __restrict__ part, int64_t pitch, int n_slices, int M, int N, int rank, int R, const T* __restrict__ B,
+                        float scale, const uint16_t* __restrict__ bias, T* __restrict__ Y, T* __restrict__ S) {
+  __shared__ float sv[16][LF_MAX_RANK];
+  const int tid = threadIdx.x, m0 = blockIdx.y * 16;
+  const int mi = tid >> 4, m = m0 + mi, col = blockIdx.x * 64 + (tid & 15) * 4;   // (N % 128 == 0: no column beyond N)
+  lf_f32x4 y = {0.f, 0.f, 0.f, 0.f};
+  lf_u32x4 b0[4];
+  if (m < M) {
+    y = sum_parts(part + (int64_t)m * pitch + col, (int64_t)M * pitch, n_slices);
+#pragma unroll
+    for (int c = 0; c < 4; c++) b0[c] = *(const lf_u32x4*)(B + (int64_t)(col + c) * rank);
+  }
+  for (int o = tid; o < 4 * R; o += 256) {   // four columns of one row each
+    const int r = o / (R / 4), j = o % (R / 4) * 4, sm = m0 + r;
+    lf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (sm < M && j < rank) v = sum_parts(part + (int64_t)sm * pitch + N + j, (int64_t)M * pitch, n_slices);
+    const lf_u32x2 h = pack4<T>(v);
+#pragma unroll
+    for (int e = 0; e < 4; e++) sv[r][j + e] = (float)(T)v[e];
+    if (blockIdx.x == 0 && sm < M) *(lf_u32x2*)((uint16_t*)S + (int64_t)sm * R + j) = h;
+  }
+  __syncthreads();
+  if (m >= M) return;
+  lf_f32x4 t = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < rank; j += 8) {
+    lf_u32x4 bn[4];
+    if (j + 8 < rank) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) bn[c] = *(const lf_u32x4*)(B + (int64_t)(col + c) * rank + j + 8);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      float f[8];
+      unpack8<T>(b0[c], f);
+#pragma unroll
+      for (int e = 0; e < 8; e++) t[c] = __builtin_fmaf(f[e], sv[mi][j + e], t[c]);
+      b0[c] = bn[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    y[c] += t[c] * scale;
+    if (bias != nullptr) y[c] += (float)__builtin_bit_cast(T, bias[col + c]);
+  }
+  *(lf_u32x2*)((uint16_t*)Y + (int64_t)m * N + col) = pack4<T>(y);
+}
+
+// Slices of K.  Compute units share the workgroups evenly or not at all: 65 groups in 4 slices are 260 workgroups, and four
+// of the 256 compute units take twice as long as the rest.  So: the count (at most sixteen, none shorter than four
+// steps) with the shortest modelled time -- the busiest compute unit's share of the stream (a full walk of K = 4096 by one
+// workgroup takes 22 us), the partial sums written and read back, and the second stage where one slice needs none.
+// 6 x 4096 x 4096 (65 groups), first and second stage: 3 slices 12.0 us, 4: 13.3, 7: 12.5, 8: 14.0; 8576 rows, K = 28672,
+// rank 64 (134 groups): 1 slice 216 us, 3: 157, 4: 170, 7: 147.
+int slices_for(int64_t groups, int K, double partial_bytes, bool second_stage) {
+  const int most = K / 256 < 1 ? 1 : K / 256 > 16 ? 16 : K / 256;
+  int best = 1;
+  double best_cost = 1e300;
+  for (int n = 1; n <= most; n++) {
+    const double share = (double)((groups * n + 255) / 256) / n;
+    const double cost = share * K * 0.0054 + n * partial_bytes / 1.5e6 + (n > 1 || second_stage ? 4.0 : 0.0);
+    if (cost < best_cost) { best_cost = cost; best = n; }
+  }
+  return best;
+}
+
+template <typename T, int RT, int MODE, bool FWD>
+int stream_launch(const StreamArgs& a, const LfSegTable& seg, int groups, hipStream_t st) {
+  auto kern = lora_stream_kernel<T, RT, MODE, FWD>;
+  constexpr int SMEM = st_smem(RT, MODE);
+  static_assert(2 * SMEM <= 160 * 1024, "two workgroups per CU");
+  static LfLdsFlags lds_ok;
+  if (!lf_allow_lds(kern, SMEM, lds_ok)) return LF_ELAUNCH;
+  return lf_launch(kern, dim3(groups, a.folded ? 1 : a.n_slices), dim3(256), SMEM, st, a, seg);
+}
+template <typename T, int RT>
+int stream_mode(const StreamArgs& a, const LfSegTable& seg, int groups, hipStream_t st) {
+  if (a.q != nullptr) return stream_launch<T, RT, 0, true>(a, seg, groups, st);
+  if (a.mask_out != nullptr) return stream_launch<T, RT, 3, false>(a, seg, groups, st);
+  if (a.mask != nullptr) return a.mask_bytes ? stream_launch<T, RT, 1, false>(a, seg, groups, st) : stream_launch<T, RT, 2, false>(a, seg, groups, st);
+  return stream_launch<T, RT, 0, false>(a, seg, groups, st);
+}
+template <typename T>
+int stream_rt(const StreamArgs& a, const LfSegTable& seg, int cols, int groups, hipStream_t st) {
+  switch (rt_of(cols)) {
+    case 1: return stream_mode<T, 1>(a, seg, groups, st);
+    case 2: return stream_mode<T, 2>(a, seg, groups, st);
+    case 4: return stream_mode<T, 4>(a, seg, groups, st);
+    default: return stream_mode<T, 8>(a, seg, groups, st);
+  }
+}
+
+template <typename T>
+int xa_stream_impl(StreamArgs a, const LfSegTable& seg, float* ws, hipStream_t st) {
+  const int groups = (a.n0 + SROWS - 1) / SROWS;
+  a.folded = a.n_slices > 1 && ws == nullptr;
+  a.part = a.n_slices > 1 ? ws : nullptr;
+  int rc = stream_rt<T>(a, seg, a.R, groups, st);
+  if (rc != LF_OK || a.part == nullptr) return rc;
+  const int64_t n4 = ((int64_t)a.n0 * a.R + 3) / 4;
+  return lf_launch((stream_reduce_kernel<T>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const float*)ws, (T*)a.S, a.n_slices, a.M,
+                   a.R, (a.mask != nullptr || a.mask_out != nullptr) ? 1 : 0, seg);
+}
+
+}  // namespace
+
+static int64_t xa_rows_of(int M, const LfSegTable& seg) { return seg.table ? (int64_t)seg.n_blocks * ROWS : M; }
+
+int lf_xa_stream_slices(int M, int K, int R, const LfSegTable& seg) {
+  const int64_t groups = (xa_rows_of(M, seg) + SROWS - 1) / SROWS;
+  return slices_for(groups, K, (double)xa_rows_of(M, seg) * R * sizeof(float), false);
+}
+
+size_t lf_xa_stream_workspace(int M, int K, int R, const LfSegTable& seg) {
+  const int n = lf_xa_stream_slices(M, K, R, seg);
+  return n > 1 ? (size_t)n * xa_rows_of(M, seg) * R * sizeof(float) : 0;
+}
+
+// ws == nullptr: no room for the slices' sums (the result is the same, bit for bit)
+int lf_launch_xa_stream(const void* X, const uint8_t* mask, uint8_t* mask_out, int mask_bits, uint64_t seed, void* S, float* ws, int M, int K, int R,
+                        const LfSegTable& seg, int dtype, hipStream_t st) {
+  StreamArgs a{};
+  a.p0 = X; a.n0 = (int)xa_rows_of(M, seg); a.K = K; a.n_slices = lf_xa_stream_slices(M, K, R, seg);
+  a.mask = mask; a.mask_out = mask_out; a.mask_bytes = !mask_bits; a.seed_lo = (uint32_t)seed; a.seed_hi = (uint32_t)(seed >> 32);
+  a.S = S; a.M = M; a.R = R;
+  return dtype == LF_BF16 ? xa_stream_impl<__bf16>(a, seg, ws, st) : xa_stream_impl<_Float16>(a, seg, ws, st);
+}
+
+// ---- forward of a short batch (one adapter, no keep-mask)
+static int short_pitch(int N, int rank) { return N + (rank + 15) / 16 * 16; }
+static int short_groups(int N, int rank) { return N / SROWS + (rank + SROWS - 1) / SROWS; }
+
+// Up to 64 rows the pass reads W at 4-5 TB/s where tiles of 64 columns leave most of the chip idle (6 x 4096 x 4096: 23.7 ->
+// 12.0 us, 64 rows: 24.9 -> 14.5; 6 x 4096 over 14336: 38.2 -> 24.0).  Up to 128 rows a workgroup fetches twice as many bytes
+// of X from L2 as of W: still ahead where the output is too narrow to fill the chip with tiles (128 x 4096 x 4096: 25.3 ->
+// 20.9), behind beyond that (128 x 14336 x 4096: 33.6 -> 45.3).
+bool lf_short_fwd_applies(int M, int N) { return M <= 64 || (M <= 128 && N <= 4096); }
+
+static int short_slices(int M, int N, int K, int rank) {
+  return slices_for(short_groups(N, rank), K, (double)M * short_pitch(N, rank) * sizeof(float), true);
+}
+size_t lf_short_fwd_workspace(int M, int N, int K, int rank) {
+  return (size_t)short_slices(M, N, K, rank) * M * short_pitch(N, rank) * sizeof(float);
+}
+
+template <typename T>
+static int short_fwd_impl(const StreamArgs& a, const LfSegTable& seg, const void* B, float scale, const void* bias, void* Y, hipStream_t st) {
+  int rc = stream_rt<T>(a, seg, a.M, short_groups(a.n0, a.n1), st);
+  if (rc != LF_OK) return rc;
+  return lf_launch((short_fwd_finish_kernel<T>), dim3(a.n0 / 64, (a.M + 15) / 16), dim3(256), 0, st, (const float*)a.part, a.pitch,
+                   a.n_slices, a.M, a.n0, a.n1, a.R, (const T*)B, scale, (const uint16_t*)bias, (T*)Y, (T*)a.S);
+}
+
+int lf_launch_short_fwd(const void* X, const void* W, const void* A, const void* B, float scale, const void* bias, void* Y, void* S, void* ws,
+                        int M, int N, int K, int rank, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
+  StreamArgs a{};
+  a.p0 = W; a.p1 = A; a.n0 = N; a.n1 = rank; a.K = K; a.n_slices = short_slices(M, N, K, rank);
+  a.part = (float*)ws; a.pitch = short_pitch(N, rank); a.S = S; a.M = M; a.R = R; a.q = X;
+  return dtype == LF_BF16 ? short_fwd_impl<__bf16>(a, seg, B, scale, bias, Y, st) : short_fwd_impl<_Float16>(a, seg, B, scale, bias, Y, st);
+}
