@@ -175,8 +175,7 @@ gemm_big_kernel(const LfGemmParams p, const LfSegTable seg) {
   // its neighbour -- identical values, since both walk K from the same start -- and no load or store needs a guard.
   struct Tile { int m0, n0, kstart; };
   auto tile_of = [&](int it) __attribute__((always_inline)) {
-    int pid = it * G + wg;
-    if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+    const int pid = lf_xcd_order(it * G + wg, total);
     const int GROUP_M = p.group_m;   // tile rows per group: 8, or 2 for a long K over few tile columns (see the launcher)
     const int width = GROUP_M * p.grid_n;
     const int group = pid / width;

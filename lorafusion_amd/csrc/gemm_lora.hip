@@ -119,10 +119,11 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
   const int wm = wave / NWN, wn = wave % NWN;
   const int l16 = lane & 15, kg = lane >> 4;  // row / column within a 16x16 block, group of 8 contraction elements
 
-  // ---- tile mapping: XCD-aware (consecutive tiles stay on one XCD's L2) + grouped along M
-  int pid = blockIdx.x;
+  // ---- tile mapping: XCD-aware (consecutive tiles, slice by slice of a split contraction, stay on one XCD's L2) + grouped along M
   const int total = p.grid_m * p.grid_n;
-  if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+  int pid = lf_xcd_order((int)(blockIdx.y * gridDim.x + blockIdx.x), total * (int)gridDim.y);
+  const int slice = p.ksplit > 1 ? pid / total : 0;
+  pid -= slice * total;
   constexpr int GROUP_M = 8;
   const int width = GROUP_M * p.grid_n;
   const int group = pid / width;
@@ -139,7 +140,7 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
   // run on one XCD, stay aligned in K and meet each other's lines in the L2 (1.5 % faster at
   // 8192x4096x4096 than an offset by row + column).
   // (split contraction: this workgroup's share of the K steps is [kbeg, kbeg + nk); an even count, like K / BK)
-  const int kbeg = p.ksplit > 1 ? (int)blockIdx.y * p.ks_steps : 0;
+  const int kbeg = slice * p.ks_steps;
   const int nk = p.ksplit > 1 ? min(p.ks_steps, p.K / BK - kbeg) : p.K / BK;
   const int kstart = (2 * (pid_n & LF_STAG)) % nk;
 
@@ -628,7 +629,7 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
   // the 64 banks once, so the 16 rows that write together land on different banks.
   if (p.ksplit > 1) {
     // split contraction: the fp32 sums of this slice, 16 bytes per lane (row l16 of a block, columns kg*4 .. +3)
-    float* __restrict__ part = p.ks_ws + (int64_t)blockIdx.y * p.M * p.N;
+    float* __restrict__ part = p.ks_ws + (int64_t)slice * p.M * p.N;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -935,7 +936,7 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
     if (cfg == 8) return lf_launch_gemm_big(q, seg, nn, dtype, 128, st);
     if (dtype != LF_BF16 && dtype != LF_F16) return (int)LF_EINVAL;
     LfGemmParams r = q;
-    r.ksplit = 1;
+    r.ksplit = 1, r.ks_steps = 0;
     if (planned && r.ks_ws != nullptr && ((uintptr_t)r.ks_ws & 15) == 0) {   // (a pinned tile configuration stays as pinned)
       const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, seg.table != nullptr ? seg.block_size_m : 0);
       if (ks.n > 1 && (size_t)ks.n * r.M * r.N * sizeof(float) <= r.ks_ws_bytes) { cfg = ks.cfg; r.ksplit = ks.n; r.ks_steps = ks.steps; }
