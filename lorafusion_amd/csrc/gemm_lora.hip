@@ -308,7 +308,7 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
     // Bit-packed keep-mask: the dword that holds the lane's four columns of each accumulator block (element n of a
     // mask row = bit n & 7 of byte n >> 3).  Requested with the operands of the first chunk where the registers allow
     // (up to 16 blocks per wave), else in one batch behind the MFMAs.
-    constexpr int GI = TM * TN <= 16 ? TM : (16 / TN > 0 ? 16 / TN : 1);   // block rows per batch of mask words
+    constexpr int GI = TM * TN <= 16 ? TM : (TM % (16 / TN) == 0 ? 16 / TN : 2);   // block rows per batch of mask words
     constexpr bool BITS_EARLY = GI == TM;
     static_assert(TM % GI == 0, "whole batches");
     uint32_t mw[GI][TN];
@@ -741,118 +741,133 @@ int launch_dtype(const LfGemmParams& p, const LfSegTable& seg, int cfg, hipStrea
     case 4: return launch_cfg<T, 128, 128, 64, 64, NN, LF_NSTAGE>(p, seg, st);
     case 5: return launch_cfg<T, 64, 64, 32, 32, NN, LF_NSTAGE_SMALL>(p, seg, st);
     case 6: return launch_cfg<T, 128, 64, 64, 32, NN, 9>(p, seg, st);
+    case 9: return launch_cfg<T, 192, 128, 96, 64, NN, 7>(p, seg, st);
     default: return LF_EINVAL;
   }
 }
 
 }  // namespace
 
-// Tile choice from a measured cost model.  A launch runs in "rounds" of resident workgroups
-// (256 CUs x workgroups per CU).  Costs are microseconds measured at K = 4096: the first round
-// costs lat0 + first_b * fill^2 (a lone tile per CU runs latency bound at boost clock, a full round
-// is power limited), every further round next_a + next_b * fill, where fill is the occupied
-// fraction of the round's slots.  For another K every term scales with K / 4096 except kRamp
-// microseconds of lat0 (launch, first loads, epilogue), which a launch pays once whatever its K:
-// a second launch for left-over rows pays off at a long K and does not at a short one.
-struct TileCand { int cfg, bm, bn, slots; double lat0, first_b, next_a, next_b; };
-static const TileCand kCands[] = {
-    {7, 256, 256, 256, 70.0, 40.0, 50.0, 30.0},   // persistent, 4 waves of 128x128 (gemm_big.hip): rounds = tiles per workgroup
-    {1, 256, 256, 256, 66.0, 50.0, 44.0, 60.0},   // 8 waves, 128x64 per wave
-    {3, 128, 256, 256, 48.0, 28.0, 28.0, 38.0},   // 8 waves, 64x64 per wave
-    {4, 128, 128, 512, 38.0, 47.0, 5.0, 70.0},    // 4 waves, two workgroups per CU
-    {5, 64, 64, 512, 19.0, 17.0, 13.0, 18.0},     // 4 waves, 32x32 per wave: spreads a short row range
-    {6, 128, 64, 256, 22.5, 4.5, 13.0, 14.0},     // 4 waves, 64x32 per wave: less operand traffic per flop than 64x64
-    {8, 128, 256, 256, 41.5, 15.0, 45.0, 30.0},   // persistent, 4 waves of 64x128 (gemm_big.hip): 2048 x 4096 outputs are one round of it
+// Tile and slice choice from a measured cost model: microseconds of one launch of an M x N product over K as `slices` shares of the
+// contraction, in rounds of 256 workgroups (one per compute unit; tiles 4 and 5 leave room for a second one, which shares
+// the unit's load path: its round is no shorter).  Every term of a round scales with the K of a slice; what does not is the
+// launch itself (`ramp`: launch, first loads, epilogue), the second kernel and the fp32 partial tiles of a split contraction, and
+// the weight's way from HBM.  Fitted to 5187 timed launches (167 shapes of 65 - 12000 rows, 1024 - 57344 columns and K, both operand
+// layouts, rank-16 term, weights rotating through 512 MB so that none comes from a cache): 5 - 8 % off, and the tile it picks costs 1.3 % more
+// than the best of all; the model before it (unsplit tiles timed on warm weights, slices by a fixed rule) picked 7.6 % more, up
+// to 1.9 times: 256 x 4096 over 28672 (NN) 160 -> 83 us, 256 x 8192 over 28672 (NT) 235 -> 147, 85 x 2304 over 4096 19.8 -> 13.2,
+// 256 x 8192 over 8192 63 -> 54, 512 x 4096 over 14336 109 -> 78.
+struct TileCand {
+  int cfg, bm, bn;
+  double ramp;     // us per launch
+  double lone;     // us per 4096 of K: one round of few workgroups
+  double fill;     //   and what a full one costs beyond it (shared load path, power)
+  double second;   //   second round
+  double more;     //   every further round
+  double last;     //   and what a full last round costs beyond an empty one
+  double reduce;   // us: the second kernel of a split contraction
+  double partial;  // us per MB of partial tiles, written and read
+  double weight;   // us per MB of weight
 };
-constexpr double kRamp = 6.0;
-static double launch_cost(const TileCand& c, int M, int N, int K) {
-  const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+static const TileCand kCands[] = {
+    {7, 256, 256, 6.3, 59.0, 30.1, 64.7, 91.2, 35.8, 0.0, 0.0, 0.121},     // persistent, 4 waves of 128x128 (gemm_big.hip)
+    {1, 256, 256, 8.9, 67.5, 15.9, 73.5, 97.7, 25.8, 0.0, 0.374, 0.046},   // 8 waves, 128x64 per wave
+    {3, 128, 256, 6.4, 45.7, 8.9, 53.5, 61.6, 15.3, 2.7, 0.304, 0.076},    // 8 waves, 64x64 per wave
+    {9, 192, 128, 6.6, 37.5, 5.5, 43.1, 55.2, 4.9, 1.2, 0.423, 0.040},     // 4 waves, 96x64 per wave (not with a routing table)
+    {4, 128, 128, 5.3, 27.0, 6.9, 20.7, 32.8, 9.6, 2.5, 0.291, 0.078},     // 4 waves, 64x64 per wave
+    {5, 64, 64, 4.6, 13.2, 3.1, 7.7, 15.6, 4.3, 2.4, 0.265, 0.061},        // 4 waves, 32x32 per wave
+    {6, 128, 64, 5.1, 17.4, 4.1, 21.5, 25.1, 3.7, 1.6, 0.479, 0.085},      // 4 waves, 64x32 per wave
+    {8, 128, 256, 6.0, 35.4, 11.3, 36.5, 54.0, 23.4, 0.0, 0.0, 0.108},     // persistent, 4 waves of 64x128 (gemm_big.hip)
+};
+static long tiles_of(int M, int N, const TileCand& c) { return (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); }
+static double launch_cost(const TileCand& c, int M, int N, int K, int slices = 1, int steps = 0) {
+  const long tiles = tiles_of(M, N, c) * slices;
   if (tiles <= 0) return 0.0;
-  const long full = tiles / c.slots;
-  const double fill = (double)(tiles % c.slots) / c.slots;
-  double at4096;
-  if (full == 0) at4096 = c.lat0 + c.first_b * fill * fill;
-  else at4096 = c.lat0 + c.first_b + (full - 1) * (c.next_a + c.next_b) + (fill > 0 ? c.next_a + c.next_b * fill : 0.0);
-  return kRamp + (at4096 - kRamp) * (K / 4096.0);
+  const long rounds = (tiles + 255) / 256;
+  const double k = (slices > 1 ? steps * (double)BK : (double)K) / 4096.0, filled = rounds > 1 ? 1.0 : tiles / 256.0;
+  double us = c.ramp + k * (c.lone + c.fill * filled) + c.weight * (2e-6 * N * K);
+  if (rounds > 1) us += k * (c.second + c.more * (double)(rounds - 2) + c.last * ((double)(tiles - (rounds - 1) * 256) / 256.0));
+  if (slices > 1) us += c.reduce + c.partial * (4e-6 * slices * M * N);
+  return us;
 }
-static int choose_cfg(int M, int N, int K, bool allow_big, double* cost_out = nullptr, bool allow_mid = true) {
+static const TileCand& cand_of(int cfg) {
+  for (const TileCand& c : kCands) if (c.cfg == cfg) return c;
+  return kCands[cfg == 2 ? 2 : 1];   // (the four-wave forms of these tiles, 0 and 2, are only run when pinned or for odd routing blocks)
+}
+// The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
+// (its 128-row tile and the other 256-column tiles leave most of the chip idle there); single: no routing table (a 96-row
+// wave may lie across two routing blocks).  The eight-wave 256x256 tile stands in for the persistent one (a long
+// contraction under a wide output prefers it: lf_plan_gemm).
+static int choose_cfg(int M, int N, int K, bool big, bool single, double* cost_out = nullptr, bool tail = false) {
   int best = 1;
   double best_cost = 1e30;
   for (const TileCand& c : kCands) {
-    if (c.cfg == 7 && (!allow_big || M < 256 || N < 256)) continue;
-    // (a lone 128x256 tile per CU takes 41 us whatever the fill, the same for both operand layouts: below half a round
-    // the smaller tiles are faster)
-    if (c.cfg == 8 && (!allow_big || !allow_mid || M < 128 || N < 256 || K < 256 || 2 * (long)((M + 127) / 128) * ((N + 255) / 256) <= c.slots)) continue;
+    if (c.cfg == 7 && (!big || tail || M < 256 || N < 256)) continue;
+    if (c.cfg == 8 && (!big || tail || M < 128 || N < 256 || K < 256)) continue;
+    if (c.cfg == 1 && (tail || (big && M >= 256 && N >= 256))) continue;
+    if (c.cfg == 3 && tail) continue;
+    if (c.cfg == 9 && (!single || tail)) continue;
     const double cost = launch_cost(c, M, N, K);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;
   return best;
 }
-// Rows [0, m_main) as 256x256 tiles, the rest as a second launch with the tile that spreads it best, when that beats
+// Rows [0, m_main) as 256x256 tiles, the rest as a second launch with the tile that spreads them best, when that beats
 // one launch (a nearly empty last round of big tiles costs a full tile time).  m_main is the multiple of 256 rows
 // with the lowest modelled cost of both launches: usually the one whose tiles fill whole rounds of the chip
 // (32 tile rows of 40 tiles are exactly five rounds; 30 rows of 40 are five rounds too, and leave a longer tail).
 // Returns m_main (0: single launch).
-static int choose_split(int M, int N, int K, bool allow_big, int* cfg_head, int* cfg_tail) {
+static int choose_split(int M, int N, int K, bool allow_big, bool single, int* cfg_head, int* cfg_tail) {
   constexpr double kLaunch = 4.0;  // a second launch
   const int grid_n = (N + 255) / 256;
   if (grid_n > 256) return 0;
   const bool big = allow_big && N >= 256;
   const TileCand& head = kCands[big ? 0 : 1];
   double best;
-  choose_cfg(M, N, K, allow_big, &best);
+  choose_cfg(M, N, K, allow_big, single, &best);
   int best_m = 0;
   for (int r = 1; r * 256 < M; r++) {
+    const double head_cost = launch_cost(head, r * 256, N, K) + kLaunch;
+    if (head_cost >= best) break;
     double tail;
-    // (left-over rows behind whole rounds of 256x256 tiles: small tiles or a split contraction, not the 128-row persistent tile)
-    const int ct = choose_cfg(M - r * 256, N, K, allow_big, &tail, false);
-    const double cost = launch_cost(head, r * 256, N, K) + tail + kLaunch;
-    if (cost < best) { best = cost; best_m = r * 256; *cfg_tail = ct; }
+    const int ct = choose_cfg(M - r * 256, N, K, allow_big, single, &tail, true);
+    if (head_cost + tail < best) { best = head_cost + tail; best_m = r * 256; *cfg_tail = ct; }
   }
   *cfg_head = big ? 7 : 1;
   return best_m;
 }
 
-// Split contraction for a launch of few tiles over a long K (left-over rows of a packed batch, short batches): K is
-// cut into slices, workgroup (tile, slice) keeps fp32 sums, a second kernel adds the slices.  Measured on the left-over
-// rows of the 8B and 70B layers (128 and 384 rows; microseconds with the second kernel, unsplit first):
-//   128 x 4096 over 28672 (NN): 64x64 tiles 134 -> 128x64 tiles in 4 slices 52;  over 6144: 31 -> 18
-//   128 x 4096 over 14336 (NT): 54 -> 35;   384 x 8192 over 57344 (NN): 128x128 tiles 580 -> 256x256 tiles in 4 slices 399
-//   384 x 8192 over 28672 (NT): 300 -> 203; 384 x 10240 over 8192: 64 unsplit, 95 in 2 slices of 256x256 tiles
-// So: when the planned tiles fill less than half of the chip's workgroup slots, the launch moves to the 128x64 tile (up
-// to 256 rows) or the eight-wave 256x256 tile (more rows) in as many slices as give every compute unit a workgroup,
-// provided a slice keeps at least 48 K steps on the small tile and 192 on the large one (their fixed cost per
-// workgroup: pipeline fill and an fp32 store of the tile) and the small tile gets at least three slices, at most 16
-// slices and at most kKsplitMaxBytes of partial tiles.  A function of the shape, the planned tile and the routing block alone: a call that is given the workspace
-// lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
-constexpr size_t kKsplitMaxBytes = (size_t)64 << 20;
+// Split contraction for launches that leave compute units idle over a long K (left-over rows of a packed batch, short
+// batches): K is cut into slices, workgroup (tile, slice) keeps fp32 sums, a second kernel adds the slices.  Larger tiles
+// move fewer operand bytes per product, and a compute unit takes in at most about 100 GB/s whatever its tile, so many slices of
+// a large tile beat one slice of many small ones once K is long: tile and slice count are chosen together by the model above, where
+// they are at least 4 % ahead of the planned launch.  A slice keeps at least 512 of K, its workgroups fit the chip at once, and the partial
+// tiles stay within a limit (the dX product's: what the library's static scratch holds).  A function of the shape, the planned tile and the routing alone: a call that is
+// given the workspace lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
+constexpr size_t kKsplitMaxBytes = (size_t)64 << 20, kKsplitMaxBytesNN = LF_STATIC_SCRATCH_BYTES;
 struct KSplit { int cfg, n, steps; };
-static long tiles_of(int M, int N, int cfg, int* slots = nullptr) {
-  int bm = 256, bn = 256, sl = 256;      // configurations 0, 1, 7
-  for (const TileCand& k : kCands) if (k.cfg == cfg) { bm = k.bm; bn = k.bn; sl = k.slots; }
-  if (cfg == 2) { bm = 128; bn = 256; }
-  if (slots != nullptr) *slots = sl;
-  return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-}
-static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block) {
+static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn) {
   const int nk = K / BK;
-  const KSplit none = {cfg, 1, nk};
-  int slots = 256;
-  if (cfg == 7 || 2 * tiles_of(M, N, cfg, &slots) > slots) return none;   // the planned launch fills half of its slots
-  const bool big_ok = routing_block <= 0 || routing_block % 128 == 0;
-  const int cand = M <= 256 ? 6 : (big_ok ? 1 : 2);
-  const int min_steps = cand == 6 ? 48 : 192;
-  const long tiles = tiles_of(M, N, cand);
-  long n = 256 / tiles;
-  n = std::min(n, (long)16);
-  n = std::min(n, (long)(nk / min_steps));
-  const size_t slice = (size_t)M * N * sizeof(float);
-  n = std::min(n, (long)(kKsplitMaxBytes / slice));
-  if (n < (cand == 6 ? 3 : 2)) return none;   // two slices of the small tile only pay for the second kernel (22 -> 24 us at K = 4096)
-  int steps = (int)((nk + n - 1) / n);
-  steps += steps & 1;                                         // an even number of steps per slice (K / BK is even)
-  return {cand, (nk + steps - 1) / steps, steps};             // no empty slice
+  KSplit best = {cfg, 1, nk};
+  const TileCand& planned = cand_of(cfg);
+  if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
+  double best_cost = 0.96 * launch_cost(planned, M, N, K);
+  const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
+  for (const TileCand& c : kCands) {
+    if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)
+    if (routing_block > 0 && (c.cfg == 9 || (c.cfg == 1 && routing_block % 128 != 0))) continue;
+    const long tiles = tiles_of(M, N, c), slots = c.cfg == 4 || c.cfg == 5 ? 512 : 256;
+    for (int n : {2, 3, 4, 5, 6, 8, 12, 16}) {
+      if (tiles * n > slots || K < n * 512 || slice * n > max_bytes) break;
+      int steps = (nk + n - 1) / n;
+      steps += steps & 1;                               // an even number of steps per slice (K / BK is even)
+      const int used = (nk + steps - 1) / steps;        // no empty slice
+      const double cost = launch_cost(c, M, N, K, used, steps);
+      if (used > 1 && cost < best_cost) { best_cost = cost; best = {c.cfg, used, steps}; }
+    }
+  }
+  return best;
 }
 
 static std::atomic<int> pinned_cfg{-1};
@@ -866,9 +881,9 @@ bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; 
 // The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned: rows [0, *rows_head)
 // with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
-  const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0);
+  const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), single = routing_block <= 0;
   int ch = 1, ct = 1;
-  const int m_main = choose_split(M, N, K, allow_big, &ch, &ct);
+  const int m_main = choose_split(M, N, K, allow_big, single, &ch, &ct);
   // A long contraction under a wide output runs faster on the eight-wave 256x256 tile than on the persistent kernel
   // (8192 x 8192 over 28672: 3.08 against 3.24 ms, over 57344: 5.74 against 5.85; at 4096 columns the two are level, and
   // at shorter contractions the persistent kernel is 3-8 % ahead): its long K loops let the tiles of an XCD drift apart
@@ -880,7 +895,7 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
   };
   if (m_main == 0) {
     *rows_head = M;
-    *cfg_head = demote(choose_cfg(M, N, K, allow_big));
+    *cfg_head = demote(choose_cfg(M, N, K, allow_big, single));
     *cfg_tail = -1;
   } else {
     *rows_head = m_main;
@@ -890,16 +905,15 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
 }
 
 // Bytes of fp32 partial tiles the split contraction of an M x N product over K may write: the largest need over the
-// launches of the plan and over the configurations a launch can be moved to at run time (the eight-wave 256x256 tile
-// and the 128x256 tile stand in for the persistent kernel where it does not apply).
-size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block) {
+// launches of the plan and over the tile a launch moves to where the persistent kernel does not apply.
+size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   if (M <= 0 || N <= 0 || K < BK) return 0;
   int rows = 0, ch = 1, ct = -1;
   lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
   size_t need = 0;
   auto part = [&](int m, int cfg) {
-    for (int c : {cfg, 1, 2, choose_cfg(m, N, K, false)}) {
-      const KSplit ks = ksplit_for(m, N, K, c, routing_block);
+    for (int c : {cfg, choose_cfg(m, N, K, false, routing_block <= 0)}) {
+      const KSplit ks = ksplit_for(m, N, K, c, routing_block, nn);
       if (ks.n > 1) need = std::max(need, (size_t)ks.n * m * N * sizeof(float));
     }
   };
@@ -925,22 +939,21 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
   const bool planned = force_cfg < 0;
   auto launch = [&](const LfGemmParams& q, int cfg) {
     if (seg.table != nullptr && seg.block_size_m % 128 != 0 && (cfg == 0 || cfg == 1 || cfg == 7)) cfg = 2;
-    // what the persistent kernel does not take goes to the eight-wave 256x256 tile: a keep-mask with one byte per
-    // element, a dX term of more than 32 rank columns and (when the library chose the tile) a contraction of one K step
-    if (cfg == 7 && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32) || (planned && q.K < 128))) cfg = 1;
-    // the 128-row persistent tile has the same limits; a product it was planned for then runs on the small tile the
-    // cost model likes best (pinned: on the four-wave 128x256 tile)
-    if (cfg == 8 && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32)))
-      cfg = planned ? choose_cfg(q.M, q.N, q.K, false) : 2;
-    if (cfg == 7) return lf_launch_gemm_big(q, seg, nn, dtype, 256, st);
-    if (cfg == 8) return lf_launch_gemm_big(q, seg, nn, dtype, 128, st);
+    // what the persistent kernel does not take (a keep-mask with one byte per element, a dX term of more than 32 rank columns)
+    // goes to the tile the cost model likes best without it (pinned: the eight-wave 256x256 or the four-wave 128x256
+    // tile), a contraction of one K step on its 256x256 tile to the eight-wave one
+    if ((cfg == 7 || cfg == 8) && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32)))
+      cfg = planned ? choose_cfg(q.M, q.N, q.K, false, seg.table == nullptr) : (cfg == 7 ? 1 : 2);
+    if (cfg == 7 && planned && q.K < 128) cfg = 1;
     if (dtype != LF_BF16 && dtype != LF_F16) return (int)LF_EINVAL;
     LfGemmParams r = q;
     r.ksplit = 1, r.ks_steps = 0;
     if (planned && r.ks_ws != nullptr && ((uintptr_t)r.ks_ws & 15) == 0) {   // (a pinned tile configuration stays as pinned)
-      const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, seg.table != nullptr ? seg.block_size_m : 0);
+      const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, seg.table != nullptr ? seg.block_size_m : 0, nn);
       if (ks.n > 1 && (size_t)ks.n * r.M * r.N * sizeof(float) <= r.ks_ws_bytes) { cfg = ks.cfg; r.ksplit = ks.n; r.ks_steps = ks.steps; }
     }
+    if (cfg == 7) return lf_launch_gemm_big(q, seg, nn, dtype, 256, st);
+    if (cfg == 8) return lf_launch_gemm_big(q, seg, nn, dtype, 128, st);
     int rc;
     if (dtype == LF_BF16) rc = nn ? launch_dtype<__bf16, true>(r, seg, cfg, st) : launch_dtype<__bf16, false>(r, seg, cfg, st);
     else rc = nn ? launch_dtype<_Float16, true>(r, seg, cfg, st) : launch_dtype<_Float16, false>(r, seg, cfg, st);

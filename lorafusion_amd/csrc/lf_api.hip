@@ -95,7 +95,7 @@ bool bad_rank_cols(int R) { return R <= 0 || R % 16 != 0 || R > LF_MAX_RANK; }
 // short forward's slices.
 size_t fwd_workspace(int M, int N, int K, int R, int rb, const LfSegTable& t) {
   const size_t sliced = !t.table && lf_short_fwd_applies(M, N) && !bad_tiled_dim(N) ? lf_short_fwd_workspace(M, N, K, t.rank[0]) : 0;
-  return std::max(sliced, align256(lf_xa_workspace(M, K, R, t)) + lf_gemm_ksplit_bytes(M, N, K, rb));
+  return std::max(sliced, align256(lf_xa_workspace(M, K, R, t)) + lf_gemm_ksplit_bytes(M, N, K, rb, false));
 }
 // What is left of a forward's workspace behind the rank-r pass's slices.
 void behind_xa(void*& ws, size_t& bytes, int M, int K, int R, const lf_routing* routing) {
@@ -144,12 +144,12 @@ size_t lf_workspace_bytes(int op, int M, int N, int K, int R, const lf_routing* 
     case LF_OP_FWD: return align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_BWD: {
       size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
-      return align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb)));
+      return align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb, true)));
     }
     case LF_OP_NF4_FWD: return align256((size_t)N * K * 2) + align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_NF4_BWD: {
       size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
-      return align256((size_t)N * K * 2) + align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb)));
+      return align256((size_t)N * K * 2) + align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb, true)));
     }
     default: return 0;
   }
@@ -364,7 +364,7 @@ int lf_lora_bwd_static(const void* dY, const void* X, const void* W, const uint8
   // what lf_workspace_bytes(LF_OP_BWD, ...) names: the rank-r passes' partial sums or the dX product's partial tiles,
   // whichever is larger (with less, the product would not split its contraction and its sums would differ in order)
   const size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
-  const size_t need = align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, t.table != nullptr ? t.block_size_m : 0)));
+  const size_t need = align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, t.table != nullptr ? t.block_size_m : 0, true)));
   if (need > (size_t)LF_STATIC_SCRATCH_BYTES) return LF_ESTATIC;
   void* ws = nullptr;
   rc = static_scratch(&ws);

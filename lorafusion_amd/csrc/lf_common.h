@@ -76,7 +76,7 @@ int lf_cu_count();
 int lf_pin_tile_cfg(int cfg);  // -1: automatic choice
 bool lf_tile_pinned();
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail);
-size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block);  // workspace of the split contraction for this product
+size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn);  // workspace of the split contraction for this product
 
 // Raise a kernel's dynamic-LDS limit once per device (the attribute belongs to the device's copy of
 // the function; one flag array per kernel instantiation; threads that race here repeat the same call).

@@ -1,0 +1,87 @@
+"""The 192x128 tile (rows and columns that end inside a tile, every form of the LoRA term and the keep-mask) and the joint choice of tile
+and slice count for short products over a long contraction, each tile that it picks.  Against fp32 sums of the same 16-bit
+inputs at the bound of the other kernel tests (|err| <= 1e-2 (|e| + rms(e)): one 16-bit rounding of the result)."""
+
+import ctypes
+
+import pytest
+import torch
+
+from oracle import lora_ref
+from tests.util import single_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, exp, name):
+    ok, rel, excess = lora_ref.check_close(got.detach().float().cpu(), exp, rtol=1e-2)
+    assert ok, f"{name}: rel {rel:.3e} excess {excess:.3e}"
+
+
+def _planned(M, N, K):
+    from lorafusion_amd import _lib as L
+
+    rows, head, tail = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    L.check(L.lib().lf_gemm_plan(M, N, K, 0, ctypes.byref(rows), ctypes.byref(head), ctypes.byref(tail)), "lf_gemm_plan")
+    return rows.value, head.value, tail.value
+
+
+@pytest.mark.parametrize("M,N,K,r,dtype", [
+    (257, 11008, 512, 16, torch.bfloat16),    # one row in the second tile row
+    (384, 11136, 512, 40, torch.float16),     # whole tile rows; rank beyond one chunk of 32 columns, not a multiple of 16
+    (350, 12160, 512, 128, torch.bfloat16),   # a last wave with rows of which some lie beyond the matrix
+])
+def test_192_row_tile(M, N, K, r, dtype):
+    from lorafusion_amd.ops import hip_ops
+
+    assert _planned(M, N, K) == (M, 9, -1)
+    d = single_inputs(M, K, N, r, p=0.0, seed=M, dtype=dtype, bias=True)
+    x, w, a, b = (d[k].cuda() for k in ("x", "w", "a", "b"))
+    ye, se = lora_ref.linear_lora_fwd_fp32(d["x"], d["w"], d["a"], d["b"], 2.0, None, 0.0, d["bias"])
+    s = se.to(dtype).cuda()
+    ye = ye + 2.0 * (s.float().cpu() - se) @ d["b"].float().T
+    _close(hip_ops.fused_lora_xw_sb(x, w, s, b, 2.0, bias=d["bias"].cuda()), ye, "y")
+    # the dX product of the transposed sizes: N columns over K, with no mask, its bytes and its bits
+    dy, wt, p = d["x"], d["w"].T.contiguous(), 0.2
+    g = torch.Generator().manual_seed(r)
+    at = ((torch.rand(r, N, generator=g) * 2 - 1) / N ** 0.5).to(dtype)
+    ds = (torch.randn(M, r, generator=g) * 0.1).to(dtype)
+    mask = torch.rand(M, N, generator=g) >= p
+    base, term = dy.float() @ wt.float(), ds.float() @ at.float()
+    dev = [t.cuda() for t in (dy, wt, ds, at)]
+    _close(hip_ops.fused_lora_dyw_dsa(*dev, 0.0), base + term, "dx")
+    expect = base + torch.where(mask, term / (1 - p), torch.zeros(()))
+    by = hip_ops.fused_lora_dyw_dsa(*dev, p, mask.cuda())
+    _close(by, expect, "dx, mask bytes")
+    _close(hip_ops.fused_lora_dyw_dsa(*dev, p, hip_ops.pack_mask(mask.cuda())), expect, "dx, mask bits")
+
+
+@pytest.mark.parametrize("M,K,N,dtype", [
+    (85, 4096, 2304, torch.bfloat16), (130, 6144, 2944, torch.float16), (256, 8192, 2048, torch.bfloat16), (283, 6144, 1024, torch.bfloat16),
+    (511, 14336, 1024, torch.float16), (700, 8192, 1024, torch.bfloat16), (2290, 9088, 1152, torch.bfloat16)])
+def test_tile_and_slices_together(M, K, N, dtype):
+    """Forward over K and dX over K (the roles of the dimensions exchanged), against the same products through the entry points
+    without a workspace, which do not split: the sums differ in order only, so by no more than one 16-bit step of the largest value."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    r, p = 16, 0.1
+    R, routing = L.round_rank(r), L.single_routing(r, 2.0, p)
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn(M, K, generator=g).to(dtype).cuda()
+    w = (torch.randn(N, K, generator=g) * 0.02).to(dtype).cuda()
+    a, b = (torch.randn(r, K, generator=g) * K ** -0.5).to(dtype).cuda(), (torch.randn(N, r, generator=g) * 0.01).to(dtype).cuda()
+    bits = hip_ops.pack_mask((torch.rand(M, K, generator=g) >= p).cuda())
+    y, s = hip_ops.lora_forward(x, w, [a], [b], routing, R, bits, None)
+    y1 = hip_ops.fused_lora_xw_sb(x, w, s[:, :r].contiguous(), b, 2.0)
+    step = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    assert float((y.float() - y1.float()).abs().max()) <= float(y1.float().abs().max()) * step
+    # dX [M, N] over K: X takes the place of dY
+    wt, at, bt = w.T.contiguous(), b.T.contiguous(), a.T.contiguous()
+    xs = torch.randn(M, N, generator=g).to(dtype).cuda()
+    bits = hip_ops.pack_mask((torch.rand(M, N, generator=g) >= p).cuda())
+    st = (torch.randn(M, R, generator=g) * 0.1).to(dtype).cuda()
+    dx = hip_ops.lora_backward(x, xs, wt, [at], [bt], st, routing, R, bits, [r])[0]
+    ds = hip_ops.fused_lora_dys_dyb(x, bt, st, 2.0)[1]
+    dx1 = hip_ops.fused_lora_dyw_dsa(x, wt, ds, at, p, bits)
+    assert float((dx.float() - dx1.float()).abs().max()) <= float(dx1.float().abs().max()) * step
