@@ -256,27 +256,42 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
     issue_first_tiles();
   } else {
     const T* __restrict__ L = (const T*)p.L;
-    const T* rp = (const T*)seg.ptr[0];
-    int rank = seg.rank[0];
-    // mult_mode 1 without a keep-mask means no dropout, whatever p says: the term is not rescaled
-    bool use_mask = p.mask != nullptr && p.mult_mode == 1 && seg.p > 0.f;
-    float mult = p.mult_mode == 0 ? seg.scale : (use_mask ? 1.f / (1.f - seg.p) : 1.f);
-    if (seg.table != nullptr) {
-      int blk = (p.row0 + wrow0) / seg.block_size_m;
-      blk = min(blk, seg.n_blocks - 1);
-      rank = seg.table[3 * blk + 0];
-      int fb = seg.table[3 * blk + 2];
+    struct Term { const T* rp; int rank; float mult; bool mask; };
+    auto term_of_block = [&](int blk) {
+      const int fb = seg.table[3 * blk + 2];
       int s = 0;
       for (int i = 1; i < seg.n_seg; i++) s = (seg.first_block[i] == fb) ? i : s;
-      rp = (const T*)seg.ptr[s];
+      Term t{(const T*)seg.ptr[s], seg.table[3 * blk + 0], 1.f, false};
       if (p.mult_mode == 0) {
-        mult = seg.block_scale[blk];
+        t.mult = seg.block_scale[blk];
       } else {
-        float pb = seg.block_p[blk];
-        use_mask = p.mask != nullptr && pb > 0.f;
-        mult = use_mask ? 1.f / (1.f - pb) : 1.f;
+        const float pb = seg.block_p[blk];
+        t.mask = p.mask != nullptr && pb > 0.f;
+        t.mult = t.mask ? 1.f / (1.f - pb) : 1.f;
+      }
+      return t;
+    };
+    // mult_mode 1 without a keep-mask means no dropout, whatever p says: the term is not rescaled
+    const bool drop = p.mask != nullptr && p.mult_mode == 1 && seg.p > 0.f;
+    Term t0{(const T*)seg.ptr[0], seg.rank[0], p.mult_mode == 0 ? seg.scale : (drop ? 1.f / (1.f - seg.p) : 1.f), drop};
+    // A wave of 96 rows may lie across two routing blocks (their size is a multiple of 128: never three): block rows from
+    // `isplit` on belong to the second, whose adapter gets a pass of its own over them.  The products of an adapter are
+    // not formed for the other's rows at all: a zero operand would still carry its infinities and NaNs over.
+    // (1280 x 4096 over 4096, ranks to 64, keep bits: 56.4 us here as 224 tiles, 69.0 as 160 of 128x256; forward 53.3 against 55.5
+    // on the persistent kernel's 128x256 tile.)
+    constexpr bool SPLIT = WM % 64 != 0;
+    Term t1 = t0;
+    int isplit = TM, nterm = 1;
+    if (seg.table != nullptr) {
+      const int row = p.row0 + wrow0, blk = min(row / seg.block_size_m, seg.n_blocks - 1);
+      t0 = term_of_block(blk);
+      if constexpr (SPLIT) {
+        const int left = (blk + 1) * seg.block_size_m - row;
+        if (left < WM && blk + 1 < seg.n_blocks) isplit = left / 16, nterm = 2, t1 = term_of_block(blk + 1);
       }
     }
+    auto second = [&](int i) { return SPLIT && i >= isplit; };
+    const bool use_mask = t0.mask || (SPLIT && nterm == 2 && t1.mask);
     // Keep-mask of this wave's sub-tile: 16-byte loads that cover whole rows of the sub-tile (issued
     // here so that their latency overlaps the seeding MFMAs), handed to the lanes that own the
     // accumulator elements through the wave's slice of the last ring stage, which no tile load
@@ -304,7 +319,6 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
 #pragma unroll
       for (int ib = 0; ib < TM32; ib++) load_mask_band(ib);
     }
-    const __amdgpu_buffer_rsrc_t rsrcR = __builtin_amdgcn_make_buffer_rsrc((void*)rp, 0, 0x7fffffff, 0x00020000);
     // Bit-packed keep-mask: the dword that holds the lane's four columns of each accumulator block (element n of a
     // mask row = bit n & 7 of byte n >> 3).  Requested with the operands of the first chunk where the registers allow
     // (up to 16 blocks per wave), else in one batch behind the MFMAs.
@@ -326,7 +340,12 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
     // All loads of a chunk are requested before the first is used (the conditions sit outside the loops over the
     // fragments): the term costs one memory round trip per chunk, not one per fragment -- with a branch and a wait
     // per fragment the NN seed of a 128x256 tile took 17 us of an 80 us launch.
-    for (int t = 0; t < (p.R + 31) / 32; t++) {
+    const int nchunk = (p.R + 31) / 32;
+    for (int u = 0; u < (SPLIT ? nterm * nchunk : nchunk); u++) {
+      const int part = SPLIT && u >= nchunk ? 1 : 0, t = u - part * nchunk;
+      const T* rp = part ? t1.rp : t0.rp;
+      const int rank = part ? t1.rank : t0.rank;
+      const __amdgpu_buffer_rsrc_t rsrcR = __builtin_amdgcn_make_buffer_rsrc((void*)rp, 0, 0x7fffffff, 0x00020000);
       const int r0 = t * 32 + kg * 8;
       lf_u32x4 rf[TN], lf[TM];
       uint32_t e[NN ? TN : 1][8];
@@ -357,7 +376,7 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
           lf[i] = *(const lf_u32x4*)(L + (int64_t)gm * p.R + r0);
         }
       }
-      if (t == 0) {
+      if (u == 0) {
         if (bits_mask && BITS_EARLY) load_bits(0);
         __builtin_amdgcn_sched_barrier(0);
         issue_first_tiles();
@@ -371,9 +390,11 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
         }
       }
 #pragma unroll
-      for (int i = 0; i < TM; i++)
+      for (int i = 0; i < TM; i++) {
+        if (SPLIT && nterm == 2 && second(i) != (part == 1)) continue;
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = MfmaOp<T>::run(rf[j], lf[i], acc[i][j]);
+      }
     }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -390,14 +411,16 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
       if constexpr (!BITS_EARLY) {
         if (bits_mask && i % GI == 0) load_bits(i);   // the next batch of block rows, all its words at once
       }
+      const float mult = second(i) ? t1.mult : t0.mult;
+      const bool masked = second(i) ? t1.mask : t0.mask;
 #pragma unroll
       for (int j = 0; j < TN; j++) {
         acc[i][j] *= mult;
-        if (bits_mask) {
+        if (masked && p.mask_bits) {
           const uint32_t bits = mw[i % GI][j];
 #pragma unroll
           for (int e = 0; e < 4; e++) acc[i][j][e] = ((bits >> e) & 1u) ? acc[i][j][e] : 0.f;
-        } else if (use_mask) {
+        } else if (masked) {
           const int dw = j * 4 + kg;  // dword of the 4 columns j*16 + kg*4 ..
           const uint32_t mk = *(const uint32_t*)(mreg + r * WN + (((dw >> 2) ^ ((r / MRW) & (MLPR - 1))) << 4) + (dw & 3) * 4);
 #pragma unroll
@@ -732,7 +755,7 @@ int launch_cfg(LfGemmParams p, const LfSegTable& seg, hipStream_t st) {
 
 template <typename T, bool NN>
 int launch_dtype(const LfGemmParams& p, const LfSegTable& seg, int cfg, hipStream_t st) {
-  // Rows of one routing block must not straddle a wave's sub-tile: WM divides block_size_m.
+  // WM divides block_size_m, but for the 96-row waves of configuration 9 (two blocks at most: block_size_m % 128 == 0).
   switch (cfg) {
     case 0: return launch_cfg<T, 256, 256, 128, 128, NN, LF_NSTAGE>(p, seg, st);
     case 1: return launch_cfg<T, 256, 256, 128, 64, NN, LF_NSTAGE>(p, seg, st);
@@ -773,7 +796,7 @@ static const TileCand kCands[] = {
     {7, 256, 256, 6.3, 59.0, 30.1, 64.7, 91.2, 35.8, 0.0, 0.0, 0.121},     // persistent, 4 waves of 128x128 (gemm_big.hip)
     {1, 256, 256, 8.9, 67.5, 15.9, 73.5, 97.7, 25.8, 0.0, 0.374, 0.046},   // 8 waves, 128x64 per wave
     {3, 128, 256, 6.4, 45.7, 8.9, 53.5, 61.6, 15.3, 2.7, 0.304, 0.076},    // 8 waves, 64x64 per wave
-    {9, 192, 128, 6.6, 37.5, 5.5, 43.1, 55.2, 4.9, 1.2, 0.423, 0.040},     // 4 waves, 96x64 per wave (not with a routing table)
+    {9, 192, 128, 6.6, 37.5, 5.5, 43.1, 55.2, 4.9, 1.2, 0.423, 0.040},     // 4 waves, 96x64 per wave
     {4, 128, 128, 5.3, 27.0, 6.9, 20.7, 32.8, 9.6, 2.5, 0.291, 0.078},     // 4 waves, 64x64 per wave
     {5, 64, 64, 4.6, 13.2, 3.1, 7.7, 15.6, 4.3, 2.4, 0.265, 0.061},        // 4 waves, 32x32 per wave
     {6, 128, 64, 5.1, 17.4, 4.1, 21.5, 25.1, 3.7, 1.6, 0.479, 0.085},      // 4 waves, 64x32 per wave
@@ -795,10 +818,11 @@ static const TileCand& cand_of(int cfg) {
   return kCands[cfg == 2 ? 2 : 1];   // (the four-wave forms of these tiles, 0 and 2, are only run when pinned or for odd routing blocks)
 }
 // The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
-// (its 128-row tile and the other 256-column tiles leave most of the chip idle there); single: no routing table (a 96-row
-// wave may lie across two routing blocks).  The eight-wave 256x256 tile stands in for the persistent one (a long
+// (its 128-row tile and the other 256-column tiles leave most of the chip idle there); wave96: a 96-row wave meets at most two
+// routing blocks.  The eight-wave 256x256 tile stands in for the persistent one (a long
 // contraction under a wide output prefers it: lf_plan_gemm).
-static int choose_cfg(int M, int N, int K, bool big, bool single, double* cost_out = nullptr, bool tail = false) {
+static bool wave96_fits(int routing_block) { return routing_block <= 0 || routing_block % 128 == 0; }
+static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_out = nullptr, bool tail = false) {
   int best = 1;
   double best_cost = 1e30;
   for (const TileCand& c : kCands) {
@@ -806,7 +830,7 @@ static int choose_cfg(int M, int N, int K, bool big, bool single, double* cost_o
     if (c.cfg == 8 && (!big || tail || M < 128 || N < 256 || K < 256)) continue;
     if (c.cfg == 1 && (tail || (big && M >= 256 && N >= 256))) continue;
     if (c.cfg == 3 && tail) continue;
-    if (c.cfg == 9 && (!single || tail)) continue;
+    if (c.cfg == 9 && (!wave96 || tail)) continue;
     const double cost = launch_cost(c, M, N, K);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
@@ -818,20 +842,20 @@ static int choose_cfg(int M, int N, int K, bool big, bool single, double* cost_o
 // with the lowest modelled cost of both launches: usually the one whose tiles fill whole rounds of the chip
 // (32 tile rows of 40 tiles are exactly five rounds; 30 rows of 40 are five rounds too, and leave a longer tail).
 // Returns m_main (0: single launch).
-static int choose_split(int M, int N, int K, bool allow_big, bool single, int* cfg_head, int* cfg_tail) {
+static int choose_split(int M, int N, int K, bool allow_big, bool wave96, int* cfg_head, int* cfg_tail) {
   constexpr double kLaunch = 4.0;  // a second launch
   const int grid_n = (N + 255) / 256;
   if (grid_n > 256) return 0;
   const bool big = allow_big && N >= 256;
   const TileCand& head = kCands[big ? 0 : 1];
   double best;
-  choose_cfg(M, N, K, allow_big, single, &best);
+  choose_cfg(M, N, K, allow_big, wave96, &best);
   int best_m = 0;
   for (int r = 1; r * 256 < M; r++) {
     const double head_cost = launch_cost(head, r * 256, N, K) + kLaunch;
     if (head_cost >= best) break;
     double tail;
-    const int ct = choose_cfg(M - r * 256, N, K, allow_big, single, &tail, true);
+    const int ct = choose_cfg(M - r * 256, N, K, allow_big, wave96, &tail, true);
     if (head_cost + tail < best) { best = head_cost + tail; best_m = r * 256; *cfg_tail = ct; }
   }
   *cfg_head = big ? 7 : 1;
@@ -856,7 +880,7 @@ static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool n
   const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
   for (const TileCand& c : kCands) {
     if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)
-    if (routing_block > 0 && (c.cfg == 9 || (c.cfg == 1 && routing_block % 128 != 0))) continue;
+    if ((c.cfg == 9 && !wave96_fits(routing_block)) || (c.cfg == 1 && routing_block > 0 && routing_block % 128 != 0)) continue;
     const long tiles = tiles_of(M, N, c), slots = c.cfg == 4 || c.cfg == 5 ? 512 : 256;
     for (int n : {2, 3, 4, 5, 6, 8, 12, 16}) {
       if (tiles * n > slots || K < n * 512 || slice * n > max_bytes) break;
@@ -881,9 +905,9 @@ bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; 
 // The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned: rows [0, *rows_head)
 // with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
-  const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), single = routing_block <= 0;
+  const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), wave96 = wave96_fits(routing_block);
   int ch = 1, ct = 1;
-  const int m_main = choose_split(M, N, K, allow_big, single, &ch, &ct);
+  const int m_main = choose_split(M, N, K, allow_big, wave96, &ch, &ct);
   // A long contraction under a wide output runs faster on the eight-wave 256x256 tile than on the persistent kernel
   // (8192 x 8192 over 28672: 3.08 against 3.24 ms, over 57344: 5.74 against 5.85; at 4096 columns the two are level, and
   // at shorter contractions the persistent kernel is 3-8 % ahead): its long K loops let the tiles of an XCD drift apart
@@ -895,7 +919,7 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
   };
   if (m_main == 0) {
     *rows_head = M;
-    *cfg_head = demote(choose_cfg(M, N, K, allow_big, single));
+    *cfg_head = demote(choose_cfg(M, N, K, allow_big, wave96));
     *cfg_tail = -1;
   } else {
     *rows_head = m_main;
@@ -912,7 +936,7 @@ size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
   size_t need = 0;
   auto part = [&](int m, int cfg) {
-    for (int c : {cfg, choose_cfg(m, N, K, false, routing_block <= 0)}) {
+    for (int c : {cfg, choose_cfg(m, N, K, false, wave96_fits(routing_block))}) {
       const KSplit ks = ksplit_for(m, N, K, c, routing_block, nn);
       if (ks.n > 1) need = std::max(need, (size_t)ks.n * m * N * sizeof(float));
     }
@@ -943,7 +967,7 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
     // goes to the tile the cost model likes best without it (pinned: the eight-wave 256x256 or the four-wave 128x256
     // tile), a contraction of one K step on its 256x256 tile to the eight-wave one
     if ((cfg == 7 || cfg == 8) && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32)))
-      cfg = planned ? choose_cfg(q.M, q.N, q.K, false, seg.table == nullptr) : (cfg == 7 ? 1 : 2);
+      cfg = planned ? choose_cfg(q.M, q.N, q.K, false, wave96_fits(seg.table != nullptr ? seg.block_size_m : 0)) : (cfg == 7 ? 1 : 2);
     if (cfg == 7 && planned && q.K < 128) cfg = 1;
     if (dtype != LF_BF16 && dtype != LF_F16) return (int)LF_EINVAL;
     LfGemmParams r = q;

@@ -56,6 +56,49 @@ def test_192_row_tile(M, N, K, r, dtype):
     _close(hip_ops.fused_lora_dyw_dsa(*dev, p, hip_ops.pack_mask(mask.cuda())), expect, "dx, mask bits")
 
 
+@pytest.mark.parametrize("seq,ranks,p_list,N,dtype", [
+    ([60, 250], [40, 16], [0.2, 0.0], 11136, torch.bfloat16),              # a wave with 32 rows of one adapter and 64 of the next
+    ([128, 1, 77], [16, 128, 8], [0.0, 0.1, 0.3], 11008, torch.float16),   # every block another adapter, one rank per kind of chunk
+])
+def test_192_row_tile_over_routing_blocks(seq, ranks, p_list, N, dtype):
+    """Waves of 96 rows that lie across two routing blocks; an adapter whose matrix holds infinities does not reach its neighbours."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+    from lorafusion_amd.ops.multi_lora import prepare_multi_lora_batch_info
+
+    K, n, scales = 512, len(seq), [1.0, 2.0, 0.5][:len(seq)]
+    info = prepare_multi_lora_batch_info(seq, list(range(n)), ranks, p_list, scales, 128)
+    padded = info.padded_seq_len_list
+    M, R, starts = sum(padded), L.round_rank(max(ranks)), [sum(padded[:i]) for i in range(n)]
+    rows, head, tail = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    L.check(L.lib().lf_gemm_plan(M, N, K, 128, ctypes.byref(rows), ctypes.byref(head), ctypes.byref(tail)), "lf_gemm_plan")
+    assert (rows.value, head.value) == (M, 9)
+    routing = hip_ops.MultiRouting(padded, ranks, info.block_to_lookup_table, info.block_to_alpha, info.block_to_dropout_p)
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) * 0.02).to(dtype)
+    s = torch.zeros(M, R, dtype=dtype)
+    side = [(torch.randn(N, r, generator=g) * 0.05).to(dtype) for r in ranks]   # B_i [N, r]; its transpose serves as A_i [r, N]
+    mask = torch.rand(M, N, generator=g) >= torch.cat([torch.full((pl, 1), p) for pl, p in zip(padded, p_list)])
+    y = x.float() @ w.float().T
+    dx = y.clone()
+    for i, (c, m, r) in enumerate(zip(starts, seq, ranks)):
+        s[c:c + m, :r] = torch.randn(m, r, generator=g).to(dtype)
+        term = s[c:c + m, :r].float() @ side[i].float().T
+        y[c:c + m] += scales[i] * term
+        dx[c:c + m] += torch.where(mask[c:c + m], term / (1 - p_list[i]), torch.zeros(())) if p_list[i] > 0 else term
+    xd, wd, sd, bd, md = x.cuda(), w.cuda(), s.cuda(), [t.cuda() for t in side], mask.cuda()
+    wt, ad = w.T.contiguous().cuda(), [t.T.contiguous().cuda() for t in side]
+    _close(hip_ops.fused_multi_lora_xw_sb(xd, wd, sd, bd, routing), y, "y")
+    for m, name in ((md, "bytes"), (hip_ops.pack_mask(md), "bits")):
+        _close(hip_ops.fused_multi_lora_dyw_dsa(xd, wt, sd, ad, routing, dropout_mask=m), dx, f"dx, mask {name}")
+    bd[1].fill_(float("inf"))
+    ad[1].fill_(float("inf"))
+    clean = torch.ones(M, dtype=torch.bool)
+    clean[starts[1]:starts[1] + padded[1]] = False
+    _close(hip_ops.fused_multi_lora_xw_sb(xd, wd, sd, bd, routing)[clean.cuda()], y[clean], "y beside infinities")
+    _close(hip_ops.fused_multi_lora_dyw_dsa(xd, wt, sd, ad, routing, dropout_mask=md)[clean.cuda()], dx[clean], "dx beside infinities")
+
+
 @pytest.mark.parametrize("M,K,N,dtype", [
     (85, 4096, 2304, torch.bfloat16), (130, 6144, 2944, torch.float16), (256, 8192, 2048, torch.bfloat16), (283, 6144, 1024, torch.bfloat16),
     (511, 14336, 1024, torch.float16), (700, 8192, 1024, torch.bfloat16), (2290, 9088, 1152, torch.bfloat16)])
