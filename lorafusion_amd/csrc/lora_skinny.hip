@@ -19,9 +19,8 @@
 // patterns are bank-conflict free: row fragments (ds_read_b128) and transposed fragments
 // (ds_read_b64_tr_b16).  Loading MFMA fragments straight from global memory would put every
 // lane on a different row (one cache line per lane) and runs at a quarter of the coalesced rate.
-// Two transports: through registers (load, keep-mask applied on the way, LDS store; xa, and
-// dys_dyb / da above rank 64), or as buffer loads that write LDS themselves, several tiles
-// ahead through a ring of stages (dys_dyb / da up to rank 64; second half of this file).
+// Two transports: through registers (xa: load, keep-mask applied on the way, LDS store), or as buffer
+// loads that write LDS themselves, several tiles ahead through a ring of stages (dys_dyb / da; second half of this file).
 //
 // MFMA 16x16x32 operand layout (64 lanes): lane l holds row/col (l & 15) and the 8
 // contraction elements of chunk (l >> 4).  Where the contraction index is the slow memory
@@ -35,15 +34,6 @@
 
 namespace {
 
-__device__ __forceinline__ lf_u32x4 tr_read8(const char* p, int pitch) {
-  // 8 contraction elements (rows r..r+3 and r+4..r+7) of this lane's column
-  lf_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lf_s16x4*)(p));
-  lf_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lf_s16x4*)(p + 4 * pitch));
-  lf_u32x2 a = __builtin_bit_cast(lf_u32x2, lo), b = __builtin_bit_cast(lf_u32x2, hi);
-  return lf_u32x4{a[0], a[1], b[0], b[1]};
-}
-
-
 constexpr int TILE_BYTES = ROWS * 128;  // 128 rows x 64 columns of 16-bit
 
 // Swizzle key of a tile row: granule g of row r sits at slot g ^ tile_key(r).  LDS serves a 16-byte read 16 lanes at
@@ -55,38 +45,6 @@ constexpr int TILE_BYTES = ROWS * 128;  // 128 rows x 64 columns of 16-bit
 __device__ __forceinline__ int tile_key(int row) {
   const int x = (row >> 1) & 7;
   return ((x & 1) << 2) | (x >> 1);
-}
-
-// One thread's share of a 128x64 tile: 4 granules of 8 elements (+ their 8 mask bytes each).
-struct TileRegs {
-  lf_u32x4 x[4];
-  lf_u32x2 m[4];
-};
-
-// Coalesced load of the tile whose first element is src[row0*ld + col0]; rows are clamped to max_row-1.
-template <typename T>
-__device__ __forceinline__ void tile_load(TileRegs& r, const T* __restrict__ src, const uint8_t* __restrict__ mask,
-                                          int64_t ld, int row0, int max_row, int col0, int tid, bool use_mask, bool mask_bits) {
-  const int srcg = (tid & 7) ^ tile_key(tid >> 3);   // rows i*32 + (tid>>3) share their key
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int row = min(row0 + i * 32 + (tid >> 3), max_row - 1);
-    const int64_t off = (int64_t)row * ld + col0 + srcg * 8;
-    r.x[i] = *((const lf_u32x4*)(src + off));
-    // (bit format: the byte is only requested here; tile_store spreads it into eight bytes)
-    if (use_mask) {
-      if (mask_bits) r.m[i][0] = mask[off >> 3];
-      else r.m[i] = *((const lf_u32x2*)(mask + off));
-    }
-  }
-}
-
-__device__ __forceinline__ void tile_store(const TileRegs& r, char* tile, int tid, bool use_mask, bool mask_bits = false) {
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const lf_u32x2 m = (use_mask && mask_bits) ? expand_keep8(r.m[i][0]) : r.m[i];
-    *(lf_u32x4*)(tile + (i * 256 + tid) * 16) = use_mask ? apply_mask8(r.x[i], m) : r.x[i];
-  }
 }
 
 // Row fragment: 8 consecutive columns (granule g) of `row`.
@@ -362,184 +320,6 @@ __device__ __forceinline__ void chunk_blocks(int b0, int b1, int group, int ch, 
   bb1 = bb0 + base + (ch < rem ? 1 : 0);
 }
 
-// ------------------------------------------------------------------------------- dys_dyb
-// grid (n_seg * max_chunks, nsplit).  Workgroup (s, ch, ns) owns the `group` consecutive 128-row blocks ch*group.. of
-// segment s and the N slice ns (tiles_per_wg <= TPW tiles of 64 columns); it walks its blocks, and per block the
-// tiles of the slice:
-//   dS partial  [128 rows, R]  += dY_tile * B_tile      (per block, over the slice; written once per block)
-//   dB partial  [64 cols, R]   += dY_tile^T * S_block    (per tile of the slice, kept in registers over ALL blocks of the
-//                                                         chunk; written once per workgroup)
-// so dB leaves the chip once per chunk of blocks, not once per block: at rank 64 and N = 28672 the per-block slabs
-// were as large as dY itself.  TPW bounds the registers of the dB accumulators (TPW * RT * 4).
-// LDS: two dY tiles, the S block [128][R] and two B tiles [64][R] (pitch 2R+32 bytes keeps the 4-row transpose reads on
-// distinct banks).  The S block is single-buffered: at a block switch one extra barrier separates its last readers
-// from the store of the next block's S (prefetched in registers one tile earlier).
-template <typename T, int RT, int TPW>
-__global__ void __launch_bounds__(256, RT == 1 ? 3 : RT <= 4 ? 2 : 1)   // waves per SIMD: the register budget follows the LDS footprint
-lora_dys_dyb_kernel(const T* __restrict__ dY, const T* __restrict__ S, float* __restrict__ ds_part,
-                    float* __restrict__ db_part, int M, int N, int R, int tiles_per_wg, int group, int max_chunks,
-                    const LfSegTable seg) {
-  constexpr int RP = RT * 32 + 32;
-  constexpr int NBR = (64 * RT * 2 + 255) / 256;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  char* ys = lds;
-  char* ss = lds + 2 * TILE_BYTES;
-  char* bs = ss + ROWS * RP;
-
-  const int s = blockIdx.x / max_chunks, ch = blockIdx.x % max_chunks, ns = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, qq = lane >> 4, j4 = li >> 2, c4 = li & 3;
-  int b0, b1;
-  segment_blocks(seg, s, M, b0, b1);
-  const int bb0 = b0 + ch * group, bb1 = min(bb0 + group, b1);
-  if (bb0 >= b1) return;  // this segment has fewer chunks (uniform for the whole workgroup)
-  const int rank = seg.rank[s];
-  const T* __restrict__ Bl = (const T*)seg.ptr[s];
-  const int Mrows = seg.table ? seg.n_blocks * ROWS : M;
-  const int n_begin = ns * tiles_per_wg * 64;
-  const int ntiles = min(tiles_per_wg, N / 64 - ns * tiles_per_wg);  // the last slice may be shorter
-  const int total = (bb1 - bb0) * ntiles;                             // (block, tile) pairs, block-major
-
-  auto valid_rows = [&](int b) { return seg.table ? seg.table[3 * b + 1] : min(ROWS, M - b * ROWS); };
-  auto load_b = [&](lf_u32x4 (&br)[NBR], int n0) {
-#pragma unroll
-    for (int i = 0; i < NBR; i++) {
-      const int g = i * 256 + tid;
-      const int row = g / (RT * 2), gc = g % (RT * 2);
-      lf_u32x4 v = {0, 0, 0, 0};
-      if (g < 64 * RT * 2 && gc * 8 < rank) v = *(const lf_u32x4*)(Bl + (int64_t)(n0 + row) * rank + gc * 8);
-      br[i] = v;
-    }
-  };
-  auto store_b = [&](const lf_u32x4 (&br)[NBR], char* dst) {
-#pragma unroll
-    for (int i = 0; i < NBR; i++) {
-      const int g = i * 256 + tid;
-      if (g < 64 * RT * 2) *(lf_u32x4*)(dst + (g / (RT * 2)) * RP + (g % (RT * 2)) * 16) = br[i];
-    }
-  };
-  // S block of row block b (rows beyond its valid count as zeros, so they add nothing to dB).  S has R columns; R may
-  // be smaller than the RT * 16 columns of the register tiling (R = 48, 80, 96, 112)
-  auto load_s = [&](lf_u32x4 (&sr)[RT], int b) {
-    const int valid = valid_rows(b);
-#pragma unroll
-    for (int i = 0; i < RT; i++) {
-      const int g = i * 256 + tid;
-      const int row = g / (RT * 2), gc = g % (RT * 2);
-      lf_u32x4 v = {0, 0, 0, 0};
-      if (row < valid && gc * 8 < R) v = *(const lf_u32x4*)(S + (int64_t)(b * ROWS + row) * R + gc * 8);
-      sr[i] = v;
-    }
-  };
-  auto store_s = [&](const lf_u32x4 (&sr)[RT]) {
-#pragma unroll
-    for (int i = 0; i < RT; i++) {
-      const int g = i * 256 + tid;
-      *(lf_u32x4*)(ss + (g / (RT * 2)) * RP + (g % (RT * 2)) * 16) = sr[i];
-    }
-  };
-  // coordinates of pair q
-  auto blk_of = [&](int q) { return bb0 + q / ntiles; };
-  auto col_of = [&](int q) { return n_begin + (q % ntiles) * 64; };
-
-  TileRegs tr;
-  lf_u32x4 br[NBR], sr[RT];
-  tile_load(tr, dY, (const uint8_t*)nullptr, N, bb0 * ROWS, Mrows, n_begin, tid, false, false);
-  load_b(br, n_begin);
-  load_s(sr, bb0);
-  store_s(sr);
-  tile_store(tr, ys, tid, false);
-  store_b(br, bs);
-  if (total > 1) {
-    tile_load(tr, dY, (const uint8_t*)nullptr, N, blk_of(1) * ROWS, Mrows, col_of(1), tid, false, false);
-    load_b(br, col_of(1));
-    if (ntiles == 1) load_s(sr, blk_of(1));
-  }
-  __syncthreads();
-
-  lf_f32x4 acc_db[TPW][RT];
-#pragma unroll
-  for (int t = 0; t < TPW; t++)
-#pragma unroll
-    for (int c = 0; c < RT; c++) acc_db[t][c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
-
-  int q = 0;
-  for (int b = bb0; b < bb1; b++) {
-    lf_f32x4 acc_ds[2][RT];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int c = 0; c < RT; c++) acc_ds[a][c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < TPW; t++) {
-      if (t < ntiles) {
-        const char* ycur = ys + (q & 1) * TILE_BYTES;
-        const char* bcur = bs + (q & 1) * 64 * RP;
-        // dS += dY_tile * B_tile : a = dY row fragment, b = B^T through the transpose read
-#pragma unroll
-        for (int step = 0; step < 2; step++) {
-          lf_u32x4 yf[2];
-#pragma unroll
-          for (int rt = 0; rt < 2; rt++) yf[rt] = tile_row_frag(ycur, wave * 32 + rt * 16 + li, step * 4 + qq);
-#pragma unroll
-          for (int c = 0; c < RT; c++) {
-            const lf_u32x4 bf = tr_read8(bcur + (step * 32 + qq * 8 + j4) * RP + (c * 16 + 4 * c4) * 2, RP);
-#pragma unroll
-            for (int rt = 0; rt < 2; rt++) acc_ds[rt][c] = Mfma16<T>::run(yf[rt], bf, acc_ds[rt][c]);
-          }
-        }
-        // dB tile: D[n][r] += sum_m dY[m][n] S[m][r]; wave w owns columns 16w..16w+15 of the tile
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-          const int mrow = kk * 32 + qq * 8 + j4;
-          const lf_u32x4 yt = tile_tr_frag(ycur, mrow, wave * 16 + 4 * c4);
-#pragma unroll
-          for (int c = 0; c < RT; c++) {
-            const lf_u32x4 sf = tr_read8(ss + mrow * RP + (c * 16 + 4 * c4) * 2, RP);
-            acc_db[t][c] = Mfma16<T>::run(yt, sf, acc_db[t][c]);
-          }
-        }
-        if (q + 1 < total) {
-          if (t + 1 == ntiles) {  // the next pair opens a new block: everyone is done with this block's S
-            __syncthreads();
-            store_s(sr);
-          }
-          tile_store(tr, ys + ((q + 1) & 1) * TILE_BYTES, tid, false);
-          store_b(br, bs + ((q + 1) & 1) * 64 * RP);
-          if (q + 2 < total) {
-            tile_load(tr, dY, (const uint8_t*)nullptr, N, blk_of(q + 2) * ROWS, Mrows, col_of(q + 2), tid, false, false);
-            load_b(br, col_of(q + 2));
-            if ((q + 2) % ntiles == 0) load_s(sr, blk_of(q + 2));
-          }
-        }
-        __syncthreads();
-        q++;
-      }
-    }
-    float* dso = ds_part + (int64_t)ns * Mrows * R;
-#pragma unroll
-    for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-      for (int c = 0; c < RT; c++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int row = b * ROWS + wave * 32 + rt * 16 + qq * 4 + e;
-          if (row < Mrows && c * 16 < R) dso[(int64_t)row * R + c * 16 + li] = acc_ds[rt][c][e];
-        }
-  }
-  // C layout: column (r) = lane & 15, rows (n) = 4*(lane >> 4) + e
-  float* dbo = db_part + (((int64_t)s * max_chunks + ch) * N + n_begin) * R;
-#pragma unroll
-  for (int t = 0; t < TPW; t++)
-    if (t < ntiles) {
-#pragma unroll
-      for (int c = 0; c < RT; c++)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (c * 16 < R) dbo[(int64_t)(t * 64 + wave * 16 + qq * 4 + e) * R + c * 16 + li] = acc_db[t][c][e];
-    }
-}
-
 // out_s = cast( mult * sum over parts of part[...] ) for segment s = blockIdx.y.
 //   transposed == 0 (dB): parts are the segment's chunks, part[(s*max_chunks + ch)][n][R] -> out [rows, rank]
 //   transposed == 1 (dA): parts are the segment's chunks, part[(s*max_chunks + ch)][R][rows] -> out [rank, rows]
@@ -595,105 +375,12 @@ reduce_ds_db_kernel(const float* __restrict__ ds_part, T* __restrict__ dS, int n
   }
 }
 
-// ------------------------------------------------------------------------------------ da
-// grid (K/64, max_chunks, n_seg).  Workgroup (kt, ch, s) owns the 64 columns kt*64.. of dA_s and
-// the `group` consecutive 128-row blocks ch*group.. of segment s; it accumulates
-//   D[r][k] = sum_m dS[m][r] * mask*X[m][k]     (1/(1-p) is applied by the reduce)
-// over its blocks and writes one fp32 partial [R][64].  Both operands are read from LDS through
-// the transpose path since the contraction index m is the slow dimension of both.
-template <typename T, int RT>
-__global__ void __launch_bounds__(256)
-lora_da_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, int mask_bits, const T* __restrict__ dS,
-               float* __restrict__ part, int M, int K, int R, int group, int max_chunks, const LfSegTable seg) {
-  constexpr int RP = RT * 32 + 32;
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  char* xs = lds;
-  char* dss = lds + 2 * TILE_BYTES;
-  const int kt = blockIdx.x, ch = blockIdx.y, s = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, qq = lane >> 4, j4 = li >> 2, c4 = li & 3;
-  int b0, b1;
-  segment_blocks(seg, s, M, b0, b1);
-  const int bb0 = b0 + ch * group, bb1 = min(bb0 + group, b1);
-  if (bb0 >= b1) return;  // this segment has fewer chunks (uniform for the whole workgroup)
-  const float p = seg.table ? (seg.block_p ? seg.block_p[b0] : 0.f) : seg.p;
-  const bool use_mask = mask != nullptr && p > 0.f;
-  const int Mrows = seg.table ? seg.n_blocks * ROWS : M;
-
-  auto valid_rows = [&](int b) { return seg.table ? seg.table[3 * b + 1] : min(ROWS, M - b * ROWS); };
-  auto load_ds = [&](lf_u32x4 (&dr)[RT], int b) {
-    const int valid = valid_rows(b);
-#pragma unroll
-    for (int i = 0; i < RT; i++) {
-      const int g = i * 256 + tid;
-      const int row = g / (RT * 2), gc = g % (RT * 2);
-      lf_u32x4 v = {0, 0, 0, 0};
-      if (row < valid && gc * 8 < R) v = *(const lf_u32x4*)(dS + (int64_t)(b * ROWS + row) * R + gc * 8);
-      dr[i] = v;
-    }
-  };
-  auto store_ds = [&](const lf_u32x4 (&dr)[RT], char* dst) {
-#pragma unroll
-    for (int i = 0; i < RT; i++) {
-      const int g = i * 256 + tid;
-      *(lf_u32x4*)(dst + (g / (RT * 2)) * RP + (g % (RT * 2)) * 16) = dr[i];
-    }
-  };
-
-  TileRegs tr;
-  lf_u32x4 dr[RT];
-  tile_load(tr, X, mask, K, bb0 * ROWS, Mrows, kt * 64, tid, use_mask, mask_bits != 0);
-  load_ds(dr, bb0);
-  tile_store(tr, xs, tid, use_mask, mask_bits != 0);
-  store_ds(dr, dss);
-  if (bb0 + 1 < bb1) {
-    tile_load(tr, X, mask, K, (bb0 + 1) * ROWS, Mrows, kt * 64, tid, use_mask, mask_bits != 0);
-    load_ds(dr, bb0 + 1);
-  }
-  __syncthreads();
-
-  lf_f32x4 acc[RT];
-#pragma unroll
-  for (int c = 0; c < RT; c++) acc[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
-
-  for (int b = bb0; b < bb1; b++) {
-    const int t = b - bb0;
-    const char* xcur = xs + (t & 1) * TILE_BYTES;
-    const char* dcur = dss + (t & 1) * ROWS * RP;
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      const int mrow = kk * 32 + qq * 8 + j4;
-      const lf_u32x4 xt = tile_tr_frag(xcur, mrow, wave * 16 + 4 * c4);
-#pragma unroll
-      for (int c = 0; c < RT; c++) {
-        const lf_u32x4 df = tr_read8(dcur + mrow * RP + (c * 16 + 4 * c4) * 2, RP);
-        acc[c] = Mfma16<T>::run(df, xt, acc[c]);
-      }
-    }
-    if (b + 1 < bb1) {
-      tile_store(tr, xs + ((t + 1) & 1) * TILE_BYTES, tid, use_mask, mask_bits != 0);
-      store_ds(dr, dss + ((t + 1) & 1) * ROWS * RP);
-      if (b + 2 < bb1) {
-        tile_load(tr, X, mask, K, (b + 2) * ROWS, Mrows, kt * 64, tid, use_mask, mask_bits != 0);
-        load_ds(dr, b + 2);
-      }
-    }
-    __syncthreads();
-  }
-  // C layout: column (k) = lane & 15, rows (r) = 4*(lane >> 4) + e
-  float* po = part + ((int64_t)s * max_chunks + ch) * R * K;
-#pragma unroll
-  for (int c = 0; c < RT; c++)
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      if (c * 16 < R) po[(int64_t)(c * 16 + qq * 4 + e) * K + kt * 64 + wave * 16 + li] = acc[c][e];  // the partial has R rows
-}
-
 // ------------------------------------------------------------------ streaming through a ring of direct-to-LDS loads
-// The passes above keep one tile per workgroup in flight (it waits in registers between its load and its LDS store);
-// the LDS footprint allows two or three workgroups per CU, so a CU has 32-48 KB on order -- half of what the HBM
-// latency asks for, less at rank 64.  The kernels below (ranks up to 64) order their tiles as buffer loads that
-// write LDS themselves (no registers, no store instructions), NS - 1 tiles ahead of the one being consumed.
+// A tile that waits in registers between its load and its LDS store leaves a workgroup one tile on order -- a CU 16-48 KB, half of
+// what the HBM latency asks for and less.  The kernels below order their tiles as buffer loads that write LDS themselves (no
+// registers, no store instructions), NS - 1 tiles ahead of the one being consumed.  (Ranks above 64, one workgroup per CU
+// either way: 3000 x 5120 at rank 128, dys_dyb 33.8 -> 26.6 us and da 35.2 -> 22.0 against the register-staged form.  What bounds
+// them there: 61 MB and 16 MB of fp32 partials beside 31 MB of operand, and the two or three stages that fit next to the side blocks.)
 //
 // A load group is waited for by count: vector memory operations complete in issue order, so "at most n younger
 // operations outstanding" means the group has landed.  The loop therefore contains no other vector memory
@@ -741,11 +428,13 @@ __device__ __forceinline__ void tile_apply_mask(char* tile, const char* mtile, i
 
 // A [rows x RT*16] side operand (S or dS block: 128 rows; B tile: 64 rows) in LDS: rows of RT*32 bytes; granule g of
 // source row r at slot g ^ side_key(r) of LDS row side_row(r).  A transposed read is served 32 lanes at a time: rows
-// j, 8+j (j = 0..3), 32 bytes of each, which must land on eight different 32-byte groups of the 64 banks.  At 128-byte
+// j, 8+j (j = 0..3), 32 bytes of each, which must land on eight different 32-byte groups of the 64 banks.  At 256-byte rows
+// (all start on one bank) the key tells all eight apart; at 128-byte
 // rows the key separates (r>>3)&1 and (r>>1)&1 (the row's parity picks the half of the banks); at 64-byte rows
 // (r>>3)&1; at 32-byte rows no key can (a row is one group): rows 8..15 of every 16 swap their halves instead.
 template <int RT>
 __device__ __forceinline__ int side_key(int row) {
+  if constexpr (RT == 8) return ((row & 3) << 1) | (((row >> 3) & 1) << 3);
   return RT >= 4 ? ((((row >> 3) & 1) << 1) | (((row >> 1) & 1) << 2)) : RT == 2 ? ((row >> 3) & 1) << 1 : 0;
 }
 template <int RT>
@@ -785,7 +474,7 @@ __device__ __forceinline__ lf_u32x4 side_tr8(const char* blk, int row, int c, in
 //   D_j[r][k] += sum_m dS[m][r] * keep*X[m][k]   per tile j of the slice, in registers over all blocks of the chunk.
 // With a keep-mask the tile is masked in place one iteration before it is consumed.
 template <typename T, int RT, int TPW, int NS, int MASK>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, RT >= 8 ? 1 : 2)
 lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, const T* __restrict__ dS, float* __restrict__ part,
                     int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg) {
   // MASK: 0 no keep-mask; 1 one byte per element (8 KB per tile, two loads per thread); 2 one bit per element (1 KB per
@@ -825,6 +514,8 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   int64_t xleft = (((int64_t)Mrows - (int64_t)bb0 * ROWS) * K - (int64_t)kt0 * 64) * 2;
   const char* sb = (const char*)(dS + (int64_t)bb0 * ROWS * R);
   int64_t sleft = ((int64_t)Mrows - (int64_t)bb0 * ROWS) * R * 2;
+  // (rows of the segment's last block behind its valid ones read as zeros)
+  const int64_t slast = (int64_t)to_sgpr(seg.table ? seg.table[3 * (b1 - 1) + 1] : ROWS) * R * 2;
   const int64_t xnext = (int64_t)ROWS * K * 2 - (int64_t)nt * 128;   // from behind a block's last tile to the next block's first
   auto issue = [&]() {
     tile_dma(window_rsrc(xb, xleft), xv, lds0 + ist * STAGE, wave);
@@ -840,7 +531,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
       dma4(window_rsrc(mask != nullptr ? (const char*)mask + boff : (const char*)X, mask != nullptr ? (xleft >> 4) : 0), mv[0],
            lds0 + ist * STAGE + TILE_BYTES + wave * 256);
     }
-    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, sleft), dv, lds0 + NS * STAGE + ((ib - bb0) & 1) * SIDE, wave);
+    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), dv, lds0 + NS * STAGE + ((ib - bb0) & 1) * SIDE, wave);
     ist = ist + 1 == ns ? 0 : ist + 1;
     if (ib < bb1) {
       if (++ij < nt) {
@@ -969,12 +660,13 @@ lora_dys_dyb_ring_kernel(const T* __restrict__ dY, const T* __restrict__ S, floa
   int64_t bleft = ((int64_t)N - (int64_t)t0 * 64) * rank * 2;
   const char* sb = (const char*)(S + (int64_t)bb0 * ROWS * R);
   int64_t sleft = ((int64_t)Mrows - (int64_t)bb0 * ROWS) * R * 2;
+  const int64_t slast = (int64_t)to_sgpr(seg.table ? seg.table[3 * (b1 - 1) + 1] : ROWS) * R * 2;   // (as in the da kernel)
   const int64_t ynext = (int64_t)ROWS * N * 2 - (int64_t)nt * 128;   // from behind a block's last tile to the next block's first
   const int64_t bstep = (int64_t)64 * rank * 2;
   auto issue = [&]() {
     tile_dma(window_rsrc(yb, yleft), yv, lds0 + ist * STAGE, wave);
     side_dma<NIB>(window_rsrc(bp, bleft), bv, lds0 + ist * STAGE + TILE_BYTES, wave);
-    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, sleft), sv, lds0 + NS * STAGE + ((ib - bb0) & 1) * SIDE, wave);
+    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), sv, lds0 + NS * STAGE + ((ib - bb0) & 1) * SIDE, wave);
     ist = ist + 1 == ns ? 0 : ist + 1;
     if (ib < bb1) {
       if (++ij < nt) {
@@ -1080,65 +772,6 @@ lora_dys_dyb_ring_kernel(const T* __restrict__ dY, const T* __restrict__ S, floa
 
 }  // namespace
 
-// Split of a length-`len` axis into slices (multiples of 64) so that blocks * split fills the
-// chip; `min_split` bounds the slice length from above.
-// Work split of the streaming passes.  A launch runs in rounds of resident workgroups (LDS-limited
-// slots per CU x 256 CUs); a workgroup walks `t` tiles in sequence, so the pass takes about
-// rounds * t tile times, plus a little per extra partial sum that the second stage must add.
-// Picks the t that minimises that (ties: larger t, fewer partials).  count(t) = workgroups at t.
-template <typename Count>
-static int pick_tiles_per_wg(int max_t, int slots, Count count) {
-  int best = 1;
-  double best_cost = 1e30;
-  for (int t = 1; t <= max_t; t++) {
-    const long wgs = count(t);
-    const double cost = (double)((wgs + slots - 1) / slots) * t + 0.15 * (double)wgs / (double)count(max_t);
-    if (cost <= best_cost) { best_cost = cost; best = t; }
-  }
-  return best;
-}
-static int dys_smem(int rt) { return 2 * TILE_BYTES + ROWS * (rt * 32 + 32) + 2 * 64 * (rt * 32 + 32); }
-// Shape of a dys_dyb launch: tiles per workgroup (<= the kernel's TPW), row blocks per chunk, chunks of the longest
-// segment.  Chosen by bytes moved: the dY stream counted in whole rounds of resident workgroups (a partly filled
-// round streams as long as a full one) plus the fp32 partial sums, written by the first stage and read by the second:
-// dS partials grow with the number of N slices, dB partials with the number of chunks.
-constexpr int dys_tpw(int rt) { return rt <= 2 ? 16 : rt == 4 ? 6 : 4; }   // dB accumulators: TPW * RT * 4 registers, next to 8 * RT of dS
-struct DysPlan { int tiles_per_wg, group, max_chunks, nsplit; };
-static DysPlan dys_plan(int M, int N, int R, const LfSegTable& seg) {
-  const int rt = rt_of(R), T = N / 64, nseg = seg.table ? seg.n_seg : 1;
-  const int nblk = n_row_blocks(M, seg);
-  const int64_t rows = seg.table ? (int64_t)nblk * ROWS : M;
-  int blocks[LF_MAX_SEG];
-  for (int s = 0; s < nseg; s++) {
-    const int b0 = seg.table ? seg.first_block[s] : 0;
-    const int b1 = seg.table ? ((s + 1 < nseg) ? seg.first_block[s + 1] : seg.n_blocks) : nblk;
-    blocks[s] = b1 - b0;
-  }
-  // two workgroups per CU from rank 32 on (registers), else what the LDS footprint allows
-  const int slots = rt >= 8 ? 256 : rt >= 2 ? 512 : lds_slots(dys_smem(rt));
-  DysPlan best{1, 1, 1, T};
-  double best_cost = 1e300;
-  for (int t = 1; t <= dys_tpw(rt) && t <= T; t++) {
-    const int nsplit = (T + t - 1) / t;
-    for (int g = 1; g <= 32; g *= 2) {
-      long chunks = 0;
-      int max_chunks = 1;
-      for (int s = 0; s < nseg; s++) {
-        const int c = (blocks[s] + g - 1) / g;
-        chunks += c;
-        max_chunks = c > max_chunks ? c : max_chunks;
-      }
-      const long wgs = chunks * nsplit;
-      const double rounds = (double)((wgs + slots - 1) / slots);
-      const double stream = rounds * slots * g * t * (double)TILE_BYTES;
-      const double partial = 2.0 * 4.0 * R * ((double)nsplit * rows + (double)nseg * max_chunks * N);
-      const double cost = stream + partial;
-      if (cost < best_cost) { best_cost = cost; best = DysPlan{t, g, max_chunks, nsplit}; }
-    }
-  }
-  return best;
-}
-
 // ---- work split of the ring kernels.  Workgroups (slice x chunk) of w tiles each run on `slots` resident slots; the
 // pass lasts about as long as its busiest slot.  Two upper bounds of that (in tiles): whole rounds of the largest
 // workgroup, and the list-scheduling bound sum / slots + largest; the smaller one is the estimate.
@@ -1186,8 +819,8 @@ static int all_group_stats(const int* blocks, int nseg, GroupStats (&st)[kNGroup
   return n;
 }
 
-constexpr int dysr_tpw(int rt) { return rt >= 2 ? 12 : 16; }
-constexpr int dysr_ns(int rt) { return rt >= 4 ? 5 : 3; }
+constexpr int dysr_tpw(int rt) { return rt >= 8 ? 4 : rt >= 2 ? 12 : 16; }   // dB accumulators: TPW * RT * 4 registers, next to 8 * RT of dS
+constexpr int dysr_ns(int rt) { return rt == 4 ? 5 : 3; }   // (rank 128: three stages of 32 KB and two S blocks of 32 KB are all of the LDS)
 static int dysr_smem(int rt) { return dysr_ns(rt) * (TILE_BYTES + (rt >= 2 ? rt / 2 : 1) * 4096) + 2 * ROWS * rt * 32; }
 struct DysRingPlan { int n_slices, group, max_chunks; };
 // By bytes: the dY (+ B tile) stream over the busiest slot, the S blocks every workgroup fetches (from L2: half weight),
@@ -1293,12 +926,8 @@ size_t lf_dys_dyb_workspace(int M, int N, int R, const LfSegTable& seg) {
   const int nblk = n_row_blocks(M, seg);
   const int64_t rows = seg.table ? (int64_t)nblk * ROWS : M;
   const int nseg = seg.table ? seg.n_seg : 1;
-  if (rt_of(R) <= 4) {
-    const DysRingPlan pl = dysr_plan(M, N, R, seg);
-    return ((size_t)pl.n_slices * rows * R + (size_t)nseg * pl.max_chunks * N * R) * sizeof(float);
-  }
-  const DysPlan pl = dys_plan(M, N, R, seg);
-  return ((size_t)pl.nsplit * rows * R + (size_t)nseg * pl.max_chunks * N * R) * sizeof(float);
+  const DysRingPlan pl = dysr_plan(M, N, R, seg);
+  return ((size_t)pl.n_slices * rows * R + (size_t)nseg * pl.max_chunks * N * R) * sizeof(float);
 }
 
 template <typename T, int RT>
@@ -1312,39 +941,20 @@ static int dysr_launch(const void* dY, const void* S, float* ds_part, float* db_
                    pl.n_slices, pl.group, pl.max_chunks, seg);
 }
 
-template <typename T, int RT>
-static int dys_launch(const void* dY, const void* S, float* ds_part, float* db_part, int M, int N, int R, const DysPlan& pl,
-                      dim3 grid, const LfSegTable& seg, hipStream_t st) {
-  auto kern = lora_dys_dyb_kernel<T, RT, dys_tpw(RT)>;
-  const int smem = dys_smem(RT);
-  static LfLdsFlags lds_ok;
-  if (!lf_allow_lds(kern, smem, lds_ok)) return LF_ELAUNCH;
-  return lf_launch(kern, grid, dim3(256), smem, st, (const T*)dY, (const T*)S, ds_part, db_part, M, N, R, pl.tiles_per_wg,
-                   pl.group, pl.max_chunks, seg);
-}
-
 template <typename T>
 static int dys_dyb_impl(const void* dY, const void* S, void* dS, void* ws, int M, int N, int R, const LfSegTable& seg, hipStream_t st) {
   const int nblk = n_row_blocks(M, seg);
   const int64_t rows = seg.table ? (int64_t)nblk * ROWS : M;
   const int nseg = seg.table ? seg.n_seg : 1;
   float* ds_part = (float*)ws;   // [slices][rows][R], then the dB partials [nseg * max_chunks][N][R]
-  float* db_part;
-  int rc, nparts, group, max_chunks;
-  if (rt_of(R) <= 4) {
-    const DysRingPlan pl = dysr_plan(M, N, R, seg);
-    db_part = ds_part + (int64_t)pl.n_slices * rows * R;
-    nparts = pl.n_slices, group = pl.group, max_chunks = pl.max_chunks;
-    switch (rt_of(R)) {
-      case 1: rc = dysr_launch<T, 1>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
-      case 2: rc = dysr_launch<T, 2>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
-      default: rc = dysr_launch<T, 4>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
-    }
-  } else {
-    const DysPlan pl = dys_plan(M, N, R, seg);
-    db_part = ds_part + (int64_t)pl.nsplit * rows * R;
-    nparts = pl.nsplit, group = pl.group, max_chunks = pl.max_chunks;
-    rc = dys_launch<T, 8>(dY, S, ds_part, db_part, M, N, R, pl, dim3(nseg * pl.max_chunks, pl.nsplit), seg, st);
+  const DysRingPlan pl = dysr_plan(M, N, R, seg);
+  float* db_part = ds_part + (int64_t)pl.n_slices * rows * R;
+  int rc;
+  switch (rt_of(R)) {
+    case 1: rc = dysr_launch<T, 1>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
+    case 2: rc = dysr_launch<T, 2>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
+    case 4: rc = dysr_launch<T, 4>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
+    default: rc = dysr_launch<T, 8>(dY, S, ds_part, db_part, M, N, R, pl, nseg, seg, st); break;
   }
   if (rc != LF_OK) return rc;
   const int64_t n = rows * R;
@@ -1353,7 +963,7 @@ static int dys_dyb_impl(const void* dY, const void* S, void* dS, void* ws, int M
   const int64_t nout = (int64_t)N * maxrank;
   const int nb_rows = (int)((n + 1023) / 1024), nb_seg = (int)((nout + 1023) / 1024);  // four outputs per thread
   return lf_launch((reduce_ds_db_kernel<T>), dim3((unsigned)(nb_rows + nb_seg * nseg)), dim3(256), 0, st, (const float*)ds_part,
-                     (T*)dS, nparts, M, R, nb_rows, (const float*)db_part, N, nb_seg, group, max_chunks, seg);
+                     (T*)dS, pl.n_slices, M, R, nb_rows, (const float*)db_part, N, nb_seg, pl.group, pl.max_chunks, seg);
 }
 
 int lf_launch_dys_dyb(const void* dY, const void* S, void* dS, void* ws, size_t ws_bytes, int M, int N, int R,
@@ -1371,33 +981,13 @@ int lf_launch_dys_dyb(const void* dY, const void* S, void* dS, void* ws, size_t 
   return LF_EINVAL;
 }
 
-// dA chunking: `group` consecutive 128-row blocks of a segment per workgroup, chosen by the same
-// round model as the other passes (a segment of b blocks gives ceil(b / group) chunks per K tile).
-static int da_smem(int rt) { return 2 * TILE_BYTES + 2 * ROWS * (rt * 32 + 32); }
-static void da_shape(int M, int K, int R, const LfSegTable& seg, int& group, int& max_chunks) {
-  const int nseg = seg.table ? seg.n_seg : 1;
-  int blocks[LF_MAX_SEG];
-  int max_blocks = 0;
-  for (int s = 0; s < nseg; s++) {
-    int b0 = seg.table ? seg.first_block[s] : 0;
-    int b1 = seg.table ? ((s + 1 < nseg) ? seg.first_block[s + 1] : seg.n_blocks) : (M + ROWS - 1) / ROWS;
-    blocks[s] = b1 - b0;
-    max_blocks = blocks[s] > max_blocks ? blocks[s] : max_blocks;
-  }
-  if (max_blocks < 1) max_blocks = 1;
-  group = pick_tiles_per_wg(max_blocks < 16 ? max_blocks : 16, lds_slots(da_smem(rt_of(R))), [&](int g) {
-    long chunks = 0;
-    for (int s = 0; s < nseg; s++) chunks += (blocks[s] + g - 1) / g;
-    return (long)(K / 64) * chunks;
-  });
-  max_chunks = (max_blocks + group - 1) / group;
-  if (max_chunks < 1) max_chunks = 1;
-}
-
 // Ring kernel shapes by rank tiles: tiles per slice (registers: TPW * RT * 4 accumulators) and ring depth (LDS: NS
 // stages of 16 KB, 24 KB with a keep-mask, plus two dS blocks of RT * 4 KB; two workgroups per CU where that fits).
 constexpr int da_tpw(int rt) { return rt >= 4 ? 8 : 16; }
-constexpr int da_ns(int rt, int maskfmt) { return maskfmt ? (rt == 1 ? 3 : 5) : (rt == 4 ? 3 : 4); }
+constexpr int da_ns(int rt, int maskfmt) {
+  if (rt == 8) return maskfmt == 1 ? 4 : 5;
+  return maskfmt ? (rt == 1 ? 3 : 5) : (rt == 4 ? 3 : 4);
+}
 static int da_ring_smem(int rt, int maskfmt) { return da_ns(rt, maskfmt) * (TILE_BYTES + da_mask_tile_bytes(maskfmt)) + 2 * ROWS * rt * 32; }
 struct DaPlan { int n_slices, group, max_chunks; };
 // Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by bytes moved: the
@@ -1429,28 +1019,10 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg) {
 
 size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg) {
   const int nseg = seg.table ? seg.n_seg : 1;
-  int max_chunks;
-  if (rt_of(R) <= 4) {
-    // the launch plans with or without a keep-mask (one byte or one bit per element): room for any
-    const int a = da_plan(M, K, R, 1, seg).max_chunks, b = da_plan(M, K, R, 0, seg).max_chunks, c = da_plan(M, K, R, 2, seg).max_chunks;
-    max_chunks = a > b ? a : b;
-    max_chunks = c > max_chunks ? c : max_chunks;
-  } else {
-    int group;
-    da_shape(M, K, R, seg, group, max_chunks);
-  }
+  // the launch plans with or without a keep-mask (one byte or one bit per element): room for any
+  int max_chunks = 1;
+  for (int fmt = 0; fmt < 3; fmt++) max_chunks = std::max(max_chunks, da_plan(M, K, R, fmt, seg).max_chunks);
   return (size_t)nseg * max_chunks * R * K * sizeof(float);
-}
-
-template <typename T, int RT>
-static int da_launch(const void* X, const uint8_t* mask, int mask_bits, const void* dS, float* part, int M, int K, int R, int group,
-                     int max_chunks, dim3 grid, const LfSegTable& seg, hipStream_t st) {
-  auto kern = lora_da_kernel<T, RT>;
-  constexpr int RP = RT * 32 + 32;
-  const int smem = 2 * TILE_BYTES + 2 * ROWS * RP;
-  static LfLdsFlags lds_ok;
-  if (!lf_allow_lds(kern, smem, lds_ok)) return LF_ELAUNCH;
-  return lf_launch(kern, grid, dim3(256), smem, st, (const T*)X, mask, mask_bits, (const T*)dS, part, M, K, R, group, max_chunks, seg);
 }
 
 template <typename T, int RT, int MASK>
@@ -1468,31 +1040,25 @@ template <typename T>
 static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, int M, int K, int R, const LfSegTable& seg, hipStream_t st) {
   const int nseg = seg.table ? seg.n_seg : 1;
   float* part = (float*)ws;
-  int group, max_chunks, rc;
-  if (rt_of(R) <= 4) {
-    const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
-    const DaPlan pl = da_plan(M, K, R, fmt, seg);
-    group = pl.group;
-    max_chunks = pl.max_chunks;
+  int rc;
+  const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
+  const DaPlan pl = da_plan(M, K, R, fmt, seg);
 #define LF_DA_RING(RTV)                                                                                                   \
   rc = fmt == 2   ? da_ring_launch<T, RTV, 2>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
        : fmt == 1 ? da_ring_launch<T, RTV, 1>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
                   : da_ring_launch<T, RTV, 0>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)
-    switch (rt_of(R)) {
-      case 1: LF_DA_RING(1); break;
-      case 2: LF_DA_RING(2); break;
-      default: LF_DA_RING(4); break;
-    }
-#undef LF_DA_RING
-  } else {
-    da_shape(M, K, R, seg, group, max_chunks);
-    rc = da_launch<T, 8>(X, mask, mask_bits, dS, part, M, K, R, group, max_chunks, dim3(K / 64, max_chunks, nseg), seg, st);
+  switch (rt_of(R)) {
+    case 1: LF_DA_RING(1); break;
+    case 2: LF_DA_RING(2); break;
+    case 4: LF_DA_RING(4); break;
+    default: LF_DA_RING(8); break;
   }
+#undef LF_DA_RING
   if (rc != LF_OK) return rc;
   int maxrank = 0;
   for (int s = 0; s < nseg; s++) maxrank = seg.rank[s] > maxrank ? seg.rank[s] : maxrank;
   const int64_t nout = (int64_t)K * maxrank;
-  return lf_launch((reduce_segments_kernel<T>), dim3((unsigned)((nout + 1023) / 1024), nseg), dim3(256), 0, st, (const float*)part, K, R, 1, mask != nullptr ? 1 : 2, M, group, max_chunks, seg);
+  return lf_launch((reduce_segments_kernel<T>), dim3((unsigned)((nout + 1023) / 1024), nseg), dim3(256), 0, st, (const float*)part, K, R, 1, mask != nullptr ? 1 : 2, M, pl.group, pl.max_chunks, seg);
 }
 
 int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, size_t ws_bytes, int M, int K, int R,

@@ -88,3 +88,50 @@ def test_short_forward(M, K, N, r, dtype, bias):
     _close(y, ye, "Y")
     _close(s[:, :r], se, "S")
     assert not s[:, r:].any()
+
+
+@pytest.mark.parametrize("mask_form", ["none", "bytes", "bits"])
+@pytest.mark.parametrize("M,N,r,dtype", [(1, 128, 72, torch.bfloat16), (129, 640, 128, torch.float16), (700, 1152, 96, torch.bfloat16),
+                                         (2500, 256, 120, torch.float16)])
+def test_backward_passes_of_high_ranks(M, N, r, dtype, mask_form):
+    """dS, dB and dA above 64 rank columns: one and several blocks and slices, ranks that fill the tiling and ranks that do not."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    g = torch.Generator().manual_seed(M + r)
+    dy, s = torch.randn(M, N, generator=g).to(dtype), torch.randn(M, r, generator=g).to(dtype)
+    b = (torch.randn(N, r, generator=g) * 0.05).to(dtype)
+    db, ds = hip_ops.fused_lora_dys_dyb(dy.cuda(), b.cuda(), s.cuda(), 2.0)
+    _close(ds[:, :r], 2.0 * (dy.float() @ b.float()), "dS")
+    _close(db, 2.0 * (dy.float().T @ s.float()), "dB")
+    assert not ds[:, r:].any()
+    p = 0.0 if mask_form == "none" else 0.2
+    mask = torch.rand(M, N, generator=g) >= p
+    x = torch.where(mask, dy.float() / (1 - p), torch.zeros(())) if p else dy.float()
+    md = None if p == 0 else hip_ops.pack_mask(mask.cuda()) if mask_form == "bits" else mask.cuda()
+    _close(hip_ops.fused_lora_da(dy.cuda(), s.cuda(), r, p, md), s.float().T @ x, "dA")
+
+
+@pytest.mark.parametrize("ranks", [[128, 72], [64, 16]])
+def test_backward_passes_leave_padding_out(ranks):
+    """Rows behind an adapter's tokens add nothing to its gradients, whatever S and dS hold there."""
+    from lorafusion_amd.ops import hip_ops
+    from lorafusion_amd.ops.multi_lora import prepare_multi_lora_batch_info
+
+    seq, N = [200, 70], 384
+    info = prepare_multi_lora_batch_info(seq, [0, 1], ranks, [0.0, 0.0], [1.0, 2.0], 128)
+    routing = hip_ops.MultiRouting(info.padded_seq_len_list, ranks, info.block_to_lookup_table, info.block_to_alpha, info.block_to_dropout_p)
+    g = torch.Generator().manual_seed(3)
+    M, R = routing.M, routing.R
+    dy, s = torch.randn(M, N, generator=g).bfloat16(), torch.randn(M, R, generator=g).bfloat16()   # (padding not zero)
+    b = [(torch.randn(N, r, generator=g) * 0.05).bfloat16() for r in ranks]
+    db, ds = hip_ops.fused_multi_lora_dys_dyb(dy.cuda(), s.cuda(), [t.cuda() for t in b], routing)
+    da = hip_ops.fused_multi_lora_da(dy.cuda(), s.cuda(), routing)
+    c = 0
+    for i, (q, pl, r) in enumerate(zip(seq, info.padded_seq_len_list, ranks)):
+        y, si, sc = dy[c:c + q].float(), s[c:c + q, :r].float(), [1.0, 2.0][i]
+        _close(ds[c:c + q, :r], sc * (y @ b[i].float()), f"dS {i}")
+        _close(db[i], sc * (y.T @ si), f"dB {i}")
+        _close(da[i], si.T @ y, f"dA {i}")
+        assert not ds[c + q:c + pl].any()
+        c += pl
