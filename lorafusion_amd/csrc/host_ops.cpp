@@ -43,6 +43,21 @@ template <typename... A>
   throw py::value_error(s.str());
 }
 
+class NotImplemented : public py::builtin_exception {
+ public:
+  using builtin_exception::builtin_exception;
+  void set_error() const override { PyErr_SetString(PyExc_NotImplementedError, what()); }
+};
+// The kernels read the values alone: a forward-mode tangent of an operand would be lost without a word.
+template <typename... L>
+void refuse_tangents(const L&... operands) {
+  if ((torch::autograd::isFwGradDefined(operands) || ...))
+    throw NotImplemented("the fused LoRA, norm and activation functions have no forward-mode derivative.");
+}
+void refuse_tangents_of(const std::vector<Tensor>& t) {
+  for (const Tensor& v : t) refuse_tangents(v);
+}
+
 void check(int rc, const char* what) {
   if (rc != LF_OK) throw std::runtime_error(std::string(what) + " failed: " + lf_strerror(rc) + " (code " + std::to_string(rc) + ")");
 }
@@ -92,7 +107,10 @@ struct Ptrs {
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 
 bool is_bits(const Tensor& mask, int64_t K) { return mask.defined() && mask.scalar_type() == at::kByte && mask.size(-1) * 8 == K; }
-int64_t rows_of(const Tensor& t) { return t.numel() / t.size(-1); }
+int64_t rows_of(const Tensor& t) {
+  if (t.size(-1) == 0) throw std::runtime_error("the number of rows of a tensor of shape " + shape_name(t.sizes()) + " is not defined.");
+  return t.numel() / t.size(-1);
+}
 
 Tensor scratch(size_t bytes, const Tensor& like) {
   return bytes ? at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)) : Tensor();
@@ -358,6 +376,7 @@ Tensor linear_lora(const Tensor& x, const Tensor& w, const Tensor& a, const Tens
   check_dims(M, N, K);
   check_rank(rank);
   if (!(p >= 0.0 && p < 1.0)) bad_value("dropout_p must be in [0, 1), got ", p, ".");
+  refuse_tangents(x, w, a, b, bias);
 
   Weight wt;
   const int R = round_rank((int)rank);
@@ -393,6 +412,9 @@ Weight weight_at(const OptTensor& w, uintptr_t nf4, const std::vector<Tensor>& k
 std::tuple<Tensor, Tensor, OptTensor, OptTensor> py_forward(const Tensor& x, const OptTensor& w, uintptr_t nf4, int N, const std::vector<Tensor>& a,
                                                            const std::vector<Tensor>& b, uintptr_t routing, int R, const OptTensor& mask,
                                                            std::optional<uint64_t> seed, bool packed, const OptTensor& bias, bool keep_dense) {
+  refuse_tangents(x, w, bias);
+  refuse_tangents_of(a);
+  refuse_tangents_of(b);
   const at::AutoDispatchBelowADInplaceOrView below;
   const c10::DeviceGuard device(x.device());
   Weight wt = weight_at(w, nf4, {});
@@ -429,6 +451,7 @@ Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tenso
   variable_list edges = inputs;
   edges.insert(edges.end(), a.begin(), a.end());
   edges.insert(edges.end(), b.begin(), b.end());
+  refuse_tangents_of(edges);
   if (at::GradMode::is_enabled() && torch::autograd::any_variable_requires_grad(edges))
     attach(out, edges, x, weight_at(w, nf4, keep), as, bs, mask.value_or(Tensor()), s, dense.value_or(Tensor()), act, routing_at(routing), tables, R, label);
   return out;
@@ -484,6 +507,7 @@ Tensor rms_norm(const Tensor& x, const Tensor& w, double eps) {
   if (w.scalar_type() != x.scalar_type()) bad_value("RMSNorm weight dtype ", dtype_name(w.scalar_type()), " differs from the input's ", dtype_name(x.scalar_type()), ".");
   const int64_t H = x.size(-1);
   if (w.dim() != 1 || w.size(0) != H) bad_value("RMSNorm weight shape ", shape_name(w.sizes()), " does not match the hidden size ", H, ".");
+  refuse_tangents(x, w);
   Tensor xs, ws, y, rstd;
   {
     const at::AutoDispatchBelowADInplaceOrView below;
@@ -553,6 +577,7 @@ Tensor silu_mul(const Tensor& a, const Tensor& b) {
   if (a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type())
     bad_value("silu_mul operands differ: ", shape_name(a.sizes()), " ", dtype_name(a.scalar_type()), " vs ", shape_name(b.sizes()), " ", dtype_name(b.scalar_type()), ".");
   if (a.size(-1) % 8 != 0) bad_value("the last dimension must be a multiple of 8, got ", a.size(-1), ".");
+  refuse_tangents(a, b);
   Tensor c;
   {
     const at::AutoDispatchBelowADInplaceOrView below;
@@ -579,6 +604,7 @@ Tensor silu_mul_merged(const Tensor& gu) {
   require_gpu(gu, "gate_up");
   const int64_t I2 = gu.size(-1), I = I2 / 2;
   if (I2 % 16 != 0) bad_value("the merged width must be a multiple of 16, got ", I2, ".");
+  refuse_tangents(gu);
   Tensor g, c;
   std::vector<int64_t> cs = gu.sizes().vec();
   cs.back() = I;
