@@ -170,13 +170,13 @@ gemm_big_kernel(const LfGemmParams p, const LfSegTable seg) {
   const int nk = p.K / BK;
 
   // Tile `it` of this workgroup -> first row / column and the start of its K walk.  XCD-aware (workgroup ids that
-  // differ by a multiple of 8 share an XCD and its L2: they get neighbouring tiles), grouped 8 tile rows deep.  A tile
+  // differ by a multiple of 8 share an XCD and its L2: they get neighbouring tiles), grouped a few tile rows deep.  A tile
   // that would cross the matrix edge is shifted inwards instead (M, N >= 256): it recomputes a few rows / columns of
   // its neighbour -- identical values, since both walk K from the same start -- and no load or store needs a guard.
   struct Tile { int m0, n0, kstart; };
   auto tile_of = [&](int it) __attribute__((always_inline)) {
     const int pid = lf_xcd_order(it * G + wg, total);
-    const int GROUP_M = p.group_m;   // tile rows per group: 8, or 2 for a long K over few tile columns (see the launcher)
+    const int GROUP_M = p.group_m;   // tile rows per group (group_rows below)
     const int width = GROUP_M * p.grid_n;
     const int group = pid / width;
     const int first_m = group * GROUP_M;
@@ -823,6 +823,25 @@ gemm_big_kernel(const LfGemmParams p, const LfSegTable seg) {
 #endif
 }
 
+// Tile rows per group of the tile order.  An XCD's 32 concurrent tiles form a block of group_rows tile rows x 32 / group_rows columns:
+// 4, 6 and 8 rows fetch 12 operand panels at a time, 2 fetch 18.  More columns side by side walk K from more different offsets, which
+// spreads their loads over the memory channels; six does not divide the 32, so neighbouring XCDs are out of step
+// too.  Timed for 298 products of 2048 - 16384 rows, 2048 - 57344 columns and K, both operand layouts, cold weights; relative to 8
+// everywhere but 2 for K >= 8192 under 16 columns, which was the rule before:
+//   short K                       6   0.97 (16384 x 14336 x 4096 NN 1352 -> 1283 us, 8192 x 8192 x 5120 NT 0.88)
+//   A beyond the 256 MB cache     4   0.96 (16384 x 14336 x 10240 NT 3926 -> 3498); up to 16 columns 2 stays: every pass over A
+//                                     comes from HBM, and 2 x 16 tiles read it once per round (16384 x 4096 x 14336 NT 1402, 4: 1457)
+//   long K, many columns, NN      4   0.98; NT 8 (4 level, 6 1.04)
+//   128-row tile                  8   0.95 from K = 10240 (2048 x 4096 x 28672 NT 460 -> 430), level below
+// Short K over many columns stays at 8 in the NT product once A takes half of that cache (16384 x 28672 x 4096: 2524, 6: 2577).
+int group_rows(int M, int K, int grid_n, int tile_rows, bool nn) {
+  const int64_t a_bytes = (int64_t)M * K * 2, cache = (int64_t)256 << 20;
+  if (tile_rows == 128) return 8;
+  if (K >= 8192 && a_bytes > cache) return grid_n <= 16 ? 2 : 4;
+  if (K < 8192 || grid_n <= 16) return !nn && grid_n > 32 && 2 * a_bytes >= cache ? 8 : 6;
+  return nn && grid_n > 32 ? 4 : 8;
+}
+
 template <typename T, bool NN, bool LORA, int TI>
 int launch_big(LfGemmParams p, const LfSegTable& seg, int max_wgs, hipStream_t st) {
   constexpr int BM = TI * 32;
@@ -832,12 +851,7 @@ int launch_big(LfGemmParams p, const LfSegTable& seg, int max_wgs, hipStream_t s
   static LfLdsFlags lds_ok;
   constexpr int SMEM_BYTES = Lds<NN, TI>::BYTES;
   if (!lf_allow_lds(kern, SMEM_BYTES, lds_ok)) return LF_ELAUNCH;
-  // Tile order: an XCD's 32 concurrent tiles form a block of group_m tile rows x 32 / group_m columns.  8 x 4 fetches
-  // the fewest operand panels (8 + 4).  With a long K and at most 16 tile columns the left operand does not fit the
-  // 256 MB memory-side cache and every pass over it is an HBM pass: 2 rows x 16 columns read it once per round
-  // (and as 16 neighbouring 128-byte pieces per row at a time) and leave the re-reads to the right operand, which the
-  // cache holds (16384x4096x14336: 1614 -> 1554 us; 16384x4096x28672: 3010 -> 2964 us; at K = 6144 it loses 8 %).
-  p.group_m = (p.K >= 8192 && p.grid_n <= 16) ? 2 : 8;
+  p.group_m = group_rows(p.M, p.K, p.grid_n, BM, NN);
   const long total = (long)p.grid_m * p.grid_n;
   const int grid = (int)(total < max_wgs ? total : max_wgs);
   return lf_launch(kern, dim3(grid), dim3(256), SMEM_BYTES, st, p, seg);
