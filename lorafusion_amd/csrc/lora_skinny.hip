@@ -65,7 +65,8 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 }
 
 // ------------------------------------------------------------------------------------ xa
-// One workgroup of 8 waves (2 above rank 64) per 16 rows (64 at ranks 48-64, 32 above); no partial sums leave the workgroup.  The K range is dealt
+// Ranks to 32, and every rank with the activation prologue (the sliced pass of lora_stream.hip takes the rest: lf_xa_streams).
+// One workgroup of 8 waves (2 above rank 64) per 16 rows (32 above rank 32); no partial sums leave the workgroup.  The K range is dealt
 // to the waves in 64-column steps (step s goes to wave s % waves), each wave streams its steps of the
 // 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), all loads of a batch
 // of steps in flight at once, applies the keep-mask in registers and turns the row-major
@@ -74,14 +75,12 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 // loads would put the four lanes of every quad on four different rows, a quarter of the
 // coalesced rate in the texture addresser.  The eight partial [16, R] accumulators are added in a fixed order through LDS,
 // scaled by 1/(1-p), zeroed in padded rows and beyond the adapter's rank, and stored as S.
-// Rows per workgroup: every workgroup reads the whole adapter matrix (from L2), which at rank 64 is four times the
-// bytes of 16 rows of X: with 32 rows per workgroup the pass ran at the L2's rate, not HBM's (268 workgroups x 1 MB of
-// A next to 140 MB of X at 8576 x 8192).  Ranks 48-64 take 64 rows (four row blocks share one set of A fragments)
-// and eight waves: 0.50 -> 0.40 ms over the four linears of the rank-64 layer.  At rank 16 two row blocks per
-// workgroup measured slower (0.27 -> 0.34 ms at the 8B layer: the registers of the second block cost loads in flight).
-// (with the activation prologue the up-half registers of four row blocks do not fit next to the rest at ranks 48-64: two)
-constexpr int xa_nb(int rt, bool act = false) { return rt == 4 ? (act ? 2 : 4) : rt > 4 ? 2 : 1; }
-constexpr int xa_rows(int rt, bool act = false) { return 16 * xa_nb(rt, act); }
+// Rows per workgroup: every workgroup reads the whole adapter matrix (from L2), which above rank 32 is several times the bytes of
+// 16 rows of X: two row blocks share a set of A fragments there (the up-half registers of four do not fit next to the rest).  At
+// rank 16 two row blocks per workgroup measured slower (0.27 -> 0.34 ms at the 8B layer: the registers of the second block cost
+// loads in flight).
+constexpr int xa_nb(int rt) { return rt >= 4 ? 2 : 1; }
+constexpr int xa_rows(int rt) { return 16 * xa_nb(rt); }
 // waves per workgroup and steps in flight per wave, by rank tiles (LDS: 2 KB * (1+RT) per wave; registers: 8 * RT per step)
 constexpr int xa_waves(int rt) { return rt <= 4 ? 8 : 2; }
 constexpr int xa_unroll(int rt) { return rt <= 1 ? 4 : rt <= 2 ? 2 : 1; }
@@ -99,7 +98,7 @@ __global__ void __launch_bounds__(xa_waves(RT) * 64)
 lora_xa_kernel(const T* __restrict__ X, const T* __restrict__ U, int64_t ldx, T* __restrict__ act_out,
                const uint8_t* __restrict__ mask, uint8_t* __restrict__ mask_out, int mask_bits,
                uint32_t seed_lo, uint32_t seed_hi, T* __restrict__ S, int M, int K, int R, const LfSegTable seg) {
-  constexpr int XA_WAVES = xa_waves(RT), XA_U = xa_unroll(RT), NB = xa_nb(RT, ACT), XA_ROWS = xa_rows(RT, ACT);
+  constexpr int XA_WAVES = xa_waves(RT), XA_U = xa_unroll(RT), NB = xa_nb(RT), XA_ROWS = xa_rows(RT);
   // the partial accumulators of the final sum reuse the patches (a barrier separates the two uses): at
   // rank 64 the separate 16 KB pushed the workgroup over 40 KB, and a CU then holds two workgroups, not four
   constexpr int PATCH_BYTES = XA_WAVES * 2048 * (NB + RT), RED_BYTES = XA_WAVES * XA_ROWS * RT * 16 * 4;
@@ -873,16 +872,20 @@ template <typename T, int RT>
 static int xa_launch(const void* X, const void* U, int64_t ldx, void* act_out, const uint8_t* mask, uint8_t* mask_out, int mask_bits,
                      uint64_t seed, void* S, int M, int K, int R, int64_t rows, const LfSegTable& seg, hipStream_t st) {
   const bool gen = mask_out != nullptr, act = U != nullptr;
-  const int wg_rows = xa_rows(RT, act);
+  constexpr int wg_rows = xa_rows(RT);
   const unsigned grid = (unsigned)((rows + wg_rows - 1) / wg_rows);
   const uint32_t lo = gen ? (uint32_t)seed : 0u, hi = gen ? (uint32_t)(seed >> 32) : 0u;
 #define LF_XA(GEN, ACT)                                                                                              \
   return lf_launch((lora_xa_kernel<T, RT, GEN, ACT>), dim3(grid), dim3(xa_waves(RT) * 64), 0, st, (const T*)X,       \
                    (const T*)U, ldx, (T*)act_out, mask, mask_out, mask_bits, lo, hi, (T*)S, M, K, R, seg)
   if (gen && act) LF_XA(true, true);
-  if (gen) LF_XA(true, false);
   if (act) LF_XA(false, true);
-  LF_XA(false, false);
+  if constexpr (RT <= 2) {
+    if (gen) LF_XA(true, false);
+    LF_XA(false, false);
+  } else {
+    return LF_EINVAL;   // (without the prologue these ranks take the sliced pass)
+  }
 #undef LF_XA
 }
 
