@@ -65,7 +65,7 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 }
 
 // ------------------------------------------------------------------------------------ xa
-// Ranks to 32, and every rank with the activation prologue (the sliced pass of lora_stream.hip takes the rest: lf_xa_streams).
+// Ranks to 32 (but for short batches: lf_xa_streams), and every rank with the activation prologue (the sliced pass of lora_stream.hip takes the rest).
 // One workgroup of 8 waves (2 above rank 64) per 16 rows (32 above rank 32); no partial sums leave the workgroup.  The K range is dealt
 // to the waves in 64-column steps (step s goes to wave s % waves), each wave streams its steps of the
 // 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), all loads of a batch
@@ -859,13 +859,15 @@ int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, vo
 // 10.1 us; 3000 x 5120, rank 128: 67 -> 19; 8576 x 28672, rank 64: 201 -> 148; 8576 x 8192: 40.6 -> 38.9), and with a
 // keep-mask up to 1024 rows, where drawing it on a few compute units is what takes the time (300 x 4096, rank 16: -2.5 us
 // drawn, level when read).  Elsewhere the second stage costs more than the slices give (4096 x 4096, rank 16: 7.9 against
-// 9.6 us).  The same choice for every mask format, drawn or read: S does not depend on how the mask came.
-bool lf_xa_streams(int M, int R, bool masked, const LfSegTable& seg) {
+// 9.6 us).  Without a mask up to 1024 rows from K = 8192, or from 4096 at ranks 17 - 32 up to 512 rows: the whole forward of
+// 333 x 14336 x 4096 71.7 -> 65.5 us at rank 16, 75.5 -> 65.5 at 32, of 1000 rows 125.4 -> 119.3, of 333 x 4096 x 14336 at rank 32 53.1 ->
+// 52.2; level at 4096 and rank 16, and at K = 1024 the second stage costs 20 % (333 x 1024 x 2048: 12.1 against 14.8).  The same choice for every mask format, drawn or read: S does not depend on how the mask came.
+bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
-  return R > 32 || (masked && rows <= 1024);
+  return R > 32 || (rows <= 1024 && (masked || K >= 8192 || (R > 16 && K >= 4096 && rows <= 512)));
 }
 size_t lf_xa_workspace(int M, int K, int R, const LfSegTable& seg) {
-  return lf_xa_streams(M, R, true, seg) ? lf_xa_stream_workspace(M, K, R, seg) : 0;
+  return lf_xa_streams(M, K, R, true, seg) ? lf_xa_stream_workspace(M, K, R, seg) : 0;
 }
 
 template <typename T, int RT>
@@ -916,7 +918,7 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
     if (ldx < K || ldx % 8 != 0 || (((uintptr_t)X | (uintptr_t)U | (uintptr_t)act_out) & 15) != 0) return LF_ESHAPE;
   } else {
     ldx = K;
-    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_streams(M, R, mask != nullptr || mask_out != nullptr, seg))
+    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_streams(M, K, R, mask != nullptr || mask_out != nullptr, seg))
       return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, seg) ? (float*)ws : nullptr, M, K,
                                  R, seg, dtype, st);
   }
