@@ -65,7 +65,7 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 }
 
 // ------------------------------------------------------------------------------------ xa
-// Ranks to 32 (but for short batches: lf_xa_streams), and every rank with the activation prologue (the sliced pass of lora_stream.hip takes the rest).
+// Ranks to 32, but for short batches (lf_xa_streams; the sliced pass of lora_stream.hip takes the rest).
 // One workgroup of 8 waves (2 above rank 64) per 16 rows (32 above rank 32); no partial sums leave the workgroup.  The K range is dealt
 // to the waves in 64-column steps (step s goes to wave s % waves), each wave streams its steps of the
 // 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), all loads of a batch
@@ -882,12 +882,8 @@ static int xa_launch(const void* X, const void* U, int64_t ldx, void* act_out, c
                    (const T*)U, ldx, (T*)act_out, mask, mask_out, mask_bits, lo, hi, (T*)S, M, K, R, seg)
   if (gen && act) LF_XA(true, true);
   if (act) LF_XA(false, true);
-  if constexpr (RT <= 2) {
-    if (gen) LF_XA(true, false);
-    LF_XA(false, false);
-  } else {
-    return LF_EINVAL;   // (without the prologue these ranks take the sliced pass)
-  }
+  if (gen) LF_XA(true, false);
+  LF_XA(false, false);
 #undef LF_XA
 }
 
@@ -899,8 +895,7 @@ static int xa_impl(const void* X, const void* U, int64_t ldx, void* act_out, con
   switch (rt_of(R)) {
     case 1: return xa_launch<T, 1>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
     case 2: return xa_launch<T, 2>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
-    case 4: return xa_launch<T, 4>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
-    default: return xa_launch<T, 8>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
+    default: return LF_ESHAPE;   // (lf_xa_streams: above rank 32 the sliced pass, behind an activation pass of its own)
   }
 }
 
