@@ -104,7 +104,8 @@ struct Ptrs {
   }
 };
 
-void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
+// (a host tensor has no stream: the nodes run on host tensors where the kernels are stood in for)
+void* stream_of(const Tensor& t) { return t.is_cuda() ? (void*)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream() : nullptr; }
 
 bool is_bits(const Tensor& mask, int64_t K) { return mask.defined() && mask.scalar_type() == at::kByte && mask.size(-1) * 8 == K; }
 int64_t rows_of(const Tensor& t) {
@@ -128,13 +129,30 @@ lf_routing single_routing(int rank, float scale, float p) {
 }
 int round_rank(int r) { return (r + 15) / 16 * 16; }
 
-// The base weight of a call: a 16-bit tensor, or NF4 codes with the tensors of their quant state.
+// The base weight of a call: a 16-bit tensor [N, K], or NF4 codes with the tensors of their quant state (whose owner the caller holds).
 struct Weight {
-  Tensor w;                    // 16-bit [N, K], or the packed codes
+  Tensor w;
   bool nf4 = false;
-  lf_nf4_weight c{};           // nf4: pointers into `w` and `keep`
-  std::vector<Tensor> keep;
+  lf_nf4_weight c{};
 };
+
+// NF4, for a backward: a Python callable, codes -> (address of their lf_nf4_weight, its owner).  The struct holds addresses, and a
+// weight may move between forward and backward (`p.data = ...` of an offloaded or gathered parameter, a hook that unpacks a
+// copy, a quant state moved along with it): it is made from what codes and state are when the backward runs.
+using PyRef = std::shared_ptr<py::object>;   // (let go of under the interpreter's lock, by whichever thread)
+PyRef py_ref(py::handle h) {
+  if (h.is_none()) return nullptr;
+  return PyRef(new py::object(py::reinterpret_borrow<py::object>(h)), [](py::object* o) {
+    py::gil_scoped_acquire gil;
+    delete o;
+  });
+}
+PyRef resolve_nf4(const py::object& of, const Tensor& codes, lf_nf4_weight& c) {
+  py::gil_scoped_acquire gil;
+  const py::tuple t = of(codes);
+  c = *(const lf_nf4_weight*)t[0].cast<uintptr_t>();
+  return py_ref(t[1]);
+}
 
 struct Forward { Tensor y, s, mask, dense; };
 
@@ -232,7 +250,7 @@ Tensor incoming(const variable_list& g, size_t i, at::IntArrayRef sizes, const a
 struct LoraBackward : Node {
   SavedVariable x, w, mask, s, dense;
   std::vector<SavedVariable> a, b, act;   // act: the merged gate/up tensor, or gate and up
-  Weight weight;                          // (its tensor sits in `w`)
+  PyRef nf4;                              // `w` holds NF4 codes: what makes their struct
   lf_routing r{};
   std::vector<Tensor> tables;
   int R = 0;
@@ -251,16 +269,19 @@ struct LoraBackward : Node {
     std::lock_guard<std::mutex> lock(mutex_);
     const Tensor xs = x.unpack(), ms = mask.unpack(), ss = s.unpack(), dn = dense.unpack();
     const std::vector<Tensor> as = unpack_all(a), bs = unpack_all(b), in = unpack_all(act);
+    Weight weight;
     weight.w = w.unpack();
+    weight.nf4 = nf4 != nullptr;
     const size_t n_in = has_act ? in.size() : 1;
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard device(xs.device());
     const Tensor dy = incoming(grads, 0, y_sizes, options);
     bool need = task_should_compute_output(0) || (n_in > 1 && task_should_compute_output(1));
+    // (no struct where nothing will be dequantised: the weight is at hand, or not needed)
+    const PyRef owner = weight.nf4 && need && !dn.defined() ? resolve_nf4(*nf4, weight.w, weight.c) : nullptr;
     const int64_t K = xs.size(-1), M = rows_of(xs);
     const std::vector<int64_t> flat = {M, K};
     Backward g = run_backward(dy, xs.contiguous(), weight, as, bs, ss, r, R, ms, dn, need, has_act ? at::IntArrayRef(flat) : at::IntArrayRef(in_sizes));
-    weight.w = Tensor();
     variable_list out;
     out.reserve(n_in + as.size() + bs.size());
     if (!has_act) {
@@ -294,13 +315,13 @@ struct LoraBackward : Node {
 
 // Make `y` the output of a LoraBackward whose inputs are `edges` (the differentiable input(s), then A_i, then B_i as the caller
 // holds them).  x, w, a, b: what the kernels read -- the same tensors where those are contiguous.
-void attach(const Tensor& y, const variable_list& edges, const Tensor& x, const Weight& w, const std::vector<Tensor>& a,
+void attach(const Tensor& y, const variable_list& edges, const Tensor& x, const Tensor& w, const PyRef& nf4, const std::vector<Tensor>& a,
             const std::vector<Tensor>& b, const Tensor& mask, const Tensor& s, const Tensor& dense, const std::vector<Tensor>& act,
             const lf_routing& r, const std::vector<Tensor>& tables, int R, const char* label) {
   std::shared_ptr<LoraBackward> n(new LoraBackward(), torch::autograd::deleteNode);
   n->set_next_edges(torch::autograd::collect_next_edges(edges));
   n->x = SavedVariable(x, false);
-  n->w = SavedVariable(w.w, false);
+  n->w = SavedVariable(w, false);
   n->mask = SavedVariable(mask, false);
   n->s = SavedVariable(s, false);
   n->dense = SavedVariable(dense, false);
@@ -308,8 +329,7 @@ void attach(const Tensor& y, const variable_list& edges, const Tensor& x, const 
   n->b = save_all(b);
   n->act = save_all(act);
   n->has_act = !act.empty();
-  n->weight = w;
-  n->weight.w = Tensor();
+  n->nf4 = nf4;
   n->r = r;
   n->tables = tables;
   n->R = R;
@@ -394,18 +414,18 @@ Tensor linear_lora(const Tensor& x, const Tensor& w, const Tensor& a, const Tens
     ys.back() = N;
     f = run_forward(xs, wt, as, bs, r, R, (int)N, mask, p > 0 ? seed : std::nullopt, true, bias.defined() ? bias.contiguous() : bias, false, ys);
   }
-  if (wants_grad({x, a, b})) attach(f.y, {x, a, b}, xs, wt, as, bs, f.mask, f.s, Tensor(), {}, r, {}, R, "FusedLinearLoRABackward");
+  if (wants_grad({x, a, b})) attach(f.y, {x, a, b}, xs, wt.w, nullptr, as, bs, f.mask, f.s, Tensor(), {}, r, {}, R, "FusedLinearLoRABackward");
   return f.y;
 }
 
 // ------------------------------------------------------------------------------------------- calls of the Python layer
 
 lf_routing routing_at(uintptr_t addr) { return *(const lf_routing*)addr; }
-Weight weight_at(const OptTensor& w, uintptr_t nf4, const std::vector<Tensor>& keep) {
+Weight weight_at(const OptTensor& w, uintptr_t nf4) {
   Weight t;
   t.w = w.value_or(Tensor());
   t.nf4 = nf4 != 0;
-  if (t.nf4) t.c = *(const lf_nf4_weight*)nf4, t.keep = keep;
+  if (t.nf4) t.c = *(const lf_nf4_weight*)nf4;
   return t;
 }
 
@@ -417,7 +437,7 @@ std::tuple<Tensor, Tensor, OptTensor, OptTensor> py_forward(const Tensor& x, con
   refuse_tangents_of(b);
   const at::AutoDispatchBelowADInplaceOrView below;
   const c10::DeviceGuard device(x.device());
-  Weight wt = weight_at(w, nf4, {});
+  Weight wt = weight_at(w, nf4);
   Forward f = run_forward(x, wt, a, b, routing_at(routing), R, N, mask.value_or(Tensor()), seed, packed, bias.value_or(Tensor()), keep_dense, {rows_of(x), N});
   return {f.y, f.s, f.mask.defined() ? OptTensor(f.mask) : std::nullopt, f.dense.defined() ? OptTensor(f.dense) : std::nullopt};
 }
@@ -428,16 +448,19 @@ std::tuple<OptTensor, std::vector<Tensor>, std::vector<Tensor>> py_backward(cons
                                                                            bool need_dx) {
   const at::AutoDispatchBelowADInplaceOrView below;
   const c10::DeviceGuard device(dy.device());
-  const Weight wt = weight_at(w, nf4, {});
+  const Weight wt = weight_at(w, nf4);
   Backward g = run_backward(dy, x, wt, a, b, s, routing_at(routing), R, mask.value_or(Tensor()), dense.value_or(Tensor()), need_dx, x.sizes());
   return {g.dx.defined() ? OptTensor(g.dx) : std::nullopt, g.da, g.db};
 }
 
 // `y` [M, N] as the differentiable result of a linear over `inputs` (x; or the merged gate/up tensor; or gate and up), of shape
 // inputs[0].shape[:-1] + [N].  x: the contiguous [.., K] input of the kernels; a, b: as the caller holds them.
-Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tensor& x, const OptTensor& w, uintptr_t nf4, const std::vector<Tensor>& keep,
-                 const std::vector<Tensor>& a, const std::vector<Tensor>& b, const OptTensor& mask, const Tensor& s, const OptTensor& dense,
+// nf4: None (or 0), or what makes the struct of the codes `w`.
+Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tensor& x, const OptTensor& w, const py::object& nf4_of,
+                 const std::vector<Tensor>&, const std::vector<Tensor>& a, const std::vector<Tensor>& b, const OptTensor& mask, const Tensor& s, const OptTensor& dense,
                  const std::vector<Tensor>& act, uintptr_t routing, const std::vector<Tensor>& tables, int R, const char* label) {
+  const PyRef nf4 = PyCallable_Check(nf4_of.ptr()) ? py_ref(nf4_of) : nullptr;
+  const py::gil_scoped_release nogil;
   Tensor out;
   std::vector<Tensor> as, bs;
   std::vector<int64_t> ys = inputs[0].sizes().vec();
@@ -453,7 +476,7 @@ Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tenso
   edges.insert(edges.end(), b.begin(), b.end());
   refuse_tangents_of(edges);
   if (at::GradMode::is_enabled() && torch::autograd::any_variable_requires_grad(edges))
-    attach(out, edges, x, weight_at(w, nf4, keep), as, bs, mask.value_or(Tensor()), s, dense.value_or(Tensor()), act, routing_at(routing), tables, R, label);
+    attach(out, edges, x, w.value_or(Tensor()), nf4, as, bs, mask.value_or(Tensor()), s, dense.value_or(Tensor()), act, routing_at(routing), tables, R, label);
   return out;
 }
 
@@ -637,7 +660,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("linear_lora", &linear_lora, nogil());
   m.def("forward", &py_forward, nogil());
   m.def("backward", &py_backward, nogil());
-  m.def("attach", &py_attach, nogil());
+  m.def("attach", &py_attach);   // (takes a Python object: lets go of the lock itself)
   m.def("check_adapters", &check_adapters, nogil());
   m.def("rms_norm", &rms_norm, nogil());
   m.def("silu_mul", &silu_mul, nogil());

@@ -208,12 +208,12 @@ class FusedLinearMultiLoRA:
         x2d = padded_x.detach().contiguous().view(padded_x.shape[-2], padded_x.shape[-1])
         a_list, b_list = list(ab[:n_adapters]), list(ab[n_adapters:])
         M, K = x2d.shape
-        wref = None
+        wref, nf4 = None, None
         if quant_state is not None:
             # NF4 base weight: linear_w holds the packed codes, quant_state its bitsandbytes-style state
-            from lorafusion_amd.ops.nf4 import NF4WeightRef
+            from lorafusion_amd.ops.nf4 import NF4WeightRef, nf4_struct_of
 
-            wref = NF4WeightRef(linear_w, quant_state)
+            wref, nf4 = NF4WeightRef(linear_w, quant_state), nf4_struct_of(quant_state)
             w_shape, w_dtype = tuple(wref.shape), wref.dtype
         else:
             linear_w = linear_w.contiguous()
@@ -254,8 +254,7 @@ class FusedLinearMultiLoRA:
                 if not hip_ops.is_packed_mask(mask, K):
                     mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
             y, s = hip_ops.lora_forward(x2d, linear_w, a_run, b_run, routing.c, routing.R, mask, bias)
-        nf4, keep = (ctypes.addressof(wref.c), wref.keep) if wref is not None else (0, [])
-        return host.attach(y, [padded_x], x2d, linear_w, nf4, [t for t in keep if t is not None], a_list, b_list, mask, s, dense, [],
+        return host.attach(y, [padded_x], x2d, linear_w, nf4, [], a_list, b_list, mask, s, dense, [],
                            ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
 
 

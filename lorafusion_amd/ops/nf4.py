@@ -126,6 +126,17 @@ class NF4WeightRef:
                            dense.data_ptr(), 1 if valid else 0, 0)
 
 
+def nf4_struct_of(quant_state):
+    """What a backward node holds of an NF4 weight: codes -> (address of their ``lf_nf4_weight``, its owner), from codes and
+    state as they are when it is called (either may have moved since the forward)."""
+
+    def at(packed: torch.Tensor):
+        ref = NF4WeightRef(packed, quant_state)
+        return ctypes.addressof(ref.c), ref
+
+    return at
+
+
 dequantize_nf4 = dequantize_nf4_triton
 
 
@@ -211,8 +222,8 @@ class FusedLinearLoRANF4:
         routing, R = L.single_routing(r, alpha, dropout_p if mask is not None else 0.0), L.round_rank(r)
         y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, [lora_a.contiguous()], [lora_b.contiguous()], routing, R, mask, bias,
                                                keep_dense=keep_dequantized)
-        return L.host().attach(y, [x], x2d, packed_w, ctypes.addressof(wref.c), [t for t in wref.keep if t is not None], [lora_a], [lora_b],
-                               mask, s, kept[0] if kept else None, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
+        return L.host().attach(y, [x], x2d, packed_w, nf4_struct_of(quant_state), [], [lora_a], [lora_b], mask, s,
+                               kept[0] if kept else None, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
 
 
 def fused_linear_lora_nf4(x, packed_w, quant_state, lora_a, lora_b, alpha, seed=None, dropout_p=0.0,
