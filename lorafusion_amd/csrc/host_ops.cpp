@@ -261,9 +261,12 @@ struct LoraBackward : Node {
 
   std::string name() const override { return label; }
   void release_variables() override {
+    PyRef state;   // (let go of behind the lock: that takes the interpreter's)
     std::lock_guard<std::mutex> lock(mutex_);
     for (SavedVariable* v : {&x, &w, &mask, &s, &dense}) v->reset_data();
     for (auto* l : {&a, &b, &act}) for (SavedVariable& v : *l) v.reset_data();
+    tables.clear();
+    state.swap(nf4);
   }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);

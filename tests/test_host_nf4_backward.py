@@ -78,6 +78,16 @@ P.data = P.data.clone()
 gc.collect()
 assert old() is None
 """,
+    "a_freed_graph_holds_neither_state_nor_tables": """
+t = torch.zeros(8)
+y, table, state = attach([t]), weakref.ref(t.untyped_storage()), weakref.ref(q)
+del t, q
+gc.collect()
+assert table() is not None and state() is not None
+y.backward(torch.ones_like(y))
+gc.collect()
+assert table() is None and state() is None and y.grad_fn is not None
+""",
 }
 
 
