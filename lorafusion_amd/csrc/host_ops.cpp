@@ -312,12 +312,13 @@ struct LoraBackward : Node {
     }
     for (Tensor& t : g.da) out.push_back(std::move(t));
     for (Tensor& t : g.db) out.push_back(std::move(t));
+    out.resize(num_outputs());   // (none for the base weight and the bias)
     return out;
   }
 };
 
-// Make `y` the output of a LoraBackward whose inputs are `edges` (the differentiable input(s), then A_i, then B_i as the caller
-// holds them).  x, w, a, b: what the kernels read -- the same tensors where those are contiguous.
+// Make `y` the output of a LoraBackward whose inputs are `edges` (the differentiable input(s), then A_i, then B_i, then base weight
+// and bias, as the caller holds them).  x, w, a, b: what the kernels read -- the same tensors where those are contiguous.
 void attach(const Tensor& y, const variable_list& edges, const Tensor& x, const Tensor& w, const PyRef& nf4, const std::vector<Tensor>& a,
             const std::vector<Tensor>& b, const Tensor& mask, const Tensor& s, const Tensor& dense, const std::vector<Tensor>& act,
             const lf_routing& r, const std::vector<Tensor>& tables, int R, const char* label) {
@@ -417,7 +418,8 @@ Tensor linear_lora(const Tensor& x, const Tensor& w, const Tensor& a, const Tens
     ys.back() = N;
     f = run_forward(xs, wt, as, bs, r, R, (int)N, mask, p > 0 ? seed : std::nullopt, true, bias.defined() ? bias.contiguous() : bias, false, ys);
   }
-  if (wants_grad({x, a, b})) attach(f.y, {x, a, b}, xs, wt.w, nullptr, as, bs, f.mask, f.s, Tensor(), {}, r, {}, R, "FusedLinearLoRABackward");
+  // (a base weight or bias that requires a gradient makes y differentiable; it receives none)
+  if (wants_grad({x, a, b, w, bias})) attach(f.y, {x, a, b, w, bias}, xs, wt.w, nullptr, as, bs, f.mask, f.s, Tensor(), {}, r, {}, R, "FusedLinearLoRABackward");
   return f.y;
 }
 
@@ -458,9 +460,10 @@ std::tuple<OptTensor, std::vector<Tensor>, std::vector<Tensor>> py_backward(cons
 
 // `y` [M, N] as the differentiable result of a linear over `inputs` (x; or the merged gate/up tensor; or gate and up), of shape
 // inputs[0].shape[:-1] + [N].  x: the contiguous [.., K] input of the kernels; a, b: as the caller holds them.
+// others: operands that make y differentiable where they require a gradient, and receive none (base weight, bias).
 // nf4: None (or 0), or what makes the struct of the codes `w`.
 Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tensor& x, const OptTensor& w, const py::object& nf4_of,
-                 const std::vector<Tensor>&, const std::vector<Tensor>& a, const std::vector<Tensor>& b, const OptTensor& mask, const Tensor& s, const OptTensor& dense,
+                 const std::vector<OptTensor>& others, const std::vector<Tensor>& a, const std::vector<Tensor>& b, const OptTensor& mask, const Tensor& s, const OptTensor& dense,
                  const std::vector<Tensor>& act, uintptr_t routing, const std::vector<Tensor>& tables, int R, const char* label) {
   const PyRef nf4 = PyCallable_Check(nf4_of.ptr()) ? py_ref(nf4_of) : nullptr;
   const py::gil_scoped_release nogil;
@@ -478,6 +481,7 @@ Tensor py_attach(const Tensor& y, const std::vector<Tensor>& inputs, const Tenso
   edges.insert(edges.end(), a.begin(), a.end());
   edges.insert(edges.end(), b.begin(), b.end());
   refuse_tangents_of(edges);
+  for (const OptTensor& t : others) edges.push_back(t.value_or(Tensor()));
   if (at::GradMode::is_enabled() && torch::autograd::any_variable_requires_grad(edges))
     attach(out, edges, x, w.value_or(Tensor()), nf4, as, bs, mask.value_or(Tensor()), s, dense.value_or(Tensor()), act, routing_at(routing), tables, R, label);
   return out;

@@ -254,7 +254,7 @@ class FusedLinearMultiLoRA:
                 if not hip_ops.is_packed_mask(mask, K):
                     mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
             y, s = hip_ops.lora_forward(x2d, linear_w, a_run, b_run, routing.c, routing.R, mask, bias)
-        return host.attach(y, [padded_x], x2d, linear_w, nf4, [], a_list, b_list, mask, s, dense, [],
+        return host.attach(y, [padded_x], x2d, linear_w, nf4, [linear_w, linear_bias], a_list, b_list, mask, s, dense, [],
                            ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
 
 

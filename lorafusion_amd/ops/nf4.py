@@ -222,7 +222,7 @@ class FusedLinearLoRANF4:
         routing, R = L.single_routing(r, alpha, dropout_p if mask is not None else 0.0), L.round_rank(r)
         y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, [lora_a.contiguous()], [lora_b.contiguous()], routing, R, mask, bias,
                                                keep_dense=keep_dequantized)
-        return L.host().attach(y, [x], x2d, packed_w, nf4_struct_of(quant_state), [], [lora_a], [lora_b], mask, s,
+        return L.host().attach(y, [x], x2d, packed_w, nf4_struct_of(quant_state), [linear_bias], [lora_a], [lora_b], mask, s,
                                kept[0] if kept else None, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
 
 

@@ -109,8 +109,8 @@ class FusedSwiGLULinearLoRA:
         routing_c = routing.c if routing is not None else L.single_routing(rank_list[0], alpha, p_used)
         x, y, s, mask = _swiglu_lora_forward(gv, uv, ld, linear_w, a_list, b_list, routing_c, R, mask, draw, bias)
         tables = [routing.table, routing.scale, routing.p] if routing is not None else []
-        return L.host().attach(y, inputs, x, linear_w, 0, [], list(ab[:n_adapters]), list(ab[n_adapters:]), mask, s, None, saved_in,
-                               ctypes.addressof(routing_c), tables, R, "FusedSwiGLULinearLoRABackward")
+        return L.host().attach(y, inputs, x, linear_w, 0, [linear_w, linear_bias], list(ab[:n_adapters]), list(ab[n_adapters:]), mask, s,
+                               None, saved_in, ctypes.addressof(routing_c), tables, R, "FusedSwiGLULinearLoRABackward")
 
 
 def fused_swiglu_linear_lora(gate_up, linear_w, lora_a, lora_b, alpha: float, seed: int | None = None,

@@ -41,6 +41,50 @@ def test_saved_tensor_hooks_run_and_raise_through():
     assert {(4, 128), (16, 128), (128, 16), (128, 128), (4, 16)} <= set(seen)
 
 
+def test_weight_and_bias_make_the_result_differentiable():
+    from lorafusion_amd import _lib as L
+
+    x, w, a, b = torch.randn(4, 128), torch.randn(128, 128), torch.randn(16, 128), torch.randn(128, 16)
+    r = L.single_routing(16, 1.0, 0.0)
+    for which in range(3):
+        others = [w.clone().requires_grad_(which == 0), None if which == 2 else torch.randn(128).requires_grad_(which == 1)]
+        y = L.host().attach(torch.zeros(4, 128), [x], x, w, 0, others, [a], [b], None, torch.zeros(4, 16), None, [], ctypes.addressof(r), [], 16, "Node")
+        assert y.requires_grad == (which < 2)
+        assert which == 2 or len(y.grad_fn.next_functions) == 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["linear_w", "linear_bias"])
+def test_backward_from_a_result_that_only_weight_or_bias_makes_differentiable(which):
+    """It runs, and leaves both without a gradient."""
+    from lorafusion_amd.ops.lora_v1 import fused_linear_lora
+    from lorafusion_amd.ops.multi_lora import fused_linear_multi_lora, prepare_multi_lora_batch_info
+    from lorafusion_amd.ops.nf4 import fused_linear_lora_nf4, quantize_nf4
+    from lorafusion_amd.ops.swiglu_lora import fused_swiglu_linear_lora
+
+    t = lambda *s: torch.randn(*s, device="cuda", dtype=torch.bfloat16)
+    M, K, N, r = 128, 256, 128, 16
+    x, gu, w, bias, a, b = t(M, K), t(M, 2 * K), t(N, K), t(N), t(r, K), t(N, r)
+    codes, state = quantize_nf4(w)
+    frozen = {"linear_w": w, "linear_bias": bias}[which].requires_grad_()
+    info = prepare_multi_lora_batch_info([M], [0], [r], [0.0], [2.0], 128)
+    kw = dict(lora_a_list=[a], lora_b_list=[b], seq_len_list=[M], padded_seq_len_list=[M], block_to_lookup_table=info.block_to_lookup_table,
+              block_to_dropout_p=info.block_to_dropout_p, block_to_alpha=info.block_to_alpha, enable_dropout=False, same_dropout_p_value=0.0,
+              max_r=r, linear_bias=bias)
+    calls = [lambda: fused_linear_lora(x, w, a, b, 2.0, linear_bias=bias), lambda: fused_linear_multi_lora(x[None], w, **kw),
+             lambda: fused_swiglu_linear_lora(gu, w, a, b, 2.0, linear_bias=bias)]
+    if which == "linear_bias":
+        calls += [lambda: fused_linear_lora_nf4(x, codes, state, a, b, 2.0, linear_bias=bias),
+                  lambda: fused_linear_multi_lora(x[None], codes, quant_state=state, **kw)]
+    for call in calls:
+        y = call()
+        y.backward(torch.ones_like(y))
+        assert frozen.grad is None
+        (call().sum() + frozen.sum()).backward()
+        assert torch.equal(frozen.grad, torch.ones_like(frozen))
+        frozen.grad = None
+
+
 @pytest.mark.gpu
 def test_public_functions_refuse_tangents_and_empty_rows():
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
