@@ -218,7 +218,7 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
           const int col = c * 16 + li;
           if (c * 16 < a.R) {
             if (a.part != nullptr) a.part[((int64_t)sl * rows_all + row) * a.R + col] = acc[c][e];
-            else ((uint16_t*)a.S)[row * a.R + col] = real && col < bi.rank ? Mfma16<T>::cvt(acc[c][e] * mult) : (uint16_t)0;
+            else ((uint16_t*)a.S)[row * a.R + col] = real && col < bi.rank ? Mfma16<T>::cvt(fp32_product(acc[c][e], mult)) : (uint16_t)0;
           }
         }
       }

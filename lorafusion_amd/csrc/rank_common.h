@@ -132,6 +132,14 @@ __device__ __forceinline__ lf_u32x2 pack4(lf_f32x4 v) {
                   (uint32_t)Mfma16<T>::cvt(v[2]) | ((uint32_t)Mfma16<T>::cvt(v[3]) << 16)};
 }
 
+// A product that is rounded to fp32 before anything else happens to it.  The compiler folds fp32 multiply and conversion to fp16 into one
+// instruction (v_fma_mixlo_f16), which rounds once where the two round twice: kernels that have to agree bit for bit would not.
+__device__ __forceinline__ float fp32_product(float a, float b) {
+  float v = a * b;
+  asm("" : "+v"(v));
+  return v;
+}
+
 __device__ __forceinline__ uint32_t to_sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
 __device__ __forceinline__ lf_u32x4 window_rsrc(const void* base, int64_t bytes) {

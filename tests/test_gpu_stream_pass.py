@@ -74,6 +74,77 @@ def test_rank_pass_packed(seq, ranks, K, mode):
         row += pl
 
 
+def _xa_entries(x, gu, a_list, routing_c, R):
+    """The rank-r entry points that take no workspace, and lf_lora_xa with and without one; each returns S."""
+    import ctypes
+
+    from lorafusion_amd import _lib as L
+
+    M, K = x.shape
+    lib, st, ap = L.lib(), L.stream_of(x), L.ptr_array(a_list)
+    dt = L.dtype_id(x.dtype) | L.LF_MASK_BITS
+    nbytes = lib.lf_workspace_bytes(L.LF_OP_XA, M, 0, K, R, routing_c)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device="cuda")
+
+    def call(name, *args):
+        s = torch.full((M, R), float("nan"), dtype=x.dtype, device="cuda")
+        L.check(getattr(lib, name)(*[s.data_ptr() if v is s_here else v for v in args]), name)
+        return s
+
+    s_here = object()
+    tail = (M, K, R, routing_c)
+    return dict(
+        given=lambda size, m=None: call("lf_lora_xa", x.data_ptr(), L.ptr(m), ap, s_here, ws.data_ptr() if size else None, nbytes if size else 0, *tail, dt, st),
+        drawn=lambda m: call("lf_lora_xa_seeded", x.data_ptr(), m.data_ptr(), ap, s_here, *tail, ctypes.c_uint64(7), dt, st),
+        silu=lambda c, given, m: call("lf_lora_xa_silu_mul", gu.data_ptr(), gu[:, K:].data_ptr(), 2 * K, c.data_ptr(), L.ptr(given), L.ptr(m),
+                                      ctypes.c_uint64(7), ap, s_here, *tail, dt, st)), nbytes
+
+
+def _rank_pass_setup(M, K, ranks, dtype):
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops, norm_act
+    from lorafusion_amd.ops.multi_lora import prepare_multi_lora_batch_info
+
+    g = torch.Generator().manual_seed(M + K)
+    n, p_list = len(ranks), [0.1, 0.0, 0.3][:len(ranks)]
+    keep, p_rows = None, 0.1
+    if n == 1:
+        routing_c, R = L.single_routing(ranks[0], 1.0, 0.1), L.round_rank(ranks[0])
+    else:
+        info = prepare_multi_lora_batch_info([100, 128, 3], list(range(n)), ranks, p_list, [1.0] * n, 128, output_dtype=torch.float32)
+        keep = hip_ops.MultiRouting(info.padded_seq_len_list, ranks, info.block_to_lookup_table, info.block_to_alpha, info.block_to_dropout_p)
+        routing_c, R, p_rows = keep.c, keep.R, np.repeat(np.asarray(p_list, np.float32), 128)
+    gu = (torch.randn(M, 2 * K, generator=g) * 1.5).to(dtype).cuda()
+    a = [(torch.randn(r, K, generator=g) * K ** -0.5).to(dtype).cuda() for r in ranks]
+    c = norm_act.silu_mul_merged(gu)
+    xa, nbytes = _xa_entries(c, gu, a, routing_c, R)
+    bits = torch.from_numpy(np.packbits(od.keep_mask(M, K, p_rows, 7), axis=1, bitorder="little")).cuda()
+    return xa, nbytes, c, bits, (a, keep)
+
+
+def _without_a_workspace(xa, c, bits):
+    """S of the entry points that take no workspace and of lf_lora_xa without one: the same, bit for bit, like the masks they draw."""
+    drawn, drawn2 = torch.zeros_like(bits), torch.zeros_like(bits)
+    s = xa["given"](False, bits)
+    assert torch.isfinite(s).all()
+    assert torch.equal(xa["drawn"](drawn), s) and torch.equal(drawn, bits)
+    for given, m in ((bits, None), (None, drawn2)):
+        x = torch.empty_like(c)
+        assert torch.equal(xa["silu"](x, given, m), s) and torch.equal(x, c)
+    assert torch.equal(drawn2, bits)
+    return s
+
+
+@pytest.mark.parametrize("M,K,ranks,dtype", [(500, 5120, [128], torch.float16), (2900, 2560, [72], torch.float16), (65, 1152, [128], torch.bfloat16),
+                                             (384, 2048, [8, 128, 16], torch.float16)])
+def test_high_ranks_without_a_workspace(M, K, ranks, dtype):
+    """Above 64 rank columns S is the sliced pass's whether or not the caller gives memory for the slices' sums, bit for bit."""
+    xa, nbytes, c, bits, keep = _rank_pass_setup(M, K, ranks, dtype)
+    assert nbytes > 0, "several slices"
+    assert torch.equal(_without_a_workspace(xa, c, bits), xa["given"](True, bits))
+    assert torch.equal(xa["given"](False), xa["given"](True))
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 64, 65, 128])
 @pytest.mark.parametrize("K,N,r,dtype,bias", [(128, 128, 8, torch.bfloat16, True), (1152, 384, 72, torch.float16, False), (512, 4096, 128, torch.bfloat16, True)])
 def test_short_forward(M, K, N, r, dtype, bias):
