@@ -111,7 +111,9 @@ size_t lf_workspace_bytes(int op, int M, int N, int K, int R, const lf_routing* 
 /* S = drop(X) A^T.  Stands in for seeded_dropout + `masked_scaled_x @ lora_a.T`
  * (lorafusion/ops/lora_v1.py:111-119) and fused_dropout_matmul
  * (lorafusion/ops/triton_ops/fused_dropout_matmul.py:280-354); multi-LoRA: the `full_s` product
- * (lorafusion/ops/multi_lora.py:481-513).  mask may be NULL (no dropout). */
+ * (lorafusion/ops/multi_lora.py:481-513).  mask may be NULL (no dropout).  Given the workspace that
+ * lf_workspace_bytes(LF_OP_XA, ...) names, a product that is faster that way adds its sums in slices of K; without, it runs
+ * on the kernel that needs none (lf_lora_xa_seeded and lf_lora_xa_silu_mul, which take no workspace, always do). */
 int lf_lora_xa(const void* X, const uint8_t* mask, const void* const* a_ptrs, void* S, void* workspace,
                size_t ws_bytes, int M, int K, int R, const lf_routing* routing, int dtype, void* stream);
 
@@ -304,7 +306,7 @@ int lf_silu_mul_fwd(const void* A, const void* B, void* C, int M, int I, int64_t
  * up tensors [M,K] (rows `ld` elements apart: the halves of a merged projection output, or two tensors; ld >= K,
  * ld % 8 == 0, 16-byte aligned) and written once to X_out [M,K] for the base GEMM and the backward: the activation
  * pass and the rank-r pass's own read of X disappear.  X_out is bit-identical to lf_silu_mul_fwd's output and S to
- * lf_lora_xa's on it.  mask: explicit keep-mask [M,K] or NULL; mask_out != NULL: the mask is drawn from `seed` as
+ * lf_lora_xa's on it without a workspace (with one, sums may be added in another order).  mask: explicit keep-mask [M,K] or NULL; mask_out != NULL: the mask is drawn from `seed` as
  * lf_lora_xa_seeded draws it and written there (mask and mask_out exclude each other); both NULL: no dropout.
  * lf_swiglu_lora_fwd adds the fused GEMM of lf_lora_xw_sb on X_out: Y = X_out W^T + scale S B^T + bias
  * (workspace as for lf_lora_fwd: lf_workspace_bytes(LF_OP_FWD, ...), or NULL).

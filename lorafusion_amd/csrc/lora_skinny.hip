@@ -65,25 +65,23 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 }
 
 // ------------------------------------------------------------------------------------ xa
-// Ranks to 32, but for short batches (lf_xa_streams; the sliced pass of lora_stream.hip takes the rest).
-// One workgroup of 8 waves (2 above rank 64) per 16 rows (32 above rank 32); no partial sums leave the workgroup.  The K range is dealt
-// to the waves in 64-column steps (step s goes to wave s % waves), each wave streams its steps of the
-// 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), all loads of a batch
-// of steps in flight at once, applies the keep-mask in registers and turns the row-major
+// Ranks to 64, where the sliced pass of lora_stream.hip is not the faster one or has no memory for its sums (lf_xa_takes_stream).
+// One workgroup of 8 waves per 16 rows (64 at ranks 48-64); no partial sums leave the workgroup.  The K range is dealt
+// to the waves in 64-column steps (step s goes to wave s % 8), each wave streams its steps of the
+// 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), the next step's loads in flight while one is used
+// (ranks to 32), applies the keep-mask in registers and turns the row-major
 // granules into MFMA row fragments through a 2 KB LDS patch of its own (same-wave LDS traffic is
 // ordered: no barrier).  The adapter matrix A (L2 resident) takes the same route: fragment-shaped
 // loads would put the four lanes of every quad on four different rows, a quarter of the
 // coalesced rate in the texture addresser.  The eight partial [16, R] accumulators are added in a fixed order through LDS,
 // scaled by 1/(1-p), zeroed in padded rows and beyond the adapter's rank, and stored as S.
-// Rows per workgroup: every workgroup reads the whole adapter matrix (from L2), which above rank 32 is several times the bytes of
-// 16 rows of X: two row blocks share a set of A fragments there (the up-half registers of four do not fit next to the rest).  At
-// rank 16 two row blocks per workgroup measured slower (0.27 -> 0.34 ms at the 8B layer: the registers of the second block cost
-// loads in flight).
-constexpr int xa_nb(int rt) { return rt >= 4 ? 2 : 1; }
-constexpr int xa_rows(int rt) { return 16 * xa_nb(rt); }
-// waves per workgroup and steps in flight per wave, by rank tiles (LDS: 2 KB * (1+RT) per wave; registers: 8 * RT per step)
-constexpr int xa_waves(int rt) { return rt <= 4 ? 8 : 2; }
-constexpr int xa_unroll(int rt) { return rt <= 1 ? 4 : rt <= 2 ? 2 : 1; }
+// Rows per workgroup: every workgroup reads the whole adapter matrix (from L2), which at rank 64 is four times the
+// bytes of 16 rows of X: ranks 48-64 take 64 rows (four row blocks share one set of A fragments; with the activation prologue the
+// up-half registers of four do not fit next to the rest: two).  At rank 16 two row blocks per
+// workgroup measured slower (0.27 -> 0.34 ms at the 8B layer: the registers of the second block cost loads in flight).
+constexpr int XA_WAVES = 8;
+constexpr int xa_nb(int rt, bool act) { return rt == 4 ? (act ? 2 : 4) : 1; }
+constexpr int xa_rows(int rt, bool act) { return 16 * xa_nb(rt, act); }
 
 // GEN: the keep-mask is not read but drawn here (Philox, the definition of the standalone mask
 // kernel) from (seed, element index) and written to `mask_out` for the backward pass: the integer
@@ -94,11 +92,11 @@ constexpr int xa_unroll(int rt) { return rt <= 1 ? 4 : rt <= 2 ? 2 : 1; }
 // base GEMM and the backward, and fed to the rank-r product from registers: the activation pass and this pass's own
 // read of X disappear.
 template <typename T, int RT, bool GEN, bool ACT>
-__global__ void __launch_bounds__(xa_waves(RT) * 64)
+__global__ void __launch_bounds__(XA_WAVES * 64)
 lora_xa_kernel(const T* __restrict__ X, const T* __restrict__ U, int64_t ldx, T* __restrict__ act_out,
                const uint8_t* __restrict__ mask, uint8_t* __restrict__ mask_out, int mask_bits,
                uint32_t seed_lo, uint32_t seed_hi, T* __restrict__ S, int M, int K, int R, const LfSegTable seg) {
-  constexpr int XA_WAVES = xa_waves(RT), XA_U = xa_unroll(RT), NB = xa_nb(RT), XA_ROWS = xa_rows(RT);
+  constexpr int NB = xa_nb(RT, ACT), XA_ROWS = xa_rows(RT, ACT);
   // the partial accumulators of the final sum reuse the patches (a barrier separates the two uses): at
   // rank 64 the separate 16 KB pushed the workgroup over 40 KB, and a CU then holds two workgroups, not four
   constexpr int PATCH_BYTES = XA_WAVES * 2048 * (NB + RT), RED_BYTES = XA_WAVES * XA_ROWS * RT * 16 * 4;
@@ -146,7 +144,7 @@ lora_xa_kernel(const T* __restrict__ X, const T* __restrict__ U, int64_t ldx, T*
   // start together and would otherwise sit in the same phase -- everyone waiting for memory, then everyone
   // computing.  Measured at 16512 x 4096, rank 16, mask drawn in the kernel: one set of four steps 44.5 us, two sets
   // of two steps 45.4 (126 registers: half the waves per SIMD), two sets of one step 42.2.
-  constexpr int NSET = XA_U >= 2 ? 2 : 1, UB = 1;
+  constexpr int NSET = RT <= 2 ? 2 : 1, UB = 1;
   lf_u32x4 xv[NSET][UB][2 * NB], av[NSET][UB][RT][2];
   lf_u32x4 uv[NSET][UB][ACT ? 2 * NB : 1];
   lf_u32x2 mv[NSET][UB][2 * NB];
@@ -851,9 +849,11 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
 }
 
 // (lora_stream.hip)
+int lf_xa_stream_slices(int, int, int, const LfSegTable&);
 size_t lf_xa_stream_workspace(int, int, int, const LfSegTable&);
 int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, void*, float*, int, int, int, const LfSegTable&, int, hipStream_t);
 
+// The products that the sliced pass (lora_stream.hip) is there for, given memory for the slices' sums:
 // The sliced pass (lora_stream.hip) in place of lora_xa_kernel: above 32 rank columns, where that kernel reads the adapter matrix
 // once per 16-64 rows through wave-private patches and has too few workgroups (1000 x 4096, rank 64, keep bits read: 22.5 ->
 // 10.1 us; 3000 x 5120, rank 128: 67 -> 19; 8576 x 28672, rank 64: 201 -> 148; 8576 x 8192: 40.6 -> 38.9), and with a
@@ -862,9 +862,15 @@ int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, vo
 // 9.6 us).  Without a mask up to 1024 rows from K = 8192, or from 4096 at ranks 17 - 32 up to 512 rows: the whole forward of
 // 333 x 14336 x 4096 71.7 -> 65.5 us at rank 16, 75.5 -> 65.5 at 32, of 1000 rows 125.4 -> 119.3, of 333 x 4096 x 14336 at rank 32 53.1 ->
 // 52.2; level at 4096 and rank 16, and at K = 1024 the second stage costs 20 % (333 x 1024 x 2048: 12.1 against 14.8).  The same choice for every mask format, drawn or read: S does not depend on how the mask came.
-bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& seg) {
+static bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   return R > 32 || (rows <= 1024 && (masked || K >= 8192 || (R > 16 && K >= 4096 && rows <= 512)));
+}
+// ... and those it takes.  Without the memory (entry points that have no workspace to give, or too small a one) this file's kernel
+// runs to rank 64; above, and where a single slice needs none, the sliced pass all the same.
+bool lf_xa_takes_stream(int M, int K, int R, bool masked, const LfSegTable& seg, const void* ws, size_t ws_bytes) {
+  return lf_xa_streams(M, K, R, masked, seg) && (R > 64 || lf_xa_stream_slices(M, K, R, seg) == 1 ||
+                                                 (ws != nullptr && ws_bytes >= lf_xa_stream_workspace(M, K, R, seg)));
 }
 size_t lf_xa_workspace(int M, int K, int R, const LfSegTable& seg) {
   return lf_xa_streams(M, K, R, true, seg) ? lf_xa_stream_workspace(M, K, R, seg) : 0;
@@ -874,11 +880,11 @@ template <typename T, int RT>
 static int xa_launch(const void* X, const void* U, int64_t ldx, void* act_out, const uint8_t* mask, uint8_t* mask_out, int mask_bits,
                      uint64_t seed, void* S, int M, int K, int R, int64_t rows, const LfSegTable& seg, hipStream_t st) {
   const bool gen = mask_out != nullptr, act = U != nullptr;
-  constexpr int wg_rows = xa_rows(RT);
+  const int wg_rows = xa_rows(RT, act);
   const unsigned grid = (unsigned)((rows + wg_rows - 1) / wg_rows);
   const uint32_t lo = gen ? (uint32_t)seed : 0u, hi = gen ? (uint32_t)(seed >> 32) : 0u;
 #define LF_XA(GEN, ACT)                                                                                              \
-  return lf_launch((lora_xa_kernel<T, RT, GEN, ACT>), dim3(grid), dim3(xa_waves(RT) * 64), 0, st, (const T*)X,       \
+  return lf_launch((lora_xa_kernel<T, RT, GEN, ACT>), dim3(grid), dim3(XA_WAVES * 64), 0, st, (const T*)X,       \
                    (const T*)U, ldx, (T*)act_out, mask, mask_out, mask_bits, lo, hi, (T*)S, M, K, R, seg)
   if (gen && act) LF_XA(true, true);
   if (act) LF_XA(false, true);
@@ -895,7 +901,8 @@ static int xa_impl(const void* X, const void* U, int64_t ldx, void* act_out, con
   switch (rt_of(R)) {
     case 1: return xa_launch<T, 1>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
     case 2: return xa_launch<T, 2>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
-    default: return LF_ESHAPE;   // (lf_xa_streams: above rank 32 the sliced pass, behind an activation pass of its own)
+    case 4: return xa_launch<T, 4>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, rows, seg, st);
+    default: return LF_ESHAPE;   // (lf_xa_takes_stream: above rank 64 the sliced pass, behind an activation pass of its own)
   }
 }
 
@@ -913,9 +920,10 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
     if (ldx < K || ldx % 8 != 0 || (((uintptr_t)X | (uintptr_t)U | (uintptr_t)act_out) & 15) != 0) return LF_ESHAPE;
   } else {
     ldx = K;
-    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_streams(M, K, R, mask != nullptr || mask_out != nullptr, seg))
-      return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, seg) ? (float*)ws : nullptr, M, K,
-                                 R, seg, dtype, st);
+    const bool masked = mask != nullptr || mask_out != nullptr;
+    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_takes_stream(M, K, R, masked, seg, ws, ws_bytes))
+      return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, seg) ? (float*)ws : nullptr, M,
+                                 K, R, seg, dtype, st);
   }
   if (dtype == LF_BF16) return xa_impl<__bf16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);
   if (dtype == LF_F16) return xa_impl<_Float16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);

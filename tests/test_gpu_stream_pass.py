@@ -145,6 +145,45 @@ def test_high_ranks_without_a_workspace(M, K, ranks, dtype):
     assert torch.equal(xa["given"](False), xa["given"](True))
 
 
+@pytest.mark.parametrize("M,K,ranks,dtype", [
+    (300, 4096, [16], torch.bfloat16), (1000, 4480, [24], torch.float16), (17, 1920, [64], torch.bfloat16), (65, 2560, [48], torch.float16),
+    (2901, 5120, [64], torch.bfloat16), (384, 2048, [8, 64, 16], torch.float16), (384, 4096, [16, 8, 16], torch.bfloat16)])
+def test_rank_pass_without_a_workspace(M, K, ranks, dtype):
+    """To 64 rank columns the sums are in another order without the memory: one rounding of S apart."""
+    xa, nbytes, c, bits, keep = _rank_pass_setup(M, K, ranks, dtype)
+    assert nbytes > 0, "the sliced pass, given memory"
+    _close(_without_a_workspace(xa, c, bits), xa["given"](True, bits).float().cpu(), "S")
+    _close(xa["given"](False), xa["given"](True).float().cpu(), "S, no mask")
+
+
+@pytest.mark.parametrize("M,K,r", [(300, 4096, 16), (64, 14336, 32)])
+def test_rank_pass_without_a_workspace_shares_k(M, K, r):
+    """... and takes at most about three times as long (one workgroup that walks all of K: 4 to 8 times)."""
+    from lorafusion_amd import _lib as L
+
+    x, a = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(r, K, device="cuda").bfloat16()
+    bits = torch.full((M, K // 8), 255, dtype=torch.uint8, device="cuda")
+    xa, _ = _xa_entries(x, x, [a], L.single_routing(r, 1.0, 0.1), r)
+
+    def us(f):
+        best = float("inf")
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            f()
+            t0.record()
+            for _ in range(20):
+                f()
+            t1.record()
+            torch.cuda.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 50)
+        return best
+
+    drawn = bits.clone()
+    with_ws, without, seeded = us(lambda: xa["given"](True, bits)), us(lambda: xa["given"](False, bits)), us(lambda: xa["drawn"](drawn))
+    print(f"{M} x {K}, rank {r}: {with_ws:.1f} us with a workspace, {without:.1f} without, {seeded:.1f} drawn", flush=True)
+    assert without <= 3 * with_ws + 10 and seeded <= 3 * with_ws + 10
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 64, 65, 128])
 @pytest.mark.parametrize("K,N,r,dtype,bias", [(128, 128, 8, torch.bfloat16, True), (1152, 384, 72, torch.float16, False), (512, 4096, 128, torch.bfloat16, True)])
 def test_short_forward(M, K, N, r, dtype, bias):
