@@ -101,8 +101,8 @@ const char* lf_strerror(int code);
  * the backward's rank-r passes, which a call must be given, and what a call does without when the
  * workspace is smaller or NULL: for LF_OP_FWD / BWD / NF4_* the fp32 partial tiles of a split
  * contraction (launches with few tiles and a long K: left-over rows of a packed batch, short
- * batches), for LF_OP_XA / FWD / NF4_FWD the slices of the forward's rank-r pass (more than 32 rank
- * columns, short batches), for LF_OP_FWD / NF4_FWD the slices of a short batch's single pass. 0 also for a
+ * batches), for LF_OP_XA / FWD / NF4_FWD the slices of the forward's rank-r pass (high ranks, and
+ * short batches over a long K), for LF_OP_FWD / NF4_FWD the slices of a short batch's single pass. 0 also for a
  * shape or routing the entry point itself would refuse (M <= 0, R not a multiple of 16 in 16..128, a tiled dimension
  * -- N for DYS_DYB / BWD / NF4_*, K for XA / DA / FWD / BWD / NF4_* -- that is not a positive multiple
  * of 128, bad routing): the size query never fails harder than the call. */

@@ -849,31 +849,49 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
 }
 
 // (lora_stream.hip)
-int lf_xa_stream_slices(int, int, int, const LfSegTable&);
-size_t lf_xa_stream_workspace(int, int, int, const LfSegTable&);
+int lf_xa_stream_slices(int, int, int, bool, const LfSegTable&);
+size_t lf_xa_stream_workspace(int, int, int, bool, const LfSegTable&);
 int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, void*, float*, int, int, int, const LfSegTable&, int, hipStream_t);
 
-// The products that the sliced pass (lora_stream.hip) is there for, given memory for the slices' sums:
-// The sliced pass (lora_stream.hip) in place of lora_xa_kernel: above 32 rank columns, where that kernel reads the adapter matrix
-// once per 16-64 rows through wave-private patches and has too few workgroups (1000 x 4096, rank 64, keep bits read: 22.5 ->
-// 10.1 us; 3000 x 5120, rank 128: 67 -> 19; 8576 x 28672, rank 64: 201 -> 148; 8576 x 8192: 40.6 -> 38.9), and with a
-// keep-mask up to 1024 rows, where drawing it on a few compute units is what takes the time (300 x 4096, rank 16: -2.5 us
-// drawn, level when read).  Elsewhere the second stage costs more than the slices give (4096 x 4096, rank 16: 7.9 against
-// 9.6 us).  Without a mask up to 1024 rows from K = 8192, or from 4096 at ranks 17 - 32 up to 512 rows: the whole forward of
-// 333 x 14336 x 4096 71.7 -> 65.5 us at rank 16, 75.5 -> 65.5 at 32, of 1000 rows 125.4 -> 119.3, of 333 x 4096 x 14336 at rank 32 53.1 ->
-// 52.2; level at 4096 and rank 16, and at K = 1024 the second stage costs 20 % (333 x 1024 x 2048: 12.1 against 14.8).  The same choice for every mask format, drawn or read: S does not depend on how the mask came.
+// The products that the sliced pass (lora_stream.hip) is the faster one for, given memory for the slices' sums.  Microseconds below: mask drawn /
+// keep bits read / no mask, this file's kernel against the sliced pass, launches replayed from a graph.
+// - Above 64 rank columns, always: 64 x 1024 at rank 128 22.4 / 18.6 / 15.4 -> 10.2 / 8.7 / 8.0, 14000 x 8192 194 / 145 / 105 -> 92 / 81 / 53.
+// - 33 to 64: this kernel reads A once per 64 rows and has a workgroup per 64 rows, each of which walks K alone.  Up to 48 of
+//   them always (1000 x 4096 38 / 24 / 17 -> 12 / 10 / 9); beyond, the second stage and the partial sums cost a fixed part
+//   and the slices give one that grows with K: the table.  One round of the chip full of workgroups (170 to 256) leaves nothing to
+//   gain (16384 x 4096 44 / 30 / 27 against 46 / 31 / 28), a second round does (20000 x 4096 79 / 52 / 42 -> 58 / 43 / 35).  Without
+//   a mask there is half as much to share, and K has to be twice as long.  Either side of the lines:
+//     64 groups   K 1024  13.5/10.0/ 8.0 -> 11.4/ 9.7/ 8.8   2048  21.9/15.0/11.1 -> 14.4/11.5/10.1
+//     110         K 1024  13.7/10.2/ 8.2 -> 14.4/11.3/10.1   1536  18.8/13.3/10.4 -> 17.3/12.9/10.7   3072 31.7/21.0/16.0 -> 23.4/17.5/15.3
+//     141         K 1536  19.2/13.6/10.9 -> 18.5/14.5/12.4   2048  24.5/17.2/13.6 -> 22.6/16.5/14.0   4096 40.5/26.7/20.2 -> 34.1/22.8/19.9
+//     192         K 4096  41.7/28.3/23.7 -> 38.7/28.9/24.8   8192  75.0/47.8/38.6 -> 65.6/46.2/39.8   14336 149/110/90 -> 111/100/82
+//     219         K 8192  75.6/49.2/42.2 -> 77.9/64.4/49.7 (eight slices; two: 80.3/49.3/42.8)
+// - To 32: up to 1024 rows from K = 4096 with a mask (300 rows at rank 16: K = 3072 8.8 / 6.1 -> 9.0 / 7.1, 4096 10.9 / 7.3 -> 8.9 / 7.2, 8192 19.1 /
+//   11.6 -> 11.7 / 8.7; a second launch costs what a short K saves), without one from 8192 (8.3 -> 7.3), and at ranks 17 - 32
+//   up to 512 rows from 4096 (300 rows: 4096 7.0 -> 6.9, 5120 8.0 -> 7.2; 1000 rows, 5120: 8.0 -> 7.7).
+// The same choice for every mask format, drawn or read: S does not depend on how the mask came.
 static bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
-  return R > 32 || (rows <= 1024 && (masked || K >= 8192 || (R > 16 && K >= 4096 && rows <= 512)));
+  if (R > 64) return true;
+  if (R > 32) {
+    const int64_t groups = (rows + 63) / 64;
+    if (groups <= 48 || groups > 256) return true;
+    const int k_min = groups <= 64 ? 1024 : groups <= 128 ? 1536 : groups <= 170 ? 2048 : groups <= 192 ? 8192 : 1 << 30;
+    return K >= (masked || k_min == 1 << 30 ? k_min : 2 * k_min);
+  }
+  return rows <= 1024 && (masked ? K >= 4096 : K >= 8192 || (R > 16 && K >= 4096 && rows <= 512));
 }
 // ... and those it takes.  Without the memory (entry points that have no workspace to give, or too small a one) this file's kernel
 // runs to rank 64; above, and where a single slice needs none, the sliced pass all the same.
 bool lf_xa_takes_stream(int M, int K, int R, bool masked, const LfSegTable& seg, const void* ws, size_t ws_bytes) {
-  return lf_xa_streams(M, K, R, masked, seg) && (R > 64 || lf_xa_stream_slices(M, K, R, seg) == 1 ||
-                                                 (ws != nullptr && ws_bytes >= lf_xa_stream_workspace(M, K, R, seg)));
+  return lf_xa_streams(M, K, R, masked, seg) && (R > 64 || lf_xa_stream_slices(M, K, R, masked, seg) == 1 ||
+                                                 (ws != nullptr && ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg)));
 }
 size_t lf_xa_workspace(int M, int K, int R, const LfSegTable& seg) {
-  return lf_xa_streams(M, K, R, true, seg) ? lf_xa_stream_workspace(M, K, R, seg) : 0;
+  size_t n = 0;
+  for (const bool masked : {false, true})
+    if (lf_xa_streams(M, K, R, masked, seg)) n = std::max(n, lf_xa_stream_workspace(M, K, R, masked, seg));
+  return n;
 }
 
 template <typename T, int RT>
@@ -922,7 +940,7 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
     ldx = K;
     const bool masked = mask != nullptr || mask_out != nullptr;
     if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_takes_stream(M, K, R, masked, seg, ws, ws_bytes))
-      return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, seg) ? (float*)ws : nullptr, M,
+      return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg) ? (float*)ws : nullptr, M,
                                  K, R, seg, dtype, st);
   }
   if (dtype == LF_BF16) return xa_impl<__bf16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);

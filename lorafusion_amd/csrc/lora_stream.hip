@@ -298,17 +298,22 @@ short_fwd_finish_kernel(const float* __restrict__ part, int64_t pitch, int n_sli
 
 // Slices of K.  Compute units share the workgroups evenly or not at all: 65 groups in 4 slices are 260 workgroups, and four
 // of the 256 compute units take twice as long as the rest.  So: the count (at most sixteen, none shorter than four
-// steps) with the shortest modelled time -- the busiest compute unit's share of the stream (a full walk of K = 4096 by one
-// workgroup takes 22 us), the partial sums written and read back, and the second stage where one slice needs none.
-// 6 x 4096 x 4096 (65 groups), first and second stage: 3 slices 12.0 us, 4: 13.3, 7: 12.5, 8: 14.0; 8576 rows, K = 28672,
-// rank 64 (134 groups): 1 slice 216 us, 3: 157, 4: 170, 7: 147.
-int slices_for(int64_t groups, int K, double partial_bytes, bool second_stage) {
-  const int most = K / 256 < 1 ? 1 : K / 256 > 16 ? 16 : K / 256;
+// steps) with the shortest modelled time -- the busiest compute unit's share of the walk (us per column of K: `walk`), the partial sums written and
+// read back, and what a second stage costs where a single slice needs none.
+// Forward: a full walk of K = 4096 takes 22 us; 6 x 4096 x 4096 (65 groups), first and second stage: 3 slices 12.0 us, 4: 13.3, 7: 12.5, 8: 14.0.
+// xa: below K = 768 one; a walk of 4096 takes 18 - 24 us without a mask, 26 - 33 with one read and 48 - 53 with one drawn (the integer work of a workgroup that
+// has a compute unit to itself); the constants are those with the smallest loss against the best count over 64 - 20000 rows, K of
+// 1024 - 14336 and ranks 64 and 128 (masked 13 % -> 3.5 %, against one walk figure of 22 us for all; 9000 x 3072 at rank 64, mask drawn: one
+// slice 41 us, three 27.5; 6000 x 1536 at rank 128: one 27, two 21).
+struct SliceModel { double walk; bool single_is_direct; };   // single_is_direct: one slice writes no partial sums and needs no second stage (1.5 us)
+constexpr SliceModel kFwdSlices = {0.0054, false}, kXaSlices = {0.008, true}, kXaMaskedSlices = {0.0105, true};
+int slices_for(int64_t groups, int K, double partial_bytes, const SliceModel& m) {
+  const int most = K / 256 < 1 || (m.single_is_direct && K < 768) ? 1 : K / 256 > 16 ? 16 : K / 256;
   int best = 1;
   double best_cost = 1e300;
   for (int n = 1; n <= most; n++) {
     const double share = (double)((groups * n + 255) / 256) / n;
-    const double cost = share * K * 0.0054 + n * partial_bytes / 1.5e6 + (n > 1 || second_stage ? 4.0 : 0.0);
+    const double cost = share * K * m.walk + (n == 1 && m.single_is_direct ? 0.0 : n * partial_bytes / 1.5e6 + 1.5);
     if (cost < best_cost) { best_cost = cost; best = n; }
   }
   return best;
@@ -356,13 +361,14 @@ int xa_stream_impl(StreamArgs a, const LfSegTable& seg, float* ws, hipStream_t s
 
 static int64_t xa_rows_of(int M, const LfSegTable& seg) { return seg.table ? (int64_t)seg.n_blocks * ROWS : M; }
 
-int lf_xa_stream_slices(int M, int K, int R, const LfSegTable& seg) {
+int lf_xa_stream_slices(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int64_t groups = (xa_rows_of(M, seg) + SROWS - 1) / SROWS;
-  return slices_for(groups, K, (double)xa_rows_of(M, seg) * R * sizeof(float), false);
+  const double slab = (double)xa_rows_of(M, seg) * R * sizeof(float);
+  return slices_for(groups, K, slab, masked ? kXaMaskedSlices : kXaSlices);
 }
 
-size_t lf_xa_stream_workspace(int M, int K, int R, const LfSegTable& seg) {
-  const int n = lf_xa_stream_slices(M, K, R, seg);
+size_t lf_xa_stream_workspace(int M, int K, int R, bool masked, const LfSegTable& seg) {
+  const int n = lf_xa_stream_slices(M, K, R, masked, seg);
   return n > 1 ? (size_t)n * xa_rows_of(M, seg) * R * sizeof(float) : 0;
 }
 
@@ -370,7 +376,7 @@ size_t lf_xa_stream_workspace(int M, int K, int R, const LfSegTable& seg) {
 int lf_launch_xa_stream(const void* X, const uint8_t* mask, uint8_t* mask_out, int mask_bits, uint64_t seed, void* S, float* ws, int M, int K, int R,
                         const LfSegTable& seg, int dtype, hipStream_t st) {
   StreamArgs a{};
-  a.p0 = X; a.n0 = (int)xa_rows_of(M, seg); a.K = K; a.n_slices = lf_xa_stream_slices(M, K, R, seg);
+  a.p0 = X; a.n0 = (int)xa_rows_of(M, seg); a.K = K; a.n_slices = lf_xa_stream_slices(M, K, R, mask != nullptr || mask_out != nullptr, seg);
   a.mask = mask; a.mask_out = mask_out; a.mask_bytes = !mask_bits; a.seed_lo = (uint32_t)seed; a.seed_hi = (uint32_t)(seed >> 32);
   a.S = S; a.M = M; a.R = R;
   return dtype == LF_BF16 ? xa_stream_impl<__bf16>(a, seg, ws, st) : xa_stream_impl<_Float16>(a, seg, ws, st);
@@ -387,7 +393,7 @@ static int short_groups(int N, int rank) { return N / SROWS + (rank + SROWS - 1)
 bool lf_short_fwd_applies(int M, int N) { return M <= 64 || (M <= 128 && N <= 4096); }
 
 static int short_slices(int M, int N, int K, int rank) {
-  return slices_for(short_groups(N, rank), K, (double)M * short_pitch(N, rank) * sizeof(float), true);
+  return slices_for(short_groups(N, rank), K, (double)M * short_pitch(N, rank) * sizeof(float), kFwdSlices);
 }
 size_t lf_short_fwd_workspace(int M, int N, int K, int rank) {
   return (size_t)short_slices(M, N, K, rank) * M * short_pitch(N, rank) * sizeof(float);

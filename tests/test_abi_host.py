@@ -141,6 +141,26 @@ def test_launch_plan_takes_the_contraction_length():
     assert plan(8192, 8192, 8192)[1] == 7 and plan(16384, 4096, 28672)[1] == 7
 
 
+def test_rank_pass_is_sliced_where_that_is_faster():
+    """Host logic: the workspace of the forward's rank-r pass is the slices' sums, nothing where the pass runs on the kernel that needs none."""
+    from lorafusion_amd import _lib as L
+
+    def slabs(M, K, R):
+        n = L.lib().lf_workspace_bytes(L.LF_OP_XA, M, 0, K, R, L.single_routing(R, 1.0, 0.1))
+        return -(-(n - 255) // (M * R * 4)) if n else 0
+
+    for M in (64, 300, 1000):
+        # a second launch costs more than the slices of a short K give at low ranks (300 x 1024, rank 16: 4.7 against 8.6 us)
+        assert [slabs(M, K, 16) for K in (1024, 2048, 3968)] == [0, 0, 0] and slabs(M, 4096, 16) == 16
+        # ... and several slices give more than one at high ranks (300 x 1024, rank 64: 16.4 against 9.4)
+        assert slabs(M, 1024, 64) > 1 and slabs(M, 1024, 128) > 1
+    assert slabs(1025, 8192, 16) == 0
+    # rank 64, a compute unit per 64 rows: the kernel without a second stage, but for a long K or more than 256 of them
+    assert slabs(7000, 1024, 64) == 0 and slabs(7000, 3072, 64) > 1
+    assert slabs(10500, 4096, 64) > 1 and slabs(14000, 8192, 64) == 0 and slabs(20000, 4096, 64) > 1
+    assert slabs(2500, 1536, 128) > 1 and slabs(6000, 1536, 128) > 1
+
+
 def test_python_layer_refuses_cpu_tensors():
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
     from lorafusion_amd.ops.nf4 import QuantState, dequantize_nf4_triton
