@@ -238,18 +238,14 @@ int lf_lora_xw_sb(const void* X, const void* W, const void* bias, const void* S,
 }
 
 // The forward of a short batch of one adapter without a keep-mask: one pass over W and A together (lora_stream.hip).
-// False where it does not apply, or where the general path refuses the call itself; a pinned tile stays as pinned.
-static bool short_fwd(const void* X, const void* W, const void* bias, const void* const* a_ptrs, const void* const* b_ptrs, void* Y, void* S,
-                      void* workspace, size_t ws_bytes, int M, int N, int K, int R, const lf_routing* routing, int dtype, void* stream, int* rc) {
-  dtype &= ~LF_MASK_BITS;
+// False where it does not apply, where its workspace is not there, or where the general path refuses the call itself; a pinned tile stays as pinned.
+static bool short_fits(const void* X, const void* W, const void* const* a_ptrs, const void* const* b_ptrs, const void* Y, const void* S,
+                       const void* workspace, size_t ws_bytes, int M, int N, int K, int R, const lf_routing* routing, int dtype, LfSegTable& t) {
   if (lf_tile_pinned() || bad_dtype(dtype) || !X || !W || !Y || !S || !a_ptrs || !b_ptrs || M <= 0 || bad_tiled_dim(N) || bad_tiled_dim(K) ||
       bad_rank_cols(R) || (((uintptr_t)Y | (uintptr_t)S) & 15) != 0)
     return false;
-  LfSegTable t;
   if (make_seg(routing, M, a_ptrs, nullptr, t) != LF_OK || t.table || !lf_short_fwd_applies(M, N) || !t.ptr[0] || !b_ptrs[0] || t.rank[0] > R) return false;
-  if (!workspace || ws_bytes < lf_short_fwd_workspace(M, N, K, t.rank[0])) return false;
-  *rc = lf_launch_short_fwd(X, W, t.ptr[0], b_ptrs[0], t.scale, bias, Y, S, workspace, M, N, K, t.rank[0], R, t, dtype, (hipStream_t)stream);
-  return true;
+  return workspace != nullptr && ws_bytes >= lf_short_fwd_workspace(M, N, K, t.rank[0]);
 }
 
 int lf_swiglu_lora_fwd(const void* G, const void* U, int64_t ld, void* X_out, const void* W, const void* bias,
@@ -257,11 +253,12 @@ int lf_swiglu_lora_fwd(const void* G, const void* U, int64_t ld, void* X_out, co
                        const void* const* b_ptrs, void* Y, void* S_out, void* workspace, size_t ws_bytes, int M, int N,
                        int K, int R, const lf_routing* routing, int dtype, void* stream) {
   const int et = dtype & ~LF_MASK_BITS;
-  // (as lf_lora_fwd on the activation's output would: short batches without a mask take the single pass)
-  if (!mask && !mask_out && routing && !routing->block_table && lf_short_fwd_applies(M, N) && G && U && X_out && !bad_tiled_dim(K)) {
+  LfSegTable t;
+  // (as lf_lora_fwd on the activation's output would: short batches without a mask take the single pass, behind an activation pass)
+  if (!mask && !mask_out && short_fits(X_out, W, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, et, t)) {
     int rc = lf_silu_mul_fwd(G, U, X_out, M, K, ld, ld, K, et, stream);
     if (rc != LF_OK) return rc;
-    return lf_lora_fwd(X_out, W, bias, nullptr, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, et, stream);
+    return lf_launch_short_fwd(X_out, W, t.ptr[0], b_ptrs[0], t.scale, bias, Y, S_out, workspace, M, N, K, t.rank[0], R, t, et, (hipStream_t)stream);
   }
   int rc = xa_silu_mul_ws(G, U, ld, X_out, mask, mask_out, seed, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;
@@ -319,9 +316,11 @@ int lf_lora_dyw_dsa(const void* dY, const void* W, const void* dS, const void* c
 int lf_lora_fwd(const void* X, const void* W, const void* bias, const uint8_t* mask, const void* const* a_ptrs,
                 const void* const* b_ptrs, void* Y, void* S_out, void* workspace, size_t ws_bytes, int M, int N,
                 int K, int R, const lf_routing* routing, int dtype, void* stream) {
-  int rc;
-  if (mask == nullptr && short_fwd(X, W, bias, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, dtype, stream, &rc)) return rc;
-  rc = lf_lora_xa(X, mask, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
+  const int et = dtype & ~LF_MASK_BITS;
+  LfSegTable t;
+  if (mask == nullptr && short_fits(X, W, a_ptrs, b_ptrs, Y, S_out, workspace, ws_bytes, M, N, K, R, routing, et, t))
+    return lf_launch_short_fwd(X, W, t.ptr[0], b_ptrs[0], t.scale, bias, Y, S_out, workspace, M, N, K, t.rank[0], R, t, et, (hipStream_t)stream);
+  int rc = lf_lora_xa(X, mask, a_ptrs, S_out, workspace, ws_bytes, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;
   behind_xa(workspace, ws_bytes, M, K, R, routing);
   return xw_sb_ws(X, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);

@@ -157,6 +157,56 @@ def test_fused_layer_single_adapter_with_bias(p):
     _close(b.grad, dbe, "db")
 
 
+@pytest.mark.parametrize("M,K,N,r,dtype", [(1, 128, 128, 8, torch.bfloat16), (64, 1152, 5120, 72, torch.float16), (65, 512, 384, 16, torch.bfloat16),
+                                           (128, 4096, 4096, 32, torch.bfloat16), (128, 256, 4224, 16, torch.bfloat16)])
+def test_short_batches(M, K, N, r, dtype):
+    """Either side of the rule of the single pass (up to 64 rows, or 128 under at most 4096 columns): the oracle, and the unfused ops bit for bit."""
+    from lorafusion_amd.ops import norm_act
+    from lorafusion_amd.ops.lora_v1 import fused_linear_lora
+    from lorafusion_amd.ops.swiglu_lora import fused_swiglu_linear_lora
+
+    d = single_inputs(M, K, N, r, p=0.0, seed=M + K, dtype=dtype, bias=True)
+    gu = _gate_up(M, K, dtype, 3)
+    w, a, b, bias = (d[k].cuda() for k in ("w", "a", "b", "bias"))
+    y = fused_swiglu_linear_lora(gu.cuda(), w, a, b, 0.5, linear_bias=bias)
+    assert torch.equal(y, fused_linear_lora(norm_act.silu_mul_merged(gu.cuda()), w, a, b, 0.5, linear_bias=bias))
+    c = norm_act.silu_mul_merged(gu.cuda()).cpu()
+    ye, _ = lora_ref.linear_lora_fwd_fp32(c, d["w"], d["a"], d["b"], 0.5, None, 0.0, d["bias"])
+    _close(y, ye, "y")
+
+
+def test_short_batch_without_a_workspace_and_refused():
+    """Without memory for the single pass the activation stays the prologue of the rank-r pass; a refused call writes nothing."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import norm_act
+
+    M, K, N, r = 40, 512, 256, 16
+    d = single_inputs(M, K, N, r, p=0.0, seed=1)
+    gu = _gate_up(M, K, torch.bfloat16, 4).cuda()
+    w, a, b = (d[k].cuda() for k in ("w", "a", "b"))
+    x, y, s = (torch.full((M, n), 3.0, dtype=torch.bfloat16, device="cuda") for n in (K, N, 16))
+    routing = L.single_routing(r, 2.0, 0.0)
+    nbytes = L.lib().lf_workspace_bytes(L.LF_OP_FWD, M, N, K, 16, routing)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+
+    def call(s_ptr, ws_ptr, n, routing=routing):
+        return L.lib().lf_swiglu_lora_fwd(gu.data_ptr(), gu[:, K:].data_ptr(), 2 * K, x.data_ptr(), w.data_ptr(), None, None, None, ctypes.c_uint64(0),
+                                          L.ptr_array([a]), L.ptr_array([b]), y.data_ptr(), s_ptr, ws_ptr, n, M, N, K, 16, routing, 0, L.stream_of(gu))
+
+    assert call(None, ws.data_ptr(), nbytes) == L.LF_EINVAL
+    assert call(s.data_ptr(), ws.data_ptr(), nbytes, L.single_routing(12, 2.0, 0.0)) == L.LF_ESHAPE
+    torch.cuda.synchronize()
+    assert bool((x == 3.0).all()) and bool((y == 3.0).all())
+    c = norm_act.silu_mul_merged(gu)
+    ye, se = lora_ref.linear_lora_fwd_fp32(c.cpu(), d["w"], d["a"], d["b"], 2.0, None, 0.0, None)
+    for ptr, n in ((None, 0), (ws.data_ptr(), nbytes)):
+        assert call(s.data_ptr(), ptr, n) == 0
+        assert torch.equal(x, c)
+        _close(y, ye, "y")
+        _close(s, se, "S")
+        y.fill_(3.0), s.fill_(3.0), x.fill_(3.0)
+
+
 def test_layer_harness_takes_the_prologue_path(monkeypatch):
     """``DecoderLayerLoRAProjections`` without a caller-supplied activation runs the down projection through
     ``lf_swiglu_lora_fwd`` and gives what the activation kernel followed by the plain LoRA linear gives."""
