@@ -8,7 +8,7 @@ int lf_launch_nf4_dequant(const uint8_t*, const void*, const float*, const float
 int lf_launch_xa(const void*, const void*, int64_t, void*, const uint8_t*, uint8_t*, int, uint64_t, void*, void*, size_t, int, int, int,
                  const LfSegTable&, int, hipStream_t);
 bool lf_xa_takes_stream(int M, int K, int R, bool masked, const LfSegTable& seg, const void* ws, size_t ws_bytes);
-bool lf_short_fwd_applies(int M, int N);
+bool lf_short_fwd_applies(int M, int N, int K, int rank);
 size_t lf_short_fwd_workspace(int M, int N, int K, int rank);
 int lf_launch_short_fwd(const void*, const void*, const void*, const void*, float, const void*, void*, void*, void*, int, int, int, int, int,
                         const LfSegTable&, int, hipStream_t);
@@ -94,7 +94,7 @@ bool bad_rank_cols(int R) { return R <= 0 || R % 16 != 0 || R > LF_MAX_RANK; }
 // Scratch of a forward: the rank-r pass's slices and, behind them, a split contraction's partial tiles (Y = [M,N] over K); or the
 // short forward's slices.
 size_t fwd_workspace(int M, int N, int K, int R, int rb, const LfSegTable& t) {
-  const size_t sliced = !t.table && lf_short_fwd_applies(M, N) && !bad_tiled_dim(N) ? lf_short_fwd_workspace(M, N, K, t.rank[0]) : 0;
+  const size_t sliced = !t.table && !bad_tiled_dim(N) && lf_short_fwd_applies(M, N, K, t.rank[0]) ? lf_short_fwd_workspace(M, N, K, t.rank[0]) : 0;
   return std::max(sliced, align256(lf_xa_workspace(M, K, R, t)) + lf_gemm_ksplit_bytes(M, N, K, rb, false));
 }
 // What is left of a forward's workspace behind the rank-r pass's slices.
@@ -244,7 +244,7 @@ static bool short_fits(const void* X, const void* W, const void* const* a_ptrs, 
   if (lf_tile_pinned() || bad_dtype(dtype) || !X || !W || !Y || !S || !a_ptrs || !b_ptrs || M <= 0 || bad_tiled_dim(N) || bad_tiled_dim(K) ||
       bad_rank_cols(R) || (((uintptr_t)Y | (uintptr_t)S) & 15) != 0)
     return false;
-  if (make_seg(routing, M, a_ptrs, nullptr, t) != LF_OK || t.table || !lf_short_fwd_applies(M, N) || !t.ptr[0] || !b_ptrs[0] || t.rank[0] > R) return false;
+  if (make_seg(routing, M, a_ptrs, nullptr, t) != LF_OK || t.table || !lf_short_fwd_applies(M, N, K, t.rank[0]) || !t.ptr[0] || !b_ptrs[0] || t.rank[0] > R) return false;
   return workspace != nullptr && ws_bytes >= lf_short_fwd_workspace(M, N, K, t.rank[0]);
 }
 

@@ -387,10 +387,18 @@ static int short_pitch(int N, int rank) { return N + (rank + 15) / 16 * 16; }
 static int short_groups(int N, int rank) { return N / SROWS + (rank + SROWS - 1) / SROWS; }
 
 // Up to 64 rows the pass reads W at 4-5 TB/s where tiles of 64 columns leave most of the chip idle (6 x 4096 x 4096: 23.7 ->
-// 12.0 us, 64 rows: 24.9 -> 14.5; 6 x 4096 over 14336: 38.2 -> 24.0).  Up to 128 rows a workgroup fetches twice as many bytes
+// 12.0 us, 64 rows: 24.9 -> 14.5).  Up to 128 rows a workgroup fetches twice as many bytes
 // of X from L2 as of W: still ahead where the output is too narrow to fill the chip with tiles (128 x 4096 x 4096: 25.3 ->
-// 20.9), behind beyond that (128 x 14336 x 4096: 33.6 -> 45.3).
-bool lf_short_fwd_applies(int M, int N) { return M <= 64 || (M <= 128 && N <= 4096); }
+// 20.9).  What it loses is the second stage, whose workgroups (64 columns x 16 rows) form the LoRA term one column per lane, in time
+// with their number and the rank, while the general path's disadvantage grows with K: the line is fitted to 620 shapes of 8 - 128 rows,
+// K of 1024 - 14336, 1024 - 14336 columns and ranks 16 - 128, where the faster path is 0.4 % ahead of the chosen one on average
+// (64 x 14336 over 1024: rank 16 17.2 against 14.7 us, rank 128 48.7 against 21.1; over 4096 at rank 16 38.5 against 38.3;
+// 48 x 7168 over 2048: 14.6 against 16.7 at rank 16, 26.2 against 22.3 at 128).
+bool lf_short_fwd_applies(int M, int N, int K, int rank) {
+  if (M > 128 || (M > 64 && N > 4096)) return false;
+  const double finish = (double)(N / 64) * ((M + 15) / 16) * (M > 64 ? 1.5 : 1.0);
+  return finish <= 255.0 + (200.0 + 0.2 * (K - 1024)) * (28.0 / (12 + rank));
+}
 
 static int short_slices(int M, int N, int K, int rank) {
   return slices_for(short_groups(N, rank), K, (double)M * short_pitch(N, rank) * sizeof(float), kFwdSlices);

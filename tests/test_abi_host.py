@@ -161,6 +161,19 @@ def test_rank_pass_is_sliced_where_that_is_faster():
     assert slabs(2500, 1536, 128) > 1 and slabs(6000, 1536, 128) > 1
 
 
+def test_short_forward_takes_the_single_pass_where_that_is_faster():
+    """Host logic: the single pass keeps its slices in the forward's workspace; the general path of these shapes needs none."""
+    from lorafusion_amd import _lib as L
+
+    def single(M, K, N, R):
+        return L.lib().lf_workspace_bytes(L.LF_OP_FWD, M, N, K, R, L.single_routing(R, 1.0, 0.0)) > 0
+
+    assert single(6, 4096, 4096, 16) and single(64, 1024, 4096, 16) and single(64, 3072, 10240, 16)
+    # a second stage of many workgroups behind a short walk (64 x 14336 over 1024: 17.2 against 14.7 us)
+    assert not single(64, 1024, 14336, 16) and not single(48, 1024, 14336, 32) and not single(96, 1024, 4096, 16)
+    assert not single(129, 1024, 4096, 16)
+
+
 def test_python_layer_refuses_cpu_tensors():
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
     from lorafusion_amd.ops.nf4 import QuantState, dequantize_nf4_triton

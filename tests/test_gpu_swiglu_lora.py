@@ -160,7 +160,7 @@ def test_fused_layer_single_adapter_with_bias(p):
 @pytest.mark.parametrize("M,K,N,r,dtype", [(1, 128, 128, 8, torch.bfloat16), (64, 1152, 5120, 72, torch.float16), (65, 512, 384, 16, torch.bfloat16),
                                            (128, 4096, 4096, 32, torch.bfloat16), (128, 256, 4224, 16, torch.bfloat16)])
 def test_short_batches(M, K, N, r, dtype):
-    """Either side of the rule of the single pass (up to 64 rows, or 128 under at most 4096 columns): the oracle, and the unfused ops bit for bit."""
+    """Either side of the rule of the single pass (few rows, narrow outputs, low ranks): the oracle, and the unfused ops bit for bit."""
     from lorafusion_amd.ops import norm_act
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
     from lorafusion_amd.ops.swiglu_lora import fused_swiglu_linear_lora
