@@ -14,12 +14,13 @@ int lf_launch_short_fwd(const void*, const void*, const void*, const void*, floa
                         const LfSegTable&, int, hipStream_t);
 int lf_launch_mask_pack(const uint8_t*, uint8_t*, int64_t, hipStream_t);
 int lf_launch_mask_unpack(const uint8_t*, uint8_t*, int64_t, hipStream_t);
-int lf_launch_dys_dyb(const void*, const void*, void*, void*, size_t, int, int, int, const LfSegTable&, int, hipStream_t);
-int lf_launch_da(const void*, const uint8_t*, int, const void*, void*, size_t, int, int, int, const LfSegTable&, int, hipStream_t);
+int lf_launch_dys_dyb(const void*, const void*, void*, void*, size_t, size_t, int, int, int, const LfSegTable&, int, hipStream_t);
+int lf_launch_da(const void*, const uint8_t*, int, const void*, void*, size_t, size_t, int, int, int, const LfSegTable&, int, hipStream_t);
 int lf_launch_dropout_mask(uint8_t*, int, int, float, const float*, int, uint64_t, hipStream_t);
 size_t lf_xa_workspace(int, int, int, const LfSegTable&);
-size_t lf_dys_dyb_workspace(int, int, int, const LfSegTable&);
-size_t lf_da_workspace(int, int, int, const LfSegTable&);
+// limit: bytes the split of the pass is to stay within, where one does (a call and its size query name the same)
+size_t lf_dys_dyb_workspace(int, int, int, const LfSegTable&, size_t limit = SIZE_MAX);
+size_t lf_da_workspace(int, int, int, const LfSegTable&, size_t limit = SIZE_MAX);
 
 // Scratch of lf_lora_bwd_static: part of the device image, one copy per GPU at its own address.  In
 // host code the array's name is only a handle for hipGetSymbolAddress; kernels and launch code
@@ -266,24 +267,34 @@ int lf_swiglu_lora_fwd(const void* G, const void* U, int64_t ld, void* X_out, co
   return xw_sb_ws(X_out, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);
 }
 
-int lf_lora_dys_dyb(const void* dY, const void* S, const void* const* b_ptrs, void* dS, void* const* db_ptrs,
-                    void* workspace, size_t ws_bytes, int M, int N, int R, const lf_routing* routing, int dtype,
-                    void* stream) {
+static int dys_dyb_within(const void* dY, const void* S, const void* const* b_ptrs, void* dS, void* const* db_ptrs, void* workspace, size_t ws_bytes,
+                          size_t limit, int M, int N, int R, const lf_routing* routing, int dtype, void* stream) {
   if (bad_dtype(dtype) || !b_ptrs || !db_ptrs) return LF_EINVAL;
   LfSegTable t;
   int rc = make_seg(routing, M, b_ptrs, db_ptrs, t);
   if (rc != LF_OK) return rc;
-  return lf_launch_dys_dyb(dY, S, dS, workspace, ws_bytes, M, N, R, t, dtype, (hipStream_t)stream);
+  return lf_launch_dys_dyb(dY, S, dS, workspace, ws_bytes, limit, M, N, R, t, dtype, (hipStream_t)stream);
 }
 
-int lf_lora_da(const void* X, const uint8_t* mask, const void* dS, void* const* da_ptrs, void* workspace,
-               size_t ws_bytes, int M, int K, int R, const lf_routing* routing, int dtype, void* stream) {
+int lf_lora_dys_dyb(const void* dY, const void* S, const void* const* b_ptrs, void* dS, void* const* db_ptrs,
+                    void* workspace, size_t ws_bytes, int M, int N, int R, const lf_routing* routing, int dtype,
+                    void* stream) {
+  return dys_dyb_within(dY, S, b_ptrs, dS, db_ptrs, workspace, ws_bytes, SIZE_MAX, M, N, R, routing, dtype, stream);
+}
+
+static int da_within(const void* X, const uint8_t* mask, const void* dS, void* const* da_ptrs, void* workspace, size_t ws_bytes, size_t limit, int M,
+                     int K, int R, const lf_routing* routing, int dtype, void* stream) {
   const int mb = take_mask_bits(dtype);
   if (bad_dtype(dtype) || !da_ptrs) return LF_EINVAL;
   LfSegTable t;
   int rc = make_seg(routing, M, nullptr, da_ptrs, t);
   if (rc != LF_OK) return rc;
-  return lf_launch_da(X, mask, mb, dS, workspace, ws_bytes, M, K, R, t, dtype, (hipStream_t)stream);
+  return lf_launch_da(X, mask, mb, dS, workspace, ws_bytes, limit, M, K, R, t, dtype, (hipStream_t)stream);
+}
+
+int lf_lora_da(const void* X, const uint8_t* mask, const void* dS, void* const* da_ptrs, void* workspace,
+               size_t ws_bytes, int M, int K, int R, const lf_routing* routing, int dtype, void* stream) {
+  return da_within(X, mask, dS, da_ptrs, workspace, ws_bytes, SIZE_MAX, M, K, R, routing, dtype, stream);
 }
 
 static int dyw_dsa_ws(const void* dY, const void* W, const void* dS, const void* const* a_ptrs, const uint8_t* mask,
@@ -335,18 +346,24 @@ int lf_lora_fwd_seeded(const void* X, const void* W, const void* bias, uint8_t* 
   return xw_sb_ws(X, W, bias, S_out, b_ptrs, Y, workspace, ws_bytes, M, N, K, R, routing, dtype & ~LF_MASK_BITS, stream);
 }
 
-int lf_lora_bwd(const void* dY, const void* X, const void* W, const uint8_t* mask, const void* S,
-                const void* const* a_ptrs, const void* const* b_ptrs, void* dX, void* const* da_ptrs,
-                void* const* db_ptrs, void* dS_out, void* workspace, size_t ws_bytes, int M, int N, int K, int R,
-                const lf_routing* routing, int dtype, void* stream) {
-  int rc = lf_lora_dys_dyb(dY, S, b_ptrs, dS_out, db_ptrs, workspace, ws_bytes, M, N, R, routing, dtype & ~LF_MASK_BITS, stream);
+static int bwd_within(const void* dY, const void* X, const void* W, const uint8_t* mask, const void* S, const void* const* a_ptrs,
+                      const void* const* b_ptrs, void* dX, void* const* da_ptrs, void* const* db_ptrs, void* dS_out, void* workspace, size_t ws_bytes,
+                      size_t limit, int M, int N, int K, int R, const lf_routing* routing, int dtype, void* stream) {
+  int rc = dys_dyb_within(dY, S, b_ptrs, dS_out, db_ptrs, workspace, ws_bytes, limit, M, N, R, routing, dtype & ~LF_MASK_BITS, stream);
   if (rc != LF_OK) return rc;
-  rc = lf_lora_da(X, mask, dS_out, da_ptrs, workspace, ws_bytes, M, K, R, routing, dtype, stream);
+  rc = da_within(X, mask, dS_out, da_ptrs, workspace, ws_bytes, limit, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;
   // (stream order: the partial sums of the two rank-r passes are consumed by now, so the product's split contraction
   // may reuse the workspace from its start)
   if (dX) rc = dyw_dsa_ws(dY, W, dS_out, a_ptrs, mask, dX, workspace, ws_bytes, M, N, K, R, routing, dtype, stream);
   return rc;
+}
+
+int lf_lora_bwd(const void* dY, const void* X, const void* W, const uint8_t* mask, const void* S,
+                const void* const* a_ptrs, const void* const* b_ptrs, void* dX, void* const* da_ptrs,
+                void* const* db_ptrs, void* dS_out, void* workspace, size_t ws_bytes, int M, int N, int K, int R,
+                const lf_routing* routing, int dtype, void* stream) {
+  return bwd_within(dY, X, W, mask, S, a_ptrs, b_ptrs, dX, da_ptrs, db_ptrs, dS_out, workspace, ws_bytes, SIZE_MAX, M, N, K, R, routing, dtype, stream);
 }
 
 int lf_lora_bwd_static(const void* dY, const void* X, const void* W, const uint8_t* mask, const void* S,
@@ -361,15 +378,16 @@ int lf_lora_bwd_static(const void* dY, const void* X, const void* W, const uint8
   int rc = make_seg(routing, M, nullptr, nullptr, t);
   if (rc != LF_OK) return rc;
   // what lf_workspace_bytes(LF_OP_BWD, ...) names: the rank-r passes' partial sums or the dX product's partial tiles,
-  // whichever is larger (with less, the product would not split its contraction and its sums would differ in order)
-  const size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
+  // whichever is larger (with less, the product would not split its contraction and its sums would differ in order).  Above rank 64, where
+  // the fastest split has up to twice the partial sums of a slightly slower one, a split that fits is taken if there is one.
+  const size_t limit = R > 64 ? (size_t)LF_STATIC_SCRATCH_BYTES : SIZE_MAX;
+  const size_t a = lf_dys_dyb_workspace(M, N, R, t, limit), b = lf_da_workspace(M, K, R, t, limit);
   const size_t need = align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, t.table != nullptr ? t.block_size_m : 0, true)));
   if (need > (size_t)LF_STATIC_SCRATCH_BYTES) return LF_ESTATIC;
   void* ws = nullptr;
   rc = static_scratch(&ws);
   if (rc != LF_OK) return rc;
-  return lf_lora_bwd(dY, X, W, mask, S, a_ptrs, b_ptrs, dX, da_ptrs, db_ptrs, dS_out, ws, LF_STATIC_SCRATCH_BYTES, M, N, K,
-                     R, routing, dtype, stream);
+  return bwd_within(dY, X, W, mask, S, a_ptrs, b_ptrs, dX, da_ptrs, db_ptrs, dS_out, ws, LF_STATIC_SCRATCH_BYTES, limit, M, N, K, R, routing, dtype, stream);
 }
 
 int lf_set_tile_cfg(int tile_cfg) { return lf_pin_tile_cfg(tile_cfg); }

@@ -822,8 +822,8 @@ static int dysr_smem(int rt) { return dysr_ns(rt) * (TILE_BYTES + (rt >= 2 ? rt 
 struct DysRingPlan { int n_slices, group, max_chunks; };
 // By bytes: the dY (+ B tile) stream over the busiest slot, the S blocks every workgroup fetches (from L2: half weight),
 // and the fp32 partials written here and read by the reduce (dS: one [rows, R] slab per slice; dB: one [N, R] slab per
-// chunk).
-static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
+// chunk).  The cheapest plan whose partials take at most `limit` bytes (if none does: the cheapest of all).
+static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = N / 64;
   int blocks[LF_MAX_SEG], nseg;
   seg_block_counts(M, seg, blocks, nseg);
@@ -835,6 +835,7 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
   GroupStats stats[kNGroups];
   const int ng = all_group_stats(blocks, nseg, stats);
   double best_cost = 1e300;
+  bool best_fits = false;
   for (int t = dysr_tpw(rt); t >= 2; t--) {   // tiles of the longest slice -> fewest slices that reach it
     const int nsl = (T + t - 1) / t;
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
@@ -842,7 +843,8 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg) {
       const GroupStats& st = stats[k];
       const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
                           2.0 * 4.0 * R * ((double)nsl * rows + (double)st.chunks * N);
-      if (cost < best_cost) { best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks}; }
+      const bool fits = ((size_t)nsl * rows * R + (size_t)nseg * st.max_chunks * N * R) * sizeof(float) <= limit;
+      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks}; }
     }
   }
   return best;
@@ -948,11 +950,11 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
   return LF_EINVAL;
 }
 
-size_t lf_dys_dyb_workspace(int M, int N, int R, const LfSegTable& seg) {
+size_t lf_dys_dyb_workspace(int M, int N, int R, const LfSegTable& seg, size_t limit) {
   const int nblk = n_row_blocks(M, seg);
   const int64_t rows = seg.table ? (int64_t)nblk * ROWS : M;
   const int nseg = seg.table ? seg.n_seg : 1;
-  const DysRingPlan pl = dysr_plan(M, N, R, seg);
+  const DysRingPlan pl = dysr_plan(M, N, R, seg, limit);
   return ((size_t)pl.n_slices * rows * R + (size_t)nseg * pl.max_chunks * N * R) * sizeof(float);
 }
 
@@ -968,12 +970,12 @@ static int dysr_launch(const void* dY, const void* S, float* ds_part, float* db_
 }
 
 template <typename T>
-static int dys_dyb_impl(const void* dY, const void* S, void* dS, void* ws, int M, int N, int R, const LfSegTable& seg, hipStream_t st) {
+static int dys_dyb_impl(const void* dY, const void* S, void* dS, void* ws, size_t limit, int M, int N, int R, const LfSegTable& seg, hipStream_t st) {
   const int nblk = n_row_blocks(M, seg);
   const int64_t rows = seg.table ? (int64_t)nblk * ROWS : M;
   const int nseg = seg.table ? seg.n_seg : 1;
   float* ds_part = (float*)ws;   // [slices][rows][R], then the dB partials [nseg * max_chunks][N][R]
-  const DysRingPlan pl = dysr_plan(M, N, R, seg);
+  const DysRingPlan pl = dysr_plan(M, N, R, seg, limit);
   float* db_part = ds_part + (int64_t)pl.n_slices * rows * R;
   int rc;
   switch (rt_of(R)) {
@@ -992,7 +994,7 @@ static int dys_dyb_impl(const void* dY, const void* S, void* dS, void* ws, int M
                      (T*)dS, pl.n_slices, M, R, nb_rows, (const float*)db_part, N, nb_seg, pl.group, pl.max_chunks, seg);
 }
 
-int lf_launch_dys_dyb(const void* dY, const void* S, void* dS, void* ws, size_t ws_bytes, int M, int N, int R,
+int lf_launch_dys_dyb(const void* dY, const void* S, void* dS, void* ws, size_t ws_bytes, size_t limit, int M, int N, int R,
                       const LfSegTable& seg, int dtype, hipStream_t st) {
   if (!dY || !S || !dS || M <= 0 || N <= 0) return LF_EINVAL;
   if (N % 128 != 0 || R % 16 != 0 || R <= 0 || R > LF_MAX_RANK) return LF_ESHAPE;
@@ -1001,9 +1003,9 @@ int lf_launch_dys_dyb(const void* dY, const void* S, void* dS, void* ws, size_t 
   for (int s = 0; s < nseg; s++) if (!seg.out[s] || !seg.ptr[s] || seg.rank[s] % 8 != 0 || seg.rank[s] > R) return LF_EINVAL;
   for (int s = 0; s < nseg; s++) if (((uintptr_t)seg.out[s] & 7) != 0) return LF_ESHAPE;  // 8-byte stores of dB
   if (((uintptr_t)dS & 7) != 0) return LF_ESHAPE;
-  if (!ws || ws_bytes < lf_dys_dyb_workspace(M, N, R, seg)) return LF_EWORKSPACE;
-  if (dtype == LF_BF16) return dys_dyb_impl<__bf16>(dY, S, dS, ws, M, N, R, seg, st);
-  if (dtype == LF_F16) return dys_dyb_impl<_Float16>(dY, S, dS, ws, M, N, R, seg, st);
+  if (!ws || ws_bytes < lf_dys_dyb_workspace(M, N, R, seg, limit)) return LF_EWORKSPACE;
+  if (dtype == LF_BF16) return dys_dyb_impl<__bf16>(dY, S, dS, ws, limit, M, N, R, seg, st);
+  if (dtype == LF_F16) return dys_dyb_impl<_Float16>(dY, S, dS, ws, limit, M, N, R, seg, st);
   return LF_EINVAL;
 }
 
@@ -1018,8 +1020,8 @@ static int da_ring_smem(int rt, int maskfmt) { return da_ns(rt, maskfmt) * (TILE
 struct DaPlan { int n_slices, group, max_chunks; };
 // Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by bytes moved: the
 // X stream in whole rounds of resident workgroups, the dS blocks every workgroup fetches, and the fp32 partials
-// (one [R, K] slab per chunk, written here and read by the reduce).
-static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg) {
+// (one [R, K] slab per chunk, written here and read by the reduce).  `limit`: as for dysr_plan.
+static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = K / 64;
   int blocks[LF_MAX_SEG], nseg;
   seg_block_counts(M, seg, blocks, nseg);
@@ -1030,6 +1032,7 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg) {
   GroupStats stats[kNGroups];
   const int ng = all_group_stats(blocks, nseg, stats);
   double best_cost = 1e300;
+  bool best_fits = false;
   for (int t = da_tpw(rt); t >= 2; t--) {   // tiles of the longest slice -> fewest slices that reach it
     const int nsl = (T + t - 1) / t;
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
@@ -1037,17 +1040,18 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg) {
       const GroupStats& st = stats[k];
       const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
                           2.0 * 4.0 * R * K * (double)st.chunks;
-      if (cost < best_cost) { best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks}; }
+      const bool fits = (size_t)nseg * st.max_chunks * R * K * sizeof(float) <= limit;
+      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks}; }
     }
   }
   return best;
 }
 
-size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg) {
+size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit) {
   const int nseg = seg.table ? seg.n_seg : 1;
   // the launch plans with or without a keep-mask (one byte or one bit per element): room for any
   int max_chunks = 1;
-  for (int fmt = 0; fmt < 3; fmt++) max_chunks = std::max(max_chunks, da_plan(M, K, R, fmt, seg).max_chunks);
+  for (int fmt = 0; fmt < 3; fmt++) max_chunks = std::max(max_chunks, da_plan(M, K, R, fmt, seg, limit).max_chunks);
   return (size_t)nseg * max_chunks * R * K * sizeof(float);
 }
 
@@ -1063,12 +1067,13 @@ static int da_ring_launch(const void* X, const uint8_t* mask, const void* dS, fl
 }
 
 template <typename T>
-static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, int M, int K, int R, const LfSegTable& seg, hipStream_t st) {
+static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, size_t limit, int M, int K, int R, const LfSegTable& seg,
+                   hipStream_t st) {
   const int nseg = seg.table ? seg.n_seg : 1;
   float* part = (float*)ws;
   int rc;
   const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
-  const DaPlan pl = da_plan(M, K, R, fmt, seg);
+  const DaPlan pl = da_plan(M, K, R, fmt, seg, limit);
 #define LF_DA_RING(RTV)                                                                                                   \
   rc = fmt == 2   ? da_ring_launch<T, RTV, 2>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
        : fmt == 1 ? da_ring_launch<T, RTV, 1>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
@@ -1087,7 +1092,7 @@ static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void
   return lf_launch((reduce_segments_kernel<T>), dim3((unsigned)((nout + 1023) / 1024), nseg), dim3(256), 0, st, (const float*)part, K, R, 1, mask != nullptr ? 1 : 2, M, pl.group, pl.max_chunks, seg);
 }
 
-int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, size_t ws_bytes, int M, int K, int R,
+int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* dS, void* ws, size_t ws_bytes, size_t limit, int M, int K, int R,
                  const LfSegTable& seg, int dtype, hipStream_t st) {
   if (!X || !dS || M <= 0 || K <= 0) return LF_EINVAL;
   if (K % 128 != 0 || R % 16 != 0 || R <= 0 || R > LF_MAX_RANK) return LF_ESHAPE;
@@ -1095,10 +1100,10 @@ int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* 
   const int nseg = seg.table ? seg.n_seg : 1;
   for (int s = 0; s < nseg; s++) if (!seg.out[s] || seg.rank[s] % 8 != 0 || seg.rank[s] > R) return LF_EINVAL;
   for (int s = 0; s < nseg; s++) if (((uintptr_t)seg.out[s] & 7) != 0) return LF_ESHAPE;  // 8-byte stores of dA
-  if (!ws || ws_bytes < lf_da_workspace(M, K, R, seg)) return LF_EWORKSPACE;
+  if (!ws || ws_bytes < lf_da_workspace(M, K, R, seg, limit)) return LF_EWORKSPACE;
   if (mask != nullptr && mask_bits && ((uintptr_t)mask & 3) != 0) return LF_ESHAPE;   // 4-byte loads of the keep bits
-  if (dtype == LF_BF16) return da_impl<__bf16>(X, mask, mask_bits, dS, ws, M, K, R, seg, st);
-  if (dtype == LF_F16) return da_impl<_Float16>(X, mask, mask_bits, dS, ws, M, K, R, seg, st);
+  if (dtype == LF_BF16) return da_impl<__bf16>(X, mask, mask_bits, dS, ws, limit, M, K, R, seg, st);
+  if (dtype == LF_F16) return da_impl<_Float16>(X, mask, mask_bits, dS, ws, limit, M, K, R, seg, st);
   return LF_EINVAL;
 }
 

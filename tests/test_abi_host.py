@@ -107,6 +107,32 @@ def test_size_query_and_static_backward_refuse_untiled_shapes():
     assert call(256, 256, 256, 16, dy=None) == _lib.LF_EINVAL
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="an accepted call would launch on the test's made-up pointers")
+def test_static_backward_takes_high_ranks_whose_fastest_split_does_not_fit():
+    """The call gets as far as looking for a device.  One adapter, and packed rows."""
+    from lorafusion_amd import _lib
+
+    lib, one, ptrs = _lib.lib(), ctypes.c_void_p(256), (ctypes.c_void_p * 6)(*[256] * 6)
+
+    def call(M, N, K, R, r):
+        return lib.lf_lora_bwd_static(one, one, one, None, one, ptrs, ptrs, one, ptrs, ptrs, one, M, N, K, R, r, 0, None)
+
+    def packed(blocks, ranks):
+        n = sum(blocks)
+        keep = torch.zeros((n, 3), dtype=torch.int32), torch.ones(n), torch.zeros(n)
+        return _lib.multi_routing([128 * b for b in blocks], ranks, *keep, 128), keep
+
+    for M, N, K, rank in ((1318, 7040, 256, 96), (531, 10240, 9472, 128), (969, 7680, 128, 128)):
+        r = _lib.single_routing(rank, 1.0, 0.1)
+        assert lib.lf_workspace_bytes(_lib.LF_OP_BWD, M, N, K, rank, r) > _lib.LF_STATIC_SCRATCH_BYTES
+        assert call(M, N, K, rank, r) == _lib.LF_ELAUNCH
+    for blocks, N, K in (([1, 1, 1], 13952, 3456), ([1, 1, 4, 2, 2], 5120, 256), ([2, 16, 1, 3, 1], 1280, 256)):
+        r, keep = packed(blocks, [128] * len(blocks))
+        assert call(128 * sum(blocks), N, K, 128, r) == _lib.LF_ELAUNCH
+    assert call(9000, 8192, 8192, 128, _lib.single_routing(128, 1.0, 0.1)) == _lib.LF_ESTATIC    # no split fits
+    assert call(128, 28672, 256, 64, _lib.single_routing(64, 1.0, 0.1)) != _lib.LF_OK
+
+
 def test_launch_plan_takes_the_contraction_length():
     """Host logic of the tile choice: left-over rows get a launch of their own when the contraction is long enough to
     pay for it, and one launch covers everything when it is short."""

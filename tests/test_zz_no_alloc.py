@@ -25,7 +25,7 @@ def _outputs(M, N, K, ranks, dev, dtype):
     return dx, da, db, ds
 
 
-def _both(dy, x, w, mask, a_list, b_list, routing_c, R, ranks):
+def _both(dy, x, w, mask, a_list, b_list, routing_c, R, ranks, fits=True):
     """Run lf_lora_bwd (with a torch workspace) and lf_lora_bwd_static; return both output sets."""
     from lorafusion_amd import _lib as L
     from lorafusion_amd.ops import hip_ops
@@ -36,7 +36,7 @@ def _both(dy, x, w, mask, a_list, b_list, routing_c, R, ranks):
     y, s = hip_ops.lora_forward(x, w, a_list, b_list, routing_c, R, mask, None)
     lib = L.lib()
     need = lib.lf_workspace_bytes(L.LF_OP_BWD, M, N, K, R, routing_c)
-    assert 0 < need <= L.LF_STATIC_SCRATCH_BYTES
+    assert need > 0 and (need <= L.LF_STATIC_SCRATCH_BYTES) == fits
     ws = torch.empty(need, dtype=torch.uint8, device=dev)
     ref = _outputs(M, N, K, ranks, dev, dtype)
     rc = lib.lf_lora_bwd(L.ptr(dy), L.ptr(x), L.ptr(w), L.ptr(mask), L.ptr(s), L.ptr_array(a_list), L.ptr_array(b_list),
@@ -89,6 +89,29 @@ def test_static_scratch_backward_matches_workspace_backward():
     ref2, got2 = _both(e["dy"].to(dev), e["x"].to(dev), e["w"].to(dev), e["mask"].to(dev), [e["a"].to(dev)],
                        [e["b"].to(dev)], rs, 16, [r2])
     _assert_same(ref2, got2, "single adapter, smaller call")
+
+
+def test_static_scratch_backward_with_a_split_that_fits():
+    """Ranks above 64 whose fastest split needs more than the buffer: another one of the same sums (32-bit, so one rounding of each
+    result apart: 2^-7 of the largest value of a tensor in bf16)."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+    from lorafusion_amd.ops.multi_lora import prepare_multi_lora_batch_info
+
+    dev = "cuda"
+    e = single_inputs(969, 256, 7680, 128, p=0.1, seed=6)
+    one = _both(e["dy"].to(dev), e["x"].to(dev), e["w"].to(dev), e["mask"].to(dev), [e["a"].to(dev)], [e["b"].to(dev)],
+                L.single_routing(128, 2.0, 0.1), 128, [128], fits=False)
+    seq, ranks = [100, 128, 500, 200, 129], [128, 72, 128, 8, 128]
+    d = multi_inputs(seq, 256, 5120, ranks, [0.1] * 5, seed=7)
+    info = prepare_multi_lora_batch_info(seq, list(range(5)), ranks, [0.1] * 5, [1.0] * 5, 128)
+    routing = hip_ops.MultiRouting(info.padded_seq_len_list, ranks, info.block_to_lookup_table, info.block_to_alpha, info.block_to_dropout_p)
+    five = _both(d["dy"].to(dev), d["x"].to(dev), d["w"].to(dev), d["mask"].to(dev), [t.to(dev) for t in d["a_list"]],
+                 [t.to(dev) for t in d["b_list"]], routing.c, routing.R, ranks, fits=False)
+    for ref, got in (one, five):
+        for r, g in ((ref[0], got[0]), *zip(ref[1], got[1]), *zip(ref[2], got[2]), (ref[3], got[3])):
+            assert torch.isfinite(g.float()).all()
+            assert float((r.float() - g.float()).abs().max()) <= 2.0 ** -7 * float(r.float().abs().max())
 
 
 def test_static_scratch_rejects_oversized_call():
