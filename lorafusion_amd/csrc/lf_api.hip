@@ -7,7 +7,7 @@ int lf_launch_nf4_dequant(const uint8_t*, const void*, const float*, const float
                           int, int, int, hipStream_t);
 int lf_launch_xa(const void*, const void*, int64_t, void*, const uint8_t*, uint8_t*, int, uint64_t, void*, void*, size_t, int, int, int,
                  const LfSegTable&, int, hipStream_t);
-bool lf_xa_takes_stream(int M, int K, int R, bool masked, const LfSegTable& seg, const void* ws, size_t ws_bytes);
+bool lf_xa_takes_stream(int M, int K, int R, const uint8_t* mask, int mask_bits, bool drawn, const LfSegTable& seg, const void* ws, size_t ws_bytes);
 bool lf_short_fwd_applies(int M, int N, int K, int rank);
 size_t lf_short_fwd_workspace(int M, int N, int K, int rank);
 int lf_launch_short_fwd(const void*, const void*, const void*, const void*, float, const void*, void*, void*, void*, int, int, int, int, int,
@@ -195,7 +195,7 @@ static int xa_silu_mul_ws(const void* G, const void* U, int64_t ld, void* X_out,
   if (rc != LF_OK) return rc;
   for (int s = 0; s < t.n_seg; s++) if (!t.ptr[s]) return LF_EINVAL;
   // (what the fused kernel refuses is refused here too; where the sliced pass takes the product, the activation is a pass of its own)
-  if (M > 0 && K > 0 && S != nullptr && lf_xa_takes_stream(M, K, R, mask != nullptr || mask_out != nullptr, t, workspace, ws_bytes)) {
+  if (M > 0 && K > 0 && S != nullptr && lf_xa_takes_stream(M, K, R, mask, mb, mask_out != nullptr, t, workspace, ws_bytes)) {
     if (K % 128 != 0 || bad_rank_cols(R) || ld < K || ld % 8 != 0 || (((uintptr_t)G | (uintptr_t)U | (uintptr_t)X_out) & 15) != 0) return LF_ESHAPE;
     rc = lf_silu_mul_fwd(G, U, X_out, M, K, ld, ld, K, dtype, stream);
     if (rc != LF_OK) return rc;

@@ -422,6 +422,20 @@ __device__ __forceinline__ void tile_apply_mask(char* tile, const char* mtile, i
 #pragma unroll
   for (int i = 0; i < 4; i++) *(lf_u32x4*)(tile + (i * 256 + tid) * 16) = apply_mask8(x[i], m[i]);
 }
+// the same for a mask of bytes that is read from memory here, `mask` at the tile's first element: any address, rows of K bytes, `rows` of them
+__device__ __forceinline__ void tile_apply_bytes(char* tile, const uint8_t* mask, int64_t K, int64_t rows, int tid) {
+  lf_u32x4 x[4];
+  lf_u32x2 m[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int p = i * 256 + tid, row = p >> 3, g = (p & 7) ^ tile_key(row);
+    x[i] = *(const lf_u32x4*)(tile + p * 16);
+    m[i] = lf_u32x2{0, 0};
+    if (row < rows) m[i] = keep_bytes8(mask + row * K + g * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) *(lf_u32x4*)(tile + (i * 256 + tid) * 16) = apply_mask8(x[i], m[i]);
+}
 
 // A [rows x RT*16] side operand (S or dS block: 128 rows; B tile: 64 rows) in LDS: rows of RT*32 bytes; granule g of
 // source row r at slot g ^ side_key(r) of LDS row side_row(r).  A transposed read is served 32 lanes at a time: rows
@@ -475,7 +489,8 @@ __global__ void __launch_bounds__(256, RT >= 8 ? 1 : 2)
 lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, const T* __restrict__ dS, float* __restrict__ part,
                     int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg) {
   // MASK: 0 no keep-mask; 1 one byte per element (8 KB per tile, two loads per thread); 2 one bit per element (1 KB per
-  // tile, one 4-byte load per thread)
+  // tile, one 4-byte load per thread); 3 one byte per element at an address that the direct loads do not take, read where it is applied (the compiler's
+  // waits for those loads empty the ring every tile)
   constexpr int STAGE = TILE_BYTES + da_mask_tile_bytes(MASK);
   constexpr int SIDE = ROWS * RT * 32;
   constexpr int G = 4 + (MASK == 1 ? 2 : MASK == 2 ? 1 : 0);   // operations per load group and thread, not counting a dS block
@@ -552,10 +567,18 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
     for (int c = 0; c < RT; c++) acc[t][c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
 
   int cst = 0;   // stage of the pair being consumed
+  auto apply_mask = [&](char* stage, int b, int t) {   // (tile t of block b)
+    if constexpr (MASK == 3) {
+      const int64_t row = (int64_t)b * ROWS;
+      tile_apply_bytes(stage, mask + row * K + (kt0 + t) * 64, K, Mrows - row, tid);
+    } else {
+      tile_apply_mask<MASK == 2>(stage, stage + TILE_BYTES, tid);
+    }
+  };
   if constexpr (MASK) {
     wait_groups<G>(ns - 2);
     ring_barrier();
-    if (use_mask) tile_apply_mask<MASK == 2>(ring, ring + TILE_BYTES, tid);
+    if (use_mask) apply_mask(ring, bb0, 0);
   }
   for (int b = bb0; b < bb1; b++) {
     const char* dcur = side + ((b - bb0) & 1) * SIDE;
@@ -569,7 +592,8 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
         issue();
         if constexpr (MASK) {
           const int nst = cst + 1 == ns ? 0 : cst + 1;
-          if (use_mask) tile_apply_mask<MASK == 2>(ring + nst * STAGE, ring + nst * STAGE + TILE_BYTES, tid);
+          // (behind the last pair the last tile is there again, unconsumed: any mask of the matrix does)
+          if (use_mask) apply_mask(ring + nst * STAGE, t + 1 < nt || b + 1 == bb1 ? b : b + 1, t + 1 < nt ? t + 1 : 0);
         }
         const char* xcur = ring + cst * STAGE;
         // all fragments of the tile first, then the MFMAs: with one or two waves per SIMD nothing else hides the LDS
@@ -885,7 +909,10 @@ static bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& se
 }
 // ... and those it takes.  Without the memory (entry points that have no workspace to give, or too small a one) this file's kernel
 // runs to rank 64; above, and where a single slice needs none, the sliced pass all the same.
-bool lf_xa_takes_stream(int M, int K, int R, bool masked, const LfSegTable& seg, const void* ws, size_t ws_bytes) {
+// A mask read from an address that the direct loads do not take also stays with this file's kernel to rank 64.
+bool lf_xa_takes_stream(int M, int K, int R, const uint8_t* mask, int mask_bits, bool drawn, const LfSegTable& seg, const void* ws, size_t ws_bytes) {
+  const bool masked = mask != nullptr || drawn;
+  if (R <= 64 && mask_off_grid(mask, mask_bits)) return false;
   return lf_xa_streams(M, K, R, masked, seg) && (R > 64 || lf_xa_stream_slices(M, K, R, masked, seg) == 1 ||
                                                  (ws != nullptr && ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg)));
 }
@@ -941,7 +968,7 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
   } else {
     ldx = K;
     const bool masked = mask != nullptr || mask_out != nullptr;
-    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_takes_stream(M, K, R, masked, seg, ws, ws_bytes))
+    if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_takes_stream(M, K, R, mask, mask_bits, mask_out != nullptr, seg, ws, ws_bytes))
       return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg) ? (float*)ws : nullptr, M,
                                  K, R, seg, dtype, st);
   }
@@ -1073,9 +1100,11 @@ static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void
   float* part = (float*)ws;
   int rc;
   const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
+  const bool off_grid = fmt == 1 && mask_off_grid(mask, 0);   // (the same split, and the same sums)
   const DaPlan pl = da_plan(M, K, R, fmt, seg, limit);
 #define LF_DA_RING(RTV)                                                                                                   \
-  rc = fmt == 2   ? da_ring_launch<T, RTV, 2>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
+  rc = off_grid   ? da_ring_launch<T, RTV, 3>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
+       : fmt == 2 ? da_ring_launch<T, RTV, 2>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
        : fmt == 1 ? da_ring_launch<T, RTV, 1>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
                   : da_ring_launch<T, RTV, 0>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)
   switch (rt_of(R)) {

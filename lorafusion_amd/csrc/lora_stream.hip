@@ -44,7 +44,8 @@ struct StreamArgs {
   const void* q;         // forward: X [M, K]
 };
 
-// grid (64-row groups of P, slices of K).  MODE: 0 no keep-mask, 1 keep bytes read, 2 keep bits read, 3 mask drawn and written.
+// grid (64-row groups of P, slices of K).  MODE: 0 no keep-mask, 1 keep bytes read, 2 keep bits read, 3 mask drawn and written, 4 bytes or bits
+// read from an address that the direct loads do not take (the compiler's waits for these loads empty the ring every step).
 // FWD: Q = X (the second use above), D is stored transposed, [m][row of P].
 template <typename T, int RT, int MODE, bool FWD>
 __global__ void __launch_bounds__(256, 2)
@@ -165,6 +166,16 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
         const char* mt = lds + cst * STAGE + SROWS * 128 + QB + wave * 256;
 #pragma unroll
         for (int h = 0; h < 2; h++) xf[h] &= select8(*(const uint8_t*)(mt + li * 8 + h * 4 + qq));
+      }
+    }
+    if constexpr (MODE == 4) {
+      if (use_mask && my_row < rows_all) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const uint64_t el = (uint64_t)(my_row * K + k0) + (uint64_t)(s * 64 + (h * 4 + qq) * 8);
+          if (a.mask_bytes) xf[h] = apply_mask8(xf[h], keep_bytes8(a.mask + el));
+          else xf[h] &= select8(a.mask[el >> 3]);
+        }
       }
     }
     if constexpr (MODE == 3) {
@@ -332,6 +343,10 @@ template <typename T, int RT>
 int stream_mode(const StreamArgs& a, const LfSegTable& seg, int groups, hipStream_t st) {
   if (a.q != nullptr) return stream_launch<T, RT, 0, true>(a, seg, groups, st);
   if (a.mask_out != nullptr) return stream_launch<T, RT, 3, false>(a, seg, groups, st);
+  if (mask_off_grid(a.mask, !a.mask_bytes)) {
+    if constexpr (RT == 8) return stream_launch<T, RT, 4, false>(a, seg, groups, st);
+    else return LF_ESHAPE;   // (lf_xa_takes_stream)
+  }
   if (a.mask != nullptr) return a.mask_bytes ? stream_launch<T, RT, 1, false>(a, seg, groups, st) : stream_launch<T, RT, 2, false>(a, seg, groups, st);
   return stream_launch<T, RT, 0, false>(a, seg, groups, st);
 }

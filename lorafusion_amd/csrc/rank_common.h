@@ -62,6 +62,15 @@ __device__ __forceinline__ lf_u32x4 apply_mask8(lf_u32x4 x, lf_u32x2 m) {
   return r;
 }
 
+// The direct-to-LDS loads of a keep-mask fetch 4 bytes of bits or 16 bytes of bytes at a time: a mask that does not lie on such an address is
+// read by each lane for itself.
+inline bool mask_off_grid(const uint8_t* mask, int mask_bits) { return mask != nullptr && ((uintptr_t)mask & (mask_bits ? 3 : 15)) != 0; }
+__device__ __forceinline__ lf_u32x2 keep_bytes8(const uint8_t* p) {
+  lf_u32x2 m;
+  __builtin_memcpy(&m, p, 8);
+  return m;
+}
+
 // Bit-packed keep-masks: element k of a row = bit k & 7 of byte k >> 3 of the row (K / 8 bytes per row).
 // The eight keep bytes (0/1 each, `lo` = the first four) as eight bits, and back: one multiply gathers / spreads four
 // single bits (no two partial products meet in one bit position, so nothing carries).

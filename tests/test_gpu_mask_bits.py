@@ -139,3 +139,34 @@ def test_whole_op_with_a_packed_mask_equals_the_bool_mask():
         res.append((y.detach(), x.grad, a.grad, b.grad))
     for t1, t2 in zip(*res):
         assert torch.equal(t1, t2)
+
+
+@pytest.mark.parametrize("M,K,r,p", [(300, 4096, 16, 0.1), (70, 1152, 48, 0.3), (513, 640, 128, 0.1), (130, 2048, 96, 0.0), (2500, 1024, 72, 0.2)])
+@pytest.mark.parametrize("fmt,offset", [("bits", 1), ("bits", 2), ("bytes", 1), ("bytes", 8)])
+def test_masks_at_addresses_the_direct_loads_do_not_take(M, K, r, p, fmt, offset):
+    """A contiguous mask somewhere in a larger buffer: the rank-r passes give what the same mask gives at an aligned address (dA and, above
+    rank 64, S bit for bit)."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    a = (torch.randn(r, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    ds = (torch.randn(M, r, generator=g) * 0.1).bfloat16().cuda()
+    mask = (torch.rand(M, K, generator=g) >= 0.2).cuda()
+    mask = hip_ops.pack_mask(mask) if fmt == "bits" else mask.to(torch.uint8)
+    buf = torch.zeros(mask.numel() + 64, dtype=torch.uint8, device="cuda")
+    odd = buf[offset:offset + mask.numel()].view(mask.shape)
+    odd.copy_(mask)
+    assert odd.is_contiguous() and odd.data_ptr() % 16 == offset
+    routing, R = L.single_routing(r, 1.0, p), L.round_rank(r)
+    s, s_odd = (hip_ops._xa(x, m, [a], routing, M, K, R) for m in (mask, odd))
+    print(f"{M} x {K}, rank {r}, {fmt} + {offset}", flush=True)
+    if r > 64:
+        assert torch.equal(s, s_odd)
+    _close(s_odd, s.float().cpu(), "S")
+    if fmt == "bytes":
+        assert torch.equal(hip_ops.fused_lora_da(x, ds, r, p, mask), hip_ops.fused_lora_da(x, ds, r, p, odd))
+    else:
+        with pytest.raises(RuntimeError, match="-2"):   # 4-byte loads of the keep bits
+            hip_ops.fused_lora_da(x, ds, r, 0.1, odd)
