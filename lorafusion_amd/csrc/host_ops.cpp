@@ -402,6 +402,8 @@ Tensor linear_lora(const Tensor& x, const Tensor& w, const Tensor& a, const Tens
   if (!(p >= 0.0 && p < 1.0)) bad_value("dropout_p must be in [0, 1), got ", p, ".");
   refuse_tangents(x, w, a, b, bias);
 
+  Tensor mask;   // (as autograd sees it: an alias made below would not share its version counter)
+  if (p > 0 && !seed) mask = checked_mask(*mask_, M, K);
   Weight wt;
   const int R = round_rank((int)rank);
   const lf_routing r = single_routing((int)rank, (float)alpha, (float)p);
@@ -412,8 +414,7 @@ Tensor linear_lora(const Tensor& x, const Tensor& w, const Tensor& a, const Tens
     const at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard device(x.device());
     xs = x.contiguous(), wt.w = w.contiguous(), as = {a.contiguous()}, bs = {b.contiguous()};
-    Tensor mask;
-    if (p > 0 && !seed) mask = packed_mask(checked_mask(*mask_, M, K), K);
+    if (mask.defined()) mask = packed_mask(mask, K);
     std::vector<int64_t> ys = x.sizes().vec();
     ys.back() = N;
     f = run_forward(xs, wt, as, bs, r, R, (int)N, mask, p > 0 ? seed : std::nullopt, true, bias.defined() ? bias.contiguous() : bias, false, ys);

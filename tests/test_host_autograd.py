@@ -86,6 +86,21 @@ def test_backward_from_a_result_that_only_weight_or_bias_makes_differentiable(wh
 
 
 @pytest.mark.gpu
+def test_a_mask_that_changes_before_the_backward_is_noticed():
+    from lorafusion_amd.ops import hip_ops
+    from lorafusion_amd.ops.lora_v1 import fused_linear_lora
+
+    t = lambda *s: torch.randn(*s, device="cuda", dtype=torch.bfloat16)
+    x, w, a, b = t(2, 64, 256).requires_grad_(), t(128, 256), t(16, 256), t(128, 16)
+    bits = hip_ops.pack_mask(torch.rand(128, 256, device="cuda") >= 0.1)
+    for mask in (bits, bits.view(2, 64, 32)):
+        y = fused_linear_lora(x, w, a, b, 1.0, dropout_p=0.1, dropout_mask=mask)
+        mask.zero_()
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
+
+
+@pytest.mark.gpu
 def test_public_functions_refuse_tangents_and_empty_rows():
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
     from lorafusion_amd.ops.norm_act import rms_norm, silu_mul, silu_mul_merged
