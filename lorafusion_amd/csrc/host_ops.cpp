@@ -609,12 +609,14 @@ Tensor silu_mul(const Tensor& a, const Tensor& b) {
     bad_value("silu_mul operands differ: ", shape_name(a.sizes()), " ", dtype_name(a.scalar_type()), " vs ", shape_name(b.sizes()), " ", dtype_name(b.scalar_type()), ".");
   if (a.size(-1) % 8 != 0) bad_value("the last dimension must be a multiple of 8, got ", a.size(-1), ".");
   refuse_tangents(a, b);
-  Tensor c;
+  Tensor c, as = a, bs = b;   // what the backward keeps: the caller's tensor where the kernel reads it as it lies, else the copy
   {
     const at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard device(a.device());
     const auto [a2, lda] = rows_view(a);
     const auto [b2, ldb] = rows_view(b);
+    if (!a2.is_alias_of(a)) as = a2;
+    if (!b2.is_alias_of(b)) bs = b2;
     c = at::empty(a.sizes(), a.options());
     if (a2.size(0) > 0)
       check(lf_silu_mul_fwd(ptr(a2), ptr(b2), mptr(c), (int)a2.size(0), (int)a2.size(1), lda, ldb, a2.size(1), dtype_id(a.scalar_type()), stream_of(a)), "lf_silu_mul_fwd");
@@ -622,8 +624,8 @@ Tensor silu_mul(const Tensor& a, const Tensor& b) {
   if (wants_grad({a, b})) {
     std::shared_ptr<SiLUMulBackward> n(new SiLUMulBackward(), torch::autograd::deleteNode);
     n->set_next_edges(torch::autograd::collect_next_edges(a, b));
-    n->a = SavedVariable(a, false);
-    n->b = SavedVariable(b, false);
+    n->a = SavedVariable(as, false);
+    n->b = SavedVariable(bs, false);
     n->sizes = a.sizes().vec();
     n->c_sizes = n->sizes;
     torch::autograd::set_history(c, n);

@@ -101,6 +101,29 @@ def test_a_mask_that_changes_before_the_backward_is_noticed():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("copied", [True, False])
+def test_activation_inputs_that_change_before_the_backward(copied):
+    """Inputs the kernel cannot read as they lie are copied for it, and the backward works on the copies; others are the caller's, and noticed."""
+    from lorafusion_amd.ops.norm_act import silu_mul
+
+    t = lambda: torch.randn(64, 128, device="cuda", dtype=torch.bfloat16)
+    a, b = (t().t().contiguous().t() if copied else t() for _ in range(2))
+    dc = t()
+    grads = lambda: torch.autograd.grad(silu_mul(x, y), (x, y), dc)
+    x, y = a.requires_grad_(), b.requires_grad_()
+    expect = grads()
+    c = silu_mul(x, y)
+    with torch.no_grad():
+        x.zero_(), y.zero_()
+    if not copied:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(c, (x, y), dc)
+        return
+    for g, e in zip(torch.autograd.grad(c, (x, y), dc), expect):
+        assert torch.equal(g, e)
+
+
+@pytest.mark.gpu
 def test_public_functions_refuse_tangents_and_empty_rows():
     from lorafusion_amd.ops.lora_v1 import fused_linear_lora
     from lorafusion_amd.ops.norm_act import rms_norm, silu_mul, silu_mul_merged
