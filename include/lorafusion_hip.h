@@ -212,9 +212,9 @@ int lf_set_tile_cfg(int tile_cfg);
 
 /* The launches the library makes for an M x N output contracted over K when no configuration is pinned: rows
  * [0, *rows_head) as one launch of tile configuration *cfg_head and, when *rows_head < M, the rest
- * as a second launch of *cfg_tail (-1 when there is none).  A launch may still move to another tile: tile 9
- * (192x128) stands in for 8 where its grid fills the chip better, and a launch that leaves compute units idle over a long K is
- * cut into slices.  routing_block_size_m: 0 for a
+ * as a second launch of *cfg_tail (-1 when there is none).  A launch may still move to another tile: a call whose keep-mask
+ * or rank the persistent kernel (7, 8) does not take goes to the best of the others, and a launch that leaves compute units idle over a long
+ * K is cut into slices.  routing_block_size_m: 0 for a
  * single-adapter call, else the routing block size.  For benchmarks that time one kernel of a
  * fused call on its own; no counterpart in the reference (Triton's autotuner picks there). */
 int lf_gemm_plan(int M, int N, int K, int routing_block_size_m, int* rows_head, int* cfg_head, int* cfg_tail);

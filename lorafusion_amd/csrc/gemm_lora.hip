@@ -820,7 +820,9 @@ static const TileCand& cand_of(int cfg) {
 // The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
 // (its 128-row tile and the other 256-column tiles leave most of the chip idle there); wave96: a 96-row wave meets at most two
 // routing blocks.  The eight-wave 256x256 tile stands in for the persistent one (a long
-// contraction under a wide output prefers it: lf_plan_gemm).
+// contraction under a wide output prefers it: lf_plan_gemm).  Where the persistent kernel's 128x256 tile fills 0.7 to one round of the chip, the
+// 192x128 tile often fills it better and reads a B panel fewer times: ahead from K = 4096 (1536 x 4096 over 6144 NT: 101.7 -> 75.5 us, NN 79.6 ->
+// 72.5; over 4096: 55.5 -> 51.9, 53.4 -> 49.3), level or behind at K = 2048 (1920 x 3072: 24.5 against 25.3).
 static bool wave96_fits(int routing_block) { return routing_block <= 0 || routing_block % 128 == 0; }
 static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_out = nullptr, bool tail = false) {
   int best = 1;
@@ -835,17 +837,7 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_o
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;
-  // (0.7 to one round of the persistent kernel's 128x256 tile are planned as that tile; settle_tile has the last word)
-  const long mid = (long)((M + 127) / 128) * ((N + 255) / 256);
-  if (best == 9 && big && M >= 128 && N >= 256 && K >= 256 && mid <= 256 && 10 * mid > 7 * 256) best = 8;
   return best;
-}
-// The tile a single launch of the plan runs on.  Where the persistent kernel's 128x256 tile fills 0.7 to one round of the chip,
-// the 192x128 tile often fills it better and reads a B panel fewer times: ahead from K = 4096 (1536 x 4096 over 6144 NT: 101.7 -> 75.5 us,
-// NN 79.6 -> 72.5; over 4096: 55.5 -> 51.9, 53.4 -> 49.3), level or behind at K = 2048 (1920 x 3072: 24.5 against 25.3).
-static int settle_tile(int cfg, int M, int N, int K, int routing_block) {
-  if (cfg != 8 || !wave96_fits(routing_block)) return cfg;
-  return launch_cost(cand_of(9), M, N, K) < launch_cost(cand_of(8), M, N, K) ? 9 : 8;
 }
 // Rows [0, m_main) as 256x256 tiles, the rest as a second launch with the tile that spreads them best, when that beats
 // one launch (a nearly empty last round of big tiles costs a full tile time).  m_main is the multiple of 256 rows
@@ -946,7 +938,7 @@ size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
   size_t need = 0;
   auto part = [&](int m, int cfg) {
-    for (int c : {settle_tile(cfg, m, N, K, routing_block), choose_cfg(m, N, K, false, wave96_fits(routing_block))}) {
+    for (int c : {cfg, choose_cfg(m, N, K, false, wave96_fits(routing_block))}) {
       const KSplit ks = ksplit_for(m, N, K, c, routing_block, nn);
       if (ks.n > 1) need = std::max(need, (size_t)ks.n * m * N * sizeof(float));
     }
@@ -979,7 +971,6 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
     if ((cfg == 7 || cfg == 8) && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32)))
       cfg = planned ? choose_cfg(q.M, q.N, q.K, false, wave96_fits(seg.table != nullptr ? seg.block_size_m : 0)) : (cfg == 7 ? 1 : 2);
     if (cfg == 7 && planned && q.K < 128) cfg = 1;
-    if (planned) cfg = settle_tile(cfg, q.M, q.N, q.K, seg.table != nullptr ? seg.block_size_m : 0);
     if (dtype != LF_BF16 && dtype != LF_F16) return (int)LF_EINVAL;
     LfGemmParams r = q;
     r.ksplit = 1, r.ks_steps = 0;

@@ -153,9 +153,9 @@ def test_launch_plan_takes_the_contraction_length():
         assert plan(16512, 4096, K) == (16512, 7, -1)
     assert plan(2048, 4096, 4096)[0] == 2048        # nothing left over: one launch
     assert L.lib().lf_gemm_plan(16, 16, 0, 0, None, None, None) == L.LF_EINVAL
-    # The persistent kernel's 128x256 tile (8) takes single launches between half a round and one round of its tiles
-    # on 256 compute units; fewer rows go to small tiles, more to its 256x256 tile (7), left-over rows never to 8.
-    assert plan(2048, 4096, 4096) == (2048, 8, -1) and plan(1536, 4096, 6144) == (1536, 8, -1)
+    # The persistent kernel's 128x256 tile (8) takes single launches of about one round of its tiles on 256 compute units, the
+    # 192x128 tile (9) those that leave it part of a round idle; fewer rows go to small tiles, more to the 256x256 tile (7), left-over rows never to 8.
+    assert plan(2048, 4096, 4096) == (2048, 8, -1) and plan(1536, 4096, 6144) == (1536, 9, -1)
     assert plan(1024, 4096, 4096)[1] not in (7, 8)
     assert plan(4096, 4096, 4096) == (4096, 7, -1) and plan(2048, 8192, 8192) == (2048, 7, -1)
     assert plan(2048, 4096, 128)[1] != 8            # its K loop needs four steps of 64
