@@ -774,11 +774,15 @@ def main():
         small = argparse.Namespace(steps=max(5, args.steps // 2), warmup=max(2, args.warmup // 2))
         res["workloads"] = {name: raw_workload(name, args if name == "c2" else small, dev)
                             for name in ("c1", "c2", "c3", "c4_qkv_merged", "c4_separate", "c5")}
-        res["workloads"]["fig5"] = fig5_block(small, dev)
-        res["gemm_ref"] = {"random_operands": gemm_ref_block(dev, reps=10), "all_zero_operands": gemm_ref_block(dev, reps=10, zero=True)}
+        # (the grid of single linears and the plain-GEMM comparison: --only fig5, gemm_ref, gemm_ref_zero)
     if not args.no_cpu_baseline:
         res["cpu_baseline"] = cpu_baseline_c4()
-    print(json.dumps(res))
+    print(json.dumps(without_launches(res)))
+
+
+def without_launches(v):
+    """The line without the launches behind each roofline (``--only <workload>`` prints them): it is read from logs that cut long lines."""
+    return {k: without_launches(x) for k, x in v.items() if k != "launches"} if isinstance(v, dict) else v
 
 
 if __name__ == "__main__":
