@@ -833,7 +833,9 @@ gemm_big_kernel(const LfGemmParams p, const LfSegTable seg) {
 //                                     comes from HBM, and 2 x 16 tiles read it once per round (16384 x 4096 x 14336 NT 1402, 4: 1457)
 //   long K, many columns, NN      4   0.98; NT 8 (4 level, 6 1.04)
 //   128-row tile                  8   0.95 from K = 10240 (2048 x 4096 x 28672 NT 460 -> 430), level below
-// Short K over many columns stays at 8 in the NT product once A takes half of that cache (16384 x 28672 x 4096: 2524, 6: 2577).
+// Short K over many columns stays at 8 in the NT product once A takes half of that cache, where the time of 6 relative to 8 crosses one: A of 32 - 64 MB
+// 0.94 - 1.01 (8192 x 14336 x 4096 640 / 653 us), 96 MB 0.93 - 1.01 (12288 x 28672 x 4096 1918 / 1990), 128 MB 1.00 - 1.03 (16384 x 14336 x 4096 1272 /
+// 1273, x 57344 5217 / 5075), 144 MB 0.97 - 1.02, 192 MB 1.00 - 1.05 (16384 x 28672 x 6144 4332 / 4163).
 int group_rows(int M, int K, int grid_n, int tile_rows, bool nn) {
   const int64_t a_bytes = (int64_t)M * K * 2, cache = (int64_t)256 << 20;
   if (tile_rows == 128) return 8;

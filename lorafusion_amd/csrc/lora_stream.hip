@@ -32,7 +32,7 @@ struct StreamArgs {
   const void* p0;        // rows [0, n0) of P
   const void* p1;        // rows [n0, n0 + n1) (forward: the adapter's rows), or nullptr
   int n0, n1, K, n_slices;
-  int folded;            // no memory for the slices' sums: one workgroup walks all slices and adds their sums in the order the second stage would
+  int folded;            // (rank tilings of 128 columns) no memory for the slices' sums: one workgroup walks all slices and adds their sums in the order the second stage would
   const uint8_t* mask;   // keep-mask read: bits [rows, K / 8] (MODE 2) or bytes [rows, K] (MODE 1)
   uint8_t* mask_out;     //           or drawn and written (MODE 3), as bits or as bytes
   int mask_bytes;
@@ -53,6 +53,7 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
   constexpr int NS = st_ns(RT, MODE), STAGE = st_bytes(RT, MODE), QB = st_q_bytes(RT);
   constexpr int NQ = RT == 1 ? 1 : RT / 2;              // loads of Q per wave and step
   constexpr int G = 2 + NQ + (MODE == 1 || MODE == 2 ? 1 : 0);       // loads per wave and step
+  constexpr bool FOLDS = RT == 8 && !FWD;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int tid = threadIdx.x, lane = tid & 63, wave = to_sgpr(tid >> 6);
@@ -138,7 +139,7 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
     wait_groups<G>(NS - 2);
     ring_barrier();   // this step's stage has landed for every wave; everyone is done with the stage refilled next
     issue();
-    if (!FWD && a.folded && s == fold_at) {
+    if (FOLDS && a.folded && s == fold_at) {
 #pragma unroll
       for (int c = 0; c < RT; c++) sum[c] += acc[c], acc[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
       fold_at = 2 * slice_begin(fold_next++);
@@ -217,8 +218,10 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
   } else {
     // lane: column li of each 16, rows 4 qq + e of the wave
     const float mult = use_mask ? 1.f / (1.f - bi.p) : 1.f;
+    if constexpr (FOLDS) {
 #pragma unroll
-    for (int c = 0; c < RT; c++) acc[c] = sum[c] + acc[c];
+      for (int c = 0; c < RT; c++) acc[c] = sum[c] + acc[c];
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int64_t row = row0 + wave * 16 + qq * 4 + e;
@@ -387,7 +390,7 @@ size_t lf_xa_stream_workspace(int M, int K, int R, bool masked, const LfSegTable
   return n > 1 ? (size_t)n * xa_rows_of(M, seg) * R * sizeof(float) : 0;
 }
 
-// ws == nullptr: no room for the slices' sums (the result is the same, bit for bit)
+// ws == nullptr: no room for the slices' sums (ranks above 64 or a single slice; the result is the same, bit for bit)
 int lf_launch_xa_stream(const void* X, const uint8_t* mask, uint8_t* mask_out, int mask_bits, uint64_t seed, void* S, float* ws, int M, int K, int R,
                         const LfSegTable& seg, int dtype, hipStream_t st) {
   StreamArgs a{};

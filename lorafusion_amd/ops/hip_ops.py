@@ -509,7 +509,8 @@ def lora_forward_seeded(x, w, a_list, b_list, routing_c, R, seed: int, bias, *, 
 
 
 def lora_backward(dy, x, w, a_list, b_list, s, routing_c, R, mask, rank_list, requires_dx: bool = True):
-    """One C call: dS/dB, dA and (optionally) dX.  Returns (dx | None, da_list, db_list)."""
+    """One C call: dS/dB, dA and (optionally) dX.  Returns (dx | None, da_list, db_list).  ``rank_list`` is not read: the adapters say
+    their ranks."""
     return L.host().backward(dy, x, w, 0, a_list, b_list, s, ctypes.addressof(routing_c), R, mask, None, requires_dx)
 
 
@@ -526,7 +527,7 @@ def nf4_lora_forward(x, wref, a_list, b_list, routing_c, R, mask, bias, *, keep_
 def nf4_lora_backward(dy, x, wref, a_list, b_list, s, routing_c, R, mask, rank_list, requires_dx: bool = True,
                       dense: torch.Tensor | None = None):
     """``lora_backward`` with the base weight given as NF4.  ``dense``: the dequantised weight a forward with
-    ``keep_dense`` left behind (nothing is dequantised then).  Returns (dx | None, da_list, db_list)."""
+    ``keep_dense`` left behind (nothing is dequantised then).  Returns (dx | None, da_list, db_list); ``rank_list`` is not read."""
     N, K = dy.shape[1], x.shape[1]
     if dense is not None and (tuple(dense.shape) != (N, K) or dense.dtype != dy.dtype or not dense.is_contiguous()):
         raise ValueError(f"dense must be a contiguous [{N}, {K}] tensor of dtype {dy.dtype}.")

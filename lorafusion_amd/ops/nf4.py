@@ -117,14 +117,6 @@ class NF4WeightRef:
         self.shape, self.dtype = shape, out_dtype
         self.c = L.NF4Weight(L.ptr(A), L.ptr(absmax), L.ptr(code), L.ptr(absmax2), L.ptr(offset), blocksize, bs2, None, 0, 0)
 
-    def with_dense(self, dense, *, valid: bool):
-        """The struct with ``dense`` (a [N, K] tensor for the dequantised weight, or None) filled in."""
-        if dense is None:
-            return self.c
-        c = self.c
-        return L.NF4Weight(c.packed, c.absmax, c.code2, c.absmax2, c.offset, c.blocksize, c.blocksize2,
-                           dense.data_ptr(), 1 if valid else 0, 0)
-
 
 def nf4_struct_of(quant_state):
     """What a backward node holds of an NF4 weight: codes -> (address of their ``lf_nf4_weight``, its owner), from codes and

@@ -99,17 +99,21 @@ def test_192_row_tile_over_routing_blocks(seq, ranks, p_list, N, dtype):
     _close(hip_ops.fused_multi_lora_dyw_dsa(xd, wt, sd, ad, routing, dropout_mask=md)[clean.cuda()], dx[clean], "dx beside infinities")
 
 
-@pytest.mark.parametrize("M,K,N,dtype", [
-    (85, 4096, 2304, torch.bfloat16), (130, 6144, 2944, torch.float16), (256, 8192, 2048, torch.bfloat16), (283, 6144, 1024, torch.bfloat16),
-    (511, 14336, 1024, torch.float16), (700, 8192, 1024, torch.bfloat16), (2290, 9088, 1152, torch.bfloat16)])
-def test_tile_and_slices_together(M, K, N, dtype):
-    """Forward over K and dX over K (the roles of the dimensions exchanged), against the same products through the entry points
-    without a workspace, which do not split: the sums differ in order only, so by no more than one 16-bit step of the largest value."""
+@pytest.mark.parametrize("M,K,N,slices,dtype", [
+    (85, 4096, 2304, 6, torch.bfloat16), (130, 6144, 2944, 8, torch.float16), (256, 8192, 2048, 8, torch.bfloat16), (283, 6144, 1024, 6, torch.bfloat16),
+    (511, 14336, 1024, 8, torch.float16), (700, 8192, 1024, 5, torch.bfloat16), (2290, 9088, 1152, 2, torch.bfloat16)])
+def test_tile_and_slices_together(M, K, N, slices, dtype):
+    """Forward over K and dX over K (the roles of the dimensions exchanged), cut into the slices that the size query makes room for: against
+    fp32 sums, and against the same products through the entry points without a workspace, which do not split: the sums
+    differ in order only, so by no more than one 16-bit step of the largest value."""
     from lorafusion_amd import _lib as L
     from lorafusion_amd.ops import hip_ops
 
     r, p = 16, 0.1
     R, routing = L.round_rank(r), L.single_routing(r, 2.0, p)
+    size = lambda op, n, k: L.lib().lf_workspace_bytes(op, M, n, k, R, routing)
+    tiles = slices * M * N * 4   # fp32 partial tiles of Y, behind the rank-r pass's slices, and of dX
+    assert 0 <= size(L.LF_OP_FWD, N, K) - size(L.LF_OP_XA, 0, K) - tiles < 512 and 0 <= size(L.LF_OP_BWD, K, N) - tiles < 256
     g = torch.Generator().manual_seed(M + K)
     x = torch.randn(M, K, generator=g).to(dtype).cuda()
     w = (torch.randn(N, K, generator=g) * 0.02).to(dtype).cuda()
@@ -117,6 +121,7 @@ def test_tile_and_slices_together(M, K, N, dtype):
     bits = hip_ops.pack_mask((torch.rand(M, K, generator=g) >= p).cuda())
     y, s = hip_ops.lora_forward(x, w, [a], [b], routing, R, bits, None)
     y1 = hip_ops.fused_lora_xw_sb(x, w, s[:, :r].contiguous(), b, 2.0)
+    _close(y, (x.float() @ w.float().T + 2.0 * s[:, :r].float() @ b.float().T).cpu(), "y")
     step = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
     assert float((y.float() - y1.float()).abs().max()) <= float(y1.float().abs().max()) * step
     # dX [M, N] over K: X takes the place of dY
@@ -127,4 +132,6 @@ def test_tile_and_slices_together(M, K, N, dtype):
     dx = hip_ops.lora_backward(x, xs, wt, [at], [bt], st, routing, R, bits, [r])[0]
     ds = hip_ops.fused_lora_dys_dyb(x, bt, st, 2.0)[1]
     dx1 = hip_ops.fused_lora_dyw_dsa(x, wt, ds, at, p, bits)
+    term = ds[:, :r].float() @ at.float() / (1 - p)
+    _close(dx, (x.float() @ wt.float() + torch.where(hip_ops.unpack_mask(bits), term, torch.zeros_like(term))).cpu(), "dx")
     assert float((dx.float() - dx1.float()).abs().max()) <= float(dx1.float().abs().max()) * step

@@ -23,7 +23,9 @@ def _close(got, exp, name):
 @pytest.mark.parametrize("M,K,r,dtype", [
     (1, 128, 40, torch.bfloat16), (63, 256, 48, torch.float16), (64, 384, 64, torch.bfloat16), (65, 640, 72, torch.bfloat16),
     (127, 1152, 128, torch.float16), (300, 4096, 64, torch.bfloat16), (1025, 512, 128, torch.bfloat16),
-    (1, 128, 8, torch.bfloat16), (65, 1152, 16, torch.float16), (1000, 256, 24, torch.bfloat16)])   # (ranks up to 32: the drawn mask only)
+    (1, 128, 8, torch.bfloat16), (65, 1152, 16, torch.float16), (1000, 256, 24, torch.bfloat16),
+    (1, 4096, 8, torch.bfloat16), (65, 4224, 16, torch.float16), (1000, 4096, 24, torch.bfloat16),   # (ranks up to 32: sliced from K = 4096, with a mask)
+    (3000, 1536, 56, torch.float16), (7040, 1152, 64, torch.bfloat16)])                              # rank 64: sliced, and too short a K for its rows
 def test_rank_pass(M, K, r, dtype, mode):
     from lorafusion_amd import _lib as L
     from lorafusion_amd.ops import hip_ops
@@ -40,6 +42,8 @@ def test_rank_pass(M, K, r, dtype, mode):
         mask = torch.from_numpy(expect).bool()
     else:
         y, s = hip_ops.lora_forward(x, w, [a], [b], routing, R, None if mask is None else hip_ops.pack_mask(mask.cuda()), None)
+        if mask is not None:
+            assert torch.equal(hip_ops._xa(x, mask.cuda(), [a], routing, M, K, R), s), "one byte per element"
     ye, se = lora_ref.linear_lora_fwd_fp32(d["x"], d["w"], d["a"], d["b"], 2.0, mask, p)
     _close(s[:, :r], se, "S")
     _close(y, ye, "Y")
@@ -47,7 +51,7 @@ def test_rank_pass(M, K, r, dtype, mode):
 
 
 @pytest.mark.parametrize("mode", ["given", "drawn"])
-@pytest.mark.parametrize("seq,ranks,K", [([1, 129, 64], [64, 8, 40], 512), ([200, 130], [128, 16], 1280)])
+@pytest.mark.parametrize("seq,ranks,K", [([1, 129, 64], [64, 8, 40], 512), ([200, 130], [128, 16], 1280), ([70, 1, 300], [16, 8, 24], 4096)])
 def test_rank_pass_packed(seq, ranks, K, mode):
     from lorafusion_amd.ops import hip_ops
     from lorafusion_amd.ops.multi_lora import prepare_multi_lora_batch_info
