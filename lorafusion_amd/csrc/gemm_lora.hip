@@ -791,6 +791,7 @@ struct TileCand {
   double reduce;   // us: the second kernel of a split contraction
   double partial;  // us per MB of partial tiles, written and read
   double weight;   // us per MB of weight
+  bool mid = false;  // gemm_mid.hip
 };
 static const TileCand kCands[] = {
     {7, 256, 256, 6.3, 59.0, 30.1, 64.7, 91.2, 35.8, 0.0, 0.0, 0.121},     // persistent, 4 waves of 128x128 (gemm_big.hip)
@@ -801,6 +802,12 @@ static const TileCand kCands[] = {
     {5, 64, 64, 4.6, 13.2, 3.1, 7.7, 15.6, 4.3, 2.4, 0.265, 0.061},        // 4 waves, 32x32 per wave
     {6, 128, 64, 5.1, 17.4, 4.1, 21.5, 25.1, 3.7, 1.6, 0.479, 0.085},      // 4 waves, 64x32 per wave
     {8, 128, 256, 6.0, 35.4, 11.3, 36.5, 54.0, 23.4, 0.0, 0.0, 0.108},     // persistent, 4 waves of 64x128 (gemm_big.hip)
+    // gemm_mid.hip: 4 waves of 96x64, 80x64, 64x64, 64x32.  Fitted to 10800 launches of 420 shapes (40 - 4100 rows, 512 - 14336 columns and
+    // K) the same way: 6 - 8 % off.
+    {9, 192, 128, 7.3, 28.8, 5.2, 40.4, 50.8, 5.8, 2.0, 0.384, 0.040, true},
+    {10, 160, 128, 6.5, 25.4, 3.0, 36.5, 44.3, 1.6, 2.0, 0.386, 0.057, true},
+    {11, 128, 128, 5.7, 22.0, 2.6, 31.3, 36.2, 3.4, 2.1, 0.364, 0.075, true},
+    {12, 128, 64, 4.4, 14.5, 2.8, 20.4, 24.3, 1.9, 1.8, 0.402, 0.082, true},
 };
 static long tiles_of(int M, int N, const TileCand& c) { return (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); }
 static double launch_cost(const TileCand& c, int M, int N, int K, int slices = 1, int steps = 0) {
@@ -813,10 +820,16 @@ static double launch_cost(const TileCand& c, int M, int N, int K, int slices = 1
   if (slices > 1) us += c.reduce + c.partial * (4e-6 * slices * M * N);
   return us;
 }
-static const TileCand& cand_of(int cfg) {
-  for (const TileCand& c : kCands) if (c.cfg == cfg) return c;
+static const TileCand& cand_of(int cfg, bool mid) {
+  for (const TileCand& c : kCands) if (c.cfg == cfg && (!c.mid || mid) && (c.cfg != 9 || c.mid == mid)) return c;
   return kCands[cfg == 2 ? 2 : 1];   // (the four-wave forms of these tiles, 0 and 2, are only run when pinned or for odd routing blocks)
 }
+// gemm_mid.hip takes whole tiles of columns, at least four K steps of 64 and routing blocks that a wave meets two of at most.
+static bool mid_shape(const TileCand& c, int N, int K) { return N % c.bn == 0 && K >= (c.cfg == 10 ? 1024 : 256); }   // (160x128: level with 192x128 at K = 512)
+// What a tile of gemm_mid.hip has to be ahead by in the model to be taken: in one round, in several, sliced.  The two models were
+// fitted apart and are 6 - 8 % off each.  Without: 64 of 840 products more than 3 % behind the plan before (worst 1.46 times), with: 15 (worst 1.1);
+// all of them together gain 8.6 % either way.
+static double mid_margin(long tiles, int slices) { return slices > 1 ? 1.06 : (tiles <= 256 ? 1.05 : 1.12); }
 // The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
 // (its 128-row tile and the other 256-column tiles leave most of the chip idle there); wave96: a 96-row wave meets at most two
 // routing blocks.  The eight-wave 256x256 tile stands in for the persistent one (a long
@@ -824,7 +837,7 @@ static const TileCand& cand_of(int cfg) {
 // 192x128 tile often fills it better and reads a B panel fewer times: ahead from K = 4096 (1536 x 4096 over 6144 NT: 101.7 -> 75.5 us, NN 79.6 ->
 // 72.5; over 4096: 55.5 -> 51.9, 53.4 -> 49.3), level or behind at K = 2048 (1920 x 3072: 24.5 against 25.3).
 static bool wave96_fits(int routing_block) { return routing_block <= 0 || routing_block % 128 == 0; }
-static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_out = nullptr, bool tail = false) {
+static int choose_cfg(int M, int N, int K, bool big, bool wave96, bool mid, double* cost_out = nullptr, bool tail = false) {
   int best = 1;
   double best_cost = 1e30;
   for (const TileCand& c : kCands) {
@@ -832,8 +845,9 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_o
     if (c.cfg == 8 && (!big || tail || M < 128 || N < 256 || K < 256)) continue;
     if (c.cfg == 1 && (tail || (big && M >= 256 && N >= 256))) continue;
     if (c.cfg == 3 && tail) continue;
-    if (c.cfg == 9 && (!wave96 || tail)) continue;
-    const double cost = launch_cost(c, M, N, K);
+    if (c.cfg == 9 && !c.mid && (!wave96 || tail)) continue;
+    if (c.mid && (!mid || !mid_shape(c, N, K) || (tail && c.cfg < 11))) continue;
+    const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1) : 1.0);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;
@@ -844,20 +858,20 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, double* cost_o
 // with the lowest modelled cost of both launches: usually the one whose tiles fill whole rounds of the chip
 // (32 tile rows of 40 tiles are exactly five rounds; 30 rows of 40 are five rounds too, and leave a longer tail).
 // Returns m_main (0: single launch).
-static int choose_split(int M, int N, int K, bool allow_big, bool wave96, int* cfg_head, int* cfg_tail) {
+static int choose_split(int M, int N, int K, bool allow_big, bool wave96, bool mid, int* cfg_head, int* cfg_tail) {
   constexpr double kLaunch = 4.0;  // a second launch
   const int grid_n = (N + 255) / 256;
   if (grid_n > 256) return 0;
   const bool big = allow_big && N >= 256;
   const TileCand& head = kCands[big ? 0 : 1];
   double best;
-  choose_cfg(M, N, K, allow_big, wave96, &best);
+  choose_cfg(M, N, K, allow_big, wave96, mid, &best);
   int best_m = 0;
   for (int r = 1; r * 256 < M; r++) {
     const double head_cost = launch_cost(head, r * 256, N, K) + kLaunch;
     if (head_cost >= best) break;
     double tail;
-    const int ct = choose_cfg(M - r * 256, N, K, allow_big, wave96, &tail, true);
+    const int ct = choose_cfg(M - r * 256, N, K, allow_big, wave96, mid, &tail, true);
     if (head_cost + tail < best) { best = head_cost + tail; best_m = r * 256; *cfg_tail = ct; }
   }
   *cfg_head = big ? 7 : 1;
@@ -873,15 +887,16 @@ static int choose_split(int M, int N, int K, bool allow_big, bool wave96, int* c
 // given the workspace lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
 constexpr size_t kKsplitMaxBytes = (size_t)64 << 20, kKsplitMaxBytesNN = LF_STATIC_SCRATCH_BYTES;
 struct KSplit { int cfg, n, steps; };
-static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn) {
+static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
   const int nk = K / BK;
   KSplit best = {cfg, 1, nk};
-  const TileCand& planned = cand_of(cfg);
+  const TileCand& planned = cand_of(cfg, mid);
   if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
-  double best_cost = 0.96 * launch_cost(planned, M, N, K);
+  double best_cost = launch_cost(planned, M, N, K) * (planned.mid ? mid_margin(tiles_of(M, N, planned), 1) : 1.0);
   const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
   for (const TileCand& c : kCands) {
     if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)
+    if (c.mid && (!mid || !mid_shape(c, N, K))) continue;
     if ((c.cfg == 9 && !wave96_fits(routing_block)) || (c.cfg == 1 && routing_block > 0 && routing_block % 128 != 0)) continue;
     const long tiles = tiles_of(M, N, c), slots = c.cfg == 4 || c.cfg == 5 ? 512 : 256;
     for (int n : {2, 3, 4, 5, 6, 8, 12, 16}) {
@@ -889,7 +904,8 @@ static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool n
       int steps = (nk + n - 1) / n;
       steps += steps & 1;                               // an even number of steps per slice (K / BK is even)
       const int used = (nk + steps - 1) / steps;        // no empty slice
-      const double cost = launch_cost(c, M, N, K, used, steps);
+      if (c.mid && nk - (used - 1) * steps < 8) continue; // (four K steps of 64 in the last slice too)
+      const double cost = launch_cost(c, M, N, K, used, steps) * (c.mid ? mid_margin(tiles, n) : 1.0 / 0.96);
       if (used > 1 && cost < best_cost) { best_cost = cost; best = {c.cfg, used, steps}; }
     }
   }
@@ -898,7 +914,7 @@ static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool n
 
 static std::atomic<int> pinned_cfg{-1};
 int lf_pin_tile_cfg(int cfg) {
-  if (cfg < -1 || cfg > 8) return LF_EINVAL;
+  if (cfg < -1 || cfg == 9 || cfg > 12) return LF_EINVAL;
   pinned_cfg.store(cfg, std::memory_order_relaxed);
   return LF_OK;
 }
@@ -909,7 +925,7 @@ bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; 
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
   const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), wave96 = wave96_fits(routing_block);
   int ch = 1, ct = 1;
-  const int m_main = choose_split(M, N, K, allow_big, wave96, &ch, &ct);
+  const int m_main = choose_split(M, N, K, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
   // A long contraction under a wide output runs faster on the eight-wave 256x256 tile than on the persistent kernel
   // (8192 x 8192 over 28672: 3.08 against 3.24 ms, over 57344: 5.74 against 5.85; at 4096 columns the two are level, and
   // at shorter contractions the persistent kernel is 3-8 % ahead): its long K loops let the tiles of an XCD drift apart
@@ -921,7 +937,7 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
   };
   if (m_main == 0) {
     *rows_head = M;
-    *cfg_head = demote(choose_cfg(M, N, K, allow_big, wave96));
+    *cfg_head = demote(choose_cfg(M, N, K, allow_big, wave96, /*mid=*/wave96));
     *cfg_tail = -1;
   } else {
     *rows_head = m_main;
@@ -931,16 +947,20 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
 }
 
 // Bytes of fp32 partial tiles the split contraction of an M x N product over K may write: the largest need over the
-// launches of the plan and over the tile a launch moves to where the persistent kernel does not apply.
+// launches of the plan and over the tiles a launch moves to where the persistent kernel or gemm_mid.hip does not apply.
 size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   if (M <= 0 || N <= 0 || K < BK) return 0;
   int rows = 0, ch = 1, ct = -1;
   lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
   size_t need = 0;
+  const bool wave96 = wave96_fits(routing_block), allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0);
   auto part = [&](int m, int cfg) {
-    for (int c : {cfg, choose_cfg(m, N, K, false, wave96_fits(routing_block))}) {
-      const KSplit ks = ksplit_for(m, N, K, c, routing_block, nn);
-      if (ks.n > 1) need = std::max(need, (size_t)ks.n * m * N * sizeof(float));
+    for (bool mid : {true, false}) {
+      if (mid && !wave96) continue;
+      for (int c : {mid || cfg < 9 ? cfg : choose_cfg(m, N, K, allow_big, wave96, false), choose_cfg(m, N, K, false, wave96, mid)}) {
+        const KSplit ks = ksplit_for(m, N, K, c, routing_block, nn, mid);
+        if (ks.n > 1) need = std::max(need, (size_t)ks.n * m * N * sizeof(float));
+      }
     }
   };
   part(rows, ch);
@@ -963,20 +983,32 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
   if (256 * p.lda * 2 >= 0x7fffffffLL || (int64_t)(nn ? p.K : 256) * p.ldb * 2 >= 0x7fffffffLL) return LF_ESHAPE;
   if (seg.table != nullptr && (seg.block_size_m % 64 != 0)) return LF_ESHAPE;
   const bool planned = force_cfg < 0;
+  const int rblock = seg.table != nullptr ? seg.block_size_m : 0;
+  // gemm_mid.hip reads keep-masks as bits and fetches the skinny operand with 16-byte direct loads (4-byte aligned addresses)
+  bool mid = wave96_fits(rblock) && (p.mask == nullptr || (p.mask_bits && p.N % 32 == 0));
+  if (p.L != nullptr)
+    for (int i = 0; i < std::max(1, seg.n_seg); i++) mid = mid && ((uintptr_t)seg.ptr[i] & 3) == 0;
   auto launch = [&](const LfGemmParams& q, int cfg) {
     if (seg.table != nullptr && seg.block_size_m % 128 != 0 && (cfg == 0 || cfg == 1 || cfg == 7)) cfg = 2;
+    if (planned && cfg >= 9 && !mid) cfg = choose_cfg(q.M, q.N, q.K, rblock == 0 || q.M % 128 == 0, true, false);
     // what the persistent kernel does not take (a keep-mask with one byte per element, a dX term of more than 32 rank columns)
     // goes to the tile the cost model likes best without it (pinned: the eight-wave 256x256 or the four-wave 128x256
     // tile), a contraction of one K step on its 256x256 tile to the eight-wave one
     if ((cfg == 7 || cfg == 8) && ((q.mask != nullptr && (!q.mask_bits || q.N % 128 != 0)) || (nn && q.L != nullptr && q.R > 32)))
-      cfg = planned ? choose_cfg(q.M, q.N, q.K, false, wave96_fits(seg.table != nullptr ? seg.block_size_m : 0)) : (cfg == 7 ? 1 : 2);
+      cfg = planned ? choose_cfg(q.M, q.N, q.K, false, wave96_fits(rblock), mid) : (cfg == 7 ? 1 : 2);
     if (cfg == 7 && planned && q.K < 128) cfg = 1;
     if (dtype != LF_BF16 && dtype != LF_F16) return (int)LF_EINVAL;
     LfGemmParams r = q;
     r.ksplit = 1, r.ks_steps = 0;
     if (planned && r.ks_ws != nullptr && ((uintptr_t)r.ks_ws & 15) == 0) {   // (a pinned tile configuration stays as pinned)
-      const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, seg.table != nullptr ? seg.block_size_m : 0, nn);
+      const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, rblock, nn, mid);
       if (ks.n > 1 && (size_t)ks.n * r.M * r.N * sizeof(float) <= r.ks_ws_bytes) { cfg = ks.cfg; r.ksplit = ks.n; r.ks_steps = ks.steps; }
+    }
+    if (cfg >= 10 || (cfg == 9 && mid && mid_shape(cand_of(9, true), q.N, q.K) && (r.ksplit == 1 || q.K / BK - (r.ksplit - 1) * r.ks_steps >= 8))) {
+      if (!mid) return (int)LF_ESHAPE;
+      const int rc = lf_launch_gemm_mid(r, seg, nn, dtype, cfg, st);
+      if (rc != LF_OK || r.ksplit <= 1) return rc;
+      return dtype == LF_BF16 ? launch_ksplit_reduce<__bf16>(r, st) : launch_ksplit_reduce<_Float16>(r, st);
     }
     if (cfg == 7) return lf_launch_gemm_big(q, seg, nn, dtype, 256, st);
     if (cfg == 8) return lf_launch_gemm_big(q, seg, nn, dtype, 128, st);
