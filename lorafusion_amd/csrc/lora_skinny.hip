@@ -479,13 +479,13 @@ __device__ __forceinline__ lf_u32x4 side_tr8(const char* blk, int row, int c, in
 }
 
 // ---- da.  grid (n_slices, max_chunks, n_seg).  Workgroup (ks, ch, s): the k-tiles of slice ks (at most TPW, at least
-// two: slices are balanced) and the `group` row blocks ch*group.. of segment s; pairs (block, tile) in block-major
-// order, the dS block of a row block is fetched once, with the block's first tile, into one of two buffers (a slice
-// of nt tiles keeps at most min(NS, nt + 1) stages of the ring busy, so a third block is never on order).
+// two -- one in the direct form, which has no partials -- and slices are balanced) and the `group` row blocks ch*group.. of segment s; pairs (block, tile) in block-major
+// order, the dS block of a row block is fetched once, with the block's first tile, into one of NSB buffers (a slice
+// of nt tiles keeps at most min(NS, (NSB - 1) nt + 1) stages of the ring busy, so one block more is never on order).
 //   D_j[r][k] += sum_m dS[m][r] * keep*X[m][k]   per tile j of the slice, in registers over all blocks of the chunk.
 // With a keep-mask the tile is masked in place one iteration before it is consumed.
-template <typename T, int RT, int TPW, int NS, int MASK>
-__global__ void __launch_bounds__(256, RT >= 8 ? 1 : 2)
+template <typename T, int RT, int TPW, int NS, int MASK, int NSB, bool DIRECT>
+__global__ void __launch_bounds__(256, RT >= 8 || DIRECT ? 1 : 2)
 lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, const T* __restrict__ dS, float* __restrict__ part,
                     int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg) {
   // MASK: 0 no keep-mask; 1 one byte per element (8 KB per tile, two loads per thread); 2 one bit per element (1 KB per
@@ -504,14 +504,20 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   int b0, b1, bb0, bb1;
   segment_blocks(seg, s, M, b0, b1);
   chunk_blocks(b0, b1, group, ch, bb0, bb1);
-  if (bb0 >= bb1) return;  // this segment has fewer chunks (uniform for the whole workgroup)
+  if (bb0 >= bb1) {  // this segment has fewer chunks (uniform for the whole workgroup)
+    if constexpr (DIRECT) {   // no rows at all: a sum of nothing
+      const int T64 = K / 64, k0 = (ks * (T64 / n_slices) + min(ks, T64 % n_slices)) * 64, nk = (T64 / n_slices + (ks < T64 % n_slices ? 1 : 0)) * 64;
+      for (int i = tid; i < seg.rank[s] * nk; i += 256) ((uint16_t*)seg.out[s])[(int64_t)(i / nk) * K + k0 + i % nk] = 0;
+    }
+    return;
+  }
   const float p = seg.table ? (seg.block_p ? seg.block_p[b0] : 0.f) : seg.p;
   const bool use_mask = MASK && mask != nullptr && p > 0.f;
   const int64_t Mrows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   const int T64 = K / 64;
   const int kt0 = ks * (T64 / n_slices) + min(ks, T64 % n_slices);
   const int nt = T64 / n_slices + (ks < T64 % n_slices ? 1 : 0);
-  const int ns = min(NS, nt + 1);   // stages in use
+  const int ns = min(NS, (NSB - 1) * nt + 1);   // stages in use
 
   uint32_t xv[4], mv[2], dv[RT];
   tile_voffs(xv, K, tid);
@@ -543,7 +549,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
       dma4(window_rsrc(mask != nullptr ? (const char*)mask + boff : (const char*)X, mask != nullptr ? (xleft >> 4) : 0), mv[0],
            lds0 + ist * STAGE + TILE_BYTES + wave * 256);
     }
-    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), dv, lds0 + NS * STAGE + ((ib - bb0) & 1) * SIDE, wave);
+    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), dv, lds0 + NS * STAGE + ((ib - bb0) % NSB) * SIDE, wave);
     ist = ist + 1 == ns ? 0 : ist + 1;
     if (ib < bb1) {
       if (++ij < nt) {
@@ -581,7 +587,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
     if (use_mask) apply_mask(ring, bb0, 0);
   }
   for (int b = bb0; b < bb1; b++) {
-    const char* dcur = side + ((b - bb0) & 1) * SIDE;
+    const char* dcur = side + ((b - bb0) % NSB) * SIDE;
     lf_u32x4 df[4][RT];
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
@@ -619,6 +625,23 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   }
   wait_vm<0>();   // the unconsumed loads behind the last pair must not land in another workgroup's LDS
   // C layout: column (k) = lane & 15, rows (r) = 4*(lane >> 4) + e
+  if constexpr (DIRECT) {   // one chunk per segment: these are the sums
+    const int rank = seg.rank[s];
+    const float mult = mask != nullptr && p > 0.f ? 1.f / (1.f - p) : 1.f;
+    uint16_t* out = (uint16_t*)seg.out[s];
+#pragma unroll
+    for (int t = 0; t < TPW; t++)
+      if (t < nt) {
+#pragma unroll
+        for (int c = 0; c < RT; c++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int r = c * 16 + qq * 4 + e;
+            if (r < rank) out[(int64_t)r * K + (kt0 + t) * 64 + wave * 16 + li] = Mfma16<T>::cvt(acc[t][c][e] * mult);
+          }
+      }
+    return;
+  } else {
   float* po = part + ((int64_t)s * max_chunks + ch) * R * K;
 #pragma unroll
   for (int t = 0; t < TPW; t++)
@@ -629,6 +652,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
         for (int e = 0; e < 4; e++)
           if (c * 16 < R) po[(int64_t)(c * 16 + qq * 4 + e) * K + (kt0 + t) * 64 + wave * 16 + li] = acc[t][c][e];
     }
+  }
 }
 
 // ---- dys_dyb.  grid (n_seg * max_chunks, n_slices).  Workgroup (s, ch, ns): the tiles of N slice ns (balanced, 2 .. TPW
@@ -1044,7 +1068,7 @@ constexpr int da_ns(int rt, int maskfmt) {
   return maskfmt ? (rt == 1 ? 3 : 5) : (rt == 4 ? 3 : 4);
 }
 static int da_ring_smem(int rt, int maskfmt) { return da_ns(rt, maskfmt) * (TILE_BYTES + da_mask_tile_bytes(maskfmt)) + 2 * ROWS * rt * 32; }
-struct DaPlan { int n_slices, group, max_chunks; };
+struct DaPlan { int n_slices, group, max_chunks; double cost; };   // cost: bytes moved, by the model below
 // Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by bytes moved: the
 // X stream in whole rounds of resident workgroups, the dS blocks every workgroup fetches, and the fp32 partials
 // (one [R, K] slab per chunk, written here and read by the reduce).  `limit`: as for dysr_plan.
@@ -1054,7 +1078,7 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, s
   seg_block_counts(M, seg, blocks, nseg);
   const int slots = lds_slots(da_ring_smem(rt, maskfmt));
   const double tile_bytes = TILE_BYTES + da_mask_tile_bytes(maskfmt);
-  DaPlan best{1, 1, 1};
+  DaPlan best{1, 1, 1, 1e300};
   if (T < 2) return best;   // as in dysr_plan
   GroupStats stats[kNGroups];
   const int ng = all_group_stats(blocks, nseg, stats);
@@ -1068,7 +1092,7 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, s
       const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
                           2.0 * 4.0 * R * K * (double)st.chunks;
       const bool fits = (size_t)nseg * st.max_chunks * R * K * sizeof(float) <= limit;
-      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks}; }
+      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks, cost}; }
     }
   }
   return best;
@@ -1082,10 +1106,47 @@ size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit)
   return (size_t)nseg * max_chunks * R * K * sizeof(float);
 }
 
+// One launch without a second stage: a workgroup walks all row blocks of its segment over t tiles of columns and stores the sums as
+// they are.  Alone on its compute unit, it has a deeper ring and more dS buffers than the two-stage form: what a walk of one or
+// two tiles per block needs to keep loads on order.  It pays where segments have few blocks (a tile costs a workgroup 0.4 us, with a
+// mask 0.9, one after the other) or the partials are large (high ranks, wide inputs).  Both sides in microseconds, fitted to
+// 496 products (128 - 16384 rows in one or four segments, K 1024 - 14336, ranks 16 - 128, with keep bits and without), direct 9 % and
+// two-stage 16 % off; the choice gives 17 % over them all, 18 is the most any choice gives, 8 are behind by more than 3 % (worst 11).
+// With keep bits, two-stage -> direct: 300 x 4096 rank 16 8.8 -> 7.8, four segments of 1280 x 4096 rank 64 14.7 -> 9.3, of 2048 x 4096 rank 16
+// 13.3 -> 10.5; the other side of the line: 1000 x 4096 rank 16 in one segment 9.7 against 14.4.
+constexpr int da1_nsb(int rt) { return rt <= 2 ? 4 : rt == 4 ? 3 : 2; }
+constexpr int da1_ns(int rt, int maskfmt) { return maskfmt == 1 ? (rt <= 2 ? 5 : 4) : rt <= 2 ? 7 : rt == 4 ? 6 : 5; }
+// (the same choice for every mask format: dA does not depend on how the mask came)
+static int da_direct_slices(int M, int K, int R, bool masked, const LfSegTable& seg, size_t limit) {
+  const int rt = rt_of(R), T = K / 64;
+  if (T < 2) return 0;
+  int blocks[LF_MAX_SEG], nseg, live = 0, big = 0;
+  seg_block_counts(M, seg, blocks, nseg);
+  for (int s = 0; s < nseg; s++) live += blocks[s] > 0, big = std::max(big, blocks[s]);
+  if (live == 0) return 0;
+  int t = rt == 8 ? 2 : 1;   // (with a mask the ring holds three stages at least: two dS buffers allow t + 1)
+  while (t <= da_tpw(rt) && ((T + t - 1) / t) * live > 256) t++;   // one round of workgroups
+  if (t > da_tpw(rt)) return 0;
+  const int nsl = (T + t - 1) / t;
+  const double m = masked, tiles = (double)big * t;
+  const double direct = 3.66 + 0.40 * m + 0.20 * rt + tiles * (0.305 + 0.466 * m + 0.049 * rt) + 0.357 * big + 0.9e-3 * tiles * nsl * live;
+  return 1.05 * direct < 4.85 + 3.5 * m + da_plan(M, K, R, masked ? 2 : 0, seg, limit).cost / 5.39e6 ? nsl : 0;
+}
+
+template <typename T, int RT, int MASK>
+static int da_direct_launch(const void* X, const uint8_t* mask, const void* dS, int M, int K, int R, int n_slices, int nseg, const LfSegTable& seg, hipStream_t st) {
+  constexpr int NS = da1_ns(RT, MASK), NSB = da1_nsb(RT), smem = NS * (TILE_BYTES + da_mask_tile_bytes(MASK)) + NSB * ROWS * RT * 32;
+  static_assert(smem <= 160 * 1024, "ring and dS buffers fit the LDS");
+  auto kern = lora_da_ring_kernel<T, RT, da_tpw(RT), NS, MASK, NSB, true>;
+  static LfLdsFlags lds_ok;
+  if (!lf_allow_lds(kern, smem, lds_ok)) return LF_ELAUNCH;
+  return lf_launch(kern, dim3(n_slices, 1, nseg), dim3(256), smem, st, (const T*)X, mask, (const T*)dS, (float*)nullptr, M, K, R, n_slices, 1 << 20, 1, seg);
+}
+
 template <typename T, int RT, int MASK>
 static int da_ring_launch(const void* X, const uint8_t* mask, const void* dS, float* part, int M, int K, int R, const DaPlan& pl,
                           int nseg, const LfSegTable& seg, hipStream_t st) {
-  auto kern = lora_da_ring_kernel<T, RT, da_tpw(RT), da_ns(RT, MASK), MASK>;
+  auto kern = lora_da_ring_kernel<T, RT, da_tpw(RT), da_ns(RT, MASK), MASK, 2, false>;
   const int smem = da_ring_smem(RT, MASK);
   static LfLdsFlags lds_ok;
   if (!lf_allow_lds(kern, smem, lds_ok)) return LF_ELAUNCH;
@@ -1101,6 +1162,20 @@ static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void
   int rc;
   const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
   const bool off_grid = fmt == 1 && mask_off_grid(mask, 0);   // (the same split, and the same sums)
+  if (const int nsl = da_direct_slices(M, K, R, mask != nullptr, seg, limit)) {
+    switch (rt_of(R)) {
+#define LF_DA_DIRECT(RTV)                                                                               \
+  return off_grid   ? da_direct_launch<T, RTV, 3>(X, mask, dS, M, K, R, nsl, nseg, seg, st)               \
+         : fmt == 2 ? da_direct_launch<T, RTV, 2>(X, mask, dS, M, K, R, nsl, nseg, seg, st)               \
+         : fmt == 1 ? da_direct_launch<T, RTV, 1>(X, mask, dS, M, K, R, nsl, nseg, seg, st)               \
+                    : da_direct_launch<T, RTV, 0>(X, mask, dS, M, K, R, nsl, nseg, seg, st)
+      case 1: LF_DA_DIRECT(1);
+      case 2: LF_DA_DIRECT(2);
+      case 4: LF_DA_DIRECT(4);
+      default: LF_DA_DIRECT(8);
+#undef LF_DA_DIRECT
+    }
+  }
   const DaPlan pl = da_plan(M, K, R, fmt, seg, limit);
 #define LF_DA_RING(RTV)                                                                                                   \
   rc = off_grid   ? da_ring_launch<T, RTV, 3>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
