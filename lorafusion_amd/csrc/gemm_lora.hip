@@ -887,7 +887,7 @@ static int choose_split(int M, int N, int K, bool allow_big, bool wave96, bool m
 // given the workspace lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
 constexpr size_t kKsplitMaxBytes = (size_t)64 << 20, kKsplitMaxBytesNN = LF_STATIC_SCRATCH_BYTES;
 struct KSplit { int cfg, n, steps; };
-static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
+static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
   const int nk = K / BK;
   KSplit best = {cfg, 1, nk};
   const TileCand& planned = cand_of(cfg, mid);
@@ -912,6 +912,11 @@ static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool n
   return best;
 }
 
+static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
+  static thread_local LfMemo<KSplit, 5> memo;
+  return memo.get({M, N, K, cfg, (int64_t)routing_block * 4 + nn * 2 + mid}, [&] { return ksplit_of(M, N, K, cfg, routing_block, nn, mid); });
+}
+
 static std::atomic<int> pinned_cfg{-1};
 int lf_pin_tile_cfg(int cfg) {
   if (cfg < -1 || cfg == 9 || cfg > 12) return LF_EINVAL;
@@ -922,7 +927,7 @@ bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; 
 
 // The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned: rows [0, *rows_head)
 // with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).
-void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
+static void plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
   const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), wave96 = wave96_fits(routing_block);
   int ch = 1, ct = 1;
   const int m_main = choose_split(M, N, K, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
@@ -946,9 +951,20 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
   }
 }
 
+void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
+  struct Plan { int rows, head, tail; };
+  static thread_local LfMemo<Plan, 4> memo;
+  const Plan pl = memo.get({M, N, K, routing_block}, [&] {
+    Plan q;
+    plan_gemm(M, N, K, routing_block, &q.rows, &q.head, &q.tail);
+    return q;
+  });
+  *rows_head = pl.rows, *cfg_head = pl.head, *cfg_tail = pl.tail;
+}
+
 // Bytes of fp32 partial tiles the split contraction of an M x N product over K may write: the largest need over the
 // launches of the plan and over the tiles a launch moves to where the persistent kernel or gemm_mid.hip does not apply.
-size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
+static size_t ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   if (M <= 0 || N <= 0 || K < BK) return 0;
   int rows = 0, ch = 1, ct = -1;
   lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
@@ -966,6 +982,11 @@ size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   part(rows, ch);
   if (ct >= 0) part(M - rows, ct);
   return need;
+}
+
+size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
+  static thread_local LfMemo<size_t, 5> memo;
+  return memo.get({M, N, K, routing_block, nn}, [&] { return ksplit_bytes(M, N, K, routing_block, nn); });
 }
 
 int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int force_cfg, hipStream_t st) {

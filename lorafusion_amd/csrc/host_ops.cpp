@@ -502,6 +502,32 @@ void check_adapters(const std::vector<Tensor>& a, const std::vector<Tensor>& b, 
   for (size_t i = 0; i < b.size(); i++) one(b[i], "lora_b", N, ranks[i]);
 }
 
+// The operands of a packed batch over a 16-bit base weight against each other and the batch's routing (`rows` of it), in one call.  True:
+// the kernels can read all of them as they lie.
+bool check_multi(const Tensor& px, const Tensor& w, const std::vector<Tensor>& a, const std::vector<Tensor>& b, const std::vector<int64_t>& ranks, int64_t rows,
+                 const OptTensor& bias) {
+  if (px.dim() == 3) {
+    if (px.size(0) != 1) bad_value("currently, we only support batch size 1 for multi-linear LoRA");
+  } else if (px.dim() != 2) {
+    bad_value("padded_x must be a 3D tensor, but got ", px.dim());
+  }
+  const int64_t M = px.size(-2), K = px.size(-1);
+  if (M != rows) bad_value("padded_x has ", M, " rows but the batch info covers ", rows, ".");
+  if (w.dim() != 2 || w.size(1) != K || w.scalar_type() != px.scalar_type())
+    bad_value("linear_w must have shape [N, ", K, "] and dtype ", dtype_name(px.scalar_type()), ".");
+  const int64_t N = w.size(0);
+  require_gpu(px, "padded_x");
+  dtype_id(px.scalar_type());
+  check_dims(M, N, K);
+  check_adapters(a, b, ranks, K, N, px);
+  if (bias && (bias->dim() != 1 || bias->size(0) != N || bias->scalar_type() != px.scalar_type()))
+    bad_value("linear_bias must have shape [", N, "] and dtype ", dtype_name(px.scalar_type()), ".");
+  bool plain = px.is_contiguous() && w.is_contiguous() && (!bias || bias->is_contiguous());
+  for (const Tensor& t : a) plain = plain && t.is_contiguous();
+  for (const Tensor& t : b) plain = plain && t.is_contiguous();
+  return plain;
+}
+
 // ------------------------------------------------------------------------------------------- RMSNorm, SiLU-multiply
 
 struct RMSNormBackward : Node {
@@ -668,6 +694,7 @@ PYBIND11_MODULE(_host, m) {
   // (no Python object is touched inside; an exception is translated after the lock is back)
   using nogil = py::call_guard<py::gil_scoped_release>;
   m.def("linear_lora", &linear_lora, nogil());
+  m.def("check_multi", &check_multi, nogil());
   m.def("forward", &py_forward, nogil());
   m.def("backward", &py_backward, nogil());
   m.def("attach", &py_attach);   // (takes a Python object: lets go of the lock itself)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <string.h>
 #include <atomic>
 #include "../../include/lorafusion_hip.h"  // error codes, dtype ids, LF_MAX_SEG
 
@@ -78,6 +79,24 @@ int lf_pin_tile_cfg(int cfg);  // -1: automatic choice
 bool lf_tile_pinned();
 void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail);
 size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn);  // workspace of the split contraction for this product
+
+// The last results of a plan (a function of sizes alone) on this thread: planning a forward + backward took 5 us of host time, more than
+// two of its launches.  Direct mapped; a key is everything the plan reads.
+template <typename V, int KEYS, int SLOTS = 16>
+struct LfMemo {
+  struct Entry { int64_t key[KEYS]; V v; bool set; };
+  Entry e[SLOTS] = {};
+  template <typename F> V get(const int64_t (&key)[KEYS], F&& make) {
+    uint64_t h = 0x9e3779b97f4a7c15ull;
+    for (int i = 0; i < KEYS; i++) h = (h ^ (uint64_t)key[i]) * 0xff51afd7ed558ccdull, h ^= h >> 32;
+    Entry& s = e[h % SLOTS];
+    if (s.set && memcmp(s.key, key, sizeof s.key) == 0) return s.v;
+    const V v = make();
+    memcpy(s.key, key, sizeof s.key);
+    s.v = v, s.set = true;
+    return v;
+  }
+};
 
 // Raise a kernel's dynamic-LDS limit once per device (the attribute belongs to the device's copy of
 // the function; one flag array per kernel instantiation; threads that race here repeat the same call).

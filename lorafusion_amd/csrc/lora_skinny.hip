@@ -871,10 +871,8 @@ struct DysRingPlan { int n_slices, group, max_chunks; };
 // By bytes: the dY (+ B tile) stream over the busiest slot, the S blocks every workgroup fetches (from L2: half weight),
 // and the fp32 partials written here and read by the reduce (dS: one [rows, R] slab per slice; dB: one [N, R] slab per
 // chunk).  The cheapest plan whose partials take at most `limit` bytes (if none does: the cheapest of all).
-static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg, size_t limit) {
+static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = N / 64;
-  int blocks[LF_MAX_SEG], nseg;
-  seg_block_counts(M, seg, blocks, nseg);
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   const int slots = lds_slots(dysr_smem(rt));
   const double tile_bytes = TILE_BYTES + 64.0 * R * 2;
@@ -896,6 +894,22 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg, size_t 
     }
   }
   return best;
+}
+
+// (what the plans read: sizes, and the blocks of each segment)
+struct PlanKey { int64_t v[5 + LF_MAX_SEG / 2]; };
+static void plan_key(PlanKey& k, int M, int dim, int R, int what, size_t limit, const LfSegTable& seg, int* blocks, int& nseg) {
+  seg_block_counts(M, seg, blocks, nseg);
+  k = PlanKey{};
+  k.v[0] = M, k.v[1] = dim, k.v[2] = R, k.v[3] = (int64_t)what << 32 | (seg.table != nullptr) << 16 | nseg, k.v[4] = (int64_t)limit;
+  for (int s = 0; s < nseg; s++) k.v[5 + s / 2] |= (int64_t)(uint32_t)blocks[s] << 32 * (s & 1);
+}
+static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg, size_t limit) {
+  static thread_local LfMemo<DysRingPlan, 5 + LF_MAX_SEG / 2> memo;
+  int blocks[LF_MAX_SEG], nseg;
+  PlanKey k;
+  plan_key(k, M, N, R, 0, limit, seg, blocks, nseg);
+  return memo.get(k.v, [&] { return dysr_plan_of(M, N, R, blocks, nseg, seg, limit); });
 }
 
 // (lora_stream.hip)
@@ -1072,10 +1086,8 @@ struct DaPlan { int n_slices, group, max_chunks; double cost; };   // cost: byte
 // Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by bytes moved: the
 // X stream in whole rounds of resident workgroups, the dS blocks every workgroup fetches, and the fp32 partials
 // (one [R, K] slab per chunk, written here and read by the reduce).  `limit`: as for dysr_plan.
-static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, size_t limit) {
+static DaPlan da_plan_of(int K, int R, int maskfmt, const int* blocks, int nseg, size_t limit) {
   const int rt = rt_of(R), T = K / 64;
-  int blocks[LF_MAX_SEG], nseg;
-  seg_block_counts(M, seg, blocks, nseg);
   const int slots = lds_slots(da_ring_smem(rt, maskfmt));
   const double tile_bytes = TILE_BYTES + da_mask_tile_bytes(maskfmt);
   DaPlan best{1, 1, 1, 1e300};
@@ -1096,6 +1108,14 @@ static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, s
     }
   }
   return best;
+}
+
+static DaPlan da_plan(int M, int K, int R, int maskfmt, const LfSegTable& seg, size_t limit) {
+  static thread_local LfMemo<DaPlan, 5 + LF_MAX_SEG / 2, 32> memo;
+  int blocks[LF_MAX_SEG], nseg;
+  PlanKey k;
+  plan_key(k, M, K, R, maskfmt, limit, seg, blocks, nseg);
+  return memo.get(k.v, [&] { return da_plan_of(K, R, maskfmt, blocks, nseg, limit); });
 }
 
 size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit) {

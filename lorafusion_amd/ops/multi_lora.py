@@ -200,24 +200,40 @@ class FusedLinearMultiLoRA:
 
     @staticmethod
     def apply(padded_x, linear_w, linear_bias, dropout_mask, seed, routing: MultiRouting, quant_state, keep_dequantized, n_adapters, *ab):
+        a_list, b_list = list(ab[:n_adapters]), list(ab[n_adapters:])
+        if quant_state is None:
+            host, bias, mask = L.host(), linear_bias, None
+            x, a_run, b_run = padded_x, a_list, b_list
+            if not host.check_multi(x, linear_w, a_list, b_list, routing.rank_list, routing.M, linear_bias):
+                x, linear_w = padded_x.detach().contiguous(), linear_w.contiguous()
+                a_run, b_run = [t.contiguous() for t in a_list], [t.contiguous() for t in b_list]
+                bias = linear_bias.contiguous() if linear_bias is not None else None
+            if routing.enable_dropout and dropout_mask is None:
+                # per-block p from the routing table, mask drawn inside the rank-r pass
+                if seed is None:
+                    seed = random.randrange(int(1e6))  # noqa: S311
+                y, s, mask = hip_ops.lora_forward_seeded(x, linear_w, a_run, b_run, routing.c, routing.R, seed, bias)
+            else:
+                if routing.enable_dropout:
+                    M, K = routing.M, x.shape[-1]
+                    mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
+                    if not hip_ops.is_packed_mask(mask, K):
+                        mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
+                y, s = hip_ops.lora_forward(x, linear_w, a_run, b_run, routing.c, routing.R, mask, bias)
+            return host.attach(y, [padded_x], x, linear_w, None, [linear_w, linear_bias], a_list, b_list, mask, s, None, [],
+                               ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
         if padded_x.ndim == THREE_DIM:
             if padded_x.shape[0] != 1:
                 raise ValueError("currently, we only support batch size 1 for multi-linear LoRA")
         elif padded_x.ndim != 2:
             raise ValueError(f"padded_x must be a 3D tensor, but got {padded_x.ndim}")
         x2d = padded_x.detach().contiguous().view(padded_x.shape[-2], padded_x.shape[-1])
-        a_list, b_list = list(ab[:n_adapters]), list(ab[n_adapters:])
         M, K = x2d.shape
-        wref, nf4 = None, None
-        if quant_state is not None:
-            # NF4 base weight: linear_w holds the packed codes, quant_state its bitsandbytes-style state
-            from lorafusion_amd.ops.nf4 import NF4WeightRef, nf4_struct_of
+        # NF4 base weight: linear_w holds the packed codes, quant_state its bitsandbytes-style state
+        from lorafusion_amd.ops.nf4 import NF4WeightRef, nf4_struct_of
 
-            wref, nf4 = NF4WeightRef(linear_w, quant_state), nf4_struct_of(quant_state)
-            w_shape, w_dtype = tuple(wref.shape), wref.dtype
-        else:
-            linear_w = linear_w.contiguous()
-            w_shape, w_dtype = tuple(linear_w.shape), linear_w.dtype
+        wref, nf4 = NF4WeightRef(linear_w, quant_state), nf4_struct_of(quant_state)
+        w_shape, w_dtype = tuple(wref.shape), wref.dtype
         if M != routing.M:
             raise ValueError(f"padded_x has {M} rows but the batch info covers {routing.M}.")
         if len(w_shape) != 2 or w_shape[1] != K or w_dtype != x2d.dtype:
@@ -232,29 +248,16 @@ class FusedLinearMultiLoRA:
             raise ValueError(f"linear_bias must have shape [{N}] and dtype {x2d.dtype}.")
         a_run, b_run = [t.contiguous() for t in a_list], [t.contiguous() for t in b_list]
 
-        mask, dense = None, None
+        mask = None
         bias = linear_bias.contiguous() if linear_bias is not None else None
-        if wref is not None:
-            if routing.enable_dropout:
-                if dropout_mask is None:
-                    dropout_mask = hip_ops.make_dropout_mask((M, K), 0.0, seed, x2d.device, routing=routing)
-                mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
-                if not hip_ops.is_packed_mask(mask, K):
-                    mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-            y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing.c, routing.R, mask, bias, keep_dense=keep_dequantized)
-            dense = kept[0] if kept else None
-        elif routing.enable_dropout and dropout_mask is None:
-            # per-block p from the routing table, mask drawn inside the rank-r pass
-            if seed is None:
-                seed = random.randrange(int(1e6))  # noqa: S311
-            y, s, mask = hip_ops.lora_forward_seeded(x2d, linear_w, a_run, b_run, routing.c, routing.R, seed, bias)
-        else:
-            if routing.enable_dropout:
-                mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
-                if not hip_ops.is_packed_mask(mask, K):
-                    mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-            y, s = hip_ops.lora_forward(x2d, linear_w, a_run, b_run, routing.c, routing.R, mask, bias)
-        return host.attach(y, [padded_x], x2d, linear_w, nf4, [linear_w, linear_bias], a_list, b_list, mask, s, dense, [],
+        if routing.enable_dropout:
+            if dropout_mask is None:
+                dropout_mask = hip_ops.make_dropout_mask((M, K), 0.0, seed, x2d.device, routing=routing)
+            mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
+            if not hip_ops.is_packed_mask(mask, K):
+                mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
+        y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing.c, routing.R, mask, bias, keep_dense=keep_dequantized)
+        return host.attach(y, [padded_x], x2d, linear_w, nf4, [linear_w, linear_bias], a_list, b_list, mask, s, kept[0] if kept else None, [],
                            ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
 
 
