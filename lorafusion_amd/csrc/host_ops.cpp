@@ -166,20 +166,28 @@ Forward run_forward(const Tensor& x, Weight& w, const std::vector<Tensor>& a, co
   f.mask = mask;
   if (seed) f.mask = packed ? at::empty({M, K / 8}, x.options().dtype(at::kByte)) : at::empty({M, K}, x.options().dtype(at::kBool));
   if (keep_dense) f.dense = at::empty({N, K}, x.options());
-  const size_t n = lf_workspace_bytes(w.nf4 && !keep_dense ? LF_OP_NF4_FWD : LF_OP_FWD, M, N, K, R, &r);
-  const Tensor ws = scratch(n, x);
+  const size_t n = lf_workspace_bytes(w.nf4 && !keep_dense && !seed ? LF_OP_NF4_FWD : LF_OP_FWD, M, N, K, R, &r);
+  // (a mask drawn over NF4 codes: the weight is dequantised here, in front of the forward's own workspace, and the 16-bit forward draws)
+  const size_t head = w.nf4 && seed && !keep_dense ? ((size_t)N * K * 2 + 255) & ~(size_t)255 : 0;
+  const Tensor ws = scratch(head + n, x);
   const Ptrs pa(a), pb(b);
   const int d = dt | (is_bits(f.mask, K) ? LF_MASK_BITS : 0);
   void* st = stream_of(x);
-  if (w.nf4) {
+  if (seed) {
+    const void* dense = ptr(w.w);
+    if (w.nf4) {
+      void* to = keep_dense ? mptr(f.dense) : mptr(ws);
+      check(lf_nf4_dequant(w.c.packed, w.c.absmax, w.c.code2, w.c.absmax2, w.c.offset, to, (int64_t)N * K, w.c.blocksize, w.c.blocksize2, dt, st), "lf_nf4_dequant");
+      dense = to;
+    }
+    check(lf_lora_fwd_seeded(ptr(x), dense, ptr(bias), (uint8_t*)mptr(f.mask), pa.v, pb.v, mptr(f.y), mptr(f.s), n ? (char*)mptr(ws) + head : nullptr, n, M, N, K, R,
+                             &r, *seed, d, st), "lf_lora_fwd_seeded");
+  } else if (w.nf4) {
     lf_nf4_weight c = w.c;
     c.dense = mptr(f.dense);
     c.dense_valid = 0;
     check(lf_nf4_lora_fwd(ptr(x), &c, ptr(bias), (const uint8_t*)ptr(f.mask), pa.v, pb.v, mptr(f.y), mptr(f.s), mptr(ws), n, M, N, K, R, &r, d, st),
           "lf_nf4_lora_fwd");
-  } else if (seed) {
-    check(lf_lora_fwd_seeded(ptr(x), ptr(w.w), ptr(bias), (uint8_t*)mptr(f.mask), pa.v, pb.v, mptr(f.y), mptr(f.s), mptr(ws), n, M, N, K, R, &r, *seed,
-                             d, st), "lf_lora_fwd_seeded");
   } else {
     check(lf_lora_fwd(ptr(x), ptr(w.w), ptr(bias), (const uint8_t*)ptr(f.mask), pa.v, pb.v, mptr(f.y), mptr(f.s), mptr(ws), n, M, N, K, R, &r, d, st),
           "lf_lora_fwd");

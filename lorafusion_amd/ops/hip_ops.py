@@ -524,6 +524,13 @@ def nf4_lora_forward(x, wref, a_list, b_list, routing_c, R, mask, bias, *, keep_
     return (y, s, dense) if keep_dense else (y, s)
 
 
+def nf4_lora_forward_seeded(x, wref, a_list, b_list, routing_c, R, seed: int, bias, *, keep_dense: bool = False):
+    """``nf4_lora_forward`` with the keep-mask drawn inside the rank-r pass from ``seed``, as ``lora_forward_seeded`` draws it: the mask kernel
+    (a byte per element written), its packing and the pass's read of the bits disappear.  Returns (y, s, mask, dense | None)."""
+    return L.host().forward(x, None, ctypes.addressof(wref.c), wref.shape[0], a_list, b_list, ctypes.addressof(routing_c), R, None,
+                            int(seed) & 0xFFFFFFFFFFFFFFFF, True, bias, keep_dense)
+
+
 def nf4_lora_backward(dy, x, wref, a_list, b_list, s, routing_c, R, mask, rank_list, requires_dx: bool = True,
                       dense: torch.Tensor | None = None):
     """``lora_backward`` with the base weight given as NF4.  ``dense``: the dequantised weight a forward with

@@ -250,14 +250,18 @@ class FusedLinearMultiLoRA:
 
         mask = None
         bias = linear_bias.contiguous() if linear_bias is not None else None
-        if routing.enable_dropout:
-            if dropout_mask is None:
-                dropout_mask = hip_ops.make_dropout_mask((M, K), 0.0, seed, x2d.device, routing=routing)
-            mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
-            if not hip_ops.is_packed_mask(mask, K):
-                mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-        y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing.c, routing.R, mask, bias, keep_dense=keep_dequantized)
-        return host.attach(y, [padded_x], x2d, linear_w, nf4, [linear_w, linear_bias], a_list, b_list, mask, s, kept[0] if kept else None, [],
+        if routing.enable_dropout and dropout_mask is None:
+            if seed is None:
+                seed = random.randrange(int(1e6))  # noqa: S311
+            y, s, mask, dense = hip_ops.nf4_lora_forward_seeded(x2d, wref, a_run, b_run, routing.c, routing.R, seed, bias, keep_dense=keep_dequantized)
+        else:
+            if routing.enable_dropout:
+                mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
+                if not hip_ops.is_packed_mask(mask, K):
+                    mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
+            y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing.c, routing.R, mask, bias, keep_dense=keep_dequantized)
+            dense = kept[0] if kept else None
+        return host.attach(y, [padded_x], x2d, linear_w, nf4, [linear_w, linear_bias], a_list, b_list, mask, s, dense, [],
                            ctypes.addressof(routing.c), [routing.table, routing.scale, routing.p], routing.R, "FusedLinearMultiLoRABackward")
 
 

@@ -11,6 +11,7 @@ dependency here).
 from __future__ import annotations
 
 import ctypes
+import random
 from dataclasses import dataclass
 
 import torch
@@ -203,19 +204,23 @@ class FusedLinearLoRANF4:
             raise ValueError(f"quant_state.dtype {quant_state.dtype} must match x.dtype {x2d.dtype}.")
         wref = NF4WeightRef(packed_w, quant_state)
         M, N, K, r = _validate_shapes(x2d, tuple(wref.shape), x2d.dtype, lora_a, lora_b, linear_bias, dropout_p)
-        mask = None
         bias = linear_bias.contiguous() if linear_bias is not None else None
-        if dropout_p > 0:
-            if dropout_mask is None:
-                dropout_mask = hip_ops.make_dropout_mask((M, K), dropout_p, seed, x2d.device)
-            mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
-            if not hip_ops.is_packed_mask(mask, K):
-                mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
-        routing, R = L.single_routing(r, alpha, dropout_p if mask is not None else 0.0), L.round_rank(r)
-        y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, [lora_a.contiguous()], [lora_b.contiguous()], routing, R, mask, bias,
-                                               keep_dense=keep_dequantized)
+        routing, R = L.single_routing(r, alpha, dropout_p), L.round_rank(r)
+        a_run, b_run = [lora_a.contiguous()], [lora_b.contiguous()]
+        if dropout_p > 0 and dropout_mask is None:
+            if seed is None:
+                seed = random.randrange(int(1e6))  # noqa: S311
+            y, s, mask, dense = hip_ops.nf4_lora_forward_seeded(x2d, wref, a_run, b_run, routing, R, seed, bias, keep_dense=keep_dequantized)
+        else:
+            mask = None
+            if dropout_p > 0:
+                mask = hip_ops._check_mask(dropout_mask.reshape(M, -1), (M, K))
+                if not hip_ops.is_packed_mask(mask, K):
+                    mask = hip_ops.pack_mask(mask)   # read three times (rank-r forward, dA, dX): an eighth of the bytes each
+            y, s, *kept = hip_ops.nf4_lora_forward(x2d, wref, a_run, b_run, routing, R, mask, bias, keep_dense=keep_dequantized)
+            dense = kept[0] if kept else None
         return L.host().attach(y, [x], x2d, packed_w, nf4_struct_of(quant_state), [linear_bias], [lora_a], [lora_b], mask, s,
-                               kept[0] if kept else None, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
+                               dense, [], ctypes.addressof(routing), [], R, "FusedLinearLoRANF4Backward")
 
 
 def fused_linear_lora_nf4(x, packed_w, quant_state, lora_a, lora_b, alpha, seed=None, dropout_p=0.0,

@@ -255,3 +255,21 @@ def test_qlora_keep_dequantized_weight_is_bit_identical():
         outs.append([y.detach(), x.grad] + [t.grad for t in al + bl])
     for t0, t1 in zip(*outs):
         assert torch.equal(t0, t1)
+
+
+@pytest.mark.parametrize("M,K,N,r,keep", [(300, 512, 384, 16, False), (129, 4096, 256, 64, True)])
+def test_mask_drawn_in_the_rank_pass_is_the_mask_kernels(M, K, N, r, keep):
+    """Seeded dropout over NF4 codes: bit for bit the call that is given the mask the mask kernel draws for the seed."""
+    from lorafusion_amd.ops import hip_ops
+    from lorafusion_amd.ops.nf4 import fused_linear_lora_nf4, quantize_nf4
+
+    d = single_inputs(M, K, N, r, p=0.0, seed=M)
+    packed, qs = quantize_nf4(d["w"].cuda())
+    x, a, b = (d[k].cuda().requires_grad_() for k in ("x", "a", "b"))
+    dy = d["dy"].cuda()
+    res = []
+    for kw in (dict(seed=5), dict(dropout_mask=hip_ops.make_dropout_mask((M, K), 0.1, 5, "cuda"))):
+        y = fused_linear_lora_nf4(x, packed, qs, a, b, 2.0, dropout_p=0.1, keep_dequantized=keep, **kw)
+        res.append((y.detach(), *torch.autograd.grad(y, (x, a, b), dy)))
+    for got, exp in zip(*res):
+        assert torch.equal(got, exp)
