@@ -7,7 +7,8 @@
 //             lorafusion/ops/lora_v1.py:111-119; the multi-adapter product, multi_lora.py:481-513)
 //   forward : P = the rows of W followed by the rows of A, Q = X of at most 128 rows: one pass over the weight gives the
 //             base product and the rank-r product of a short batch; a second kernel adds the slices and forms
-//             Y = X W^T + scale (X A^T) B^T + bias (fused_lora_xw_sb, triton_ops/fused_lora_xw_sb.py:74-206)
+//             Y = X W^T + scale (X A^T) B^T + bias (fused_lora_xw_sb, triton_ops/fused_lora_xw_sb.py:74-206);
+//             up to 16 rows and rank 32 a kernel of its own does all of it in one launch (short16_fwd_kernel)
 //
 // Both are bound by the stream of P (the forward of 8 rows moves 34 MB of weights for 0.3 GFLOP), so what counts is how
 // many bytes the chip has on order.  A workgroup (4 waves) owns 64 rows of P and a slice of K: the slices are what
@@ -257,6 +258,118 @@ stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_sl
   *(lf_u32x2*)((uint16_t*)S + idx) = pack4<T>(v);
 }
 
+// Forward of up to 16 rows at ranks up to 32 in one launch.  A workgroup owns 16 G rows of W over all of K; its NW waves deal the steps of 64
+// among themselves, and each streams its steps of W, of X (16 rows) and of A through a ring of its own, so the walk has no barrier.  Every
+// workgroup forms all of S for itself; the first stores it.  The waves' sums are added in a fixed order through LDS, S is rounded,
+// and the workgroup's 16 G columns of Y leave complete: no partial sums in memory, no second launch.  What that costs is X and A once per
+// workgroup, from L2 -- as many bytes each as W at G = 1 and rank 16.  That is why the form ends at 16 rows and rank 32, and why G is 4 (with four
+// waves: the same LDS) where there are columns for it: G = 4 over G = 1 at 8192 columns 13.4 against 16.0 us, at 4096, with 64 workgroups,
+// 11.1 against 9.0.  G = 2 was never ahead of both.
+// Bound by the launch, the first loads and W's bytes: 6 x 4096 x 4096 at rank 16 (MI355X, W from the memory-side cache, captured back to back)
+// 12.8 -> 9.0 us, 3.7 TB/s of W; 6 x 1024 x 1024 7.1 -> 3.9; 6 x 14336 x 4096 (W from HBM, 4.6 TB/s) 34.2 -> 25.6.
+constexpr int short16_waves(int g) { return g == 1 ? 8 : 4; }
+constexpr int short16_stages(int rt, int g) { return 160 / (short16_waves(g) * 2 * (g + 1 + rt)); }   // what 160 KiB hold: 3, 2 (G = 1, ranks to 16, 32), 3, 2
+template <typename T, int RT, int G, int NW = short16_waves(G)>
+__global__ void __launch_bounds__(NW * 64)
+short16_fwd_kernel(const void* __restrict__ X, const void* __restrict__ W, const void* __restrict__ A, const T* __restrict__ B, float scale,
+                   const uint16_t* __restrict__ bias, T* __restrict__ Y, T* __restrict__ S, int M, int N, int K, int rank, int R) {
+  constexpr int NS = short16_stages(RT, G), STAGE = (G + 1 + RT) * 2048, GL = 2 * (G + 1 + RT), NT = NW * 64, COLS = 16 * G;
+  static_assert(NS >= 2 && (NS - 2) * GL < 64, "");
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = to_sgpr(tid >> 6);
+  const int li = lane & 15, qq = lane >> 4;
+  const int col0 = blockIdx.x * COLS;
+  const int nsteps = (K / 64 - wave + NW - 1) / NW;   // steps wave, wave + NW, ...
+  // the row of B that this thread multiplies at the end: requested first
+  const int n = tid % COLS;
+  lf_u32x4 bv[RT * 2];
+#pragma unroll
+  for (int q = 0; q < RT * 2; q++) bv[q] = q * 8 < rank ? *(const lf_u32x4*)(B + (int64_t)(col0 + n) * rank + q * 8) : lf_u32x4{0, 0, 0, 0};
+
+  char* ring = lds + wave * NS * STAGE;
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  // 8 lanes cover the 128 bytes of a row; granule c of row r at slot c ^ ((r >> 1) & 7)
+  const int lrow = lane >> 3, slot = lane & 7;
+  constexpr int NV = 2 * (G > RT ? G : RT);
+  uint32_t rv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int r = i * 8 + lrow;
+    rv[i] = (uint32_t)((int64_t)r * K * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
+  }
+  auto issue = [&](int i) {
+    const int at = i < nsteps ? i : nsteps - 1;   // (behind the last step: that one again, unconsumed)
+    const int64_t ko = (int64_t)(wave + at * NW) * 128;
+    const uint32_t st = ring0 + (i % NS) * STAGE;
+    const lf_u32x4 rw = window_rsrc((const char*)W + (int64_t)col0 * K * 2 + ko, (int64_t)COLS * K * 2 - ko);
+    const lf_u32x4 rx = window_rsrc((const char*)X + ko, (int64_t)M * K * 2 - ko);   // (rows beyond M and beyond the rank read as zeros)
+    const lf_u32x4 ra = window_rsrc((const char*)A + ko, (int64_t)rank * K * 2 - ko);
+#pragma unroll
+    for (int q = 0; q < 2 * G; q++) dma16(rw, rv[q], st + q * 1024);
+#pragma unroll
+    for (int q = 0; q < 2; q++) dma16(rx, rv[q], st + G * 2048 + q * 1024);
+#pragma unroll
+    for (int q = 0; q < 2 * RT; q++) dma16(ra, rv[q], st + (G + 1) * 2048 + q * 1024);
+  };
+  lf_f32x4 acc[G + RT];   // lane: column li of each group (of W's rows, then of A's), rows 4 qq + e of X
+#pragma unroll
+  for (int c = 0; c < G + RT; c++) acc[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int key = (li >> 1) & 7;
+  if (nsteps > 0) {
+    for (int i = 0; i < NS - 1; i++) issue(i);
+    for (int i = 0; i < nsteps; i++) {
+      wait_groups<GL>(NS - 2);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave has read the stage that is refilled now
+      issue(i + NS - 1);
+      const char* st = ring + (i % NS) * STAGE;
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const char* fr = st + li * 128 + (((h * 4 + qq) ^ key) << 4);
+        const lf_u32x4 xf = *(const lf_u32x4*)(fr + G * 2048);
+#pragma unroll
+        for (int c = 0; c < G + RT; c++) acc[c] = Mfma16<T>::run(xf, *(const lf_u32x4*)(fr + (c < G ? c : c + 1) * 2048), acc[c]);
+      }
+    }
+    wait_vm<0>();   // the unconsumed loads behind the last step
+  }
+  __syncthreads();
+  float* part = (float*)lds;                             // [NW][16 (G + RT) columns][16 rows]
+  float* sv = part + NW * (G + RT) * 256;                // [16 RT][16 rows]: S, rounded
+#pragma unroll
+  for (int c = 0; c < G + RT; c++) *(lf_f32x4*)(part + ((wave * (G + RT) + c) * 16 + li) * 16 + qq * 4) = acc[c];
+  __syncthreads();
+  for (int o = tid; o < RT * 256; o += NT) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) v += part[(w * (G + RT) + G) * 256 + o];
+    sv[o] = (float)(T)v;
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    for (int o = tid; o < M * R; o += NT) {
+      const int m = o / R, r = o % R;
+      S[o] = r < rank ? (T)sv[r * 16 + m] : (T)0.f;
+    }
+  }
+#pragma unroll
+  for (int m = tid / COLS; m < 16; m += NT / COLS) {
+    if (m >= M) break;
+    float y = 0.f, t = 0.f;
+#pragma unroll
+    for (int p = 0; p < NW; p++) y += part[(p * (G + RT) * 16 + n) * 16 + m];
+#pragma unroll
+    for (int q = 0; q < RT * 2; q++) {
+      float f[8];
+      unpack8<T>(bv[q], f);
+#pragma unroll
+      for (int e = 0; e < 8; e++) t = __builtin_fmaf(f[e], sv[(q * 8 + e) * 16 + m], t);   // (zero beyond the rank on both sides)
+    }
+    y += t * scale;
+    if (bias != nullptr) y += (float)__builtin_bit_cast(T, bias[col0 + n]);
+    Y[(int64_t)m * N + col0 + n] = (T)y;
+  }
+}
+
 // Second stage of the short forward.  grid (64-column tiles of Y, groups of 16 rows), 16 lanes per row.  A short launch is
 // as long as its chain of memory round trips: the slices of Y and the rows of B are requested before the S rows that the
 // workgroup needs are added up and rounded (each workgroup its own, r <= 128 columns, from L2; the first column tile
@@ -314,7 +427,7 @@ short_fwd_finish_kernel(const float* __restrict__ part, int64_t pitch, int n_sli
 // of the 256 compute units take twice as long as the rest.  So: the count (at most sixteen, none shorter than four
 // steps) with the shortest modelled time -- the busiest compute unit's share of the walk (us per column of K: `walk`), the partial sums written and
 // read back, and what a second stage costs where a single slice needs none.
-// Forward: a full walk of K = 4096 takes 22 us; 6 x 4096 x 4096 (65 groups), first and second stage: 3 slices 12.0 us, 4: 13.3, 7: 12.5, 8: 14.0.
+// Forward: a full walk of K = 4096 takes 22 us; 6 x 4096 x 4096 (65 groups; now a single launch), first and second stage: 3 slices 12.0 us, 4: 13.3, 7: 12.5, 8: 14.0.
 // xa: below K = 768 one; a walk of 4096 takes 18 - 24 us without a mask, 26 - 33 with one read and 48 - 53 with one drawn (the integer work of a workgroup that
 // has a compute unit to itself); the constants are those with the smallest loss against the best count over 64 - 20000 rows, K of
 // 1024 - 14336 and ranks 64 and 128 (masked 13 % -> 3.5 %, against one walk figure of 22 us for all; 9000 x 3072 at rank 64, mask drawn: one
@@ -405,7 +518,7 @@ static int short_pitch(int N, int rank) { return N + (rank + 15) / 16 * 16; }
 static int short_groups(int N, int rank) { return N / SROWS + (rank + SROWS - 1) / SROWS; }
 
 // Up to 64 rows the pass reads W at 4-5 TB/s where tiles of 64 columns leave most of the chip idle (6 x 4096 x 4096: 23.7 ->
-// 12.0 us, 64 rows: 24.9 -> 14.5).  Up to 128 rows a workgroup fetches twice as many bytes
+// 12.0 us, 9.0 in one launch, 64 rows: 24.9 -> 14.5).  Up to 128 rows a workgroup fetches twice as many bytes
 // of X from L2 as of W: still ahead where the output is too narrow to fill the chip with tiles (128 x 4096 x 4096: 25.3 ->
 // 20.9).  What it loses is the second stage, whose workgroups (64 columns x 16 rows) form the LoRA term one column per lane, in time
 // with their number and the rank, while the general path's disadvantage grows with K: the line is fitted to 620 shapes of 8 - 128 rows,
@@ -433,8 +546,41 @@ static int short_fwd_impl(const StreamArgs& a, const LfSegTable& seg, const void
                    a.n_slices, a.M, a.n0, a.n1, a.R, (const T*)B, scale, (const uint16_t*)bias, (T*)Y, (T*)a.S);
 }
 
+// The one-launch form, against the two launches, over 8 widths of 128 - 14336 columns, K of 1024 - 14336, 1 - 16 rows, ranks 8 - 32.  A workgroup walks
+// all of K at what one compute unit takes in, so it loses where K is long and the columns are few, and earlier at rank 32, which adds a third
+// to its bytes: 16 x 1024 x 6144 rank 16 10.0 against 10.3 us, x 8192 11.4 against 11.0; 6 x 1024 x 4096 rank 32 7.7 against 8.9,
+// x 5120 10.0 against 9.2.  From 3072 columns the two launches have more to stream: 16 x 3072 x 7168 rank 32 13.7 against 14.7.  In groups of 64 columns: 16 x
+// 4224 x 4096 rank 16 12.8 against 13.0, rank 32 14.8 against 14.0, 6 x 8192 rank 32 14.8 against 18.9.  More than 256 groups are a second round: 6 x 17408 x 4096
+// 47.3 against 40.8.
+static bool short16_applies(int M, int N, int K, int rank) {
+  if (M > 16 || rank > 32 || N > 256 * 64) return false;
+  if (N > 4096) return K <= (rank <= 16 || N >= 8192 ? 4096 : 2048);
+  return K <= (N >= 3072 ? 7168 : rank <= 16 ? 6144 : 4096);
+}
+
+template <typename T, int RT, int G>
+static int short16_launch(const void* X, const void* W, const void* A, const void* B, float scale, const void* bias, void* Y, void* S, int M, int N, int K,
+                          int rank, int R, hipStream_t st) {
+  auto kern = short16_fwd_kernel<T, RT, G>;
+  constexpr int SMEM = short16_waves(G) * short16_stages(RT, G) * (G + 1 + RT) * 2048;
+  static LfLdsFlags lds_ok;
+  if (!lf_allow_lds(kern, SMEM, lds_ok)) return LF_ELAUNCH;
+  return lf_launch(kern, dim3(N / (16 * G)), dim3(short16_waves(G) * 64), SMEM, st, X, W, A, (const T*)B, scale, (const uint16_t*)bias, (T*)Y, (T*)S, M, N, K,
+                   rank, R);
+}
+template <typename T>
+static int short16_impl(const void* X, const void* W, const void* A, const void* B, float scale, const void* bias, void* Y, void* S, int M, int N, int K,
+                        int rank, int R, hipStream_t st) {
+  auto launch = rank <= 16 ? (N <= 4096 ? short16_launch<T, 1, 1> : short16_launch<T, 1, 4>) : N <= 4096 ? short16_launch<T, 2, 1> : short16_launch<T, 2, 4>;
+  return launch(X, W, A, B, scale, bias, Y, S, M, N, K, rank, R, st);
+}
+
 int lf_launch_short_fwd(const void* X, const void* W, const void* A, const void* B, float scale, const void* bias, void* Y, void* S, void* ws,
                         int M, int N, int K, int rank, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
+  if (short16_applies(M, N, K, rank)) {
+    auto one = dtype == LF_BF16 ? short16_impl<__bf16> : short16_impl<_Float16>;
+    return one(X, W, A, B, scale, bias, Y, S, M, N, K, rank, R, st);
+  }
   StreamArgs a{};
   a.p0 = W; a.p1 = A; a.n0 = N; a.n1 = rank; a.K = K; a.n_slices = short_slices(M, N, K, rank);
   a.part = (float*)ws; a.pitch = short_pitch(N, rank); a.S = S; a.M = M; a.R = R; a.q = X;
