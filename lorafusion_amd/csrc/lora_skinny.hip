@@ -65,7 +65,8 @@ __device__ __forceinline__ lf_u32x4 tile_tr_frag(const char* tile, int row, int 
 }
 
 // ------------------------------------------------------------------------------------ xa
-// Ranks to 64, where the sliced pass of lora_stream.hip is not the faster one or has no memory for its sums (lf_xa_takes_stream).
+// Ranks to 64, where the sliced pass of lora_stream.hip is not the faster one or has no memory for its sums (lf_xa_takes_stream), and without a mask
+// its ring kernel is not (lf_xa_rings).
 // One workgroup of 8 waves per 16 rows (64 at ranks 48-64); no partial sums leave the workgroup.  The K range is dealt
 // to the waves in 64-column steps (step s goes to wave s % 8), each wave streams its steps of the
 // 16 rows with coalesced 16-byte loads (8 lanes cover one 128-byte line), the next step's loads in flight while one is used
@@ -915,6 +916,7 @@ static DysRingPlan dysr_plan(int M, int N, int R, const LfSegTable& seg, size_t 
 // (lora_stream.hip)
 int lf_xa_stream_slices(int, int, int, bool, const LfSegTable&);
 size_t lf_xa_stream_workspace(int, int, int, bool, const LfSegTable&);
+int lf_launch_xa_ring(const void*, void*, int, int, int, const LfSegTable&, int, hipStream_t);
 int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, void*, float*, int, int, int, const LfSegTable&, int, hipStream_t);
 
 // The products that the sliced pass (lora_stream.hip) is the faster one for, given memory for the slices' sums.  Microseconds below: mask drawn /
@@ -931,8 +933,10 @@ int lf_launch_xa_stream(const void*, const uint8_t*, uint8_t*, int, uint64_t, vo
 //     192         K 4096  41.7/28.3/23.7 -> 38.7/28.9/24.8   8192  75.0/47.8/38.6 -> 65.6/46.2/39.8   14336 149/110/90 -> 111/100/82
 //     219         K 8192  75.6/49.2/42.2 -> 77.9/64.4/49.7 (eight slices; two: 80.3/49.3/42.8)
 // - To 32: up to 1024 rows from K = 4096 with a mask (300 rows at rank 16: K = 3072 8.8 / 6.1 -> 9.0 / 7.1, 4096 10.9 / 7.3 -> 8.9 / 7.2, 8192 19.1 /
-//   11.6 -> 11.7 / 8.7; a second launch costs what a short K saves), without one from 8192 (8.3 -> 7.3), and at ranks 17 - 32
-//   up to 512 rows from 4096 (300 rows: 4096 7.0 -> 6.9, 5120 8.0 -> 7.2; 1000 rows, 5120: 8.0 -> 7.7).
+//   11.6 -> 11.7 / 8.7; a second launch costs what a short K saves).  Without one, against lora_xa_ring_kernel (us, rank to 16 / to 32): 333 rows, K = 8192
+//   6.8 / 7.4 -> 6.3 / 9.6, 14336 8.7 / 9.4 -> 12.1 / 17.0; 1000 rows, 8192 8.7 / 10.0 -> 8.4 / 10.7.  At 333 x 4096 and rank 32 the ring takes 5.7
+//   against 6.4 when X comes from the caches, but inside a forward whose weight has pushed X out of them (117 MB, 14336 columns) the sliced
+//   pass's 96 workgroups fetch it sooner than 21 and the whole forward takes 57.8 against 58.2: there it stays sliced.
 // The same choice for every mask format, drawn or read: S does not depend on how the mask came.
 static bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
@@ -943,7 +947,7 @@ static bool lf_xa_streams(int M, int K, int R, bool masked, const LfSegTable& se
     const int k_min = groups <= 64 ? 1024 : groups <= 128 ? 1536 : groups <= 170 ? 2048 : groups <= 192 ? 8192 : 1 << 30;
     return K >= (masked || k_min == 1 << 30 ? k_min : 2 * k_min);
   }
-  return rows <= 1024 && (masked ? K >= 4096 : K >= 8192 || (R > 16 && K >= 4096 && rows <= 512));
+  return rows <= 1024 && K >= (masked ? 4096 : R <= 16 ? 8320 : rows <= 512 ? 4096 : 8192);
 }
 // ... and those it takes.  Without the memory (entry points that have no workspace to give, or too small a one) this file's kernel
 // runs to rank 64; above, and where a single slice needs none, the sliced pass all the same.
@@ -953,6 +957,16 @@ bool lf_xa_takes_stream(int M, int K, int R, const uint8_t* mask, int mask_bits,
   if (R <= 64 && mask_off_grid(mask, mask_bits)) return false;
   return lf_xa_streams(M, K, R, masked, seg) && (R > 64 || lf_xa_stream_slices(M, K, R, masked, seg) == 1 ||
                                                  (ws != nullptr && ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg)));
+}
+// The products without a mask that lora_xa_ring_kernel (lora_stream.hip) is the faster one for: ranks to 32 while there are no more than one
+// workgroup per compute unit -- its LDS holds one at a time.  This file's kernel against it, us, rank 16: 333 x 2048 3.8 -> 3.6, 1000 x 4096 6.6 -> 5.3,
+// 4096 x 4096 9.2 -> 8.3, 4096 x 14336 27.7 -> 24.9; 8192 rows 15.0 -> 14.2 at K = 4096 but 9.4 -> 9.8 at 2048 and 29.7 -> 30.4 at 8192.  Direct
+// loads take addresses of whole dwords.
+static bool lf_xa_rings(const void* X, int M, int R, const LfSegTable& seg) {
+  if (R > 32 || (seg.table ? (int64_t)seg.n_blocks * ROWS : M) > 256 * 16) return false;
+  uintptr_t at = (uintptr_t)X;
+  for (int i = 0; i < (seg.table ? seg.n_seg : 1); i++) at |= (uintptr_t)seg.ptr[i];
+  return (at & 3) == 0;
 }
 size_t lf_xa_workspace(int M, int K, int R, const LfSegTable& seg) {
   size_t n = 0;
@@ -1009,6 +1023,7 @@ int lf_launch_xa(const void* X, const void* U, int64_t ldx, void* act_out, const
     if ((dtype == LF_BF16 || dtype == LF_F16) && lf_xa_takes_stream(M, K, R, mask, mask_bits, mask_out != nullptr, seg, ws, ws_bytes))
       return lf_launch_xa_stream(X, mask, mask_out, mask_bits, seed, S, ws_bytes >= lf_xa_stream_workspace(M, K, R, masked, seg) ? (float*)ws : nullptr, M,
                                  K, R, seg, dtype, st);
+    if ((dtype == LF_BF16 || dtype == LF_F16) && !masked && lf_xa_rings(X, M, R, seg)) return lf_launch_xa_ring(X, S, M, K, R, seg, dtype, st);
   }
   if (dtype == LF_BF16) return xa_impl<__bf16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);
   if (dtype == LF_F16) return xa_impl<_Float16>(X, U, ldx, act_out, mask, mask_out, mask_bits, seed, S, M, K, R, seg, st);

@@ -258,6 +258,82 @@ stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_sl
   *(lf_u32x2*)((uint16_t*)S + idx) = pack4<T>(v);
 }
 
+// Rank-r product without a keep-mask at ranks up to 32, where the rows are few (lf_xa_rings).  A workgroup of eight waves per 16 rows of X over all of K, as
+// lora_xa_kernel has it, but X and A arrive by direct loads: a wave streams its steps of both (every eighth 64 columns)
+// through a ring of its own, without a barrier, and keeps NS - 1 steps on order instead of the one or two that registers hold.  Nothing needs to come
+// through registers here: there is no mask to apply before the product.
+// Bound by what one compute unit takes in, X and A (MI355X, replayed from a graph, rank 16: 333 x 4096 5.2 -> 4.5 us, 1000 x 4096 6.6 -> 5.3,
+// 4096 x 4096 9.2 -> 8.3, 4.1 TB/s of X; whole forwards of 333 x 4096 into 4096 27.1 -> 26.1, 3000 x 8192 into 2048 at rank 32 99.6 -> 96.8).
+constexpr int xr_stages(int rt) { return rt == 1 ? 4 : 3; }
+template <typename T, int RT>
+__global__ void __launch_bounds__(512)
+lora_xa_ring_kernel(const void* __restrict__ X, T* __restrict__ S, int M, int rows, int K, int R, const LfSegTable seg) {
+  constexpr int NS = xr_stages(RT), STAGE = (1 + RT) * 2048, GL = 2 * (1 + RT);
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = to_sgpr(tid >> 6);
+  const int li = lane & 15, qq = lane >> 4;
+  const int row0 = blockIdx.x * 16;
+  const BlockInfo bi = block_info(seg, row0 / ROWS, M);
+  const char* A = (const char*)seg.ptr[bi.seg];
+  const int nsteps = (K / 64 - wave + 7) / 8;   // steps wave, wave + 8, ...
+
+  char* ring = lds + wave * NS * STAGE;
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+  // 8 lanes cover the 128 bytes of a row; granule c of row r at slot c ^ ((r >> 1) & 7)
+  const int lrow = lane >> 3, slot = lane & 7;
+  uint32_t rv[2 * RT];
+#pragma unroll
+  for (int i = 0; i < 2 * RT; i++) {
+    const int r = i * 8 + lrow;
+    rv[i] = (uint32_t)((int64_t)r * K * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
+  }
+  auto issue = [&](int i) {
+    const int at = i < nsteps ? i : nsteps - 1;   // (behind the last step: that one again, unconsumed)
+    const int64_t ko = (int64_t)(wave + at * 8) * 128;
+    const uint32_t st = ring0 + (i % NS) * STAGE;
+    const lf_u32x4 rx = window_rsrc((const char*)X + (int64_t)row0 * K * 2 + ko, (int64_t)(rows - row0) * K * 2 - ko);   // (rows beyond the last and
+    const lf_u32x4 ra = window_rsrc(A + ko, (int64_t)bi.rank * K * 2 - ko);                                              // beyond the rank read as zeros)
+#pragma unroll
+    for (int q = 0; q < 2; q++) dma16(rx, rv[q], st + q * 1024);
+#pragma unroll
+    for (int q = 0; q < 2 * RT; q++) dma16(ra, rv[q], st + 2048 + q * 1024);
+  };
+  lf_f32x4 acc[RT];
+#pragma unroll
+  for (int c = 0; c < RT; c++) acc[c] = lf_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int key = (li >> 1) & 7;
+  if (nsteps > 0) {
+    for (int i = 0; i < NS - 1; i++) issue(i);
+    for (int i = 0; i < nsteps; i++) {
+      wait_groups<GL>(NS - 2);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave has read the stage that is refilled now
+      issue(i + NS - 1);
+      const char* st = ring + (i % NS) * STAGE;
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const char* fr = st + li * 128 + (((h * 4 + qq) ^ key) << 4);
+        const lf_u32x4 xf = *(const lf_u32x4*)fr;
+#pragma unroll
+        for (int c = 0; c < RT; c++) acc[c] = Mfma16<T>::run(xf, *(const lf_u32x4*)(fr + (1 + c) * 2048), acc[c]);
+      }
+    }
+    wait_vm<0>();   // the unconsumed loads behind the last step
+  }
+  __syncthreads();
+  float* part = (float*)lds;   // [8 waves][16 RT columns][16 rows]
+#pragma unroll
+  for (int c = 0; c < RT; c++) *(lf_f32x4*)(part + ((wave * RT + c) * 16 + li) * 16 + qq * 4) = acc[c];
+  __syncthreads();
+  const int col = tid >> 4, m = tid & 15;
+  if (col < R && row0 + m < rows) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; w++) v += part[w * RT * 256 + (col % (16 * RT)) * 16 + m];
+    const bool real = (row0 + m) % ROWS < bi.valid && col < bi.rank;
+    S[(int64_t)(row0 + m) * R + col] = real ? (T)v : (T)0.f;
+  }
+}
+
 // Forward of up to 16 rows at ranks up to 32 in one launch.  A workgroup owns 16 G rows of W over all of K; its NW waves deal the steps of 64
 // among themselves, and each streams its steps of W, of X (16 rows) and of A through a ring of its own, so the walk has no barrier.  Every
 // workgroup forms all of S for itself; the first stores it.  The waves' sums are added in a fixed order through LDS, S is rounded,
@@ -501,6 +577,20 @@ int lf_xa_stream_slices(int M, int K, int R, bool masked, const LfSegTable& seg)
 size_t lf_xa_stream_workspace(int M, int K, int R, bool masked, const LfSegTable& seg) {
   const int n = lf_xa_stream_slices(M, K, R, masked, seg);
   return n > 1 ? (size_t)n * xa_rows_of(M, seg) * R * sizeof(float) : 0;
+}
+
+template <typename T, int RT>
+static int xa_ring_launch(const void* X, void* S, int M, int rows, int K, int R, const LfSegTable& seg, hipStream_t st) {
+  auto kern = lora_xa_ring_kernel<T, RT>;
+  constexpr int SMEM = 8 * xr_stages(RT) * (1 + RT) * 2048;
+  static LfLdsFlags lds_ok;
+  if (!lf_allow_lds(kern, SMEM, lds_ok)) return LF_ELAUNCH;
+  return lf_launch(kern, dim3((rows + 15) / 16), dim3(512), SMEM, st, X, (T*)S, M, rows, K, R, seg);
+}
+int lf_launch_xa_ring(const void* X, void* S, int M, int K, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
+  const int rows = (int)xa_rows_of(M, seg);
+  if (dtype == LF_BF16) return R <= 16 ? xa_ring_launch<__bf16, 1>(X, S, M, rows, K, R, seg, st) : xa_ring_launch<__bf16, 2>(X, S, M, rows, K, R, seg, st);
+  return R <= 16 ? xa_ring_launch<_Float16, 1>(X, S, M, rows, K, R, seg, st) : xa_ring_launch<_Float16, 2>(X, S, M, rows, K, R, seg, st);
 }
 
 // ws == nullptr: no room for the slices' sums (ranks above 64 or a single slice; the result is the same, bit for bit)
