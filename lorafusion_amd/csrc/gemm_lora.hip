@@ -641,7 +641,8 @@ gemm_lora_kernel(const LfGemmParams p, const LfSegTable seg) {
   __syncthreads();
   if (grp == 1) phase_barrier();
   while (kt + 5 < nk) step_pair(integral_constant<bool, true>{});
-  while (kt < nk) step_pair(integral_constant<bool, false>{});
+  do step_pair(integral_constant<bool, false>{});   // (two steps are left at least: written so that every path to the end shows its wait)
+  while (kt < nk);
   if (grp == 0) phase_barrier();
   }
 

@@ -388,7 +388,7 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
   int s = 1;
   for (; s + NST - 1 < nk; s++) k_step(s, F_{}, T_{}, T_{}, integral_constant<int, INFLIGHT>{});
   __builtin_amdgcn_sched_barrier(0);
-  // the term's skinny operand (no term: an empty buffer)
+  // the term's skinny operand (no term: an empty buffer, zeros)
   dead = cst >= STAGE ? cst - STAGE : (NST - 1) * STAGE;
   load_rop(t0, 0, 0);
   load_rop(t0, 1, 1);
@@ -398,6 +398,9 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
     k_step(s + I.value, F_{}, F_{}, std::bool_constant<(I.value < NST - 2)>{}, integral_constant<int, left >= 0 ? left * NL + 2 * TJ : -1>{});
   });
   mfma_fence();
+  // The term's operand has landed, in waves without a term too: an empty buffer still writes its zeros to LDS, and the stages take
+  // other waves' results from here on (a split contraction's later slices end here: nothing may land behind the workgroup's end).
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   barrier();   // every wave is done with the stages
 
   // ---- results into ordinary vector registers: acc + mult * (masked) term

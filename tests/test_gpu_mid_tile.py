@@ -38,6 +38,31 @@ def test_single(tile, M, K, N, r, p, scale):
     run_single(M, K, N, r, p, scale)
 
 
+@pytest.mark.parametrize("K,bias", [(256, False), (512, True), (4096, False)])
+def test_rows_in_the_upper_half_of_the_last_tile(tile, K, bias):
+    """The lower waves of the last tile have no rows and no LoRA term.  With K a multiple of 256 their (empty) skinny operand goes to the stage
+    that the upper waves' results leave through."""
+    rows = {10: 160, 11: 128, 12: 128}[tile]
+    run_single(rows + rows // 2 - 11, K, 512, 16, 0.1, 2.0, bias=bias)
+
+
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("M,N,K", [(300, 256, 256), (224, 384, 4096), (129, 128, 320)])
+def test_plain_product(tile, trans_b, M, N, K):
+    """No LoRA term in any wave; a product with the identity gives the operand back bit for bit."""
+    from lorafusion_amd.ops import hip_ops
+
+    g = torch.Generator().manual_seed(M + K)
+    a = torch.randn(M, K, generator=g).bfloat16().cuda()
+    b = torch.randn(N, K, generator=g).bfloat16().cuda()
+    c = hip_ops.gemm(a, b if trans_b else b.T.contiguous(), trans_b=trans_b, tile_cfg=tile)
+    ok, rel, excess = lora_ref.check_close(c.float().cpu(), a.float().cpu() @ b.float().cpu().T, rtol=1e-2)
+    assert ok, f"rel {rel:.3e} excess {excess:.3e}"
+    eye = torch.eye(256).bfloat16().cuda()
+    a = torch.randn(M, 256, generator=g).bfloat16().cuda()
+    assert torch.equal(hip_ops.gemm(a, eye, trans_b=trans_b, tile_cfg=tile), a)
+
+
 def test_single_bias_3d_fp16(tile):
     run_single(512, 512, 640, 16, 0.1, 2.0, bias=True, three_d=True)
     run_single(161, 512, 384, 16, 0.1, 2.0, dtype=torch.float16)
