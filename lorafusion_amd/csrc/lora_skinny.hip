@@ -550,7 +550,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
       dma4(window_rsrc(mask != nullptr ? (const char*)mask + boff : (const char*)X, mask != nullptr ? (xleft >> 4) : 0), mv[0],
            lds0 + ist * STAGE + TILE_BYTES + wave * 256);
     }
-    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), dv, lds0 + NS * STAGE + ((ib - bb0) % NSB) * SIDE, wave);
+    if (ij == 0 && ib < bb1) side_dma<RT>(window_rsrc(sb, ib == b1 - 1 ? min(sleft, slast) : sleft), dv, lds0 + NS * STAGE + ((uint32_t)(ib - bb0) % NSB) * SIDE, wave);
     ist = ist + 1 == ns ? 0 : ist + 1;
     if (ib < bb1) {
       if (++ij < nt) {
@@ -588,7 +588,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
     if (use_mask) apply_mask(ring, bb0, 0);
   }
   for (int b = bb0; b < bb1; b++) {
-    const char* dcur = side + ((b - bb0) % NSB) * SIDE;
+    const char* dcur = side + ((uint32_t)(b - bb0) % NSB) * SIDE;
     lf_u32x4 df[4][RT];
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
