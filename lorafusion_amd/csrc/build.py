@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "liblorafusion_hip.so")
 HOST = os.path.join(PKG, "_host.so")
-SOURCES = ["gemm_lora.hip", "gemm_big.hip", "gemm_mid.hip", "lora_skinny.hip", "lora_stream.hip", "nf4_dequant.hip", "dropout_mask.hip", "norm_act.hip", "lf_api.hip"]
+SOURCES = ["gemm_lora.hip", "gemm_big.hip", "gemm_mid.hip", "lora_skinny.hip", "lora_da_direct.hip", "lora_stream.hip", "nf4_dequant.hip", "dropout_mask.hip", "norm_act.hip", "lf_api.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -24,7 +24,7 @@ FLAGS = [
 
 # sources whose kernels issue memory instructions from inline assembly: their generated code is checked for the
 # hazards the compiler does not resolve there (asm_lint.py)
-LINTED = ["gemm_big.hip", "gemm_mid.hip", "gemm_lora.hip", "lora_skinny.hip", "lora_stream.hip"]
+LINTED = ["gemm_big.hip", "gemm_mid.hip", "gemm_lora.hip", "lora_skinny.hip", "lora_da_direct.hip", "lora_stream.hip"]
 
 
 def _assembly(src: str) -> str:

@@ -1,4 +1,4 @@
-// Pieces shared by the rank-r passes (lora_skinny.hip, lora_stream.hip): routing of a 128-row block, MFMA wrapper,
+// Pieces shared by the rank-r passes (lora_skinny.hip, lora_da_direct.hip, lora_stream.hip): routing of a 128-row block, MFMA wrapper,
 // keep-mask arithmetic, sums of fp32 partials, and the direct-to-LDS loads with their counted waits (internal).
 #pragma once
 #include "lf_common.h"
