@@ -8,9 +8,10 @@
 
 namespace {
 
-// Alone on its compute unit: ring stages and dS buffers.
+// Alone on its compute unit: ring stages and dS buffers.  (A seventh stage without a mask, and a wait that leaves it in flight: 128 - 1000 rows x 2048 -
+// 14336 at ranks 16 and 32 within 1 % either way.)
 constexpr int da1_nsb(int rt) { return rt <= 2 ? 4 : rt == 4 ? 3 : 2; }
-constexpr int da1_ns(int rt, int maskfmt) { return maskfmt == 1 ? (rt <= 2 ? 5 : 4) : rt <= 2 ? 7 : rt == 4 ? 6 : 5; }
+constexpr int da1_ns(int rt, int maskfmt) { return maskfmt == 1 ? (rt <= 2 ? 5 : 4) : rt <= 2 ? (maskfmt ? 7 : 6) : rt == 4 ? 6 : 5; }
 
 template <typename T, int RT, int MASK>
 int launch(const void* X, const uint8_t* mask, const void* dS, int M, int K, int R, int n_slices, const LfSegTable& seg, hipStream_t st) {

@@ -166,7 +166,8 @@ __device__ __forceinline__ void dma4(const lf_u32x4& rsrc, uint32_t voff, uint32
 }
 template <int N>
 __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// at most `groups` groups of G operations each may still be outstanding
+// at most `groups` groups of G operations each may still be outstanding (above four: four; a ring with more stages on order would not use them)
+constexpr int WAIT_MOST = 4;
 template <int G>
 __device__ __forceinline__ void wait_groups(int groups) {
   switch (groups) {
@@ -174,7 +175,7 @@ __device__ __forceinline__ void wait_groups(int groups) {
     case 1: wait_vm<G>(); break;
     case 2: wait_vm<2 * G>(); break;
     case 3: wait_vm<3 * G>(); break;
-    default: wait_vm<4 * G>(); break;
+    default: wait_vm<WAIT_MOST * G>(); break;
   }
 }
 __device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

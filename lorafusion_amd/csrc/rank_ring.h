@@ -180,6 +180,7 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   constexpr int STAGE = TILE_BYTES + da_mask_tile_bytes(MASK);
   constexpr int SIDE = ROWS * RT * 32;
   constexpr int G = 4 + (MASK == 1 ? 2 : MASK == 2 ? 1 : 0);   // operations per load group and thread, not counting a dS block
+  static_assert(NS - (MASK ? 3 : 2) <= WAIT_MOST, "every stage of the ring is used");
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   char* ring = lds;
   char* side = lds + NS * STAGE;
