@@ -435,10 +435,11 @@ short16_fwd_kernel(const void* __restrict__ X, const void* __restrict__ W, const
     for (int p = 0; p < NW; p++) y += part[(p * (G + RT) * 16 + n) * 16 + m];
 #pragma unroll
     for (int q = 0; q < RT * 2; q++) {
+      if (q * 8 >= rank) break;   // (not zeros times zeros: S beyond the rank is the zeros of A times X, NaN where X has an infinity)
       float f[8];
       unpack8<T>(bv[q], f);
 #pragma unroll
-      for (int e = 0; e < 8; e++) t = __builtin_fmaf(f[e], sv[(q * 8 + e) * 16 + m], t);   // (zero beyond the rank on both sides)
+      for (int e = 0; e < 8; e++) t = __builtin_fmaf(f[e], sv[(q * 8 + e) * 16 + m], t);
     }
     y += t * scale;
     if (bias != nullptr) y += (float)__builtin_bit_cast(T, bias[col0 + n]);

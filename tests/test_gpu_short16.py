@@ -32,3 +32,27 @@ def test_short16(M, K, N, r, dtype, bias):
         ok, rel, excess = lora_ref.check_close(got.float().cpu(), exp, rtol=1e-2)
         assert ok, f"{name}: rel {rel:.3e} excess {excess:.3e}"
     assert not s[:, r:].any()
+
+
+@pytest.mark.parametrize("r", [8, 16, 24, 32])
+@pytest.mark.parametrize("N", [256, 4224])
+def test_infinities_stay_infinities(r, N):
+    """An infinity in X against positive columns of W, A and B is an infinity in Y, at ranks below the kernel's tiling too, where the rank columns
+    behind the last are zeros times X; the other rows are untouched."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    M, K = 5, 512
+    d = single_inputs(M, K, N, r, p=0.0, seed=r)
+    x, w, a, b = d["x"], d["w"], d["a"], d["b"].abs()
+    x[1, 7], x[3, 400] = float("inf"), float("-inf")
+    for c in (7, 400):
+        w[:, c], a[:, c] = w[:, c].abs() + 0.01, a[:, c].abs() + 0.01
+    y, s = hip_ops.lora_forward(x.cuda(), w.cuda(), [a.cuda()], [b.cuda()], L.single_routing(r, 0.5, 0.0), L.round_rank(r), None, None)
+    y, s = y.float().cpu(), s.float().cpu()
+    for row, inf in ((1, float("inf")), (3, float("-inf"))):
+        assert bool((y[row] == inf).all()) and bool((s[row, :r] == inf).all())
+    assert not s[:, r:].any()
+    ye, _ = lora_ref.linear_lora_fwd_fp32(x, w, a, b, 0.5, None, 0.0, None)
+    ok, rel, excess = lora_ref.check_close(y[[0, 2, 4]], ye[[0, 2, 4]], rtol=1e-2)
+    assert ok, f"rel {rel:.3e} excess {excess:.3e}"
