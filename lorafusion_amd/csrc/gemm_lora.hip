@@ -1006,7 +1006,8 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
   if (seg.table != nullptr && (seg.block_size_m % 64 != 0)) return LF_ESHAPE;
   const bool planned = force_cfg < 0;
   const int rblock = seg.table != nullptr ? seg.block_size_m : 0;
-  // gemm_mid.hip reads keep-masks as bits and fetches the skinny operand with 16-byte direct loads (4-byte aligned addresses)
+  // gemm_mid.hip reads keep-masks as bits.  It fetches the skinny operand with 16-byte direct loads: one off a dword stays with the tiles that read it
+  // lane by lane.  (A and B of every product come by direct loads from any element's address, with the same results.)
   bool mid = wave96_fits(rblock) && (p.mask == nullptr || (p.mask_bits && p.N % 32 == 0));
   if (p.L != nullptr)
     for (int i = 0; i < std::max(1, seg.n_seg); i++) mid = mid && ((uintptr_t)seg.ptr[i] & 3) == 0;

@@ -626,8 +626,8 @@ bool lf_xa_takes_stream(int M, int K, int R, const uint8_t* mask, int mask_bits,
 }
 // The products without a mask that lora_xa_ring_kernel (lora_stream.hip) is the faster one for: ranks to 32 while there are no more than one
 // workgroup per compute unit -- its LDS holds one at a time.  This file's kernel against it, us, rank 16: 333 x 2048 3.8 -> 3.6, 1000 x 4096 6.6 -> 5.3,
-// 4096 x 4096 9.2 -> 8.3, 4096 x 14336 27.7 -> 24.9; 8192 rows 15.0 -> 14.2 at K = 4096 but 9.4 -> 9.8 at 2048 and 29.7 -> 30.4 at 8192.  Direct
-// loads take addresses of whole dwords.
+// 4096 x 4096 9.2 -> 8.3, 4096 x 14336 27.7 -> 24.9; 8192 rows 15.0 -> 14.2 at K = 4096 but 9.4 -> 9.8 at 2048 and 29.7 -> 30.4 at 8192.  X or A off a
+// dword stays with this file's kernel.
 static bool lf_xa_rings(const void* X, int M, int R, const LfSegTable& seg) {
   if (R > 32 || (seg.table ? (int64_t)seg.n_blocks * ROWS : M) > 256 * 16) return false;
   uintptr_t at = (uintptr_t)X;
