@@ -295,7 +295,8 @@ def kernel_breakdown(linears, reps: int):
                          "TFLOP/s": round(fl / (ms * 1e-3) / 1e12, 1)})
         del w, s, ds
     kern = ("gemm_big_kernel<bf16, NN, LoRA> (persistent 256x256 tiles)" if kinds == {7} else
-            "gemm_lora_kernel / gemm_big_kernel, NN (tile configurations %s)" % sorted(kinds))
+            "%s, NN (tile configurations %s)" % (" / ".join(sorted({"gemm_big_kernel" if c in (7, 8) else "gemm_mid_kernel" if c >= 10 else "gemm_lora_kernel"
+                                                                    for c in kinds})), sorted(kinds)))
     achieved = dom_flops / (dom_ms * 1e-3) / 1e12
     n = len(launches)
     roofline = {

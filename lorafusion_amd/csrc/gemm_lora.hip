@@ -805,7 +805,7 @@ static const TileCand kCands[] = {
     {8, 128, 256, 6.0, 35.4, 11.3, 36.5, 54.0, 23.4, 0.0, 0.0, 0.108},     // persistent, 4 waves of 64x128 (gemm_big.hip)
     // gemm_mid.hip: 4 waves of 96x64, 80x64, 64x64, 64x32.  Fitted to 10800 launches of 420 shapes (40 - 4100 rows, 512 - 14336 columns and
     // K) the same way: 6 - 8 % off.
-    {9, 192, 128, 7.3, 28.8, 5.2, 40.4, 50.8, 5.8, 2.0, 0.384, 0.040, true},
+    {13, 192, 128, 7.3, 28.8, 5.2, 40.4, 50.8, 5.8, 2.0, 0.384, 0.040, true},
     {10, 160, 128, 6.5, 25.4, 3.0, 36.5, 44.3, 1.6, 2.0, 0.386, 0.057, true},
     {11, 128, 128, 5.7, 22.0, 2.6, 31.3, 36.2, 3.4, 2.1, 0.364, 0.075, true},
     {12, 128, 64, 4.4, 14.5, 2.8, 20.4, 24.3, 1.9, 1.8, 0.402, 0.082, true},
@@ -821,8 +821,8 @@ static double launch_cost(const TileCand& c, int M, int N, int K, int slices = 1
   if (slices > 1) us += c.reduce + c.partial * (4e-6 * slices * M * N);
   return us;
 }
-static const TileCand& cand_of(int cfg, bool mid) {
-  for (const TileCand& c : kCands) if (c.cfg == cfg && (!c.mid || mid) && (c.cfg != 9 || c.mid == mid)) return c;
+static const TileCand& cand_of(int cfg) {
+  for (const TileCand& c : kCands) if (c.cfg == cfg) return c;
   return kCands[cfg == 2 ? 2 : 1];   // (the four-wave forms of these tiles, 0 and 2, are only run when pinned or for odd routing blocks)
 }
 // gemm_mid.hip takes whole tiles of columns, at least four K steps of 64 and routing blocks that a wave meets two of at most.
@@ -830,6 +830,7 @@ static bool mid_shape(const TileCand& c, int N, int K) { return N % c.bn == 0 &&
 // What a tile of gemm_mid.hip has to be ahead by in the model to be taken: in one round, in several, sliced.  The two models were
 // fitted apart and are 6 - 8 % off each.  Without: 64 of 840 products more than 3 % behind the plan before (worst 1.46 times), with: 15 (worst 1.1);
 // all of them together gain 8.6 % either way.
+// (A 192x128 tile that only the margin keeps with gemm_lora.hip runs here all the same: one tile, one kernel, but for what this one does not take.)
 static double mid_margin(long tiles, int slices) { return slices > 1 ? 1.06 : (tiles <= 256 ? 1.05 : 1.12); }
 // The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
 // (its 128-row tile and the other 256-column tiles leave most of the chip idle there); wave96: a 96-row wave meets at most two
@@ -846,13 +847,13 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, bool mid, doub
     if (c.cfg == 8 && (!big || tail || M < 128 || N < 256 || K < 256)) continue;
     if (c.cfg == 1 && (tail || (big && M >= 256 && N >= 256))) continue;
     if (c.cfg == 3 && tail) continue;
-    if (c.cfg == 9 && !c.mid && (!wave96 || tail)) continue;
-    if (c.mid && (!mid || !mid_shape(c, N, K) || (tail && c.cfg < 11))) continue;
+    if (c.cfg == 9 && (!wave96 || tail)) continue;
+    if (c.mid && (!mid || !mid_shape(c, N, K) || (tail && c.bm > 128))) continue;
     const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1) : 1.0);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;
-  return best;
+  return best == 9 && mid && mid_shape(cand_of(13), N, K) ? 13 : best;
 }
 // Rows [0, m_main) as 256x256 tiles, the rest as a second launch with the tile that spreads them best, when that beats
 // one launch (a nearly empty last round of big tiles costs a full tile time).  m_main is the multiple of 256 rows
@@ -891,7 +892,7 @@ struct KSplit { int cfg, n, steps; };
 static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
   const int nk = K / BK;
   KSplit best = {cfg, 1, nk};
-  const TileCand& planned = cand_of(cfg, mid);
+  const TileCand& planned = cand_of(cfg);
   if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
   double best_cost = launch_cost(planned, M, N, K) * (planned.mid ? mid_margin(tiles_of(M, N, planned), 1) : 1.0);
   const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
@@ -910,6 +911,7 @@ static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn
       if (used > 1 && cost < best_cost) { best_cost = cost; best = {c.cfg, used, steps}; }
     }
   }
+  if (best.n > 1 && best.cfg == 9 && mid && mid_shape(cand_of(13), N, K) && nk - (best.n - 1) * best.steps >= 8) best.cfg = 13;
   return best;
 }
 
@@ -920,7 +922,7 @@ static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool n
 
 static std::atomic<int> pinned_cfg{-1};
 int lf_pin_tile_cfg(int cfg) {
-  if (cfg < -1 || cfg == 9 || cfg > 12) return LF_EINVAL;
+  if (cfg < -1 || cfg == 9 || cfg > 13) return LF_EINVAL;
   pinned_cfg.store(cfg, std::memory_order_relaxed);
   return LF_OK;
 }
@@ -1027,7 +1029,7 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
       const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, rblock, nn, mid);
       if (ks.n > 1 && (size_t)ks.n * r.M * r.N * sizeof(float) <= r.ks_ws_bytes) { cfg = ks.cfg; r.ksplit = ks.n; r.ks_steps = ks.steps; }
     }
-    if (cfg >= 10 || (cfg == 9 && mid && mid_shape(cand_of(9, true), q.N, q.K) && (r.ksplit == 1 || q.K / BK - (r.ksplit - 1) * r.ks_steps >= 8))) {
+    if (cfg >= 10) {
       if (!mid) return (int)LF_ESHAPE;
       const int rc = lf_launch_gemm_mid(r, seg, nn, dtype, cfg, st);
       if (rc != LF_OK || r.ksplit <= 1) return rc;

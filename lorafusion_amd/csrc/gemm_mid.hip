@@ -563,7 +563,7 @@ int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, in
   if (seg.table != nullptr && seg.block_size_m % 128 != 0) return LF_ESHAPE;
   if (p.mask != nullptr && (!p.mask_bits || p.N % 32 != 0 || p.ldmask % 4 != 0)) return LF_ESHAPE;
   switch (cfg) {
-    case 9: return launch_mid_any<6, 4>(p, seg, nn, dtype, st);
+    case 13: return launch_mid_any<6, 4>(p, seg, nn, dtype, st);
     case 10: return launch_mid_any<5, 4>(p, seg, nn, dtype, st);
     case 11: return launch_mid_any<4, 4>(p, seg, nn, dtype, st);
     case 12: return launch_mid_any<4, 2>(p, seg, nn, dtype, st);

@@ -1,5 +1,5 @@
-"""GPU parity of the GEMM kernel for outputs of about one round (gemm_mid.hip) at its edges: its 160x128, 128x128 and 128x64 tiles are
-pinned (10, 11, 12; the 192x128 tile runs planned in test_gpu_plan.py), so that K loops of exactly four steps and a few more, ragged
+"""GPU parity of the GEMM kernel for outputs of about one round (gemm_mid.hip) at its edges: its 160x128, 128x128, 128x64 and
+192x128 tiles are pinned (10 to 13), so that K loops of exactly four steps and a few more, ragged
 rows, every kind of rank chunk, both 16-bit types, bias, and waves that lie across two adapters run against the CPU oracle.
 Tolerances as in test_gpu_lora_single.py / test_gpu_lora_multi.py."""
 
@@ -13,7 +13,7 @@ from tests.test_gpu_lora_single import _run_case as run_single
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(params=[10, 11, 12], ids=["160x128", "128x128", "128x64"])
+@pytest.fixture(params=[10, 11, 12, 13], ids=["160x128", "128x128", "128x64", "192x128"])
 def tile(request):
     from lorafusion_amd import _lib
 
@@ -42,7 +42,7 @@ def test_single(tile, M, K, N, r, p, scale):
 def test_rows_in_the_upper_half_of_the_last_tile(tile, K, bias):
     """The lower waves of the last tile have no rows and no LoRA term.  With K a multiple of 256 their (empty) skinny operand goes to the stage
     that the upper waves' results leave through."""
-    rows = {10: 160, 11: 128, 12: 128}[tile]
+    rows = {10: 160, 11: 128, 12: 128, 13: 192}[tile]
     run_single(rows + rows // 2 - 11, K, 512, 16, 0.1, 2.0, bias=bias)
 
 
