@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from oracle import lora_ref
+from tests.util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -13,6 +14,13 @@ pytestmark = pytest.mark.gpu
 def _close(got, exp, name):
     ok, rel, excess = lora_ref.check_close(got.detach().float().cpu(), exp, rtol=1e-2)
     assert ok, f"{name}: rel {rel:.3e} excess {excess:.3e}"
+
+
+def _direct(fn):
+    """What ``fn`` returns, from one launch: no second stage over partial sums."""
+    out, names = kernels_of(fn)
+    assert "lora_da_ring_kernel" in names and "reduce_segments_kernel" not in names, names
+    return out
 
 
 @pytest.mark.parametrize("M,K,r,dtype", [
@@ -28,10 +36,11 @@ def test_one_segment(M, K, r, dtype, p):
     keep = torch.rand(M, K, generator=g) >= p
     exp = ds.float().T @ torch.where(keep, x.float(), torch.zeros(())) / (1 - p)
     m = keep.cuda() if p else None
-    da = hip_ops.fused_lora_da(x.cuda(), ds.cuda(), r, p, hip_ops.pack_mask(m) if p else None)
+    xd, dsd, bits = x.cuda(), ds.cuda(), hip_ops.pack_mask(m) if p else None
+    da = _direct(lambda: hip_ops.fused_lora_da(xd, dsd, r, p, bits))
     _close(da, exp, "bits" if p else "no mask")
     if p:
-        assert torch.equal(da, hip_ops.fused_lora_da(x.cuda(), ds.cuda(), r, p, m))
+        assert torch.equal(da, _direct(lambda: hip_ops.fused_lora_da(xd, dsd, r, p, m)))
 
 
 @pytest.mark.parametrize("seq,ranks,p_list,K", [
@@ -59,5 +68,6 @@ def test_segments(seq, ranks, p_list, K):
         exp.append(ds[at:at + m, :r].float().T @ xs)
         at += pl
     mask = hip_ops.pack_mask(keep.cuda()) if any(p_list) else None
-    for i, got in enumerate(hip_ops.fused_multi_lora_da(x.cuda(), ds.cuda(), routing, mask)):
+    xd, dsd = x.cuda(), ds.cuda()
+    for i, got in enumerate(_direct(lambda: hip_ops.fused_multi_lora_da(xd, dsd, routing, mask))):
         _close(got, exp[i], f"adapter {i}")

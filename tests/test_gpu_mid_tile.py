@@ -9,6 +9,7 @@ import torch
 from oracle import lora_ref
 from tests.test_gpu_lora_multi import _run as run_multi
 from tests.test_gpu_lora_single import _run_case as run_single
+from tests.util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -106,19 +107,19 @@ def test_pinned_tile_refuses_what_it_does_not_take(tile):
 
 
 def test_skinny_operand_at_an_odd_address():
-    """B and A as views at a 2-byte offset: the direct loads of this kernel need 4, so the product runs on a tile that reads them lane by
-    lane (planned: 128x64 over one round)."""
+    """B and A as views at a 2-byte offset: the products run on a tile that reads them lane by lane, with them on a dword on this kernel's 128x64."""
     from lorafusion_amd.ops import hip_ops
 
     g = torch.Generator().manual_seed(3)
-    M, K, N, r = 300, 1024, 1024, 16
+    M, K, N, r = 600, 2048, 2048, 16
     x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), (torch.randn(N, K, generator=g) * 0.02).bfloat16().cuda()
     s = (torch.randn(M, r, generator=g) * 0.1).bfloat16().cuda()
     flat = (torch.randn(N * r + 1, generator=g) * 0.05).bfloat16().cuda()
     b, a = flat[1:].view(N, r), flat[1:].view(r, N)
     assert b.data_ptr() % 4 == 2
-    y = hip_ops.fused_lora_xw_sb(x, w, s, b, 2.0)
-    dx = hip_ops.fused_lora_dyw_dsa(x, w, s, a, 0.0)
+    for side, kernel in (((b.clone(), a.clone()), "gemm_mid_kernel"), ((b, a), "gemm_lora_kernel")):   # (a copy lies on a dword)
+        (y, dx), names = kernels_of(lambda: (hip_ops.fused_lora_xw_sb(x, w, s, side[0], 2.0), hip_ops.fused_lora_dyw_dsa(x, w, s, side[1], 0.0)))
+        assert [k for k in ("gemm_mid_kernel", "gemm_lora_kernel") if k in names] == [kernel], names
     for got, exp, name in ((y, x.float() @ w.float().T + 2.0 * s.float() @ b.float().T, "y"), (dx, x.float() @ w.float() + s.float() @ a.float(), "dx")):
         ok, rel, excess = lora_ref.check_close(got.float().cpu(), exp.cpu(), rtol=1e-2)
         assert ok, f"{name}: rel {rel:.3e} excess {excess:.3e}"

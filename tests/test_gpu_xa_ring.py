@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from oracle import lora_ref
+from tests.util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -16,17 +17,23 @@ def _close(got, exp):
     assert ok, f"rel {rel:.3e} excess {excess:.3e}"
 
 
-@pytest.mark.parametrize("M,K,r,dtype", [(1, 128, 8, torch.bfloat16), (15, 640, 16, torch.float16), (17, 1152, 24, torch.bfloat16), (333, 3968, 32, torch.bfloat16), (513, 4096, 32, torch.bfloat16),
-                                         (333, 4096, 32, torch.float16), (100, 8192, 16, torch.bfloat16), (1025, 8320, 8, torch.float16),
-                                         (4095, 256, 32, torch.bfloat16), (4097, 256, 16, torch.bfloat16)])
-def test_xa_ring(M, K, r, dtype):
+RING, SLICED, GENERAL = "lora_xa_ring_kernel", "lora_stream_kernel", "lora_xa_kernel"
+
+
+@pytest.mark.parametrize("M,K,r,dtype,kernel", [
+    (1, 128, 8, torch.bfloat16, RING), (15, 640, 16, torch.float16, RING), (17, 1152, 24, torch.bfloat16, RING), (333, 3968, 32, torch.bfloat16, RING),
+    (513, 4096, 32, torch.bfloat16, RING), (333, 4096, 32, torch.float16, SLICED), (100, 8192, 16, torch.bfloat16, RING), (100, 8320, 16, torch.bfloat16, SLICED),
+    (1025, 8320, 8, torch.float16, RING), (1000, 8192, 24, torch.bfloat16, SLICED), (4095, 256, 32, torch.bfloat16, RING), (4097, 256, 16, torch.bfloat16, GENERAL)])
+def test_xa_ring(M, K, r, dtype, kernel):
     from lorafusion_amd import _lib as L
     from lorafusion_amd.ops import hip_ops
 
     g = torch.Generator().manual_seed(M + r)
     x, a = torch.randn(M + 1, K, generator=g).to(dtype), (torch.randn(r + 1, K, generator=g) * K ** -0.5).to(dtype)
     x[M], a[r] = float("nan"), float("nan")   # what lies beyond the operands must not reach the result
-    s = hip_ops._xa(x.cuda()[:M], None, [a.cuda()[:r]], L.single_routing(r, 2.0, 0.0), M, K, L.round_rank(r))
+    xd, ad = x.cuda()[:M], a.cuda()[:r]
+    s, names = kernels_of(lambda: hip_ops._xa(xd, None, [ad], L.single_routing(r, 2.0, 0.0), M, K, L.round_rank(r)))
+    assert [k for k in (RING, SLICED, GENERAL) if k in names] == [kernel], names
     _close(s[:, :r], x[:M].double() @ a[:r].double().t())
     assert not s[:, r:].any()
 
@@ -42,7 +49,9 @@ def test_xa_ring_packed(seq, ranks, K):
     g = torch.Generator().manual_seed(n)
     x = torch.randn(routing.M, K, generator=g).bfloat16()
     a = [(torch.randn(r, K, generator=g) * K ** -0.5).bfloat16() for r in ranks]
-    s = hip_ops._xa(x.cuda(), None, [t.cuda() for t in a], routing.c, routing.M, K, routing.R)
+    xd, ad = x.cuda(), [t.cuda() for t in a]
+    s, names = kernels_of(lambda: hip_ops._xa(xd, None, ad, routing.c, routing.M, K, routing.R))
+    assert RING in names, names
     row = 0
     for q, pl, r, at in zip(seq, info.padded_seq_len_list, ranks, a):
         _close(s[row:row + q, :r], x[row:row + q].double() @ at.double().t())

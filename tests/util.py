@@ -23,6 +23,17 @@ def single_inputs(M, K, N, r, p=0.1, seed=0, dtype=torch.bfloat16, bias=False):
     return dict(x=x, w=w, a=a, b=b, dy=dy, mask=mask, bias=bias_t)
 
 
+def kernels_of(fn):
+    """(what ``fn()`` returns, the names of the GPU kernels it ran, as one text)."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, " ".join(e.key for e in prof.key_averages())
+
+
 def lognormal_segments(total_tokens, n_adapters, seed=0, mu=6.5, sigma=0.8, lo=64, hi=4096):
     """Lengths ~ lognormal clipped to [lo, hi], drawn until they sum to total_tokens (last one
     truncated), dealt round-robin to the adapters; returns tokens per adapter."""
