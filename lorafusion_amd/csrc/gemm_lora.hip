@@ -880,6 +880,13 @@ static int choose_split(int M, int N, int K, bool allow_big, bool wave96, bool m
   return best_m;
 }
 
+// ... and what an unsplit round of it has to be ahead of slices by, beyond that margin, over a long K: there the model says too little for it (NT: 11 % at
+// K = 8192, 16 % at 13000; NN: 7 % to 20000, 17 % beyond) and not for the large tiles in slices.  Forward + backward of 1000 shapes, launches traced
+// against the plans before gemm_mid.hip: of 314 NT products of one round 22 were more than 3 % slower (1408 x 2176 over 13312: 97 -> 118 us, 638 x 4864 over
+// 13568: 91 -> 126), of 418 NN products 10 (1468 x 2176 over 25728: 190 -> 220); without those that this sends back to slices 7 and 3 remain, and all of them
+// together are another 0.6 % and 0.05 % faster (400 shapes that were not fitted: 15 of 539 products more than 3 % slower, all together 9 % faster).
+static double mid_long_k(long tiles, int K, bool nn) { return tiles > 256 ? 0.0 : (nn ? 0.02 * std::max(0, K - 16384) : 0.015 * std::max(0, K - 4096)) / 1024; }
+
 // Split contraction for launches that leave compute units idle over a long K (left-over rows of a packed batch, short
 // batches): K is cut into slices, workgroup (tile, slice) keeps fp32 sums, a second kernel adds the slices.  Larger tiles
 // move fewer operand bytes per product, and a compute unit takes in at most about 100 GB/s whatever its tile, so many slices of
@@ -894,7 +901,8 @@ static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn
   KSplit best = {cfg, 1, nk};
   const TileCand& planned = cand_of(cfg);
   if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
-  double best_cost = launch_cost(planned, M, N, K) * (planned.mid ? mid_margin(tiles_of(M, N, planned), 1) : 1.0);
+  double best_cost = launch_cost(planned, M, N, K);
+  if (const long tiles = tiles_of(M, N, planned); planned.mid) best_cost *= mid_margin(tiles, 1) + mid_long_k(tiles, K, nn);
   const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
   for (const TileCand& c : kCands) {
     if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import lora_ref
-from tests.util import single_inputs
+from tests.util import kernels_of, single_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -135,3 +135,28 @@ def test_tile_and_slices_together(M, K, N, slices, dtype):
     term = ds[:, :r].float() @ at.float() / (1 - p)
     _close(dx, (x.float() @ wt.float() + torch.where(hip_ops.unpack_mask(bits), term, torch.zeros_like(term))).cpu(), "dx")
     assert float((dx.float() - dx1.float()).abs().max()) <= float(dx1.float().abs().max()) * step
+
+
+@pytest.mark.parametrize("M,N,K,nn,sliced", [
+    (1408, 2176, 13312, False, True), (638, 4864, 13568, False, True), (1468, 2176, 25728, True, True),   # slices of 256x256 and 128x256 tiles
+    (1921, 1920, 8576, False, False), (1408, 2176, 4224, True, False), (1408, 2176, 13312, True, False)])
+def test_one_round_over_a_long_contraction(M, N, K, nn, sliced):
+    """Products of one round of 128x128 tiles: cut into slices of larger tiles where K is long, earlier for Y = X W^T than for dX = dY W."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    r, g = 16, torch.Generator(device="cuda").manual_seed(M + K)
+    randn = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    routing, R = L.single_routing(r, 2.0, 0.0), L.round_rank(r)
+    x, w = randn(M, K), randn(N, K, std=0.02)
+    a, b = randn(r, K, std=K ** -0.5), randn(N, r, std=0.05)
+    if not nn:
+        (got, s), names = kernels_of(lambda: hip_ops.lora_forward(x, w, [a], [b], routing, R, None, None))
+        exp = x.float() @ w.float().T + 2.0 * s[:, :r].float() @ b.float().T
+    else:   # x in the place of dY, w^T in the place of W: dX [M, N] over K
+        wt, at, bt, xs, s = w.T.contiguous(), b.T.contiguous(), a.T.contiguous(), randn(M, N), randn(M, R, std=0.1)
+        (got, _, _), names = kernels_of(lambda: hip_ops.lora_backward(x, xs, wt, [at], [bt], s, routing, R, None, [r]))
+        ds = hip_ops.fused_lora_dys_dyb(x, bt, s, 2.0)[1]
+        exp = x.float() @ wt.float() + ds[:, :r].float() @ at.float()
+    assert ("ksplit_reduce_kernel" in names) == sliced and ("gemm_mid_kernel" in names) != sliced, names
+    _close(got, exp.cpu(), "dX" if nn else "Y")
