@@ -8,7 +8,8 @@
 //
 // What bounds it: the path into a compute unit's LDS.  A unit takes in 100 - 130 GB/s of direct loads, whatever the number of stages in
 // flight beyond two (four here; five and six measured level) -- a loads-only loop over the tiles of 300 x 4096 x 4096 takes 17 us, the
-// kernel 19 on warm weights -- and the MFMAs of a 160x128 tile take about as long as its loads.  Hence:
+// kernel 19 on warm weights -- and the MFMAs of a 160x128 tile take about as long as its loads.  (Where a large weight comes from HBM, the reads from there:
+// loads alone over the tiles of 333 x 14336 x 4096 take 45 us cold and 29 warm, the kernel 46 - 50.)  Hence:
 //  * whole 128-byte lines per load (K steps of 64), one every few MFMAs over the whole step: gemm_lora.hip's four-wave tiles load
 //    half lines in pairs, all of them in every second step of 32, more than the texture addresser takes there;
 //  * the LoRA term behind the K loop: its rows of L and keep bits come into registers while the first tiles land, its skinny operand
