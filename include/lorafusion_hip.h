@@ -201,21 +201,21 @@ int lf_gemm(const void* A, const void* B, const void* bias, void* C, int M, int 
             int tile_cfg, void* stream);
 
 /* Tile configuration of every later MFMA GEMM launch of this process that does not name one itself
- * (the fused entry points, lf_gemm with tile_cfg = -1): 0..8 or 10..13 pins it, -1 (the initial state)
+ * (the fused entry points, lf_gemm with tile_cfg = -1): 0..8 or 10..15 pins it, -1 (the initial state)
  * returns to the library's own choice.  A process-wide setting meant for tests and tuning runs --
  * parity of every tile shape at small sizes; the reference has the same kind of knob in the
  * Triton autotune configs of its kernels (lorafusion/ops/triton_ops/config.py).  A launch whose
  * shape the pinned configuration cannot take fails with LF_ESHAPE (7, the persistent kernel's
  * 256x256 tile, needs M, N >= 256 and K >= 128; 8, its 128x256 tile, M >= 128, N >= 256 and
- * K >= 256; 10 = 160x128, 11 = 128x128, 12 = 128x64 and 13 = 192x128 of the kernel for outputs of about one round need whole tiles of columns,
- * K >= 256 and bit-packed keep-masks).  Returns LF_EINVAL for 9 and outside -1..13. */
+ * K >= 256; 10 = 160x128, 11 = 128x128, 12 = 128x64, 13 = 192x128, 14 = 96x64 and 15 = 64x64 of the kernel for outputs of about one round need whole tiles of columns,
+ * K >= 256 and bit-packed keep-masks).  Returns LF_EINVAL for 9 and outside -1..15. */
 int lf_set_tile_cfg(int tile_cfg);
 
 /* The launches the library makes for an M x N output contracted over K when no configuration is pinned: rows
  * [0, *rows_head) as one launch of tile configuration *cfg_head and, when *rows_head < M, the rest
  * as a second launch of *cfg_tail (-1 when there is none).  Every number names one kernel and tile: 4, 6 and 9 are the 128x128, 128x64 and
- * 192x128 tiles of the general kernel, 11, 12 and 13 those of the kernel for outputs of about one round.  A launch may still move to another tile: a call whose
- * keep-mask or rank the persistent kernel (7, 8) does not take, or whose keep-mask (one byte per element) the kernel for about one round (10..13) does not,
+ * 192x128 tiles of the general kernel, 11, 12 and 13 (with 10, 14 and 15) those of the kernel for outputs of about one round.  A launch may still move to another tile: a call whose
+ * keep-mask or rank the persistent kernel (7, 8) does not take, or whose keep-mask (one byte per element) the kernel for about one round (10..15) does not,
  * goes to the best of the others, and a launch that leaves compute units idle over a long K is cut into slices.  routing_block_size_m: 0 for a
  * single-adapter call, else the routing block size.  For benchmarks that time one kernel of a
  * fused call on its own; no counterpart in the reference (Triton's autotuner picks there). */

@@ -21,6 +21,15 @@
 //
 // One workgroup per tile of 32 TI x 32 TJ, four waves of 16 TI x 16 TJ (16x16x32 MFMA blocks, accumulators in the accumulation
 // registers, the loop's memory instructions in assembly: see gemm_big.hip for the reasons).
+//
+// Tiles of up to 128x128 leave room in the register file for four waves more (LOADERS), which do nothing but load.  A wave that does both stops multiplying
+// while the texture addresser, which four waves' loads keep 60 - 80 % busy, takes its next load; the loading waves stop in its place, and they order a
+// stage's loads as soon as it is free.  Cold weights, rank-16 term, us, NT / NN: 300 x 4096 x 4096 on 128x64 22.1 / 22.9 -> 21.2 / 21.3; 1024 x 4096 x 4096
+// on 128x128 34.9 / 38.1 -> 33.2 / 36.0; 600 x 4096 x 4096 28.8 / 30.8 -> 27.7 / 28.1.  (160x128 and 192x128 would spill at 256 registers a wave.  Measured
+// level: fragments waited for by count and a barrier behind the first MFMAs of a half, other priorities; slower: the two halves of a step on
+// two sets of four waves.)
+// The 96x64 and 64x64 tiles move fewer operand bytes per compute unit where a few hundred rows do not fill a round with larger ones: 300 x 4096 x 4096
+// on 96x64 (256 tiles) 19.7 / 19.6, 500 x 2048 x 4096 20.6 / 21.0 (128x64) -> 17.7 / 17.6.
 #include "lf_common.h"
 #include <type_traits>
 #include <utility>
@@ -85,24 +94,27 @@ template <int TI, int TJ> struct MidLds {
   static constexpr int STAGE = (TI + TJ) * 4096;   // bytes: (32 TI + 32 TJ) rows of 128
   static constexpr int NST = 4;
   static constexpr int BYTES = NST * STAGE;
+  static constexpr bool LOADERS = TI * TJ <= 16;   // four waves more, which only load
+  static constexpr int THREADS = LOADERS ? 512 : 256;
   static_assert(BYTES <= 160 * 1024, "stages fit the LDS of a CU");
 };
 
 template <typename T, bool NN, int TI, int TJ>
-__global__ void __launch_bounds__(256, 1)
+__global__ void __launch_bounds__((MidLds<TI, TJ>::THREADS), 1)
 gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub (buffer-resource types are device-only)
   using std::integral_constant;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr int BM = TI * 32, BN = TJ * 32, WROWS = TI * 16, WCOLS = TJ * 16;
   constexpr int STAGE = MidLds<TI, TJ>::STAGE, NST = MidLds<TI, TJ>::NST, STAGE_A = TI * 4096;
-  constexpr int NL = TI + TJ;          // tile loads per wave and step
+  constexpr bool LOADERS = MidLds<TI, TJ>::LOADERS;
+  constexpr int NL = TI + TJ;          // tile loads per (loading) wave and step
   constexpr int NLH = (NL + 1) / 2;    // of which in the first sub-step
   constexpr int NM = TI * TJ;          // MFMAs per wave and sub-step
   constexpr int LDP = NM / NLH;        // a tile load every LDP MFMAs
   static_assert(LDP >= 2 && NL <= NM, "a sub-step has a gap for every fragment read and two for every tile load");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (among those that multiply, or among those that load)
   const int wm = wave >> 1, wn = wave & 1;
 
   // ---- tile: XCD-aware order, grouped along M (a split contraction: slice by slice)
@@ -193,7 +205,38 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
     __builtin_amdgcn_sched_barrier(0);
   };
   // (nk >= NST: the launcher's condition)
-  sfor<NST - 1>([&](auto I) { load_stage(I.value, I); });
+  if constexpr (LOADERS) {
+    if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) != 0) {
+      // The loading waves keep NST - 1 steps on order.  Barrier of step s: step s+1 has landed and every multiplying wave has read all of
+      // step s, whose stage takes step s+NST.  They end behind the last step's barrier with nothing in flight; later barriers are the other waves' own.
+      sfor<NST>([&](auto I) { load_stage(I.value, I); });
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * NL) : "memory");
+      barrier();
+      uint32_t st = 0;
+      for (int s = 0; s + NST < nk; s++) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * NL) : "memory");
+        barrier();
+        int ka, kb;
+        kbase(s + NST, ka, kb);
+        const uint32_t mb = m0w + st;
+        sfor<NL>([&](auto I) {
+          set_m0(mb, integral_constant<int, I.value * 4096>{});
+          asm volatile("s_nop 0" ::: "memory");
+          issue_load(I.value < TI ? ra : rb, voff[I.value], I.value < TI ? ka : kb);
+        });
+        st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+      }
+      sfor<NST - 1>([&](auto I) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2 - I.value) * NL) : "memory");
+        barrier();
+      });
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      barrier();
+      return;
+    }
+  } else {
+    sfor<NST - 1>([&](auto I) { load_stage(I.value, I); });
+  }
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- LoRA term: adapters of the wave's rows.  A wave's rows meet at most two routing blocks (their size is a multiple
@@ -361,7 +404,7 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
       sfor<NM>([&](auto MM) {
         constexpr int m = MM.value;
         if constexpr (READ.value && m < NL) read_one(integral_constant<int, 1 - set>{}, integral_constant<int, 1 - set>{}, rst, MM);
-        if constexpr (LOAD.value && m / LDP < COUNT.value) {
+        if constexpr (!LOADERS && LOAD.value && m / LDP < COUNT.value) {
           constexpr int idx = BASE.value + m / LDP;
           if constexpr (m % LDP == 0) set_m0(mb, integral_constant<int, idx * 4096>{});
           if constexpr (m % LDP == 1) issue_load(idx < TI ? ra : rb, voff[idx], idx < TI ? ka : kb);
@@ -371,7 +414,7 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
       });
     };
     half(S0{}, T_{}, cur, integral_constant<int, 0>{}, integral_constant<int, NLH>{}, FIRST);
-    if constexpr (WAIT.value >= 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT.value) : "memory");
+    if constexpr (!LOADERS && WAIT.value >= 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT.value) : "memory");
     barrier();
     half(S1{}, NEXT, nxt, integral_constant<int, NLH>{}, integral_constant<int, NL - NLH>{}, F_{});
     __builtin_amdgcn_sched_barrier(0);
@@ -381,7 +424,7 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
   };
   constexpr int INFLIGHT = (NST - 3) * NL + NLH;
   static_assert(NST >= 4 && (NST - 2) * NL + 2 * TJ < 64, "vmcnt is a 6-bit counter");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * NL) : "memory");
+  if constexpr (!LOADERS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * NL) : "memory");
   barrier();
   sfor<NL>([&](auto I) { read_one(S0{}, S0{}, 0u, I); });
   lgkm0();
@@ -544,7 +587,7 @@ int launch_mid(LfGemmParams p, const LfSegTable& seg, hipStream_t st) {
   auto kern = gemm_mid_kernel<T, NN, TI, TJ>;
   static LfLdsFlags lds_ok;
   if (!lf_allow_lds(kern, MidLds<TI, TJ>::BYTES, lds_ok)) return LF_ELAUNCH;
-  return lf_launch(kern, dim3(p.grid_m * p.grid_n, p.ksplit > 1 ? p.ksplit : 1), dim3(256), MidLds<TI, TJ>::BYTES, st, p, seg);
+  return lf_launch(kern, dim3(p.grid_m * p.grid_n, p.ksplit > 1 ? p.ksplit : 1), dim3(MidLds<TI, TJ>::THREADS), MidLds<TI, TJ>::BYTES, st, p, seg);
 }
 
 template <int TI, int TJ>
@@ -558,7 +601,7 @@ int launch_mid_any(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
 
 int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int cfg, hipStream_t st) {
   // whole tiles along N; at least as many K steps as stages, in the last slice of a split contraction too
-  if (p.K % BK != 0 || p.M < 1 || p.N % (cfg == 12 ? 64 : 128) != 0 || p.R > LF_MAX_RANK) return LF_ESHAPE;
+  if (p.K % BK != 0 || p.M < 1 || p.N % (cfg == 12 || cfg >= 14 ? 64 : 128) != 0 || p.R > LF_MAX_RANK) return LF_ESHAPE;
   if (p.ksplit > 1 && p.ks_steps % 2 != 0) return LF_ESHAPE;
   if ((p.ksplit > 1 ? p.K / BK - (p.ksplit - 1) * (p.ks_steps / 2) : p.K / BK) < 4) return LF_ESHAPE;
   if (seg.table != nullptr && seg.block_size_m % 128 != 0) return LF_ESHAPE;
@@ -568,6 +611,8 @@ int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, in
     case 10: return launch_mid_any<5, 4>(p, seg, nn, dtype, st);
     case 11: return launch_mid_any<4, 4>(p, seg, nn, dtype, st);
     case 12: return launch_mid_any<4, 2>(p, seg, nn, dtype, st);
+    case 14: return launch_mid_any<3, 2>(p, seg, nn, dtype, st);
+    case 15: return launch_mid_any<2, 2>(p, seg, nn, dtype, st);
     default: return LF_EINVAL;
   }
 }

@@ -73,7 +73,7 @@ __device__ __forceinline__ int lf_xcd_order(int id, int total) {
 // launchers (one per translation unit)
 int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int force_cfg, hipStream_t st);
 int lf_launch_gemm_big(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int tile_rows, hipStream_t st);  // persistent tiles of 256 or 128 rows x 256 columns
-int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int cfg, hipStream_t st);  // about one round: 160x128 (10), 128x128 (11), 128x64 (12), 192x128 (13)
+int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int cfg, hipStream_t st);  // about one round: 160x128 (10), 128x128 (11), 128x64 (12), 192x128 (13), 96x64 (14), 64x64 (15)
 int lf_cu_count();
 int lf_pin_tile_cfg(int cfg);  // -1: automatic choice
 bool lf_tile_pinned();
