@@ -21,6 +21,10 @@ size_t lf_xa_workspace(int, int, int, const LfSegTable&);
 // limit: bytes the split of the pass is to stay within, where one does (a call and its size query name the same)
 size_t lf_dys_dyb_workspace(int, int, int, const LfSegTable&, size_t limit = SIZE_MAX);
 size_t lf_da_workspace(int, int, int, const LfSegTable&, size_t limit = SIZE_MAX);
+size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable&);
+bool lf_short_grads_apply(const void*, const void*, const uint8_t*, int, const void*, const void*, const void*, size_t, size_t, int M, int N, int K, int R, const LfSegTable&,
+                          const LfSegTable&);
+int lf_launch_short_grads(const void*, const void*, const uint8_t*, int, const void*, void*, void*, int M, int N, int K, int R, const LfSegTable&, const LfSegTable&, int, hipStream_t);
 
 // Scratch of lf_lora_bwd_static: part of the device image, one copy per GPU at its own address.  In
 // host code the array's name is only a handle for hipGetSymbolAddress; kernels and launch code
@@ -144,12 +148,12 @@ size_t lf_workspace_bytes(int op, int M, int N, int K, int R, const lf_routing* 
     // (the products of the whole-pass entry points may split their contraction: Y = [M,N] over K, dX = [M,K] over N)
     case LF_OP_FWD: return align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_BWD: {
-      size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
+      size_t a = std::max(lf_dys_dyb_workspace(M, N, R, t), lf_short_grads_workspace(M, N, K, R, t)), b = lf_da_workspace(M, K, R, t);
       return align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb, true)));
     }
     case LF_OP_NF4_FWD: return align256((size_t)N * K * 2) + align256(fwd_workspace(M, N, K, R, rb, t));
     case LF_OP_NF4_BWD: {
-      size_t a = lf_dys_dyb_workspace(M, N, R, t), b = lf_da_workspace(M, K, R, t);
+      size_t a = std::max(lf_dys_dyb_workspace(M, N, R, t), lf_short_grads_workspace(M, N, K, R, t)), b = lf_da_workspace(M, K, R, t);
       return align256((size_t)N * K * 2) + align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, rb, true)));
     }
     default: return 0;
@@ -349,7 +353,17 @@ int lf_lora_fwd_seeded(const void* X, const void* W, const void* bias, uint8_t* 
 static int bwd_within(const void* dY, const void* X, const void* W, const uint8_t* mask, const void* S, const void* const* a_ptrs,
                       const void* const* b_ptrs, void* dX, void* const* da_ptrs, void* const* db_ptrs, void* dS_out, void* workspace, size_t ws_bytes,
                       size_t limit, int M, int N, int K, int R, const lf_routing* routing, int dtype, void* stream) {
-  int rc = dys_dyb_within(dY, S, b_ptrs, dS_out, db_ptrs, workspace, ws_bytes, limit, M, N, R, routing, dtype & ~LF_MASK_BITS, stream);
+  LfSegTable sb, sg;
+  int rc;
+  if (!bad_dtype(dtype & ~LF_MASK_BITS) && b_ptrs && da_ptrs && db_ptrs && make_seg(routing, M, b_ptrs, nullptr, sb) == LF_OK &&
+      make_seg(routing, M, (const void* const*)db_ptrs, da_ptrs, sg) == LF_OK &&
+      lf_short_grads_apply(dY, X, mask, (dtype & LF_MASK_BITS) != 0, S, dS_out, workspace, ws_bytes, limit, M, N, K, R, sb, sg)) {
+    rc = lf_launch_short_grads(dY, X, mask, (dtype & LF_MASK_BITS) != 0, S, dS_out, workspace, M, N, K, R, sb, sg, dtype & ~LF_MASK_BITS, (hipStream_t)stream);
+    if (rc != LF_OK) return rc;
+    // (stream order: dS's slices are consumed by now, so the product's split contraction may reuse the workspace from its start)
+    return dX ? dyw_dsa_ws(dY, W, dS_out, a_ptrs, mask, dX, workspace, ws_bytes, M, N, K, R, routing, dtype, stream) : LF_OK;
+  }
+  rc = dys_dyb_within(dY, S, b_ptrs, dS_out, db_ptrs, workspace, ws_bytes, limit, M, N, R, routing, dtype & ~LF_MASK_BITS, stream);
   if (rc != LF_OK) return rc;
   rc = da_within(X, mask, dS_out, da_ptrs, workspace, ws_bytes, limit, M, K, R, routing, dtype, stream);
   if (rc != LF_OK) return rc;

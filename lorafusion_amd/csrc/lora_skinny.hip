@@ -534,7 +534,7 @@ static int all_group_stats(const int* blocks, int nseg, GroupStats (&st)[kNGroup
 constexpr int dysr_tpw(int rt) { return rt >= 8 ? 4 : rt >= 2 ? 12 : 16; }   // dB accumulators: TPW * RT * 4 registers, next to 8 * RT of dS
 constexpr int dysr_ns(int rt) { return rt == 4 ? 5 : 3; }   // (rank 128: three stages of 32 KB and two S blocks of 32 KB are all of the LDS)
 static int dysr_smem(int rt) { return dysr_ns(rt) * (TILE_BYTES + (rt >= 2 ? rt / 2 : 1) * 4096) + 2 * ROWS * rt * 32; }
-struct DysRingPlan { int n_slices, group, max_chunks; };
+struct DysRingPlan { int n_slices, group, max_chunks; double cost; };   // cost: as DaPlan's
 // By bytes: the dY (+ B tile) stream over the busiest slot, the S blocks every workgroup fetches (from L2: half weight),
 // and the fp32 partials written here and read by the reduce (dS: one [rows, R] slab per slice; dB: one [N, R] slab per
 // chunk).  The cheapest plan whose partials take at most `limit` bytes (if none does: the cheapest of all).
@@ -543,7 +543,7 @@ static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   const int slots = lds_slots(dysr_smem(rt));
   const double tile_bytes = TILE_BYTES + 64.0 * R * 2;
-  DysRingPlan best{1, 1, 1};
+  DysRingPlan best{1, 1, 1, 1e300};
   if (T < 2) return best;   // fewer than two column tiles: nothing to split (and no division by a zero slice count)
   GroupStats stats[kNGroups];
   const int ng = all_group_stats(blocks, nseg, stats);
@@ -557,7 +557,7 @@ static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg
       const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
                           2.0 * 4.0 * R * ((double)nsl * rows + (double)st.chunks * N);
       const bool fits = ((size_t)nsl * rows * R + (size_t)nseg * st.max_chunks * N * R) * sizeof(float) <= limit;
-      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks}; }
+      if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks, cost}; }
     }
   }
   return best;
@@ -815,25 +815,28 @@ size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit)
 // With keep bits, two-stage -> direct: 300 x 4096 rank 16 8.8 -> 7.8, four segments of 1280 x 4096 rank 64 14.7 -> 9.3, of 2048 x 4096 rank 16
 // 13.3 -> 10.5; the other side of the line: 1000 x 4096 rank 16 in one segment 9.7 against 14.4.
 // (the same choice for every mask format: dA does not depend on how the mask came)
-static int da_direct_slices(int M, int K, int R, bool masked, const LfSegTable& seg, size_t limit) {
+struct DaForm { int direct_slices; double us; };   // 0: two stages
+static DaForm da_form(int M, int K, int R, bool masked, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = K / 64;
-  if (T < 2) return 0;
+  const double m = masked, two_stage = T < 2 ? 0.0 : 4.85 + 3.5 * m + da_plan(M, K, R, masked ? 2 : 0, seg, limit).cost / 5.39e6;
+  const DaForm staged{0, two_stage};
+  if (T < 2) return staged;
   int blocks[LF_MAX_SEG], nseg, live = 0, big = 0;
   seg_block_counts(M, seg, blocks, nseg);
   for (int s = 0; s < nseg; s++) live += blocks[s] > 0, big = std::max(big, blocks[s]);
-  if (live == 0) return 0;
+  if (live == 0) return staged;
   int t = rt == 8 ? 2 : 1;   // (with a mask the ring holds three stages at least: two dS buffers allow t + 1)
   while (t <= da_tpw(rt) && ((T + t - 1) / t) * live > 256) t++;   // one round of workgroups
-  if (t > da_tpw(rt)) return 0;
+  if (t > da_tpw(rt)) return staged;
   const int nsl = (T + t - 1) / t;
-  const double m = masked, tiles = (double)big * t;
+  const double tiles = (double)big * t;
   const double direct = 3.66 + 0.40 * m + 0.20 * rt + tiles * (0.305 + 0.466 * m + 0.049 * rt) + 0.357 * big + 0.9e-3 * tiles * nsl * live;
-  return 1.05 * direct < 4.85 + 3.5 * m + da_plan(M, K, R, masked ? 2 : 0, seg, limit).cost / 5.39e6 ? nsl : 0;
+  return 1.05 * direct < two_stage ? DaForm{nsl, direct} : staged;
 }
 
 // (lora_da_direct.hip)  mask_fmt: the kernel's MASK
-int lf_launch_da_direct(const void* X, const uint8_t* mask, int mask_fmt, const void* dS, int M, int K, int R, int n_slices, const LfSegTable& seg, int dtype,
-                        hipStream_t st);
+int lf_launch_da_direct(const void* X, const uint8_t* mask, int mask_fmt, const void* dS, int M, int K, int R, int n_slices, const LfSegTable& seg, const void* dY,
+                        const void* S, int N, int n_slices_b, int dtype, hipStream_t st);
 
 template <typename T, int RT, int MASK>
 static int da_ring_launch(const void* X, const uint8_t* mask, const void* dS, float* part, int M, int K, int R, const DaPlan& pl,
@@ -843,7 +846,7 @@ static int da_ring_launch(const void* X, const uint8_t* mask, const void* dS, fl
   static LfLdsFlags lds_ok;
   if (!lf_allow_lds(kern, smem, lds_ok)) return LF_ELAUNCH;
   return lf_launch(kern, dim3(pl.n_slices, pl.max_chunks, nseg), dim3(256), smem, st, (const T*)X, mask, (const T*)dS, part, M, K, R,
-                   pl.n_slices, pl.group, pl.max_chunks, seg);
+                   pl.n_slices, pl.group, pl.max_chunks, seg, DbOperands{});
 }
 
 template <typename T>
@@ -854,8 +857,9 @@ static int da_impl(const void* X, const uint8_t* mask, int mask_bits, const void
   int rc;
   const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : 1;
   const bool off_grid = fmt == 1 && mask_off_grid(mask, 0);   // (the same split, and the same sums)
-  if (const int nsl = da_direct_slices(M, K, R, mask != nullptr, seg, limit))
-    return lf_launch_da_direct(X, mask, off_grid ? 3 : fmt, dS, M, K, R, nsl, seg, std::is_same_v<T, __bf16> ? LF_BF16 : LF_F16, st);
+  if (const int nsl = da_form(M, K, R, mask != nullptr, seg, limit).direct_slices)
+    return lf_launch_da_direct(X, mask, off_grid ? 3 : fmt, dS, M, K, R, nsl, seg, nullptr, nullptr, 0, 0,
+                               std::is_same_v<T, __bf16> ? LF_BF16 : LF_F16, st);
   const DaPlan pl = da_plan(M, K, R, fmt, seg, limit);
 #define LF_DA_RING(RTV)                                                                                                   \
   rc = off_grid   ? da_ring_launch<T, RTV, 3>(X, mask, dS, part, M, K, R, pl, nseg, seg, st)                              \
@@ -891,3 +895,69 @@ int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* 
   return LF_EINVAL;
 }
 
+
+// ---- the rank-r part of a short backward in two or three launches: dS on its own (complete, lora_stream.hip), then dA and dB side by side as sums over rows
+// (lora_da_direct.hip), where dys_dyb and da take three to five.  dY is read twice; what goes is the fp32 partials of dS and dB, their second stage and the walk of
+// da behind that of dys_dyb.  Behind where one workgroup walks many blocks (a tile costs it 0.4 us, with a mask 0.9).
+// Both sides in microseconds, fitted to 1250 backwards without the dX product (60 - 6000 rows in 1 - 8 segments, N 1024 - 14336, K 1024 - 8192, ranks 8 - 128, with keep
+// bits and without; 10 % off each) and checked on 540 more: the choice takes 0.89 of the old way's time over them, 0.876 is the least any choice takes, 30 are
+// more than 3 % slower (worst 1.25).  With keep bits, replayed from a graph: 300 x 4096 x 4096 rank 16 16.7 -> 13.0, four segments of 1280 rows rank 64 31.7 -> 24.2, 788 x 2944 x
+// 3328 rank 64 28.5 -> 23.2; the other side of the line: 2048 x 4096 x 4096 rank 16 28.0 against 31.1, 3000 x 5120 x 5120 rank 128 62 against 89.
+size_t lf_ds_workspace(int M, int N, int R, const LfSegTable& seg);   // (lora_stream.hip)
+int lf_launch_ds(const void* dY, void* dS, void* ws, int M, int N, int R, const LfSegTable& seg, int dtype, hipStream_t st);
+
+struct ShortGrads { int a, b; };   // slices of K and of N; 0: not this way
+static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfSegTable& seg) {
+  const int rt = rt_of(R), TA = K / 64, TB = N / 64;
+  if (TA < 2 || TB < 2) return {0, 0};
+  int blocks[LF_MAX_SEG], nseg, live = 0, big = 0;
+  seg_block_counts(M, seg, blocks, nseg);
+  for (int s = 0; s < nseg; s++) live += blocks[s] > 0, big = std::max(big, blocks[s]);
+  if (live == 0 || big > 64) return {0, 0};
+  int t = rt == 8 ? 2 : 1;   // (as in da_form)
+  auto slices = [](int T, int t) { return (T + t - 1) / t; };
+  while (t <= da_tpw(rt) && (slices(TA, t) + slices(TB, t)) * live > 256) t++;   // one round of workgroups
+  if (t > da_tpw(rt)) return {0, 0};
+  const ShortGrads g{slices(TA, t), slices(TB, t)};
+  const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
+  const double m = masked, tiles = (double)big * t, n = N / 4096.0;
+  double us = 7.1 + 0.59 * rt + tiles * (0.387 + 0.484 * m) + 0.196 * big + 0.9e-3 * tiles * (g.a + g.b) * live;
+  if (R <= 32) {
+    const double groups = (double)((rows + 15) / 16) / 256;
+    us += n * (0.42 + 1.7 * rt + 5.3 * std::min(groups, 1.0) + 7.6 * std::max(groups - 1.0, 0.0));
+  } else {
+    const int sl = lf_xa_stream_slices(M, N, R, false, seg);
+    const double share = (double)(((rows + 63) / 64 * sl + 255) / 256) / sl;
+    us += 1.3 + n * share * 4.28 * rt + (sl > 1 ? 1.71 * 4e-6 * sl * (double)rows * R : 0.0);
+  }
+  const double old = 4.6 + 0.63 * rt + 0.201e-6 * dysr_plan(M, N, R, seg, SIZE_MAX).cost + da_form(M, K, R, masked, seg, SIZE_MAX).us;
+  return us < old ? g : ShortGrads{0, 0};
+}
+size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {
+  for (const bool masked : {false, true})
+    if (short_grads(M, N, K, R, masked, seg).a > 0) return lf_ds_workspace(M, N, R, seg);
+  return 0;
+}
+// sb: B_i in ptr; sg: dB_i in ptr, dA_i in out.  The launcher's preconditions are the two passes' own (lf_launch_dys_dyb, lf_launch_da): where
+// one is missing, they run and say so.  (Operands at any element's address, as there.)
+bool lf_short_grads_apply(const void* dY, const void* X, const uint8_t* mask, int mask_bits, const void* S, const void* dS, const void* ws, size_t ws_bytes, size_t limit, int M,
+                          int N, int K, int R, const LfSegTable& sb, const LfSegTable& sg) {
+  if (!dY || !X || !S || !dS || !ws || M <= 0 || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0 || R % 16 != 0 || R <= 0 || R > LF_MAX_RANK) return false;
+  if (sb.table && sb.block_size_m != ROWS) return false;
+  uintptr_t at8 = (uintptr_t)dS;
+  for (int s = 0; s < (sb.table ? sb.n_seg : 1); s++) {
+    if (!sb.ptr[s] || !sg.ptr[s] || !sg.out[s] || sb.rank[s] % 8 != 0 || sb.rank[s] > R) return false;
+    at8 |= (uintptr_t)sg.ptr[s] | (uintptr_t)sg.out[s];
+  }
+  if ((at8 & 7) != 0 || (mask != nullptr && mask_bits && ((uintptr_t)mask & 3) != 0)) return false;
+  if (short_grads(M, N, K, R, mask != nullptr, sb).a == 0) return false;
+  return ws_bytes >= std::max(lf_ds_workspace(M, N, R, sb), std::max(lf_dys_dyb_workspace(M, N, R, sb, limit), lf_da_workspace(M, K, R, sb, limit)));
+}
+int lf_launch_short_grads(const void* dY, const void* X, const uint8_t* mask, int mask_bits, const void* S, void* dS, void* ws, int M, int N, int K, int R,
+                          const LfSegTable& sb, const LfSegTable& sg, int dtype, hipStream_t st) {
+  const int rc = lf_launch_ds(dY, dS, ws, M, N, R, sb, dtype, st);
+  if (rc != LF_OK) return rc;
+  const ShortGrads g = short_grads(M, N, K, R, mask != nullptr, sb);
+  const int fmt = mask == nullptr ? 0 : mask_bits ? 2 : mask_off_grid(mask, 0) ? 3 : 1;
+  return lf_launch_da_direct(X, mask, fmt, dS, M, K, R, g.a, sg, dY, S, N, g.b, dtype, st);
+}

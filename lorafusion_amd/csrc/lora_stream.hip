@@ -2,13 +2,14 @@
 //
 //   D[row][c] = sum_k keep(row, k) * P[row][k] * Q[c][k]       P: many rows, read once; Q: at most 128 rows
 //
-// Two uses:
+// Three uses:
 //   xa      : P = X, Q = A_i:             S = drop(X) A^T     (seeded_dropout + `masked_scaled_x @ lora_a.T`,
 //             lorafusion/ops/lora_v1.py:111-119; the multi-adapter product, multi_lora.py:481-513)
 //   forward : P = the rows of W followed by the rows of A, Q = X of at most 128 rows: one pass over the weight gives the
 //             base product and the rank-r product of a short batch; a second kernel adds the slices and forms
 //             Y = X W^T + scale (X A^T) B^T + bias (fused_lora_xw_sb, triton_ops/fused_lora_xw_sb.py:74-206);
 //             up to 16 rows and rank 32 a kernel of its own does all of it in one launch (short16_fwd_kernel)
+//   dS      : P = dY, Q = B_i transposed: dS = scale dY B_i, where dB comes with dA (lora_da_direct.hip)
 //
 // Both are bound by the stream of P (the forward of 8 rows moves 34 MB of weights for 0.3 GFLOP), so what counts is how
 // many bytes the chip has on order.  A workgroup (4 waves) owns 64 rows of P and a slice of K: the slices are what
@@ -20,6 +21,7 @@
 #include "lf_common.h"
 #include "act_math.h"
 #include "rank_common.h"
+#include "rank_ring.h"
 
 namespace {
 
@@ -47,8 +49,8 @@ struct StreamArgs {
 
 // grid (64-row groups of P, slices of K).  MODE: 0 no keep-mask, 1 keep bytes read, 2 keep bits read, 3 mask drawn and written, 4 bytes or bits
 // read from an address that the direct loads do not take (the compiler's waits for these loads empty the ring every step).
-// FWD: Q = X (the second use above), D is stored transposed, [m][row of P].
-template <typename T, int RT, int MODE, bool FWD>
+// FWD: Q = X (the second use above), D is stored transposed, [m][row of P].  QT: Q lies transposed in memory, [K, rank] (the third: P = dY, Q = B_i).
+template <typename T, int RT, int MODE, bool FWD, bool QT>
 __global__ void __launch_bounds__(256, 2)
 lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
   constexpr int NS = st_ns(RT, MODE), STAGE = st_bytes(RT, MODE), QB = st_q_bytes(RT);
@@ -96,14 +98,16 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
     qv[i] = (uint32_t)(((int64_t)r * K) * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
     if (RT == 1 && lane >= 32) qv[i] = 0xffffff00u;   // beyond the window: nothing is fetched
   }
+  if constexpr (QT) side_voffs<RT, NQ>(qv, q_rows, q_rows, tid);
   if constexpr (MODE == 1) mv = (uint32_t)((wave * 16 + (lane >> 2)) * (int64_t)K + (lane & 3) * 16);
   if constexpr (MODE == 2) mv = lane < 32 ? (uint32_t)((wave * 16 + (lane >> 1)) * (K >> 3) + (lane & 1) * 4) : 0xffffff00u;
 
   const int64_t k0 = (int64_t)k_lo * 128;
   pb += ((int64_t)row0 * K + k0) * 2;
   int64_t pleft = ((int64_t)(rows_all - row0) * K - k0) * 2;
-  qb += k0 * 2;
-  int64_t qleft = ((int64_t)q_rows * K - k0) * 2;
+  qb += k0 * 2 * (QT ? q_rows : 1);
+  int64_t qleft = QT ? (K - k0) * q_rows * 2 : ((int64_t)q_rows * K - k0) * 2;
+  const int qstep = QT ? 128 * q_rows : 128;
   const char* mb = (const char*)a.mask + (((int64_t)row0 * K + k0) >> (MODE == 2 ? 3 : 0));
   int64_t mleft = ((int64_t)(rows_all - row0) * K - k0) >> (MODE == 2 ? 3 : 0);
   int ord = 0, ist = 0;   // steps ordered so far (behind the last one: that one again, unconsumed), stage of the next
@@ -113,12 +117,12 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
 #pragma unroll
     for (int i = 0; i < 2; i++) dma16(rp, pv[i], st + wave * 2048 + i * 1024);
 #pragma unroll
-    for (int i = 0; i < NQ; i++) dma16(rq, qv[i], st + SROWS * 128 + (wave * NQ + i) * 1024);
+    for (int i = 0; i < NQ; i++) dma16(rq, qv[i], st + SROWS * 128 + (QT ? i * 4096 + wave * 1024 : (wave * NQ + i) * 1024));
     if constexpr (MODE == 1) dma16(window_rsrc(mb, mleft), mv, st + SROWS * 128 + QB + wave * 1024);
     if constexpr (MODE == 2) dma4(window_rsrc(mb, mleft), mv, st + SROWS * 128 + QB + wave * 256);
     ist = ist + 1 == NS ? 0 : ist + 1;
     if (++ord < nsteps) {
-      pb += 128, pleft -= 128, qb += 128, qleft -= 128;
+      pb += 128, pleft -= 128, qb += qstep, qleft -= qstep;
       if constexpr (MODE == 1) mb += 64, mleft -= 64;
       if constexpr (MODE == 2) mb += 8, mleft -= 8;
     }
@@ -154,7 +158,8 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
       xf[h] = *(const lf_u32x4*)(x + li * 128 + fo);
 #pragma unroll
       for (int c = 0; c < RT; c++)
-        qf[h][c] = *(const lf_u32x4*)(RT == 1 ? q + (li >> 2) * 1024 + (li & 3) * 128 + fo : q + (c * 16 + li) * 128 + fo);
+        if constexpr (QT) qf[h][c] = side_tr8<RT>(q, h * 32 + qq * 8 + (li >> 2), c, li & 3);
+        else qf[h][c] = *(const lf_u32x4*)(RT == 1 ? q + (li >> 2) * 1024 + (li & 3) * 128 + fo : q + (c * 16 + li) * 128 + fo);
     }
     if constexpr (MODE == 1) {
       if (use_mask) {
@@ -218,7 +223,7 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
     }
   } else {
     // lane: column li of each 16, rows 4 qq + e of the wave
-    const float mult = use_mask ? 1.f / (1.f - bi.p) : 1.f;
+    const float mult = QT ? bi.scale : use_mask ? 1.f / (1.f - bi.p) : 1.f;
     if constexpr (FOLDS) {
 #pragma unroll
       for (int c = 0; c < RT; c++) acc[c] = sum[c] + acc[c];
@@ -241,10 +246,10 @@ lora_stream_kernel(const StreamArgs a, const LfSegTable seg) {
   }
 }
 
-// Second stage of a sliced xa: S = cast(1/(1-p) * sum of the slices), zero in padded rows and beyond the rank.
+// Second stage of a sliced xa: S = cast(1/(1-p) * sum of the slices), zero in padded rows and beyond the rank.  (mult: 0 none, 1 1/(1-p), 2 the scale: dS)
 template <typename T>
 __global__ void __launch_bounds__(256)
-stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_slices, int M, int R, int dropout, const LfSegTable seg) {
+stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_slices, int M, int R, int mult, const LfSegTable seg) {
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (idx >= rows * R) return;
@@ -253,7 +258,8 @@ stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_sl
   lf_f32x4 v = {0.f, 0.f, 0.f, 0.f};
   if (row % ROWS < bi.valid && col < bi.rank) {
     v = sum_parts(part + idx, rows * R, n_slices);
-    if (dropout && bi.p > 0.f) v *= 1.f / (1.f - bi.p);
+    if (mult == 1 && bi.p > 0.f) v *= 1.f / (1.f - bi.p);
+    if (mult == 2) v *= bi.scale;
   }
   *(lf_u32x2*)((uint16_t*)S + idx) = pack4<T>(v);
 }
@@ -265,7 +271,8 @@ stream_reduce_kernel(const float* __restrict__ part, T* __restrict__ S, int n_sl
 // Bound by what one compute unit takes in, X and A (MI355X, replayed from a graph, rank 16: 333 x 4096 5.2 -> 4.5 us, 1000 x 4096 6.6 -> 5.3,
 // 4096 x 4096 9.2 -> 8.3, 4.1 TB/s of X; whole forwards of 333 x 4096 into 4096 27.1 -> 26.1, 3000 x 8192 into 2048 at rank 32 99.6 -> 96.8).
 constexpr int xr_stages(int rt) { return rt == 1 ? 4 : 3; }
-template <typename T, int RT>
+// QT: A lies transposed in memory, [K, rank], and the product is scaled: dS = scale dY B_i.
+template <typename T, int RT, bool QT>
 __global__ void __launch_bounds__(512)
 lora_xa_ring_kernel(const void* __restrict__ X, T* __restrict__ S, int M, int rows, int K, int R, const LfSegTable seg) {
   constexpr int NS = xr_stages(RT), STAGE = (1 + RT) * 2048, GL = 2 * (1 + RT);
@@ -287,16 +294,23 @@ lora_xa_ring_kernel(const void* __restrict__ X, T* __restrict__ S, int M, int ro
     const int r = i * 8 + lrow;
     rv[i] = (uint32_t)((int64_t)r * K * 2 + ((slot ^ ((r >> 1) & 7)) << 4));
   }
+  uint32_t tv[2 * RT];   // QT: 64 rows of B_i
+#pragma unroll
+  for (int i = 0; i < 2 * RT; i++) {
+    const int p = i * 64 + lane, row = side_row<RT>(p / (RT * 2)), g = (p % (RT * 2)) ^ side_key<RT>(row);
+    tv[i] = (uint32_t)(row * bi.rank * 2 + (g * 8 < bi.rank ? g : 0) * 16);   // (beyond the rank: columns that are not stored)
+  }
   auto issue = [&](int i) {
     const int at = i < nsteps ? i : nsteps - 1;   // (behind the last step: that one again, unconsumed)
     const int64_t ko = (int64_t)(wave + at * 8) * 128;
     const uint32_t st = ring0 + (i % NS) * STAGE;
     const lf_u32x4 rx = window_rsrc((const char*)X + (int64_t)row0 * K * 2 + ko, (int64_t)(rows - row0) * K * 2 - ko);   // (rows beyond the last and
-    const lf_u32x4 ra = window_rsrc(A + ko, (int64_t)bi.rank * K * 2 - ko);                                              // beyond the rank read as zeros)
+    const int64_t qo = QT ? (int64_t)(wave + at * 8) * 128 * bi.rank : ko;                                               // beyond the rank read as zeros)
+    const lf_u32x4 ra = window_rsrc(A + qo, (int64_t)bi.rank * K * 2 - qo);
 #pragma unroll
     for (int q = 0; q < 2; q++) dma16(rx, rv[q], st + q * 1024);
 #pragma unroll
-    for (int q = 0; q < 2 * RT; q++) dma16(ra, rv[q], st + 2048 + q * 1024);
+    for (int q = 0; q < 2 * RT; q++) dma16(ra, QT ? tv[q] : rv[q], st + 2048 + q * 1024);
   };
   lf_f32x4 acc[RT];
 #pragma unroll
@@ -314,7 +328,8 @@ lora_xa_ring_kernel(const void* __restrict__ X, T* __restrict__ S, int M, int ro
         const char* fr = st + li * 128 + (((h * 4 + qq) ^ key) << 4);
         const lf_u32x4 xf = *(const lf_u32x4*)fr;
 #pragma unroll
-        for (int c = 0; c < RT; c++) acc[c] = Mfma16<T>::run(xf, *(const lf_u32x4*)(fr + (1 + c) * 2048), acc[c]);
+        for (int c = 0; c < RT; c++)
+          acc[c] = Mfma16<T>::run(xf, QT ? side_tr8<RT>(st + 2048, h * 32 + qq * 8 + (li >> 2), c, li & 3) : *(const lf_u32x4*)(fr + (1 + c) * 2048), acc[c]);
       }
     }
     wait_vm<0>();   // the unconsumed loads behind the last step
@@ -330,6 +345,7 @@ lora_xa_ring_kernel(const void* __restrict__ X, T* __restrict__ S, int M, int ro
 #pragma unroll
     for (int w = 0; w < 8; w++) v += part[w * RT * 256 + (col % (16 * RT)) * 16 + m];
     const bool real = (row0 + m) % ROWS < bi.valid && col < bi.rank;
+    if constexpr (QT) v = fp32_product(v, bi.scale);
     S[(int64_t)(row0 + m) * R + col] = real ? (T)v : (T)0.f;
   }
 }
@@ -523,9 +539,9 @@ int slices_for(int64_t groups, int K, double partial_bytes, const SliceModel& m)
   return best;
 }
 
-template <typename T, int RT, int MODE, bool FWD>
+template <typename T, int RT, int MODE, bool FWD, bool QT = false>
 int stream_launch(const StreamArgs& a, const LfSegTable& seg, int groups, hipStream_t st) {
-  auto kern = lora_stream_kernel<T, RT, MODE, FWD>;
+  auto kern = lora_stream_kernel<T, RT, MODE, FWD, QT>;
   constexpr int SMEM = st_smem(RT, MODE);
   static_assert(2 * SMEM <= 160 * 1024, "two workgroups per CU");
   static LfLdsFlags lds_ok;
@@ -580,9 +596,9 @@ size_t lf_xa_stream_workspace(int M, int K, int R, bool masked, const LfSegTable
   return n > 1 ? (size_t)n * xa_rows_of(M, seg) * R * sizeof(float) : 0;
 }
 
-template <typename T, int RT>
+template <typename T, int RT, bool QT = false>
 static int xa_ring_launch(const void* X, void* S, int M, int rows, int K, int R, const LfSegTable& seg, hipStream_t st) {
-  auto kern = lora_xa_ring_kernel<T, RT>;
+  auto kern = lora_xa_ring_kernel<T, RT, QT>;
   constexpr int SMEM = 8 * xr_stages(RT) * (1 + RT) * 2048;
   static LfLdsFlags lds_ok;
   if (!lf_allow_lds(kern, SMEM, lds_ok)) return LF_ELAUNCH;
@@ -602,6 +618,26 @@ int lf_launch_xa_stream(const void* X, const uint8_t* mask, uint8_t* mask_out, i
   a.mask = mask; a.mask_out = mask_out; a.mask_bytes = !mask_bits; a.seed_lo = (uint32_t)seed; a.seed_hi = (uint32_t)(seed >> 32);
   a.S = S; a.M = M; a.R = R;
   return dtype == LF_BF16 ? xa_stream_impl<__bf16>(a, seg, ws, st) : xa_stream_impl<_Float16>(a, seg, ws, st);
+}
+
+// ---- dS = scale dY B_i, complete: to rank 32 on the ring kernel, above in slices of N.
+// ws: lf_ds_workspace bytes
+size_t lf_ds_workspace(int M, int N, int R, const LfSegTable& seg) { return R <= 32 ? 0 : lf_xa_stream_workspace(M, N, R, false, seg); }
+template <typename T>
+static int ds_impl(const void* dY, void* dS, float* ws, int M, int N, int R, const LfSegTable& seg, hipStream_t st) {
+  const int rows = (int)xa_rows_of(M, seg);
+  if (R <= 32) return R <= 16 ? xa_ring_launch<T, 1, true>(dY, dS, M, rows, N, R, seg, st) : xa_ring_launch<T, 2, true>(dY, dS, M, rows, N, R, seg, st);
+  StreamArgs a{};
+  a.p0 = dY; a.n0 = rows; a.K = N; a.n_slices = lf_xa_stream_slices(M, N, R, false, seg); a.S = dS; a.M = M; a.R = R;
+  a.part = a.n_slices > 1 ? ws : nullptr;
+  const int groups = (rows + SROWS - 1) / SROWS;
+  const int rc = rt_of(R) == 4 ? stream_launch<T, 4, 0, false, true>(a, seg, groups, st) : stream_launch<T, 8, 0, false, true>(a, seg, groups, st);
+  if (rc != LF_OK || a.part == nullptr) return rc;
+  const int64_t n4 = ((int64_t)rows * R + 3) / 4;
+  return lf_launch((stream_reduce_kernel<T>), dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, (const float*)ws, (T*)dS, a.n_slices, M, R, 2, seg);
+}
+int lf_launch_ds(const void* dY, void* dS, void* ws, int M, int N, int R, const LfSegTable& seg, int dtype, hipStream_t st) {
+  return dtype == LF_BF16 ? ds_impl<__bf16>(dY, dS, (float*)ws, M, N, R, seg, st) : ds_impl<_Float16>(dY, dS, (float*)ws, M, N, R, seg, st);
 }
 
 // ---- forward of a short batch (one adapter, no keep-mask)

@@ -170,10 +170,12 @@ __device__ __forceinline__ lf_u32x4 side_tr8(const char* blk, int row, int c, in
 // of nt tiles keeps at most min(NS, (NSB - 1) nt + 1) stages of the ring busy, so one block more is never on order).
 //   D_j[r][k] += sum_m dS[m][r] * keep*X[m][k]   per tile j of the slice, in registers over all blocks of the chunk.
 // With a keep-mask the tile is masked in place one iteration before it is consumed.
+// The direct form takes dB with dA: the workgroups of blockIdx.y = 1 walk dY beside S without a mask, the same sum with other operands.
+struct DbOperands { const void* dY; const void* S; int N, n_slices; };   // (outputs: seg.ptr)
 template <typename T, int RT, int TPW, int NS, int MASK, int NSB, bool DIRECT>
 __global__ void __launch_bounds__(256, RT >= 8 || DIRECT ? 1 : 2)
 lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, const T* __restrict__ dS, float* __restrict__ part,
-                    int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg) {
+                    int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg, const DbOperands db) {
   // MASK: 0 no keep-mask; 1 one byte per element (8 KB per tile, two loads per thread); 2 one bit per element (1 KB per
   // tile, one 4-byte load per thread); 3 one byte per element at an address that the direct loads do not take, read where it is applied (the compiler's
   // waits for those loads empty the ring every tile)
@@ -185,7 +187,12 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   char* ring = lds;
   char* side = lds + NS * STAGE;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
-  const int ks = blockIdx.x, ch = blockIdx.y, s = blockIdx.z;
+  const int ks = blockIdx.x, ch = DIRECT ? 0 : blockIdx.y, s = blockIdx.z;
+  const bool grad_b = DIRECT && blockIdx.y != 0;
+  if constexpr (DIRECT) {
+    if (grad_b) X = (const T*)db.dY, dS = (const T*)db.S, K = db.N, n_slices = db.n_slices, mask = nullptr;
+    if (ks >= n_slices) return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = to_sgpr(tid >> 6);
   const int li = lane & 15, qq = lane >> 4, j4 = li >> 2, c4 = li & 3;
   int b0, b1, bb0, bb1;
@@ -194,7 +201,8 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   if (bb0 >= bb1) {  // this segment has fewer chunks (uniform for the whole workgroup)
     if constexpr (DIRECT) {   // no rows at all: a sum of nothing
       const int T64 = K / 64, k0 = (ks * (T64 / n_slices) + min(ks, T64 % n_slices)) * 64, nk = (T64 / n_slices + (ks < T64 % n_slices ? 1 : 0)) * 64;
-      for (int i = tid; i < seg.rank[s] * nk; i += 256) ((uint16_t*)seg.out[s])[(int64_t)(i / nk) * K + k0 + i % nk] = 0;
+      if (grad_b) for (int i = tid; i < seg.rank[s] * nk; i += 256) ((uint16_t*)seg.ptr[s])[(int64_t)k0 * seg.rank[s] + i] = 0;
+      else for (int i = tid; i < seg.rank[s] * nk; i += 256) ((uint16_t*)seg.out[s])[(int64_t)(i / nk) * K + k0 + i % nk] = 0;
     }
     return;
   }
@@ -314,6 +322,20 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   // C layout: column (k) = lane & 15, rows (r) = 4*(lane >> 4) + e
   if constexpr (DIRECT) {   // one chunk per segment: these are the sums
     const int rank = seg.rank[s];
+    if (grad_b) {   // [N, rank]: a lane has four neighbours of a row
+      const float mult = seg.table ? (seg.block_scale ? seg.block_scale[b0] : 1.f) : seg.scale;
+      uint16_t* out = (uint16_t*)seg.ptr[s];
+#pragma unroll
+      for (int t = 0; t < TPW; t++)
+        if (t < nt) {
+#pragma unroll
+          for (int c = 0; c < RT; c++) {
+            const int r = c * 16 + qq * 4;
+            if (r < rank) *(lf_u32x2*)(out + (int64_t)((kt0 + t) * 64 + wave * 16 + li) * rank + r) = pack4<T>(acc[t][c] * mult);
+          }
+        }
+      return;
+    }
     const float mult = mask != nullptr && p > 0.f ? 1.f / (1.f - p) : 1.f;
     uint16_t* out = (uint16_t*)seg.out[s];
 #pragma unroll
