@@ -216,7 +216,8 @@ int lf_set_tile_cfg(int tile_cfg);
  * as a second launch of *cfg_tail (-1 when there is none).  Every number names one kernel and tile: 4, 6 and 9 are the 128x128, 128x64 and
  * 192x128 tiles of the general kernel, 11, 12 and 13 (with 10, 14 and 15) those of the kernel for outputs of about one round.  A launch may still move to another tile: a call whose
  * keep-mask or rank the persistent kernel (7, 8) does not take, or whose keep-mask (one byte per element) the kernel for about one round (10..15) does not,
- * goes to the best of the others, and a launch that leaves compute units idle over a long K is cut into slices.  routing_block_size_m: 0 for a
+ * goes to the best of the others, a launch that leaves compute units idle over a long K is cut into slices, and one of 7 over a K that is a multiple of
+ * 1024 runs on the eight-wave 256x256 tile (1) where that is the faster one for such row pitches.  routing_block_size_m: 0 for a
  * single-adapter call, else the routing block size.  For benchmarks that time one kernel of a
  * fused call on its own; no counterpart in the reference (Triton's autotuner picks there). */
 int lf_gemm_plan(int M, int N, int K, int routing_block_size_m, int* rows_head, int* cfg_head, int* cfg_tail);

@@ -803,15 +803,15 @@ static const TileCand kCands[] = {
     {5, 64, 64, 4.6, 13.2, 3.1, 7.7, 15.6, 4.3, 2.4, 0.265, 0.061},        // 4 waves, 32x32 per wave
     {6, 128, 64, 5.1, 17.4, 4.1, 21.5, 25.1, 3.7, 1.6, 0.479, 0.085},      // 4 waves, 64x32 per wave
     {8, 128, 256, 6.0, 35.4, 11.3, 36.5, 54.0, 23.4, 0.0, 0.0, 0.108},     // persistent, 4 waves of 64x128 (gemm_big.hip)
-    // gemm_mid.hip: 4 waves of 96x64, 80x64, 64x64, 64x32, 48x32, 32x32.  Timed in 32500 launches of 1400 shapes (17 - 3000 rows, 1024 - 14336 columns and
-    // K, cold weights); the figures are those with which the plan (tile and slices) costs least on seven tenths of the shapes: on the other three
-    // tenths it is 0.9 % behind the best launch timed, the plan from the figures fitted before the two smallest tiles were there 6.8 %.
-    {13, 192, 128, 7.1, 28.0, 4.2, 40.4, 50.8, 5.8, 1.5, 0.384, 0.046, true},
-    {10, 160, 128, 6.4, 26.3, 2.7, 36.5, 44.3, 1.6, 1.8, 0.413, 0.051, true},
-    {11, 128, 128, 6.1, 23.9, 1.5, 24.1, 36.0, 17.3, 1.1, 0.525, 0.061, true},
-    {12, 128, 64, 2.9, 17.3, 3.9, 17.9, 21.2, 8.4, 1.8, 0.461, 0.062, true},
-    {14, 96, 64, 3.2, 14.3, 2.5, 13.6, 17.6, 6.2, 1.8, 0.431, 0.076, true},
-    {15, 64, 64, 2.2, 12.3, 1.15, 8.5, 12.2, 6.1, 2.3, 0.423, 0.090, true},
+    // gemm_mid.hip: 4 waves of 96x64, 80x64, 64x64, 64x32, 48x32, 32x32.  Timed in 130000 launches of 6200 shapes (17 - 3000 rows, 1024 - 14336 columns, K
+    // to 57344, ranks 16 - 128, cold weights); the figures are those with which the plan (tile and slices) costs least on three quarters of the shapes: on the
+    // others it is 1.2 % behind the best launch timed, the plan from the figures fitted before the two smallest tiles were there 5.8 %.
+    {13, 192, 128, 7.4, 28.1, 4.1, 40.5, 50.8, 5.8, 1.4, 0.365, 0.046, true},
+    {10, 160, 128, 5.9, 25.6, 3.2, 31.3, 44.3, 1.6, 2.2, 0.397, 0.059, true},
+    {11, 128, 128, 6.1, 24.2, 1.8, 22.5, 36.0, 17.3, 1.1, 0.487, 0.061, true},
+    {12, 128, 64, 2.9, 17.8, 3.6, 20.3, 21.2, 8.4, 1.8, 0.398, 0.070, true},
+    {14, 96, 64, 3.1, 14.3, 2.7, 21.7, 17.6, 6.2, 1.7, 0.406, 0.075, true},
+    {15, 64, 64, 2.1, 12.3, 1.2, 8.7, 12.2, 6.1, 2.3, 0.373, 0.082, true},
 };
 static long tiles_of(int M, int N, const TileCand& c) { return (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); }
 static double launch_cost(const TileCand& c, int M, int N, int K, int slices = 1, int steps = 0) {
@@ -835,7 +835,10 @@ static bool mid_shape(const TileCand& c, int N, int K) { return N % c.bn == 0 &&
 // What a tile of gemm_mid.hip has to be ahead by in the model to be taken: in one round, in several, sliced (fitted with the figures above; in several
 // rounds the model says too little for it).
 // (A 192x128 tile that only the margin keeps with gemm_lora.hip runs here all the same: one tile, one kernel, but for what this one does not take.)
-static double mid_margin(long tiles, int slices) { return slices > 1 ? 0.99 : (tiles <= 256 ? 1.0 : 1.08); }
+// Slices of a long contraction: 1.4 % more at K = 12000, 4 % at 28000 (256 x 8192 over 28672 in two slices of 128x128 169 us, in eight of 256x256 148).
+static double mid_margin(long tiles, int slices, int K) {
+  return slices > 1 ? 0.98 + std::min(0.08, 0.0018 * std::max(0, K - 4096) / 1024) : (tiles <= 256 ? 1.0 : 1.1);
+}
 // The tile of an unsplit launch.  big: the persistent kernel applies; tail: left-over rows behind whole rounds of 256x256 tiles
 // (its 128-row tile and the other 256-column tiles leave most of the chip idle there); wave96: a 96-row wave meets at most two
 // routing blocks.  The eight-wave 256x256 tile stands in for the persistent one (a long
@@ -853,18 +856,70 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, bool mid, doub
     if (c.cfg == 3 && tail) continue;
     if (c.cfg == 9 && (!wave96 || tail)) continue;
     if (c.mid && (!mid || !mid_shape(c, N, K) || (tail && c.bm != 128))) continue;   // (left-over rows: 128x128 and 128x64; in slices any tile)
-    const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1) : 1.0);
+    const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1, K) : 1.0);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;
   return best == 9 && mid && mid_shape(cand_of(13), N, K) ? 13 : best;
 }
+// ... and what an unsplit round of it has to be ahead of slices by, beyond that margin, over a long K: there the model says too little for it (NT: 11 % at
+// K = 8192, 16 % at 13000; NN: 7 % to 20000, 17 % beyond) and not for the large tiles in slices.  Forward + backward of 1000 shapes, launches traced
+// against the plans before gemm_mid.hip: of 314 NT products of one round 22 were more than 3 % slower (1408 x 2176 over 13312: 97 -> 118 us, 638 x 4864 over
+// 13568: 91 -> 126), of 418 NN products 10 (1468 x 2176 over 25728: 190 -> 220); without those that this sends back to slices 7 and 3 remain, and all of them
+// together are another 0.6 % and 0.05 % faster (400 shapes that were not fitted: 15 of 539 products more than 3 % slower, all together 9 % faster).
+static double mid_long_k(long tiles, int K, bool nn) { return tiles > 256 ? 0.0 : (nn ? 0.02 * std::max(0, K - 16384) : 0.0155 * std::max(0, K - 4096)) / 1024; }
+
+// Split contraction for launches that leave compute units idle over a long K (left-over rows of a packed batch, short
+// batches): K is cut into slices, workgroup (tile, slice) keeps fp32 sums, a second kernel adds the slices.  Larger tiles
+// move fewer operand bytes per product, and a compute unit takes in at most about 100 GB/s whatever its tile, so many slices of
+// a large tile beat one slice of many small ones once K is long: tile and slice count are chosen together by the model above, where
+// they are at least 4 % ahead of the planned launch.  A slice keeps at least 512 of K, its workgroups fit the chip at once, and the partial
+// tiles stay within a limit (the dX product's: what the library's static scratch holds).  A function of the shape, the planned tile and the routing alone: a call that is
+// given the workspace lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
+constexpr size_t kKsplitMaxBytes = (size_t)64 << 20, kKsplitMaxBytesNN = LF_STATIC_SCRATCH_BYTES;
+struct KSplit { int cfg, n, steps; };
+// The cheapest slices below `best_cost`, which becomes theirs; `best` as it came if there are none.
+static KSplit cheapest_slices(int M, int N, int K, int routing_block, bool nn, bool mid, KSplit best, double& best_cost) {
+  const int nk = K / BK;
+  const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
+  for (const TileCand& c : kCands) {
+    if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)
+    if (c.mid && (!mid || !mid_shape(c, N, K))) continue;
+    if ((c.cfg == 9 && !wave96_fits(routing_block)) || (c.cfg == 1 && routing_block > 0 && routing_block % 128 != 0)) continue;
+    const long tiles = tiles_of(M, N, c), slots = c.cfg == 4 || c.cfg == 5 ? 512 : 256;
+    for (int n : {2, 3, 4, 5, 6, 8, 12, 16}) {
+      if (tiles * n > slots || K < n * 512 || slice * n > max_bytes) break;
+      int steps = (nk + n - 1) / n;
+      steps += steps & 1;                               // an even number of steps per slice (K / BK is even)
+      const int used = (nk + steps - 1) / steps;        // no empty slice
+      if (c.mid && nk - (used - 1) * steps < 8) continue; // (four K steps of 64 in the last slice too)
+      // (packed batches: a tile of 192, 160 or 96 rows may lie across two adapters and then multiplies two skinny operands)
+      const double cost = launch_cost(c, M, N, K, used, steps) * (c.mid ? mid_margin(tiles, n, K) + (routing_block > 0 && c.bm % 128 != 0 && c.bm > 64 ? 0.05 : 0.0) : 1.0 / 0.96);
+      if (used > 1 && cost < best_cost) { best_cost = cost; best = {c.cfg, used, steps}; }
+    }
+  }
+  return best;
+}
+static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
+  const int nk = K / BK;
+  KSplit best = {cfg, 1, nk};
+  const TileCand& planned = cand_of(cfg);
+  if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
+  double best_cost = launch_cost(planned, M, N, K);
+  if (const long tiles = tiles_of(M, N, planned); planned.mid) best_cost *= mid_margin(tiles, 1, K) + mid_long_k(tiles, K, nn);
+  best = cheapest_slices(M, N, K, routing_block, nn, mid, best, best_cost);
+  if (best.n > 1 && best.cfg == 9 && mid && mid_shape(cand_of(13), N, K) && nk - (best.n - 1) * best.steps >= 8) best.cfg = 13;
+  return best;
+}
+
 // Rows [0, m_main) as 256x256 tiles, the rest as a second launch with the tile that spreads them best, when that beats
 // one launch (a nearly empty last round of big tiles costs a full tile time).  m_main is the multiple of 256 rows
 // with the lowest modelled cost of both launches: usually the one whose tiles fill whole rounds of the chip
 // (32 tile rows of 40 tiles are exactly five rounds; 30 rows of 40 are five rounds too, and leave a longer tail).
 // Returns m_main (0: single launch).
-static int choose_split(int M, int N, int K, bool allow_big, bool wave96, bool mid, int* cfg_head, int* cfg_tail) {
+// (Left-over rows over a long K run in slices where the call has memory for them, as the whole forward and backward do, and are priced that way: unsliced, 512 rows x 8192 over
+// 57344 look 60 us dearer than 256, they are 190.)
+static int choose_split(int M, int N, int K, int routing_block, bool allow_big, bool wave96, bool mid, int* cfg_head, int* cfg_tail) {
   constexpr double kLaunch = 4.0;  // a second launch
   const int grid_n = (N + 255) / 256;
   if (grid_n > 256) return 0;
@@ -878,53 +933,11 @@ static int choose_split(int M, int N, int K, bool allow_big, bool wave96, bool m
     if (head_cost >= best) break;
     double tail;
     const int ct = choose_cfg(M - r * 256, N, K, allow_big, wave96, mid, &tail, true);
+    if (K >= 1024) cheapest_slices(M - r * 256, N, K, routing_block, /*nn=*/true, mid, {ct, 1, K / BK}, tail);
     if (head_cost + tail < best) { best = head_cost + tail; best_m = r * 256; *cfg_tail = ct; }
   }
   *cfg_head = big ? 7 : 1;
   return best_m;
-}
-
-// ... and what an unsplit round of it has to be ahead of slices by, beyond that margin, over a long K: there the model says too little for it (NT: 11 % at
-// K = 8192, 16 % at 13000; NN: 7 % to 20000, 17 % beyond) and not for the large tiles in slices.  Forward + backward of 1000 shapes, launches traced
-// against the plans before gemm_mid.hip: of 314 NT products of one round 22 were more than 3 % slower (1408 x 2176 over 13312: 97 -> 118 us, 638 x 4864 over
-// 13568: 91 -> 126), of 418 NN products 10 (1468 x 2176 over 25728: 190 -> 220); without those that this sends back to slices 7 and 3 remain, and all of them
-// together are another 0.6 % and 0.05 % faster (400 shapes that were not fitted: 15 of 539 products more than 3 % slower, all together 9 % faster).
-static double mid_long_k(long tiles, int K, bool nn) { return tiles > 256 ? 0.0 : (nn ? 0.02 * std::max(0, K - 16384) : 0.026 * std::max(0, K - 4096)) / 1024; }
-
-// Split contraction for launches that leave compute units idle over a long K (left-over rows of a packed batch, short
-// batches): K is cut into slices, workgroup (tile, slice) keeps fp32 sums, a second kernel adds the slices.  Larger tiles
-// move fewer operand bytes per product, and a compute unit takes in at most about 100 GB/s whatever its tile, so many slices of
-// a large tile beat one slice of many small ones once K is long: tile and slice count are chosen together by the model above, where
-// they are at least 4 % ahead of the planned launch.  A slice keeps at least 512 of K, its workgroups fit the chip at once, and the partial
-// tiles stay within a limit (the dX product's: what the library's static scratch holds).  A function of the shape, the planned tile and the routing alone: a call that is
-// given the workspace lf_workspace_bytes names always makes the same split, so its result does not depend on who calls.
-constexpr size_t kKsplitMaxBytes = (size_t)64 << 20, kKsplitMaxBytesNN = LF_STATIC_SCRATCH_BYTES;
-struct KSplit { int cfg, n, steps; };
-static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
-  const int nk = K / BK;
-  KSplit best = {cfg, 1, nk};
-  const TileCand& planned = cand_of(cfg);
-  if (K < 1024 || tiles_of(M, N, planned) > 512) return best;
-  double best_cost = launch_cost(planned, M, N, K);
-  if (const long tiles = tiles_of(M, N, planned); planned.mid) best_cost *= mid_margin(tiles, 1) + mid_long_k(tiles, K, nn);
-  const size_t slice = (size_t)M * N * sizeof(float), max_bytes = nn ? kKsplitMaxBytesNN : kKsplitMaxBytes;
-  for (const TileCand& c : kCands) {
-    if (c.cfg == 7 || c.cfg == 8) continue;             // (the persistent kernel does not split)
-    if (c.mid && (!mid || !mid_shape(c, N, K))) continue;
-    if ((c.cfg == 9 && !wave96_fits(routing_block)) || (c.cfg == 1 && routing_block > 0 && routing_block % 128 != 0)) continue;
-    const long tiles = tiles_of(M, N, c), slots = c.cfg == 4 || c.cfg == 5 ? 512 : 256;
-    for (int n : {2, 3, 4, 5, 6, 8, 12, 16}) {
-      if (tiles * n > slots || K < n * 512 || slice * n > max_bytes) break;
-      int steps = (nk + n - 1) / n;
-      steps += steps & 1;                               // an even number of steps per slice (K / BK is even)
-      const int used = (nk + steps - 1) / steps;        // no empty slice
-      if (c.mid && nk - (used - 1) * steps < 8) continue; // (four K steps of 64 in the last slice too)
-      const double cost = launch_cost(c, M, N, K, used, steps) * (c.mid ? mid_margin(tiles, n) : 1.0 / 0.96);
-      if (used > 1 && cost < best_cost) { best_cost = cost; best = {c.cfg, used, steps}; }
-    }
-  }
-  if (best.n > 1 && best.cfg == 9 && mid && mid_shape(cand_of(13), N, K) && nk - (best.n - 1) * best.steps >= 8) best.cfg = 13;
-  return best;
 }
 
 static KSplit ksplit_for(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
@@ -945,7 +958,7 @@ bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; 
 static void plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
   const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), wave96 = wave96_fits(routing_block);
   int ch = 1, ct = 1;
-  const int m_main = choose_split(M, N, K, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
+  const int m_main = choose_split(M, N, K, routing_block, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
   // A long contraction under a wide output runs faster on the eight-wave 256x256 tile than on the persistent kernel
   // (8192 x 8192 over 28672: 3.08 against 3.24 ms, over 57344: 5.74 against 5.85; at 4096 columns the two are level, and
   // at shorter contractions the persistent kernel is 3-8 % ahead): its long K loops let the tiles of an XCD drift apart
@@ -1004,6 +1017,18 @@ size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   return memo.get({M, N, K, routing_block, nn}, [&] { return ksplit_bytes(M, N, K, routing_block, nn); });
 }
 
+// Unsplit products planned on the persistent 256x256 tile that the eight-wave one is the faster kernel for: a left operand (and, NT, a weight) whose row
+// pitch is a multiple of 2 KB puts a K step's lines of all rows on few memory channels, and the persistent kernel, which has one step of 64 on order, waits for
+// them where the other's ring of five steps of 32 does not.  The powers of two and 3 and 7 times 2 KB are spread by the address hash.  Eight-wave over persistent in
+// 4270 launches of 1500 - 12300 rows over 2048 - 14336 columns (cold weights, rank-16 term, geometric means): NT 0.935 at K = 5120 and 6144 (9 of 358 more than 2 % behind), 0.918 from 9216
+// (7 of 805), 1.02 / 0.99 / 1.01 at 4096 / 7168 / 8192, 1.00 at pitches that are no multiple of 2 KB; NN 1.00 at 5120 - 9216, 0.956 at 10240 - 15360, 0.93
+// from 16384.  3000 x 5120 over 5120 NT 138 -> 127 us, 8192 x 4096 over 10240 547 -> 492.  To two rounds of tiles: of longer launches, which run at the power limit, the
+// faster one slows its neighbours down (16384 x 4096 over 28672 NN 2751 -> 2620 us, the decoder layer around it 12 070 -> 12 057).
+static bool pitch_prefers_eight_waves(const LfGemmParams& q, bool nn) {
+  if (q.K % 1024 != 0 || (long)((q.M + 255) / 256) * ((q.N + 255) / 256) > 512) return false;
+  return nn ? q.K >= 10240 : q.K == 5120 || q.K == 6144 || q.K >= 9216;
+}
+
 int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dtype, int force_cfg, hipStream_t st) {
   if (force_cfg < 0) force_cfg = pinned_cfg.load(std::memory_order_relaxed);
   if (p.M <= 0 || p.N <= 0 || p.K <= 0) return LF_EINVAL;
@@ -1041,6 +1066,7 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
       const KSplit ks = ksplit_for(r.M, r.N, r.K, cfg, rblock, nn, mid);
       if (ks.n > 1 && (size_t)ks.n * r.M * r.N * sizeof(float) <= r.ks_ws_bytes) { cfg = ks.cfg; r.ksplit = ks.n; r.ks_steps = ks.steps; }
     }
+    if (planned && cfg == 7 && r.ksplit <= 1 && pitch_prefers_eight_waves(q, nn)) cfg = 1;
     if (cfg >= 10) {
       if (!mid) return (int)LF_ESHAPE;
       const int rc = lf_launch_gemm_mid(r, seg, nn, dtype, cfg, st);

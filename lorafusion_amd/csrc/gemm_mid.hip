@@ -287,7 +287,10 @@ gemm_mid_kernel(const LfGemmParams p, const LfSegTable seg) {
       const int row = p.row0 + wrow0, blk = min(row / seg.block_size_m, seg.n_blocks - 1);
       t0 = term_of_block(blk);
       const int left = (blk + 1) * seg.block_size_m - row;
-      if (left < WROWS && blk + 1 < seg.n_blocks) isplit = left / 16, nterm = 2, t1 = term_of_block(blk + 1);
+      if (left < WROWS && blk + 1 < seg.n_blocks) {
+        t1 = term_of_block(blk + 1);
+        if (t1.rp != t0.rp || t1.rank != t0.rank || t1.mult != t0.mult || t1.mask != t0.mask) isplit = left / 16, nterm = 2;   // (else two blocks of one adapter)
+      }
     }
     use_mask = t0.mask || (nterm == 2 && t1.mask);
     if (use_mask) {

@@ -931,7 +931,7 @@ static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfS
     us += 1.3 + n * share * 4.28 * rt + (sl > 1 ? 1.71 * 4e-6 * sl * (double)rows * R : 0.0);
   }
   const double old = 4.6 + 0.63 * rt + 0.201e-6 * dysr_plan(M, N, R, seg, SIZE_MAX).cost + da_form(M, K, R, masked, seg, SIZE_MAX).us;
-  return us < old ? g : ShortGrads{0, 0};
+  return us * (big > 8 ? 1.06 : 1.0) < old ? g : ShortGrads{0, 0};   // (longer segments gain 1 - 2 % and are as often behind)
 }
 size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {
   for (const bool masked : {false, true})
