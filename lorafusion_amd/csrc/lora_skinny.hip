@@ -486,7 +486,7 @@ lora_dys_dyb_ring_kernel(const T* __restrict__ dY, const T* __restrict__ S, floa
 
 // ---- work split of the ring kernels.  Workgroups (slice x chunk) of w tiles each run on `slots` resident slots; the
 // pass lasts about as long as its busiest slot.  Two upper bounds of that (in tiles): whole rounds of the largest
-// workgroup, and the list-scheduling bound sum / slots + largest; the smaller one is the estimate.
+// workgroup, and the list-scheduling bound sum / slots + largest; the smaller one is the estimate (ring_us).
 struct GroupStats { long chunks, total; int max_chunks, big; };   // of one chunk length: independent of the slices
 static GroupStats group_stats(const int* blocks, int nseg, int g) {
   GroupStats r{0, 0, 1, 0};
@@ -501,14 +501,26 @@ static GroupStats group_stats(const int* blocks, int nseg, int g) {
   }
   return r;
 }
-static double ring_span(const GroupStats& r, int T, int nsl, int slots) {
+// Microseconds of a pass and its second stage: tiles and row blocks of the busiest slot, rounds of workgroups, partials in MB (dS: one [rows, R] slab per slice; dB or dA: one slab per
+// chunk), the side operand that every workgroup fetches per block in MB, and the share of a slot if all tiles were spread evenly.  Fitted, by rank tiling, to 35 plans each of 2423
+// batches (700 - 16400 rows in 1 - 8 segments, 1024 - 14336 columns): on shapes that were not fitted dys_dyb is 5.5 % behind the best plan timed, dA 2.4 % and without a mask 1.8 %;
+// the bytes moved, by which plans were chosen before, 8.5, 3.9 and 5.9 %.  2048 x 4096 rank 16: dys_dyb 15.4 -> 13.3, dA 13.6 -> 11.8; the eight-tile slices of the byte model
+// leave three quarters of the compute units idle there.
+struct RingModel { double fixed, tile, block, round, ds, slab, side, even; };
+static double ring_us(const RingModel& m, const GroupStats& r, int T, int nsl, int slots, double ds_mb, double slab_mb, double side_mb) {
   const int t_max = (T + nsl - 1) / nsl;
-  const long wgs = r.chunks * nsl;
-  const double sum = (double)r.total * T / slots, largest = (double)r.big * t_max;
-  const double by_rounds = (double)((wgs + slots - 1) / slots) * largest, by_list = sum + largest;
-  const double span = by_rounds < by_list ? by_rounds : by_list;
-  return span < sum ? sum : span;
+  const double rounds = (double)((r.chunks * nsl + slots - 1) / slots), even = (double)r.total * T / slots, largest = (double)r.big * t_max;
+  const double span = std::max(std::min(rounds * largest, even + largest), even);
+  const double blocks = std::max(std::min(rounds * r.big, (double)r.total * nsl / slots + r.big), 1.0);
+  return m.fixed + m.tile * span + m.block * blocks + m.round * rounds + m.ds * ds_mb + m.slab * slab_mb + m.side * side_mb + m.even * even;
 }
+static int model_of(int rt) { return rt >= 8 ? 3 : rt >= 4 ? 2 : rt >= 2 ? 1 : 0; }
+static const RingModel kDysModel[4] = {{8.66, 0.166, 0.237, 1.13, 0.081, 0.429, 0.609, 1.074}, {9.36, 0.276, 0.505, 0.87, 0.193, 0.434, 0.279, 0.464},
+                                       {9.19, 0.346, 0.120, 2.42, 0.251, 0.271, 0.167, 0.0}, {7.22, 0.764, 0.456, 3.44, 0.150, 0.238, 0.220, 0.064}};
+static const RingModel kDaModel[2][4] = {{{7.73, 0.243, 0.055, 0.47, 0.0, 0.846, 0.032, 0.658}, {10.27, 0.216, 0.268, 0.0, 0.0, 0.595, 0.078, 0.577},
+                                          {8.01, 0.271, 0.0, 0.89, 0.0, 0.329, 0.045, 0.617}, {10.25, 0.541, 0.002, 2.39, 0.0, 0.324, 0.055, 0.0}},
+                                         {{9.29, 0.558, 0.012, 3.44, 0.0, 0.425, 0.310, 0.760}, {9.44, 0.556, 0.082, 0.74, 0.0, 0.572, 0.322, 0.0},
+                                          {10.92, 0.622, 0.0, 1.29, 0.0, 0.431, 0.132, 0.0}, {14.39, 0.581, 0.014, 1.87, 0.0, 0.286, 0.067, 0.0}}};   // without and with a keep-mask
 static void seg_block_counts(int M, const LfSegTable& seg, int* blocks, int& nseg) {
   nseg = seg.table ? seg.n_seg : 1;
   for (int s = 0; s < nseg; s++) {
@@ -534,15 +546,12 @@ static int all_group_stats(const int* blocks, int nseg, GroupStats (&st)[kNGroup
 constexpr int dysr_tpw(int rt) { return rt >= 8 ? 4 : rt >= 2 ? 12 : 16; }   // dB accumulators: TPW * RT * 4 registers, next to 8 * RT of dS
 constexpr int dysr_ns(int rt) { return rt == 4 ? 5 : 3; }   // (rank 128: three stages of 32 KB and two S blocks of 32 KB are all of the LDS)
 static int dysr_smem(int rt) { return dysr_ns(rt) * (TILE_BYTES + (rt >= 2 ? rt / 2 : 1) * 4096) + 2 * ROWS * rt * 32; }
-struct DysRingPlan { int n_slices, group, max_chunks; double cost; };   // cost: as DaPlan's
-// By bytes: the dY (+ B tile) stream over the busiest slot, the S blocks every workgroup fetches (from L2: half weight),
-// and the fp32 partials written here and read by the reduce (dS: one [rows, R] slab per slice; dB: one [N, R] slab per
-// chunk).  The cheapest plan whose partials take at most `limit` bytes (if none does: the cheapest of all).
+struct DysRingPlan { int n_slices, group, max_chunks; double us; };   // us: by the model above
+// The cheapest plan whose partials take at most `limit` bytes (if none does: the cheapest of all).
 static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = N / 64;
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
   const int slots = lds_slots(dysr_smem(rt));
-  const double tile_bytes = TILE_BYTES + 64.0 * R * 2;
   DysRingPlan best{1, 1, 1, 1e300};
   if (T < 2) return best;   // fewer than two column tiles: nothing to split (and no division by a zero slice count)
   GroupStats stats[kNGroups];
@@ -554,8 +563,8 @@ static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
     for (int k = 0; k < ng; k++) {
       const GroupStats& st = stats[k];
-      const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
-                          2.0 * 4.0 * R * ((double)nsl * rows + (double)st.chunks * N);
+      const double cost = ring_us(kDysModel[model_of(rt)], st, T, nsl, slots, 4e-6 * R * nsl * (double)rows, 4e-6 * R * (double)st.chunks * N,
+                                  2e-6 * (double)st.chunks * nsl * kGroups[k] * ROWS * R);
       const bool fits = ((size_t)nsl * rows * R + (size_t)nseg * st.max_chunks * N * R) * sizeof(float) <= limit;
       if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks, cost}; }
     }
@@ -762,14 +771,11 @@ constexpr int da_ns(int rt, int maskfmt) {
   return maskfmt ? (rt == 1 ? 3 : 5) : (rt == 4 ? 3 : 4);
 }
 static int da_ring_smem(int rt, int maskfmt) { return da_ns(rt, maskfmt) * (TILE_BYTES + da_mask_tile_bytes(maskfmt)) + 2 * ROWS * rt * 32; }
-struct DaPlan { int n_slices, group, max_chunks; double cost; };   // cost: bytes moved, by the model below
-// Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by bytes moved: the
-// X stream in whole rounds of resident workgroups, the dS blocks every workgroup fetches, and the fp32 partials
-// (one [R, K] slab per chunk, written here and read by the reduce).  `limit`: as for dysr_plan.
+struct DaPlan { int n_slices, group, max_chunks; double us; };
+// Slices of the K axis (balanced, 2 .. TPW tiles each) x chunks of `group` row blocks per segment, by the model above.  `limit`: as for dysr_plan.
 static DaPlan da_plan_of(int K, int R, int maskfmt, const int* blocks, int nseg, size_t limit) {
   const int rt = rt_of(R), T = K / 64;
   const int slots = lds_slots(da_ring_smem(rt, maskfmt));
-  const double tile_bytes = TILE_BYTES + da_mask_tile_bytes(maskfmt);
   DaPlan best{1, 1, 1, 1e300};
   if (T < 2) return best;   // as in dysr_plan
   GroupStats stats[kNGroups];
@@ -781,8 +787,7 @@ static DaPlan da_plan_of(int K, int R, int maskfmt, const int* blocks, int nseg,
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
     for (int k = 0; k < ng; k++) {
       const GroupStats& st = stats[k];
-      const double cost = ring_span(st, T, nsl, slots) * slots * tile_bytes + 0.5 * (double)st.chunks * nsl * kGroups[k] * ROWS * R * 2 +
-                          2.0 * 4.0 * R * K * (double)st.chunks;
+      const double cost = ring_us(kDaModel[maskfmt != 0][model_of(rt)], st, T, nsl, slots, 0.0, 4e-6 * R * K * (double)st.chunks, 2e-6 * (double)st.chunks * nsl * kGroups[k] * ROWS * R);
       const bool fits = (size_t)nseg * st.max_chunks * R * K * sizeof(float) <= limit;
       if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks, cost}; }
     }
@@ -818,7 +823,7 @@ size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit)
 struct DaForm { int direct_slices; double us; };   // 0: two stages
 static DaForm da_form(int M, int K, int R, bool masked, const LfSegTable& seg, size_t limit) {
   const int rt = rt_of(R), T = K / 64;
-  const double m = masked, two_stage = T < 2 ? 0.0 : 4.85 + 3.5 * m + da_plan(M, K, R, masked ? 2 : 0, seg, limit).cost / 5.39e6;
+  const double m = masked, two_stage = T < 2 ? 0.0 : da_plan(M, K, R, masked ? 2 : 0, seg, limit).us;
   const DaForm staged{0, two_stage};
   if (T < 2) return staged;
   int blocks[LF_MAX_SEG], nseg, live = 0, big = 0;
@@ -930,7 +935,7 @@ static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfS
     const double share = (double)(((rows + 63) / 64 * sl + 255) / 256) / sl;
     us += 1.3 + n * share * 4.28 * rt + (sl > 1 ? 1.71 * 4e-6 * sl * (double)rows * R : 0.0);
   }
-  const double old = 4.6 + 0.63 * rt + 0.201e-6 * dysr_plan(M, N, R, seg, SIZE_MAX).cost + da_form(M, K, R, masked, seg, SIZE_MAX).us;
+  const double old = dysr_plan(M, N, R, seg, SIZE_MAX).us + da_form(M, K, R, masked, seg, SIZE_MAX).us;
   return us * (big > 8 ? 1.06 : 1.0) < old ? g : ShortGrads{0, 0};   // (longer segments gain 1 - 2 % and are as often behind)
 }
 size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {

@@ -99,8 +99,8 @@ def test_against_float32(tokens, ranks, N, K, p, mask_kind, dtype):
 
 
 def test_long_segments_keep_the_two_passes():
-    """One workgroup would walk the 16 blocks of 2048 rows alone: dys_dyb and da in two stages are ahead there."""
-    M, N, K = 2048, 4096, 4096
+    """One workgroup would walk the 64 blocks of 8192 rows alone: dys_dyb and da in two stages are ahead there."""
+    M, N, K = 8192, 1024, 1024
     t = lambda *sh: torch.randn(*sh, device="cuda", dtype=torch.bfloat16)
-    *_, names = _bwd(t(M, N), t(M, K), None, True, t(M, 16), [t(N, 16)], [t(16, K)], [16], [1.0], [0.0], [M])
+    *_, names = _bwd(t(M, N), t(M, K), None, True, t(M, 16), [t(N, 16)], [t(16, K)], [64], [1.0], [0.0], [M])
     assert "dys_dyb" in names, names
