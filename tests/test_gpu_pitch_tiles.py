@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nn,M,N,K,kernel", [
     (False, 2800, 4096, 5120, "gemm_lora_kernel"), (False, 2800, 4096, 5248, "gemm_big_kernel"),   # a pitch of 10 KB and one beside it
     (False, 2800, 4096, 8192, "gemm_big_kernel"),                                                  # a power of two
-    (True, 2800, 4096, 5120, "gemm_big_kernel"), (True, 4000, 4096, 10240, "gemm_lora_kernel")])
+    (True, 2800, 4096, 5120, "gemm_big_kernel"), (True, 2800, 4096, 16384, "gemm_lora_kernel")])
 def test_kernel_and_result(nn, M, N, K, kernel):
     from lorafusion_amd.ops import hip_ops
 
