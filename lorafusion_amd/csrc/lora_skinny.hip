@@ -955,6 +955,19 @@ bool lf_short_grads_apply(const void* dY, const void* X, const uint8_t* mask, in
     at8 |= (uintptr_t)sg.ptr[s] | (uintptr_t)sg.out[s];
   }
   if ((at8 & 7) != 0 || (mask != nullptr && mask_bits && ((uintptr_t)mask & 3) != 0)) return false;
+  // Outputs over inputs stay with the two passes: those write dS (caller's scratch: it may lie over S) and dB once dY, S and B_i have been read, and two-stage dA
+  // once X, the mask and dS have.
+  struct Span { uintptr_t at, bytes; };
+  const auto span = [](const void* p, int64_t bytes) { return Span{(uintptr_t)p, p != nullptr ? (uintptr_t)bytes : 0}; };
+  const Span in[] = {span(dY, (int64_t)M * N * 2), span(S, (int64_t)M * R * 2), span(X, (int64_t)M * K * 2), span(mask, mask_bits ? (int64_t)M * K / 8 : (int64_t)M * K)};
+  const Span ds = span(dS, (int64_t)M * R * 2);
+  const auto meet = [](const Span& a, const Span& b) { return a.at < b.at + b.bytes && b.at < a.at + a.bytes; };
+  for (const Span& i : in) if (meet(ds, i)) return false;
+  for (int s = 0; s < (sb.table ? sb.n_seg : 1); s++) {
+    const Span b = span(sb.ptr[s], (int64_t)N * sb.rank[s] * 2), db = span(sg.ptr[s], (int64_t)N * sb.rank[s] * 2), da = span(sg.out[s], (int64_t)K * sb.rank[s] * 2);
+    if (meet(ds, b) || meet(ds, db) || meet(ds, da)) return false;
+    for (const Span& i : in) if (meet(db, i) || meet(da, i)) return false;
+  }
   if (short_grads(M, N, K, R, mask != nullptr, sb).a == 0) return false;
   return ws_bytes >= std::max(lf_ds_workspace(M, N, R, sb), std::max(lf_dys_dyb_workspace(M, N, R, sb, limit), lf_da_workspace(M, K, R, sb, limit)));
 }

@@ -14,8 +14,8 @@ from tests.util import kernels_of
 pytestmark = pytest.mark.gpu
 
 
-def _bwd(dy, x, mask, mask_bits, s, b, a, blocks, scales, ps, valid):
-    """dS, dA_i, dB_i of one packed batch (blocks: 128-row blocks of each segment; one segment: no routing tables)."""
+def _bwd(dy, x, mask, mask_bits, s, b, a, blocks, scales, ps, valid, ds=None):
+    """dS (in `ds`, if given), dA_i, dB_i of one packed batch (blocks: 128-row blocks of each segment; one segment: no routing tables)."""
     from lorafusion_amd import _lib as L
 
     M, N, K, R, n = dy.shape[0], dy.shape[1], x.shape[1], s.shape[1], len(b)
@@ -30,7 +30,8 @@ def _bwd(dy, x, mask, mask_bits, s, b, a, blocks, scales, ps, valid):
         per = lambda v: torch.tensor([v[seg] for seg, nb in enumerate(blocks) for _ in range(nb)], dtype=torch.float32, device="cuda")
         keep = (torch.tensor(table, dtype=torch.int32, device="cuda"), per(scales), per(ps))
         r = L.multi_routing([nb * 128 for nb in blocks], ranks, *keep, 128)
-    ds, da, db = torch.full_like(s, 7), [torch.full_like(t, 7) for t in a], [torch.full_like(t, 7) for t in b]
+    ds = torch.full_like(s, 7) if ds is None else ds
+    da, db = [torch.full_like(t, 7) for t in a], [torch.full_like(t, 7) for t in b]
     dt = L.dtype_id(dy.dtype) | (L.LF_MASK_BITS if mask_bits else 0)
     nbytes = L.lib().lf_workspace_bytes(L.LF_OP_BWD, M, N, K, R, ctypes.byref(r))
     ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
@@ -96,6 +97,22 @@ def test_against_float32(tokens, ranks, N, K, p, mask_kind, dtype):
         assert not ds[rs, ranks[i]:].any() and not ds[start[i] + tokens[i]:start[i] + rows[i]].any()
         _check(da[i], ds[real, :ranks[i]].float().T @ xt[real], f"dA {i}")
         _check(db[i], scales[i] * (dy[real].float().T @ s[real, :ranks[i]].float()), f"dB {i}")
+
+
+@pytest.mark.parametrize("over", ["S", "dY", "apart"])
+def test_scratch_over_an_input(over):
+    """dS_out is the caller's scratch: over S, or over dY of a call without a dX product, the gradients are what they are with a buffer of its own."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rn = lambda *sh: torch.randn(*sh, generator=g, device="cuda").bfloat16()
+    dy, x, s, b, a = rn(300, 512), rn(300, 512), rn(300, 16), [rn(512, 16)], [rn(16, 512)]
+    dyf, xf, sf = dy.float(), x.float(), s.float()
+    ds = {"S": s, "dY": dy.view(-1)[1024:1024 + 300 * 16].view(300, 16), "apart": None}[over]
+    ds, da, db, names = _bwd(dy, x, None, True, s, b, a, [3], [2.0], [0.0], [300], ds)
+    assert ("dys_dyb" in names) == (over != "apart"), names
+    e = 2 * (dyf @ b[0].float())
+    _check(ds, e, "dS")
+    _check(da[0], ds.float().T @ xf, "dA")
+    _check(db[0], 2 * (dyf.T @ sf), "dB")
 
 
 def test_long_segments_keep_the_two_passes():
