@@ -179,9 +179,8 @@ int lf_lora_bwd(const void* dY, const void* X, const void* W, const uint8_t* mas
  * of the dX product's split contraction, where it has one) go to a buffer of
  * LF_STATIC_SCRATCH_BYTES that is part of the library's device image (one copy per GPU, held until
  * the process ends); the call allocates and frees nothing.  A call that needs more than the buffer
- * holds (lf_workspace_bytes(LF_OP_BWD, ...) > LF_STATIC_SCRATCH_BYTES, and above 64 rank columns no
- * other split of the rank-r passes that fits) returns LF_ESTATIC and
- * enqueues nothing.  All calls on one GPU share the buffer: calls that may overlap on one GPU
+ * holds (lf_workspace_bytes(LF_OP_BWD, ...) > LF_STATIC_SCRATCH_BYTES, and no other split of the
+ * rank-r passes that fits) returns LF_ESTATIC and enqueues nothing.  All calls on one GPU share the buffer: calls that may overlap on one GPU
  * (different streams, or several host threads) race -- serialise them.  Nothing in the buffer has
  * to start at zero (every partial sum is written before it is read within the call), and its
  * contents after a call are unspecified.  The first call on a device looks up the buffer's

@@ -392,9 +392,9 @@ int lf_lora_bwd_static(const void* dY, const void* X, const void* W, const uint8
   int rc = make_seg(routing, M, nullptr, nullptr, t);
   if (rc != LF_OK) return rc;
   // what lf_workspace_bytes(LF_OP_BWD, ...) names: the rank-r passes' partial sums or the dX product's partial tiles,
-  // whichever is larger (with less, the product would not split its contraction and its sums would differ in order).  Above rank 64, where
-  // the fastest split has up to twice the partial sums of a slightly slower one, a split that fits is taken if there is one.
-  const size_t limit = R > 64 ? (size_t)LF_STATIC_SCRATCH_BYTES : SIZE_MAX;
+  // whichever is larger (with less, the product would not split its contraction and its sums would differ in order).  Where the fastest split of a pass
+  // has more partial sums than the buffer holds, the fastest that fits is taken; where none fits the call is refused.
+  constexpr size_t limit = LF_STATIC_SCRATCH_BYTES;
   const size_t a = lf_dys_dyb_workspace(M, N, R, t, limit), b = lf_da_workspace(M, K, R, t, limit);
   const size_t need = align256(std::max(std::max(a, b), lf_gemm_ksplit_bytes(M, K, N, t.table != nullptr ? t.block_size_m : 0, true)));
   if (need > (size_t)LF_STATIC_SCRATCH_BYTES) return LF_ESTATIC;

@@ -108,8 +108,9 @@ def test_size_query_and_static_backward_refuse_untiled_shapes():
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="an accepted call would launch on the test's made-up pointers")
-def test_static_backward_takes_high_ranks_whose_fastest_split_does_not_fit():
-    """The call gets as far as looking for a device.  One adapter, and packed rows."""
+def test_static_backward_takes_calls_whose_fastest_split_does_not_fit():
+    """The call gets as far as looking for a device.  One adapter, and packed rows; ranks above 64, and below (where the partial sums of a few slices or chunks
+    fit and those of the fastest split do not)."""
     from lorafusion_amd import _lib
 
     lib, one, ptrs = _lib.lib(), ctypes.c_void_p(256), (ctypes.c_void_p * 6)(*[256] * 6)
@@ -129,6 +130,13 @@ def test_static_backward_takes_high_ranks_whose_fastest_split_does_not_fit():
     for blocks, N, K in (([1, 1, 1], 13952, 3456), ([1, 1, 4, 2, 2], 5120, 256), ([2, 16, 1, 3, 1], 1280, 256)):
         r, keep = packed(blocks, [128] * len(blocks))
         assert call(128 * sum(blocks), N, K, 128, r) == _lib.LF_ELAUNCH
+    for M, N, K, rank in ((1358, 13952, 4352, 64),):
+        r = _lib.single_routing(rank, 1.0, 0.1)
+        assert call(M, N, K, rank, r) == _lib.LF_ELAUNCH
+    for blocks, N, K, rank in (([37, 34, 9, 12], 3840, 11648, 16), ([3, 72], 7808, 22784, 16), ([3, 12], 10880, 5376, 48), ([4, 3, 9, 19], 15360, 12032, 8),
+                               ([15, 9, 5], 5760, 19200, 48)):
+        r, keep = packed(blocks, [rank] * len(blocks))
+        assert call(128 * sum(blocks), N, K, (rank + 15) // 16 * 16, r) == _lib.LF_ELAUNCH
     assert call(9000, 8192, 8192, 128, _lib.single_routing(128, 1.0, 0.1)) == _lib.LF_ESTATIC    # no split fits
     assert call(128, 28672, 256, 64, _lib.single_routing(64, 1.0, 0.1)) != _lib.LF_OK
 
