@@ -504,8 +504,12 @@ static GroupStats group_stats(const int* blocks, int nseg, int g) {
 // Microseconds of a pass and its second stage: tiles and row blocks of the busiest slot, rounds of workgroups, partials in MB (dS: one [rows, R] slab per slice; dB or dA: one slab per
 // chunk), the side operand that every workgroup fetches per block in MB, and the share of a slot if all tiles were spread evenly.  Fitted, by rank tiling, to 35 plans each of 2423
 // batches (700 - 16400 rows in 1 - 8 segments, 1024 - 14336 columns): on shapes that were not fitted dys_dyb is 5.5 % behind the best plan timed, dA 2.4 % and without a mask 1.8 %;
-// the bytes moved, by which plans were chosen before, 8.5, 3.9 and 5.9 %.  2048 x 4096 rank 16: dys_dyb 15.4 -> 13.3, dA 13.6 -> 11.8; the eight-tile slices of the byte model
-// leave three quarters of the compute units idle there.
+// the bytes moved, by which plans were chosen before, 8.5, 3.9 and 5.9 %.  (The eight-tile slices of the byte model leave three quarters of the compute units idle at 2048 x 4096.)
+// Then each model was put on the scale of a second campaign (a factor and a constant, which leave its choice of plans alone): there these two passes, direct dA and the short
+// backward below were timed the same way, twelve launches a graph, 10200 batches (60 - 16400 rows in 1 - 8 segments, N 1024 - 14336, K 1024 - 8192, ranks 8 - 128, with keep bits
+// and without).  On a quarter of them that was not fitted dys_dyb is 8 % off at ranks to 32 and 13 % above, dA 5 - 10 %, and the two in a row take their sum.  Measured (model), us, x
+// 4096 columns at rank 16: dys_dyb of 1000 rows 10.7 (10.7), 2048 13.6 (13.3), 3000 14.3 (15.5); dA with keep bits 9.3 (9.9), 13.6 (12.5), 14.7 (14.8), without 7.7 (8.0), 9.6 (9.7),
+// 10.5 (11.0).
 struct RingModel { double fixed, tile, block, round, ds, slab, side, even; };
 static double ring_us(const RingModel& m, const GroupStats& r, int T, int nsl, int slots, double ds_mb, double slab_mb, double side_mb) {
   const int t_max = (T + nsl - 1) / nsl;
@@ -515,12 +519,12 @@ static double ring_us(const RingModel& m, const GroupStats& r, int T, int nsl, i
   return m.fixed + m.tile * span + m.block * blocks + m.round * rounds + m.ds * ds_mb + m.slab * slab_mb + m.side * side_mb + m.even * even;
 }
 static int model_of(int rt) { return rt >= 8 ? 3 : rt >= 4 ? 2 : rt >= 2 ? 1 : 0; }
-static const RingModel kDysModel[4] = {{8.66, 0.166, 0.237, 1.13, 0.081, 0.429, 0.609, 1.074}, {9.36, 0.276, 0.505, 0.87, 0.193, 0.434, 0.279, 0.464},
-                                       {9.19, 0.346, 0.120, 2.42, 0.251, 0.271, 0.167, 0.0}, {7.22, 0.764, 0.456, 3.44, 0.150, 0.238, 0.220, 0.064}};
-static const RingModel kDaModel[2][4] = {{{7.73, 0.243, 0.055, 0.47, 0.0, 0.846, 0.032, 0.658}, {10.27, 0.216, 0.268, 0.0, 0.0, 0.595, 0.078, 0.577},
-                                          {8.01, 0.271, 0.0, 0.89, 0.0, 0.329, 0.045, 0.617}, {10.25, 0.541, 0.002, 2.39, 0.0, 0.324, 0.055, 0.0}},
-                                         {{9.29, 0.558, 0.012, 3.44, 0.0, 0.425, 0.310, 0.760}, {9.44, 0.556, 0.082, 0.74, 0.0, 0.572, 0.322, 0.0},
-                                          {10.92, 0.622, 0.0, 1.29, 0.0, 0.431, 0.132, 0.0}, {14.39, 0.581, 0.014, 1.87, 0.0, 0.286, 0.067, 0.0}}};   // without and with a keep-mask
+static const RingModel kDysModel[4] = {{5.779, 0.184, 0.263, 1.256, 0.090, 0.477, 0.677, 1.194}, {5.803, 0.358, 0.656, 1.130, 0.251, 0.564, 0.362, 0.602},
+                                       {3.217, 0.643, 0.223, 4.497, 0.466, 0.504, 0.310, 0.0}, {6.341, 0.956, 0.571, 4.305, 0.188, 0.298, 0.275, 0.080}};
+static const RingModel kDaModel[2][4] = {{{4.711, 0.256, 0.058, 0.496, 0.0, 0.892, 0.034, 0.694}, {5.569, 0.227, 0.282, 0.0, 0.0, 0.626, 0.082, 0.607},
+                                          {4.813, 0.334, 0.0, 1.095, 0.0, 0.405, 0.055, 0.759}, {3.906, 0.758, 0.003, 3.348, 0.0, 0.454, 0.077, 0.0}},
+                                         {{1.255, 0.733, 0.016, 4.521, 0.0, 0.559, 0.407, 0.999}, {5.160, 0.711, 0.105, 0.946, 0.0, 0.731, 0.412, 0.0},
+                                          {4.415, 0.829, 0.0, 1.720, 0.0, 0.575, 0.176, 0.0}, {4.659, 1.024, 0.025, 3.297, 0.0, 0.504, 0.118, 0.0}}};   // without and with a keep-mask
 static void seg_block_counts(int M, const LfSegTable& seg, int* blocks, int& nseg) {
   nseg = seg.table ? seg.n_seg : 1;
   for (int s = 0; s < nseg; s++) {
@@ -814,11 +818,10 @@ size_t lf_da_workspace(int M, int K, int R, const LfSegTable& seg, size_t limit)
 // One launch without a second stage: a workgroup walks all row blocks of its segment over t tiles of columns and stores the sums as
 // they are.  Alone on its compute unit, it has a deeper ring and more dS buffers than the two-stage form: what a walk of one or
 // two tiles per block needs to keep loads on order.  It pays where segments have few blocks (a tile costs a workgroup 0.4 us, with a
-// mask 0.9, one after the other) or the partials are large (high ranks, wide inputs).  Both sides in microseconds, fitted to
-// 496 products (128 - 16384 rows in one or four segments, K 1024 - 14336, ranks 16 - 128, with keep bits and without), direct 9 % and
-// two-stage 16 % off; the choice gives 17 % over them all, 18 is the most any choice gives, 8 are behind by more than 3 % (worst 11).
-// With keep bits, two-stage -> direct: 300 x 4096 rank 16 8.8 -> 7.8, four segments of 1280 x 4096 rank 64 14.7 -> 9.3, of 2048 x 4096 rank 16
-// 13.3 -> 10.5; the other side of the line: 1000 x 4096 rank 16 in one segment 9.7 against 14.4.
+// mask 0.9, one after the other) or the partials are large (high ranks, wide inputs).  Both sides in microseconds on one scale (ring_us): over its 14100 products direct is 6.5 % off,
+// the choice takes 0.3 % more than the faster form of each, 2.8 % of them more than 3 % (worst 1.5 times).
+// With keep bits, two-stage -> direct: 300 x 4096 rank 16 7.9 -> 7.7, four segments of 1280 x 4096 rank 64 13.6 -> 9.9; the other side of the line: 1000 x 4096 rank 16 in one
+// segment 9.3 against 13.7, without a mask 7.7 against 9.5.
 // (the same choice for every mask format: dA does not depend on how the mask came)
 struct DaForm { int direct_slices; double us; };   // 0: two stages
 static DaForm da_form(int M, int K, int R, bool masked, const LfSegTable& seg, size_t limit) {
@@ -836,7 +839,7 @@ static DaForm da_form(int M, int K, int R, bool masked, const LfSegTable& seg, s
   const int nsl = (T + t - 1) / t;
   const double tiles = (double)big * t;
   const double direct = 3.66 + 0.40 * m + 0.20 * rt + tiles * (0.305 + 0.466 * m + 0.049 * rt) + 0.357 * big + 0.9e-3 * tiles * nsl * live;
-  return 1.05 * direct < two_stage ? DaForm{nsl, direct} : staged;
+  return direct < two_stage ? DaForm{nsl, direct} : staged;
 }
 
 // (lora_da_direct.hip)  mask_fmt: the kernel's MASK
@@ -904,10 +907,10 @@ int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* 
 // ---- the rank-r part of a short backward in two or three launches: dS on its own (complete, lora_stream.hip), then dA and dB side by side as sums over rows
 // (lora_da_direct.hip), where dys_dyb and da take three to five.  dY is read twice; what goes is the fp32 partials of dS and dB, their second stage and the walk of
 // da behind that of dys_dyb.  Behind where one workgroup walks many blocks (a tile costs it 0.4 us, with a mask 0.9).
-// Both sides in microseconds, fitted to 1250 backwards without the dX product (60 - 6000 rows in 1 - 8 segments, N 1024 - 14336, K 1024 - 8192, ranks 8 - 128, with keep
-// bits and without; 10 % off each) and checked on 540 more: the choice takes 0.89 of the old way's time over them, 0.876 is the least any choice takes, 30 are
-// more than 3 % slower (worst 1.25).  With keep bits, replayed from a graph: 300 x 4096 x 4096 rank 16 16.7 -> 13.0, four segments of 1280 rows rank 64 31.7 -> 24.2, 788 x 2944 x
-// 3328 rank 64 28.5 -> 23.2; the other side of the line: 2048 x 4096 x 4096 rank 16 28.0 against 31.1, 3000 x 5120 x 5120 rank 128 62 against 89.
+// Both sides in microseconds on one scale (ring_us); the short side fitted to the same batches, 7 % off on those that were not.  On these the choice takes 0.914 of the two passes' time (the
+// faster form of dA among them) and 1.1 % more than the best of every form; 2.7 % are more than 3 % slower than the two passes (worst 1.2 times).  With keep bits, replayed from a graph, two
+// passes -> short: 300 x 4096 x 4096 rank 16 16.3 -> 12.8, four segments of 1280 rows rank 64 26.7 -> 24.1; the line: 1000 x 4096 x 4096 rank 16 20.7 either way; the other side of it: 1500 rows
+// 23.8 against 25.7, 2048 28.0 against 31.0 (without a mask 22.0 against 22.5), 3000 x 5120 x 5120 rank 128 60 against 88.
 size_t lf_ds_workspace(int M, int N, int R, const LfSegTable& seg);   // (lora_stream.hip)
 int lf_launch_ds(const void* dY, void* dS, void* ws, int M, int N, int R, const LfSegTable& seg, int dtype, hipStream_t st);
 
@@ -925,18 +928,19 @@ static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfS
   if (t > da_tpw(rt)) return {0, 0};
   const ShortGrads g{slices(TA, t), slices(TB, t)};
   const int64_t rows = seg.table ? (int64_t)seg.n_blocks * ROWS : M;
-  const double m = masked, tiles = (double)big * t, n = N / 4096.0;
-  double us = 7.1 + 0.59 * rt + tiles * (0.387 + 0.484 * m) + 0.196 * big + 0.9e-3 * tiles * (g.a + g.b) * live;
+  const double m = masked, tiles = (double)big * t, n = N / 4096.0, full = (g.a + g.b) * live / 256.0;
+  double us = 5.34 + 0.806 * rt + tiles * (0.368 + 0.517 * m) + 0.443 * big + 1.49 * t * full;
   if (R <= 32) {
     const double groups = (double)((rows + 15) / 16) / 256;
-    us += n * (0.42 + 1.7 * rt + 5.3 * std::min(groups, 1.0) + 7.6 * std::max(groups - 1.0, 0.0));
+    us += n * (0.29 + 1.73 * rt + 2.47 * std::min(groups, 1.0) + 10.7 * std::max(groups - 1.0, 0.0));
   } else {
     const int sl = lf_xa_stream_slices(M, N, R, false, seg);
     const double share = (double)(((rows + 63) / 64 * sl + 255) / 256) / sl;
-    us += 1.3 + n * share * 4.28 * rt + (sl > 1 ? 1.71 * 4e-6 * sl * (double)rows * R : 0.0);
+    us += 0.665 + n * share * 5.21 * rt + (sl > 1 ? 4e-6 * sl * (double)rows * R : 0.0);
   }
   const double old = dysr_plan(M, N, R, seg, SIZE_MAX).us + da_form(M, K, R, masked, seg, SIZE_MAX).us;
-  return us * (big > 8 ? 1.06 : 1.0) < old ? g : ShortGrads{0, 0};   // (longer segments gain 1 - 2 % and are as often behind)
+  // (longer segments gain 1 - 2 % and are as often behind; where the workgroups take almost all compute units the model is 11 % off and not 5)
+  return us * (big > 8 ? 1.06 : 1.0) * (full > 0.9 ? 1.1 : 1.0) < old ? g : ShortGrads{0, 0};
 }
 size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {
   for (const bool masked : {false, true})

@@ -71,3 +71,17 @@ def test_segments(seq, ranks, p_list, K):
     xd, dsd = x.cuda(), ds.cuda()
     for i, got in enumerate(_direct(lambda: hip_ops.fused_multi_lora_da(xd, dsd, routing, mask))):
         _close(got, exp[i], f"adapter {i}")
+
+
+@pytest.mark.parametrize("M,K,r,p", [(1000, 4096, 16, 0.1), (1000, 4096, 16, 0.0), (2048, 4096, 16, 0.1), (3000, 5120, 128, 0.1)])
+def test_long_segments_take_two_stages(M, K, r, p):
+    """One workgroup would walk 8 blocks and more alone: chunks of blocks and a second stage are ahead (1000 x 4096 with keep bits 9.3 against 13.7 us)."""
+    from lorafusion_amd.ops import hip_ops
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, ds = torch.randn(M, K, generator=g, device="cuda").bfloat16(), (torch.randn(M, r, generator=g, device="cuda") * 0.1).bfloat16()
+    keep = torch.rand(M, K, generator=g, device="cuda") >= p
+    bits = hip_ops.pack_mask(keep) if p else None
+    da, names = kernels_of(lambda: hip_ops.fused_lora_da(x, ds, r, p, bits))
+    assert "reduce_segments_kernel" in names, names
+    _close(da, (ds.float().T @ torch.where(keep, x.float(), torch.zeros((), device="cuda")) / (1 - p)).cpu(), "dA")

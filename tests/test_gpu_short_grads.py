@@ -121,3 +121,12 @@ def test_long_segments_keep_the_two_passes():
     t = lambda *sh: torch.randn(*sh, device="cuda", dtype=torch.bfloat16)
     *_, names = _bwd(t(M, N), t(M, K), None, True, t(M, 16), [t(N, 16)], [t(16, K)], [64], [1.0], [0.0], [M])
     assert "dys_dyb" in names, names
+
+
+@pytest.mark.parametrize("M,masked,short", [(300, True, True), (300, False, True), (1500, True, False), (2048, True, False), (2048, False, False)])
+def test_either_side_of_the_line(M, masked, short):
+    """4096 x 4096 at rank 16: the short way to about 1000 rows of one segment with keep bits; at 2048 the two passes are ahead with a mask (28.0 against 31.0 us) and without."""
+    t = lambda *sh: torch.randn(*sh, device="cuda", dtype=torch.bfloat16)
+    mask = torch.randint(0, 256, (M, 512), device="cuda", dtype=torch.uint8) if masked else None
+    *_, names = _bwd(t(M, 4096), t(M, 4096), mask, True, t(M, 16), [t(4096, 16)], [t(16, 4096)], [(M + 127) // 128], [2.0], [0.1 if masked else 0.0], [M])
+    assert ("dys_dyb" not in names) == short, names
