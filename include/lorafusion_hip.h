@@ -210,7 +210,8 @@ int lf_gemm(const void* A, const void* B, const void* bias, void* C, int M, int 
  * K >= 256 and bit-packed keep-masks).  Returns LF_EINVAL for 9 and outside -1..15. */
 int lf_set_tile_cfg(int tile_cfg);
 
-/* The launches the library makes for an M x N output contracted over K when no configuration is pinned: rows
+/* The launches the library makes for an M x N output contracted over K when no configuration is pinned, in a call that has the workspace of the whole forward or backward
+ * (without one left-over rows cannot run in slices of K, and fewer products have them): rows
  * [0, *rows_head) as one launch of tile configuration *cfg_head and, when *rows_head < M, the rest
  * as a second launch of *cfg_tail (-1 when there is none).  Every number names one kernel and tile: 4, 6 and 9 are the 128x128, 128x64 and
  * 192x128 tiles of the general kernel, 11, 12 and 13 (with 10, 14 and 15) those of the kernel for outputs of about one round.  A launch may still move to another tile: a call whose

@@ -900,6 +900,10 @@ static KSplit cheapest_slices(int M, int N, int K, int routing_block, bool nn, b
   }
   return best;
 }
+// Whether any tile leaves room for two slices: most of the row counts that choose_split prices do not, and need no search.
+static bool may_slice(int M, int N) {
+  return 2 * tiles_of(M, N, cand_of(1)) <= 256 || 2 * tiles_of(M, N, cand_of(4)) <= 512;
+}
 static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn, bool mid) {
   const int nk = K / BK;
   KSplit best = {cfg, 1, nk};
@@ -917,9 +921,9 @@ static KSplit ksplit_of(int M, int N, int K, int cfg, int routing_block, bool nn
 // with the lowest modelled cost of both launches: usually the one whose tiles fill whole rounds of the chip
 // (32 tile rows of 40 tiles are exactly five rounds; 30 rows of 40 are five rounds too, and leave a longer tail).
 // Returns m_main (0: single launch).
-// (Left-over rows over a long K run in slices where the call has memory for them, as the whole forward and backward do, and are priced that way: unsliced, 512 rows x 8192 over
-// 57344 look 60 us dearer than 256, they are 190.)
-static int choose_split(int M, int N, int K, int routing_block, bool allow_big, bool wave96, bool mid, int* cfg_head, int* cfg_tail) {
+// sliced: the call has memory for slices, as the whole forward and backward do: left-over rows over a long K run in slices then and are priced that way (unsliced, 512 rows x
+// 8192 over 57344 look 60 us dearer than 256, they are 190).  With the smaller limit of the two products, so that both have one plan.
+static int choose_split(int M, int N, int K, int routing_block, bool sliced, bool allow_big, bool wave96, bool mid, int* cfg_head, int* cfg_tail) {
   constexpr double kLaunch = 4.0;  // a second launch
   const int grid_n = (N + 255) / 256;
   if (grid_n > 256) return 0;
@@ -933,7 +937,7 @@ static int choose_split(int M, int N, int K, int routing_block, bool allow_big, 
     if (head_cost >= best) break;
     double tail;
     const int ct = choose_cfg(M - r * 256, N, K, allow_big, wave96, mid, &tail, true);
-    if (K >= 1024) cheapest_slices(M - r * 256, N, K, routing_block, /*nn=*/true, mid, {ct, 1, K / BK}, tail);
+    if (sliced && K >= 1024 && may_slice(M - r * 256, N)) cheapest_slices(M - r * 256, N, K, routing_block, /*nn=*/true, mid, {ct, 1, K / BK}, tail);
     if (head_cost + tail < best) { best = head_cost + tail; best_m = r * 256; *cfg_tail = ct; }
   }
   *cfg_head = big ? 7 : 1;
@@ -953,12 +957,12 @@ int lf_pin_tile_cfg(int cfg) {
 }
 bool lf_tile_pinned() { return pinned_cfg.load(std::memory_order_relaxed) >= 0; }
 
-// The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned: rows [0, *rows_head)
-// with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).
-static void plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
+// The launches lf_launch_gemm makes for an M x N product over K when no configuration is pinned (sliced: and the call has the memory that
+// lf_gemm_ksplit_bytes names): rows [0, *rows_head) with *cfg_head and, when *rows_head < M, the remaining rows with *cfg_tail (-1 otherwise).
+static void plan_gemm(int M, int N, int K, int routing_block, bool sliced, int* rows_head, int* cfg_head, int* cfg_tail) {
   const bool allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0), wave96 = wave96_fits(routing_block);
   int ch = 1, ct = 1;
-  const int m_main = choose_split(M, N, K, routing_block, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
+  const int m_main = choose_split(M, N, K, routing_block, sliced, allow_big, wave96, /*mid=*/wave96, &ch, &ct);
   // A long contraction under a wide output runs faster on the eight-wave 256x256 tile than on the persistent kernel
   // (8192 x 8192 over 28672: 3.08 against 3.24 ms, over 57344: 5.74 against 5.85; at 4096 columns the two are level, and
   // at shorter contractions the persistent kernel is 3-8 % ahead): its long K loops let the tiles of an XCD drift apart
@@ -979,12 +983,12 @@ static void plan_gemm(int M, int N, int K, int routing_block, int* rows_head, in
   }
 }
 
-void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail) {
+void lf_plan_gemm(int M, int N, int K, int routing_block, bool sliced, int* rows_head, int* cfg_head, int* cfg_tail) {
   struct Plan { int rows, head, tail; };
-  static thread_local LfMemo<Plan, 4> memo;
-  const Plan pl = memo.get({M, N, K, routing_block}, [&] {
+  static thread_local LfMemo<Plan, 5> memo;
+  const Plan pl = memo.get({M, N, K, routing_block, sliced}, [&] {
     Plan q;
-    plan_gemm(M, N, K, routing_block, &q.rows, &q.head, &q.tail);
+    plan_gemm(M, N, K, routing_block, sliced, &q.rows, &q.head, &q.tail);
     return q;
   });
   *rows_head = pl.rows, *cfg_head = pl.head, *cfg_tail = pl.tail;
@@ -995,7 +999,7 @@ void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* c
 static size_t ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
   if (M <= 0 || N <= 0 || K < BK) return 0;
   int rows = 0, ch = 1, ct = -1;
-  lf_plan_gemm(M, N, K, routing_block, &rows, &ch, &ct);
+  lf_plan_gemm(M, N, K, routing_block, /*sliced=*/true, &rows, &ch, &ct);
   size_t need = 0;
   const bool wave96 = wave96_fits(routing_block), allow_big = routing_block <= 0 || (routing_block % 128 == 0 && M % 128 == 0);
   auto part = [&](int m, int cfg) {
@@ -1083,7 +1087,8 @@ int lf_launch_gemm(const LfGemmParams& p, const LfSegTable& seg, bool nn, int dt
   };
   if (force_cfg >= 0) return launch(p, force_cfg);
   int m_main = 0, cfg_head = 1, cfg_tail = -1;
-  lf_plan_gemm(p.M, p.N, p.K, seg.table != nullptr ? seg.block_size_m : 0, &m_main, &cfg_head, &cfg_tail);
+  const bool sliced = p.ks_ws != nullptr && ((uintptr_t)p.ks_ws & 15) == 0 && p.ks_ws_bytes >= lf_gemm_ksplit_bytes(p.M, p.N, p.K, rblock, nn);
+  lf_plan_gemm(p.M, p.N, p.K, rblock, sliced, &m_main, &cfg_head, &cfg_tail);
   if (cfg_tail < 0) return launch(p, cfg_head);
   LfGemmParams head = p, tail = p;
   head.M = m_main;

@@ -408,7 +408,7 @@ int lf_set_tile_cfg(int tile_cfg) { return lf_pin_tile_cfg(tile_cfg); }
 
 int lf_gemm_plan(int M, int N, int K, int routing_block_size_m, int* rows_head, int* cfg_head, int* cfg_tail) {
   if (M <= 0 || N <= 0 || K <= 0 || rows_head == nullptr || cfg_head == nullptr || cfg_tail == nullptr) return LF_EINVAL;
-  lf_plan_gemm(M, N, K, routing_block_size_m, rows_head, cfg_head, cfg_tail);
+  lf_plan_gemm(M, N, K, routing_block_size_m, /*sliced=*/true, rows_head, cfg_head, cfg_tail);
   return LF_OK;
 }
 

@@ -77,7 +77,7 @@ int lf_launch_gemm_mid(const LfGemmParams& p, const LfSegTable& seg, bool nn, in
 int lf_cu_count();
 int lf_pin_tile_cfg(int cfg);  // -1: automatic choice
 bool lf_tile_pinned();
-void lf_plan_gemm(int M, int N, int K, int routing_block, int* rows_head, int* cfg_head, int* cfg_tail);
+void lf_plan_gemm(int M, int N, int K, int routing_block, bool sliced, int* rows_head, int* cfg_head, int* cfg_tail);
 size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn);  // workspace of the split contraction for this product
 
 // The last results of a plan (a function of sizes alone) on this thread: planning a forward + backward took 5 us of host time, more than

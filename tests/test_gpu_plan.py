@@ -160,3 +160,23 @@ def test_one_round_over_a_long_contraction(M, N, K, nn, sliced):
         exp = x.float() @ wt.float() + ds[:, :r].float() @ at.float()
     assert ("ksplit_reduce_kernel" in names) == sliced and ("gemm_mid_kernel" in names) != sliced, names
     _close(got, exp.cpu(), "dX" if nn else "Y")
+
+
+def test_left_over_rows_are_priced_in_slices_only_where_there_is_memory():
+    """Rows behind whole rounds of 256x256 tiles run in slices of K in the whole forward, which has memory for them.  Without memory they would run unsliced, and one launch of
+    128x256 tiles is the cheaper plan."""
+    from lorafusion_amd import _lib as L
+    from lorafusion_amd.ops import hip_ops
+
+    M, N, K, r = 4882, 3200, 3584, 16
+    assert _planned(M, N, K)[0] < M
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rn = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).bfloat16()
+    x, w, a, b = rn(M, K), rn(N, K, std=0.02), rn(r, K, std=K ** -0.5), rn(N, r, std=0.01)
+    exp = x.float() @ w.float().T
+    y, names = kernels_of(lambda: hip_ops.gemm(x, w))
+    assert "gemm_big_kernel" in names and "gemm_lora_kernel" not in names and "gemm_mid_kernel" not in names, names
+    _close(y, exp.cpu(), "alone")
+    (y, s), names = kernels_of(lambda: hip_ops.lora_forward(x, w, [a], [b], L.single_routing(r, 2.0, 0.0), L.round_rank(r), None, None))
+    assert "gemm_big_kernel" in names and ("gemm_lora_kernel" in names or "gemm_mid_kernel" in names) and "ksplit" in names, names
+    _close(y, (exp + 2.0 * s[:, :r].float() @ b.float().T).cpu(), "forward")
