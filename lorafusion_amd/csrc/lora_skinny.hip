@@ -30,6 +30,9 @@
 #include "lf_common.h"
 #include "act_math.h"
 #include "rank_ring.h"
+#include <algorithm>
+#include <cmath>
+#include <numeric>
 #include <type_traits>
 
 namespace {
@@ -487,9 +490,11 @@ lora_dys_dyb_ring_kernel(const T* __restrict__ dY, const T* __restrict__ S, floa
 // ---- work split of the ring kernels.  Workgroups (slice x chunk) of w tiles each run on `slots` resident slots; the
 // pass lasts about as long as its busiest slot.  Two upper bounds of that (in tiles): whole rounds of the largest
 // workgroup, and the list-scheduling bound sum / slots + largest; the smaller one is the estimate (ring_us).
-struct GroupStats { long chunks, total; int max_chunks, big; };   // of one chunk length: independent of the slices
+// Of one chunk length, independent of the slices.  busy: workgroups per slice on the busiest of the eight XCDs when the grid is [segments * max_chunks, slices] and an id's XCD is its remainder:
+// columns beyond a segment's last chunk end at once, and where the row of the grid is a multiple of 2, 4 or 8 the others can share a few remainders.
+struct GroupStats { long chunks, total; int max_chunks, big; double busy; };
 static GroupStats group_stats(const int* blocks, int nseg, int g) {
-  GroupStats r{0, 0, 1, 0};
+  GroupStats r{0, 0, 1, 0, 0.0};
   for (int s = 0; s < nseg; s++) {
     const int c = (blocks[s] + g - 1) / g;
     if (c <= 0) continue;
@@ -499,6 +504,13 @@ static GroupStats group_stats(const int* blocks, int nseg, int g) {
     r.big = sz > r.big ? sz : r.big;
     r.total += blocks[s];
   }
+  const int period = std::gcd(nseg * r.max_chunks, 8);
+  long at[8] = {};
+  for (int s = 0; s < nseg; s++) {
+    const int c = (blocks[s] + g - 1) / g;
+    for (int q = 0; q < period; q++) at[(s * r.max_chunks + q) % period] += c / period + (q < c % period ? 1 : 0);
+  }
+  r.busy = *std::max_element(at, at + period) * period / 8.0;
   return r;
 }
 // Microseconds of a pass and its second stage: tiles and row blocks of the busiest slot, rounds of workgroups, partials in MB (dS: one [rows, R] slab per slice; dB or dA: one slab per
@@ -511,9 +523,12 @@ static GroupStats group_stats(const int* blocks, int nseg, int g) {
 // 4096 columns at rank 16: dys_dyb of 1000 rows 10.7 (10.7), 2048 13.6 (13.3), 3000 14.3 (15.5); dA with keep bits 9.3 (9.9), 13.6 (12.5), 14.7 (14.8), without 7.7 (8.0), 9.6 (9.7),
 // 10.5 (11.0).
 struct RingModel { double fixed, tile, block, round, ds, slab, side, even; };
-static double ring_us(const RingModel& m, const GroupStats& r, int T, int nsl, int slots, double ds_mb, double slab_mb, double side_mb) {
+static double ring_us(const RingModel& m, const GroupStats& r, int T, int nsl, int slots, bool chunk_rows, double ds_mb, double slab_mb, double side_mb) {
   const int t_max = (T + nsl - 1) / nsl;
-  const double rounds = (double)((r.chunks * nsl + slots - 1) / slots), even = (double)r.total * T / slots, largest = (double)r.big * t_max;
+  // (chunk_rows: the grid of `busy`.  eight adapters of 7, 2, 2, 2, 2, 1, 1 and 2 blocks, 10752 columns, rank 64: 231 workgroups in chunks of two, four columns on each of two XCDs, 71.7 us; 456 in chunks
+  // of one 50.7.  With the busiest XCD's rounds the plan is 1.2 % behind the best one timed at ranks 33 - 64 and 0.9 % above, with the chip's 3.1 and 1.9)
+  const double chip = (double)((r.chunks * nsl + slots - 1) / slots), rounds = chunk_rows ? std::max(chip, std::ceil(std::ceil(r.busy * nsl) / (slots / 8))) : chip;
+  const double even = (double)r.total * T / slots, largest = (double)r.big * t_max;
   const double span = std::max(std::min(rounds * largest, even + largest), even);
   const double blocks = std::max(std::min(rounds * r.big, (double)r.total * nsl / slots + r.big), 1.0);
   return m.fixed + m.tile * span + m.block * blocks + m.round * rounds + m.ds * ds_mb + m.slab * slab_mb + m.side * side_mb + m.even * even;
@@ -567,7 +582,7 @@ static DysRingPlan dysr_plan_of(int M, int N, int R, const int* blocks, int nseg
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
     for (int k = 0; k < ng; k++) {
       const GroupStats& st = stats[k];
-      const double cost = ring_us(kDysModel[model_of(rt)], st, T, nsl, slots, 4e-6 * R * nsl * (double)rows, 4e-6 * R * (double)st.chunks * N,
+      const double cost = ring_us(kDysModel[model_of(rt)], st, T, nsl, slots, true, 4e-6 * R * nsl * (double)rows, 4e-6 * R * (double)st.chunks * N,
                                   2e-6 * (double)st.chunks * nsl * kGroups[k] * ROWS * R);
       const bool fits = ((size_t)nsl * rows * R + (size_t)nseg * st.max_chunks * N * R) * sizeof(float) <= limit;
       if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DysRingPlan{nsl, kGroups[k], st.max_chunks, cost}; }
@@ -791,7 +806,7 @@ static DaPlan da_plan_of(int K, int R, int maskfmt, const int* blocks, int nseg,
     if (nsl > T / 2 || (T + nsl - 1) / nsl != t) continue;
     for (int k = 0; k < ng; k++) {
       const GroupStats& st = stats[k];
-      const double cost = ring_us(kDaModel[maskfmt != 0][model_of(rt)], st, T, nsl, slots, 0.0, 4e-6 * R * K * (double)st.chunks, 2e-6 * (double)st.chunks * nsl * kGroups[k] * ROWS * R);
+      const double cost = ring_us(kDaModel[maskfmt != 0][model_of(rt)], st, T, nsl, slots, false, 0.0, 4e-6 * R * K * (double)st.chunks, 2e-6 * (double)st.chunks * nsl * kGroups[k] * ROWS * R);
       const bool fits = (size_t)nseg * st.max_chunks * R * K * sizeof(float) <= limit;
       if (fits == best_fits ? cost < best_cost : fits) { best_fits = fits; best_cost = cost; best = DaPlan{nsl, kGroups[k], st.max_chunks, cost}; }
     }
@@ -908,7 +923,7 @@ int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* 
 // (lora_da_direct.hip), where dys_dyb and da take three to five.  dY is read twice; what goes is the fp32 partials of dS and dB, their second stage and the walk of
 // da behind that of dys_dyb.  Behind where one workgroup walks many blocks (a tile costs it 0.4 us, with a mask 0.9).
 // Both sides in microseconds on one scale (ring_us); the short side fitted to the same batches, 7 % off on those that were not.  On these the choice takes 0.914 of the two passes' time (the
-// faster form of dA among them) and 1.1 % more than the best of every form; 2.7 % are more than 3 % slower than the two passes (worst 1.2 times).  With keep bits, replayed from a graph, two
+// faster form of dA among them) and 0.8 % more than the best of every form; 3.4 % are more than 3 % slower than the two passes (worst 1.2 times).  With keep bits, replayed from a graph, two
 // passes -> short: 300 x 4096 x 4096 rank 16 16.3 -> 12.8, four segments of 1280 rows rank 64 26.7 -> 24.1; the line: 1000 x 4096 x 4096 rank 16 20.7 either way; the other side of it: 1500 rows
 // 23.8 against 25.7, 2048 28.0 against 31.0 (without a mask 22.0 against 22.5), 3000 x 5120 x 5120 rank 128 60 against 88.
 size_t lf_ds_workspace(int M, int N, int R, const LfSegTable& seg);   // (lora_stream.hip)
@@ -940,7 +955,7 @@ static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfS
   }
   const double old = dysr_plan(M, N, R, seg, SIZE_MAX).us + da_form(M, K, R, masked, seg, SIZE_MAX).us;
   // (longer segments gain 1 - 2 % and are as often behind; where the workgroups take almost all compute units the model is 11 % off and not 5)
-  return us * (big > 8 ? 1.06 : 1.0) * (full > 0.9 ? 1.1 : 1.0) < old ? g : ShortGrads{0, 0};
+  return us * (big > 8 ? 1.03 : 1.0) * (full > 0.9 ? 1.05 : 1.0) < old ? g : ShortGrads{0, 0};
 }
 size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {
   for (const bool masked : {false, true})

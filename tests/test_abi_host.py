@@ -141,6 +141,21 @@ def test_static_backward_takes_calls_whose_fastest_split_does_not_fit():
     assert call(128, 28672, 256, 64, _lib.single_routing(64, 1.0, 0.1)) != _lib.LF_OK
 
 
+def test_chunks_of_a_packed_batch_spread_over_the_dies():
+    """Workgroups are dealt to the eight dies by their index, chunks beyond a segment's last one end at once.  Eight adapters, one of seven row blocks: in chunks of two blocks (four columns
+    of the grid per adapter) ten columns of work share five dies, two of them four columns each; in chunks of three (three columns) no die has more than two."""
+    from lorafusion_amd import _lib
+
+    blocks, N, R = [7, 2, 2, 2, 2, 1, 1, 2], 10752, 64
+    busiest = lambda per: max(sum(1 for s, b in enumerate(blocks) for c in range(-(-b // per)) if (s * -(-max(blocks) // per) + c) % 8 == die) for die in range(8))
+    assert busiest(2) == 4 and busiest(3) == 2
+    n = sum(blocks)
+    keep = torch.zeros((n, 3), dtype=torch.int32), torch.ones(n), torch.zeros(n)
+    r = _lib.multi_routing([128 * b for b in blocks], [R] * 8, *keep, 128)
+    slices, chunks = 16, 3   # fp32 partials: dS [slices, rows, R], dB [adapters * chunks, N, R]
+    assert _lib.lib().lf_workspace_bytes(_lib.LF_OP_DYS_DYB, 128 * n, N, 128, R, r) == 4 * R * (slices * 128 * n + 8 * chunks * N)
+
+
 def test_launch_plan_takes_the_contraction_length():
     """Host logic of the tile choice: left-over rows get a launch of their own when the contraction is long enough to
     pay for it, and one launch covers everything when it is short."""
