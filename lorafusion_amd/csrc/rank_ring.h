@@ -170,9 +170,9 @@ __device__ __forceinline__ lf_u32x4 side_tr8(const char* blk, int row, int c, in
 // of nt tiles keeps at most min(NS, (NSB - 1) nt + 1) stages of the ring busy, so one block more is never on order).
 //   D_j[r][k] += sum_m dS[m][r] * keep*X[m][k]   per tile j of the slice, in registers over all blocks of the chunk.
 // With a keep-mask the tile is masked in place one iteration before it is consumed.
-// The direct form takes dB with dA: the workgroups of blockIdx.y = 1 walk dY beside S without a mask, the same sum with other operands.
+// The direct form takes dB with dA (WITH_B): the workgroups of blockIdx.y = 1 walk dY beside S without a mask, the same sum with other operands.
 struct DbOperands { const void* dY; const void* S; int N, n_slices; };   // (outputs: seg.ptr)
-template <typename T, int RT, int TPW, int NS, int MASK, int NSB, bool DIRECT>
+template <typename T, int RT, int TPW, int NS, int MASK, int NSB, bool DIRECT, bool WITH_B = false>
 __global__ void __launch_bounds__(256, RT >= 8 || DIRECT ? 1 : 2)
 lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, const T* __restrict__ dS, float* __restrict__ part,
                     int M, int K, int R, int n_slices, int group, int max_chunks, const LfSegTable seg, const DbOperands db) {
@@ -188,8 +188,8 @@ lora_da_ring_kernel(const T* __restrict__ X, const uint8_t* __restrict__ mask, c
   char* side = lds + NS * STAGE;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   const int ks = blockIdx.x, ch = DIRECT ? 0 : blockIdx.y, s = blockIdx.z;
-  const bool grad_b = DIRECT && blockIdx.y != 0;
-  if constexpr (DIRECT) {
+  const bool grad_b = WITH_B && blockIdx.y != 0;
+  if constexpr (WITH_B) {
     if (grad_b) X = (const T*)db.dY, dS = (const T*)db.S, K = db.N, n_slices = db.n_slices, mask = nullptr;
     if (ks >= n_slices) return;
   }
