@@ -829,9 +829,13 @@ static const TileCand& cand_of(int cfg) {
   return kCands[cfg == 2 ? 2 : 1];   // (the four-wave forms of these tiles, 0 and 2, are only run when pinned or for odd routing blocks)
 }
 // gemm_mid.hip takes whole tiles of columns, at least four K steps of 64 and routing blocks that a wave meets two of at most.
-// (160x128: level with 192x128 at K = 512.  128x64 and smaller below K = 1024: a
-// microsecond at most ahead of gemm_lora.hip's 64x64, which gives the same bits for every mask format.)
-static bool mid_shape(const TileCand& c, int N, int K) { return N % c.bn == 0 && K >= (c.cfg == 10 || c.bn == 64 ? 1024 : 256); }
+// (160x128: level with 192x128 at K = 512.  96x64 and 64x64 below K = 1024: a microsecond at most ahead of gemm_lora.hip's 64x64, which gives the same bits for every
+// mask format.  128x64 is ahead of gemm_lora.hip's tiles there but for a few tiles, by 5 - 8 % of a forward and 10 - 13 % of dX over 284 and 276 shapes: forwards of 768 x 1664 over 640 at rank 64
+// 20.3 -> 18.2 us, 368 x 5120 over 768 at rank 32 15.9 -> 14.6.)
+static bool mid_shape(const TileCand& c, int N, int K) { return N % c.bn == 0 && K >= (c.cfg == 10 || c.cfg == 14 || c.cfg == 15 ? 1024 : 256); }
+// ... and what 128x64 costs there beyond its figures, which are those of longer contractions, in microseconds.  (Of 1280 products over 256 - 896 13 % are
+// more than 3 % behind the best launch timed; 20 % without it, 53 % without the tile.)
+static double mid_short_k(const TileCand& c, int K) { return c.cfg == 12 && K < 1024 ? 1.8 : 0.0; }
 // What a tile of gemm_mid.hip has to be ahead by in the model to be taken: in one round, in several, sliced (fitted with the figures above; in several
 // rounds the model says too little for it).
 // (A 192x128 tile that only the margin keeps with gemm_lora.hip runs here all the same: one tile, one kernel, but for what this one does not take.)
@@ -856,7 +860,7 @@ static int choose_cfg(int M, int N, int K, bool big, bool wave96, bool mid, doub
     if (c.cfg == 3 && tail) continue;
     if (c.cfg == 9 && (!wave96 || tail)) continue;
     if (c.mid && (!mid || !mid_shape(c, N, K) || (tail && c.bm != 128))) continue;   // (left-over rows: 128x128 and 128x64; in slices any tile)
-    const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1, K) : 1.0);
+    const double cost = launch_cost(c, M, N, K) * (c.mid ? mid_margin(tiles_of(M, N, c), 1, K) : 1.0) + mid_short_k(c, K);
     if (cost < best_cost) { best_cost = cost; best = c.cfg; }
   }
   if (cost_out) *cost_out = best_cost;

@@ -141,6 +141,18 @@ def test_static_backward_takes_calls_whose_fastest_split_does_not_fit():
     assert call(128, 28672, 256, 64, _lib.single_routing(64, 1.0, 0.1)) != _lib.LF_OK
 
 
+def test_short_contractions_of_a_few_hundred_rows_run_on_128x64_tiles():
+    """K below 1024: a round of 128x64 tiles runs in the kernel for outputs of about one round (12), a few tiles in the general kernel's 64x64 (5)."""
+    import ctypes
+
+    from lorafusion_amd import _lib as L
+
+    v = (ctypes.c_int * 3)()
+    p = [ctypes.cast(ctypes.byref(v, 4 * i), ctypes.POINTER(ctypes.c_int)) for i in range(3)]
+    for M, N, K, cfg in ((768, 1664, 640, 12), (368, 5120, 768, 12), (512, 3584, 640, 12), (300, 384, 256, 5), (200, 640, 384, 5)):
+        assert L.lib().lf_gemm_plan(M, N, K, 0, *p) == 0 and list(v) == [M, cfg, -1], (M, N, K, list(v))
+
+
 def test_chunks_of_a_packed_batch_spread_over_the_dies():
     """Workgroups are dealt to the eight dies by their index, chunks beyond a segment's last one end at once.  Eight adapters, one of seven row blocks: in chunks of two blocks (four columns
     of the grid per adapter) ten columns of work share five dies, two of them four columns each; in chunks of three (three columns) no die has more than two."""
