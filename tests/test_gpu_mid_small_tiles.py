@@ -2,9 +2,12 @@
 load: K loops of exactly as many steps as there are stages and a few more, ragged rows, waves of 48 and 32 rows across two adapters, and every kind of rank
 chunk, against the CPU oracle.  Tolerances as in test_gpu_lora_single.py / test_gpu_lora_multi.py."""
 
+import re
+
 import pytest
 import torch
 
+from oracle import lora_ref
 from tests.test_gpu_lora_multi import _run as run_multi
 from tests.test_gpu_lora_single import _run_case as run_single
 from tests.util import kernels_of
@@ -40,7 +43,7 @@ def test_multi(tile):
 
 
 def test_short_batches_run_on_them():
-    """The plan takes the 96x64 tile for 300 rows over 4096 columns and K (four rows of tiles fill one round) and slices of it or of the 64x64 tile for fewer."""
+    """The plan takes the 96x64 tile for 300 rows over 4096 columns and K (four rows of tiles fill one round).  (Slices of both tiles: test_gpu_split_contraction.py.)"""
     import ctypes
 
     from lorafusion_amd import _lib
@@ -50,5 +53,7 @@ def test_short_batches_run_on_them():
     p = [ctypes.cast(ctypes.byref(v, 4 * i), ctypes.POINTER(ctypes.c_int)) for i in range(3)]
     assert _lib.lib().lf_gemm_plan(300, 4096, 4096, 0, *p) == 0 and list(v) == [300, 14, -1]
     x, w = torch.randn(300, 4096).bfloat16().cuda(), torch.randn(4096, 4096).bfloat16().cuda()
-    _, names = kernels_of(lambda: hip_ops.gemm(x, w, trans_b=True))
-    assert "gemm_mid_kernel" in names, names
+    y, names = kernels_of(lambda: hip_ops.gemm(x, w, trans_b=True))
+    assert re.findall(r"gemm_mid_kernelI\w+?Lb[01]ELi(\d+)ELi(\d+)E", names) == [("3", "2")] and "ksplit" not in names, names   # (rows and columns / 32)
+    ok, rel, excess = lora_ref.check_close(y.float().cpu(), (x.float() @ w.float().T).cpu(), rtol=1e-2)
+    assert ok, f"rel {rel:.3e} excess {excess:.3e}"

@@ -130,3 +130,18 @@ def test_either_side_of_the_line(M, masked, short):
     mask = torch.randint(0, 256, (M, 512), device="cuda", dtype=torch.uint8) if masked else None
     *_, names = _bwd(t(M, 4096), t(M, 4096), mask, True, t(M, 16), [t(4096, 16)], [t(16, 4096)], [(M + 127) // 128], [2.0], [0.1 if masked else 0.0], [M])
     assert ("dys_dyb" not in names) == short, names
+
+
+def test_segment_without_rows():
+    """The last adapter has no row blocks in this batch: its gradients are sums of nothing, in both halves of the launch, and the other's are not touched."""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    rn = lambda *sh: torch.randn(*sh, generator=g, device="cuda").bfloat16()
+    M, N, K = 256, 384, 640
+    dy, x, s, b, a = rn(M, N), rn(M, K), rn(M, 16), [rn(N, 16), rn(N, 8)], [rn(16, K), rn(8, K)]
+    s[200:] = 0
+    ds, da, db, names = _bwd(dy, x, None, True, s, b, a, [2, 0], [2.0, 1.0], [0.0, 0.0], [200, 0])
+    assert "dys_dyb" not in names, names
+    assert not da[1].any() and not db[1].any()
+    _check(ds[:200], 2 * (dy[:200].float() @ b[0].float()), "dS")
+    _check(da[0], ds[:200].float().T @ x[:200].float(), "dA")
+    _check(db[0], 2 * (dy[:200].float().T @ s[:200].float()), "dB")
