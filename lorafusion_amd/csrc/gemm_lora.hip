@@ -1027,9 +1027,9 @@ size_t lf_gemm_ksplit_bytes(int M, int N, int K, int routing_block, bool nn) {
 
 // Unsplit products planned on the persistent 256x256 tile that the eight-wave one is the faster kernel for: a left operand (and, NT, a weight) whose row
 // pitch is a multiple of 2 KB puts a K step's lines of all rows on few memory channels, and the persistent kernel, which has one step of 64 on order, waits for
-// them where the other's ring of five steps of 32 does not.  The powers of two and 3 and 7 times 2 KB are spread by the address hash.  Eight-wave over persistent in
+// them where the other's ring of five steps of 32 does not.  (4, 7 and 8 times 2 KB are exceptions, 3 times was not timed, 16 times is none.)  Eight-wave over persistent in
 // 4270 launches of 1500 - 12300 rows over 2048 - 14336 columns (cold weights, rank-16 term, geometric means): NT 0.935 at K = 5120 and 6144 (9 of 358 more than 2 % behind), 0.918 from 9216
-// (7 of 805), 1.02 / 0.99 / 1.01 at 4096 / 7168 / 8192, 1.00 at pitches that are no multiple of 2 KB; NN 1.00 at 5120 - 9216, 0.956 at 10240 - 15360 (but not over a
+// (7 of 805; 16384 0.94, 28672 0.83), 1.02 / 0.99 / 1.01 at 4096 / 7168 / 8192, 1.00 at pitches that are no multiple of 2 KB; NN 1.00 at 5120 - 9216, 0.956 at 10240 - 15360 (but not over a
 // weight that was just written: 4096 x 4096 over 14336, dequantised before, 809 -> 821 for the whole forward and backward), 0.93 from 16384.  3000 x 5120 over 5120 NT 138 -> 127 us, 8192 x 4096 over 10240 547 -> 492.  To two rounds of tiles: of longer launches, which run at the power limit, the
 // faster one slows its neighbours down (16384 x 4096 over 28672 NN 2751 -> 2620 us, the decoder layer around it 12 070 -> 12 057).
 static bool pitch_prefers_eight_waves(const LfGemmParams& q, bool nn) {

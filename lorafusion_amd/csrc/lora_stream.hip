@@ -11,7 +11,7 @@
 //             up to 16 rows and rank 32 a kernel of its own does all of it in one launch (short16_fwd_kernel)
 //   dS      : P = dY, Q = B_i transposed: dS = scale dY B_i, where dB comes with dA (lora_da_direct.hip)
 //
-// Both are bound by the stream of P (the forward of 8 rows moves 34 MB of weights for 0.3 GFLOP), so what counts is how
+// All are bound by the stream of P (the forward of 8 rows moves 34 MB of weights for 0.3 GFLOP), so what counts is how
 // many bytes the chip has on order.  A workgroup (4 waves) owns 64 rows of P and a slice of K: the slices are what
 // gives every compute unit two workgroups when P has few rows, or when Q is so tall that a workgroup which walks all of K
 // (lora_xa_kernel) would read it once per 16 rows of P.  P (64 rows x 64 columns, 8 KB), Q (up to 16 KB) and the keep
