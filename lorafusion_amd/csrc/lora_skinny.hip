@@ -923,7 +923,7 @@ int lf_launch_da(const void* X, const uint8_t* mask, int mask_bits, const void* 
 // (lora_da_direct.hip), where dys_dyb and da take three to five.  dY is read twice; what goes is the fp32 partials of dS and dB, their second stage and the walk of
 // da behind that of dys_dyb.  Behind where one workgroup walks many blocks (a tile costs it 0.4 us, with a mask 0.9).
 // Both sides in microseconds on one scale (ring_us); the short side fitted to the same batches, 7 % off on those that were not.  On these the choice takes 0.914 of the two passes' time (the
-// faster form of dA among them) and 0.8 % more than the best of every form; 3.4 % are more than 3 % slower than the two passes (worst 1.2 times).  With keep bits, replayed from a graph, two
+// faster form of dA among them) and 0.7 % more than the best of every form; 5.7 % are more than 3 % slower than the two passes (worst 1.3 times), most of them for a launch less.  With keep bits, replayed from a graph, two
 // passes -> short: 300 x 4096 x 4096 rank 16 16.3 -> 12.8, four segments of 1280 rows rank 64 26.7 -> 24.1; the line: 1000 x 4096 x 4096 rank 16 20.7 either way; the other side of it: 1500 rows
 // 23.8 against 25.7, 2048 28.0 against 31.0 (without a mask 22.0 against 22.5), 3000 x 5120 x 5120 rank 128 60 against 88.
 size_t lf_ds_workspace(int M, int N, int R, const LfSegTable& seg);   // (lora_stream.hip)
@@ -953,9 +953,13 @@ static ShortGrads short_grads(int M, int N, int K, int R, bool masked, const LfS
     const double share = (double)(((rows + 63) / 64 * sl + 255) / 256) / sl;
     us += 0.665 + n * share * 5.21 * rt + (sl > 1 ? 4e-6 * sl * (double)rows * R : 0.0);
   }
-  const double old = dysr_plan(M, N, R, seg, SIZE_MAX).us + da_form(M, K, R, masked, seg, SIZE_MAX).us;
+  // (one segment above rank 64: the two passes' models are 6 % high)
+  const double old = (dysr_plan(M, N, R, seg, SIZE_MAX).us + da_form(M, K, R, masked, seg, SIZE_MAX).us) * (seg.table == nullptr && rt == 8 ? 0.94 : 1.0);
+  // One to three launches less, whose host side is 3 us each: it counts where forward and backward take less time than the host to issue them, 130 us, and for packed batches, where the host does more.
+  // 1596 rows of five adapters x 6656 x 1408 at rank 16: 25.8 us either way, the whole call 132 - 144 and 149 - 153.  (Without these the choice is 0.7 % over the best of every form.)
+  const double launches = (double)M * N * K < 2.5e10 ? (seg.table != nullptr ? 3.5 : 1.5) : 0.5;
   // (longer segments gain 1 - 2 % and are as often behind; where the workgroups take almost all compute units the model is 11 % off and not 5)
-  return us * (big > 8 ? 1.03 : 1.0) * (full > 0.9 ? 1.05 : 1.0) < old ? g : ShortGrads{0, 0};
+  return us * (big > 8 ? 1.03 : 1.0) * (full > 0.9 ? 1.05 : 1.0) < old + launches ? g : ShortGrads{0, 0};
 }
 size_t lf_short_grads_workspace(int M, int N, int K, int R, const LfSegTable& seg) {
   for (const bool masked : {false, true})
